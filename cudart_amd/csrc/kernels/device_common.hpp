@@ -332,8 +332,14 @@ __device__ __forceinline__ float slab_inverse(float c) {
     return fabsf(c) < 0x1p-64f ? copysignf(0x1p64f, c) : 1.f / c;
 }
 
-// Returns false when the ray cannot hit anything: a zero direction (det == 0 for
-// every triangle) or a NaN component (every comparison of the triangle test fails).
+// False for a direction that cannot hit anything: zero (det == 0 for every triangle)
+// or with a NaN component (every comparison of the triangle test fails).
+__device__ __forceinline__ bool can_hit(V3 d) {
+    const bool nan = d.x != d.x || d.y != d.y || d.z != d.z;
+    return !nan && !(d.x == 0.f && d.y == 0.f && d.z == 0.f);
+}
+
+// Returns can_hit(d).
 __device__ __forceinline__ bool trav_begin(TravRay& r, V3 o, V3 d) {
     r.o = o;
     r.d = d;
@@ -342,8 +348,7 @@ __device__ __forceinline__ bool trav_begin(TravRay& r, V3 o, V3 d) {
     r.iz = slab_inverse(d.z);
     r.node = 0;
     r.leaf = kNoChild;
-    const bool nan = d.x != d.x || d.y != d.y || d.z != d.z;
-    return !nan && !(d.x == 0.f && d.y == 0.f && d.z == 0.f);
+    return can_hit(d);
 }
 
 // True for a lane that a node phase can advance without a leaf set aside.

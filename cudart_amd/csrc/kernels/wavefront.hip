@@ -4,7 +4,7 @@
 // list of tiles (job, pixel range, sample range); slots are numbered tile by tile.
 // One chunk runs as a captured HIP graph:
 //
-//   setup -> generate -> [extend -> shade -> shadow] x max_depth -> resolve -> advance
+//   setup -> generate -> [extend -> shade -> shadow] x max_depth -> resolve
 //
 //   generate camera rays (origin, direction) of the chunk's pixel-samples, queued
 //            in groups of 64 that share a pixel (or a small pixel block)
@@ -13,9 +13,8 @@
 //            first iteration's camera rays are traced 64 at a time as packets)
 //   shade    shade_vertex() of every hit; survivors are compacted into the next
 //            queue and shadow rays into the shadow queue (wave ballots + one atomic
-//            per workgroup and queue), finished paths write their colour to their
-//            result slot (row-major per sample within the tile)
-//   shadow   occlusion test of every shadow ray; adds mask * direct
+//            per workgroup and queue); what a vertex adds goes to the path's result slot
+//   shadow   occlusion test of every shadow ray; adds mask * direct to the result
 //   resolve  adds the result slots of each pixel to its running sum in sample order
 //
 // All paths of a chunk are at bounce `it` during iteration `it`, and the vertex
@@ -39,23 +38,21 @@
 namespace prt {
 
 constexpr int kMaxIter = 64;
-// Same-address atomics serialise (about 11 ns each on MI355X), so work is handed
-// out by kSpread counters, one kBatch-item batch per atomic, and appends to a queue
-// are aggregated per workgroup.
+// Same-address atomics serialise (about 11 ns each on MI355X), so work beyond each
+// wave's first batch is handed out by kSpread counters, one kBatch-item batch per
+// atomic, and appends to a queue are aggregated per workgroup.
 // Fetch counters per (kernel, iteration), items per fetch atomic, and shade
 // workgroup size. With every counter on its own line, 1080p x 128 spp measured
-// within noise of 64 / 64 / 512 for spread 128, batch 128 and 1024-thread shade
-// workgroups; spread 32 and 256-thread shade workgroups were 2-4 % slower.
-#ifndef PRT_FETCH_SPREAD
-#define PRT_FETCH_SPREAD 64
-#endif
+// within noise of 64 / 512 for batch 128 and 1024-thread shade workgroups;
+// 256-thread shade workgroups were 2-4 % slower.
 #ifndef PRT_FETCH_BATCH
 #define PRT_FETCH_BATCH 64
 #endif
 #ifndef PRT_SHADE_BLOCK
 #define PRT_SHADE_BLOCK 512
 #endif
-constexpr uint32_t kSpread = PRT_FETCH_SPREAD;
+constexpr uint32_t kSpread = 64;
+constexpr uint32_t kSteal = 2;  // other counters a wave tries when its own is exhausted
 constexpr uint32_t kBatch = PRT_FETCH_BATCH;  // items per fetch atomic
 constexpr int kShadeBlock = PRT_SHADE_BLOCK;
 // Waves of wf_shade per compute unit in its grid (its occupancy limit, 4 waves per SIMD).
@@ -63,8 +60,8 @@ constexpr int kShadeBlock = PRT_SHADE_BLOCK;
 #define PRT_SHADE_GRID_WAVES 16
 #endif
 constexpr int kShadeGridWaves = PRT_SHADE_GRID_WAVES;
-// Bytes of queues and path state per slot: 2 queues x 64, hit 16 + 4, shadow 64, result 16.
-constexpr size_t kSlotBytes = 2 * 64 + 16 + 4 + 64 + 16;
+// Bytes of queues and path state per slot: 2 queues x 48, hit 16 + 4, shadow 48 + 4, result 16.
+constexpr size_t kSlotBytes = 2 * 48 + 16 + 4 + 48 + 4 + 16;
 // Counter words per 128-byte cache line. Each queue counter and each fetch counter
 // has a line of its own: atomics on one line serialize in its L2 channel, and the
 // appends of wf_shade and the batch fetches of the traversal kernels would otherwise
@@ -77,12 +74,13 @@ enum WfCounter : uint32_t {
     kExt0 = 0,                 // ray count of queue 0
     kExt1 = kCtrLine,          // ray count of queue 1
     kShadow = 2 * kCtrLine,    // shadow ray count
-    kChunk = 3 * kCtrLine,     // index of the chunk being rendered
+    kChunk = 3 * kCtrLine,     // number of the chunk being rendered, from 1
+    kStats = 4 * kCtrLine,     // kCntNum 64-bit counters (two words each)
     kFetch = 8 * kCtrLine,     // per (kernel, iteration) fetch counters: 3 * kMaxIter groups of kSpread,
                                // counter c of group g at kFetch + (g * kSpread + c) * kCtrLine
-    kStats = kFetch + 3 * kMaxIter * kSpread * kCtrLine,  // kCntNum 64-bit counters (two words each)
-    kNumCounters = kStats + 2 * kCntNum,
+    kNumCounters = kFetch + 3 * kMaxIter * kSpread * kCtrLine,
 };
+static_assert(kStats + 2 * kCntNum <= kFetch, "the statistics lie below the fetch counters");
 // First fetch counter of group g (3 * iteration + kernel: 0 extend, 2 shadow).
 constexpr uint32_t fetch_group(uint32_t g) { return kFetch + g * kSpread * kCtrLine; }
 
@@ -110,11 +108,15 @@ struct WfChunk {
 // Queue entry (structure of arrays, one float4 each, coalesced by queue index):
 //   A  origin.xyz, pixel | job << 24
 //   B  direction.xyz, sample index
-//   C  throughput.xyz, previous bsdf
-//   D  colour.xyz, slot (result index)
-// Shadow entry: E position.xyz, target | F normal.xyz, lu | G mask.xyz, light record |
-//   H lv, final flag. `target` is the path's entry in the next queue, or its result
-//   slot when the path ended at this vertex.
+//   C  throughput.xyz, slot | (previous bsdf specular or refractive) << 31
+// Shadow entry: E origin.xyz, distance to the light sample | F direction.xyz, light id |
+//   non-finite throughput channels << 28 | G contribution.xyz, slot; and the job.
+// A path's slot is its position in the chunk's first queue; result[slot] is its colour so
+// far, touched only by the vertices that change it (first vertex, emission, sky, a visible
+// light sample). Queue order and slots keep neighbouring paths together, so those accesses
+// coalesce. (Carrying the colour in the queue entries, and the light sample's position,
+// normal, coordinates and throughput in the shadow entries, took 64 bytes each, and
+// wf_shade, whose first launch runs at the memory's rate, wrote them.)
 struct WfArgs {
     const WfJob* jobs;
     const WfTile* tiles;
@@ -123,18 +125,18 @@ struct WfArgs {
     float4* qa[2];
     float4* qb[2];
     float4* qc[2];
-    float4* qd[2];
     float4* hits;    // t, u, v, record (0xFFFFFFFF = miss)
     uint32_t* hmat;  // material of the hit record
     float4* se;
     float4* sf;
     float4* sg;
-    float4* sh;
-    float4* result;  // per slot final colour
+    uint32_t* sj;    // job of the shadow entry
+    float4* result;  // per slot colour
     int* spill;
     uint32_t spill_stride;
     uint32_t max_depth;
-    uint32_t group_lg;  // log2 of the forced camera-path block side, or kNone: choose per tile
+    uint32_t one_scene;  // every job traverses the same scene
+    uint32_t group_lg;  // log2 of the forced camera-path block side, or kNone: choose per section
 };
 
 struct WavefrontState {
@@ -155,58 +157,69 @@ struct WavefrontState {
 
 namespace dev {
 
-// Hands out 64-item batches of [0, n). Batch b belongs to counter b % kSpread. A
-// wave draws from counter (wave % kSpread); issue() sends the atomic for its next
-// batch before the current batch is processed, so the round trip overlaps the
-// traversal. When its counter is exhausted the wave probes the others, with a
-// coherent load first so exhausted counters cost no atomic. resolve() returns the
-// batch's first item or 0xFFFFFFFF when every batch has been handed out.
-struct SpreadFetch {
+constexpr uint32_t kNone = 0xFFFFFFFFu;
+
+// Hands out 64-item batches of [0, n) to the waves of a launch. Wave w's first batch
+// is batch w, with no atomic; the batches from `waves` on belong to kSpread counters
+// in turn, and a wave draws from counter (wave % kSpread): issue() sends the atomic
+// for its next batch before the current batch is processed, so the round trip
+// overlaps the traversal. When its counter is exhausted the wave tries kSteal others:
+// neighbouring batches belong to different counters, so these run out at about the same
+// time and there is little to take over. A queue of at most `waves` batches costs no
+// atomic. resolve() returns the batch's first item or kNone. All of it but the atomic in
+// flight is wave-uniform and stays in scalar registers.
+// What bounds small queues is this ending: with every wave asking all other counters one
+// after the other, each launch ended in 63 dependent loads, about 45 us (256 x 256 x 16 samples
+// of a 36-triangle box, depth 5: wf_extend and wf_shadow 632 -> 400 us per frame);
+// one vector load of all 64 counters per wave still read each of their lines once
+// per wave, and cost a 0.9 ms packet launch 70 us.
+struct WaveFetch {
     uint32_t* ctr;
-    uint32_t k, nb;
-    __device__ __forceinline__ uint32_t limit(uint32_t c) const { return (nb + kSpread - 1 - c) / kSpread; }
+    uint32_t k, nb, waves;
+    __device__ __forceinline__ uint32_t limit(uint32_t c) const {
+        return nb > waves + c ? (nb - waves - c + kSpread - 1) / kSpread : 0u;
+    }
+    __device__ __forceinline__ uint32_t item(uint32_t c, uint32_t idx) const {
+        return (waves + idx * kSpread + c) * kBatch;
+    }
     __device__ __forceinline__ uint32_t issue() const {
-        uint32_t idx = 0xFFFFFFFFu;
-        if ((threadIdx.x & 63) == 0) idx = atomicAdd(ctr + k * kCtrLine, 1u);
+        uint32_t idx = kNone;
+        if (nb > waves && (threadIdx.x & 63) == 0) idx = atomicAdd(ctr + k * kCtrLine, 1u);
         return idx;
     }
     __device__ __forceinline__ uint32_t resolve(uint32_t raw) {
-        uint32_t idx = __shfl(raw, 0, 64);
-        if (idx < limit(k)) return (idx * kSpread + k) * kBatch;
-        for (uint32_t probe = 1; probe < kSpread; ++probe) {
-            k = (k + 1) % kSpread;
-            idx = 0xFFFFFFFFu;
-            if ((threadIdx.x & 63) == 0) {
-                const uint32_t lim = limit(k);
-                const uint32_t seen = __hip_atomic_load(ctr + k * kCtrLine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (seen < lim) idx = atomicAdd(ctr + k * kCtrLine, 1u);
-                if (idx >= lim) idx = 0xFFFFFFFFu;
-            }
-            idx = __shfl(idx, 0, 64);
-            if (idx != 0xFFFFFFFFu) return (idx * kSpread + k) * kBatch;
+        if (nb <= waves) return kNone;
+        uint32_t idx = uniform_u32(raw);
+        for (uint32_t tries = 0; idx >= limit(k); ++tries) {
+            if (tries == kSteal) return kNone;
+            k = (k + 21u) % kSpread;
+            idx = kNone;
+            if ((threadIdx.x & 63) == 0) idx = atomicAdd(ctr + k * kCtrLine, 1u);
+            idx = uniform_u32(idx);
         }
-        return 0xFFFFFFFFu;
+        return item(k, idx);
+    }
+    // The wave's first batch; sets up the fetch of the others.
+    __device__ __forceinline__ uint32_t start(uint32_t* counters, uint32_t n) {
+        const uint32_t wave = uniform_u32(blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64);
+        ctr = counters;
+        k = wave % kSpread;
+        nb = (n + kBatch - 1) / kBatch;
+        waves = gridDim.x * (blockDim.x / 64);
+        return wave < nb ? wave * kBatch : kNone;
     }
 };
-__device__ __forceinline__ SpreadFetch make_fetch(uint32_t* ctr, uint32_t n) {
-    const uint32_t wave = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-    return SpreadFetch{ctr, wave % kSpread, (n + kBatch - 1) / kBatch};
-}
-
-constexpr uint32_t kNone = 0xFFFFFFFFu;
-
 // Hands single items of [0, n) to individual lanes: the wave holds one 64-item
-// batch of a SpreadFetch at a time (one atomic per 64 items, the next one already
+// batch of a WaveFetch at a time (one atomic per 64 items, the next one already
 // in flight) and gives its items to whichever lanes ask, so a lane whose ray has
 // finished takes a new one while the others keep traversing. Every issued atomic
 // is resolved before more() turns false. Calls must be wave-uniform.
 struct LaneFeeder {
-    SpreadFetch fetch;
+    WaveFetch fetch;
     uint32_t n, base, used, pending;
     __device__ __forceinline__ void start(uint32_t* ctr, uint32_t count) {
-        fetch = make_fetch(ctr, count);
         n = count;
-        base = n ? fetch.resolve(fetch.issue()) : kNone;
+        base = fetch.start(ctr, count);
         used = 0;
         pending = base != kNone ? fetch.issue() : kNone;
     }
@@ -271,13 +284,12 @@ __device__ __forceinline__ const T* wave_uniform(const T* p) {
 static_assert(PRT_EXTEND_PHASE_MIN >= 0 && PRT_EXTEND_PHASE_MIN <= 64, "phase threshold out of range");
 static_assert(PRT_SHADOW_PHASE_MIN >= 0 && PRT_SHADOW_PHASE_MIN <= 64, "phase threshold out of range");
 
-// Waves per SIMD of the traversal kernels. With the scene bases in SGPRs,
-// wf_extend fits 8 (63 VGPRs; the one spill is a constant reloaded only for
-// zero-direction rays) and wf_shadow 7 (72 VGPRs; its spill is reloaded only on the
-// stack's overflow path). 1080p x 128 spp over 1M triangles: 153.7 -> 151.6 ms per
-// frame against 7 and 6; before the SGPR bases, forced occupancy spilled in the loop.
+// Waves per SIMD of the traversal kernels: with the scene bases and the feeder in SGPRs,
+// wf_extend fits 8 (64 VGPRs, 2 spilled on rarely taken paths) and wf_shadow too (54, with
+// its rays set up by wf_shade: 35.6 -> 31.6 ms per frame of 1080p x 128 spp over 1M
+// triangles, against 72 VGPRs, 7 waves and the set-up in its refill).
 #ifndef PRT_SHADOW_WAVES
-#define PRT_SHADOW_WAVES __attribute__((amdgpu_waves_per_eu(7)))
+#define PRT_SHADOW_WAVES __attribute__((amdgpu_waves_per_eu(8)))
 #endif
 #ifndef PRT_EXTEND_WAVES
 #define PRT_EXTEND_WAVES __attribute__((amdgpu_waves_per_eu(8)))
@@ -320,88 +332,96 @@ __device__ __forceinline__ uint32_t find_tile(const WfTile* t, uint32_t first, u
     return lo;
 }
 
-__global__ void wf_setup(WfArgs a) {
-    for (uint32_t k = threadIdx.x; k < 3 * kMaxIter * kSpread; k += blockDim.x) a.ctr[kFetch + k * kCtrLine] = 0;
-    if (threadIdx.x != 0) return;
+// Goes on to the next chunk: its path count, empty queues, and the fetch counters of
+// the iterations it will run (one workgroup clearing all of them took 9 us).
+__global__ __launch_bounds__(256) void wf_setup(WfArgs a) {
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < 3 * a.max_depth * kSpread; k += gridDim.x * blockDim.x)
+        a.ctr[kFetch + k * kCtrLine] = 0;
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
     const uint32_t c = a.ctr[kChunk];
+    a.ctr[kChunk] = c + 1;
     a.ctr[kExt0] = a.chunks[c].paths;
     a.ctr[kExt1] = 0;
     a.ctr[kShadow] = 0;
 }
-
-__global__ void wf_advance(WfArgs a) {
-    if (threadIdx.x == 0) a.ctr[kChunk] = a.ctr[kChunk] + 1;
+// The chunk that wf_setup has gone on to.
+__device__ __forceinline__ WfChunk current_chunk(const WfArgs& a) {
+    return a.chunks[__builtin_amdgcn_readfirstlane(a.ctr[kChunk]) - 1];
 }
 
-// Path order within a tile. Where a tile covers whole rows of its image, each run
-// of 64 paths (one wave's batch) is a g x g pixel block times 64 / g^2 consecutive
-// samples of those pixels: blocks band by band and left to right, sample groups
-// outermost. g is the smallest of 1, 2, 4, 8 that divides the tile (its sample count
-// by 64 / g^2, its width and rows by g), so at 128 spp a wave traces 64 samples of
-// one pixel: nearly the same primary ray in every lane, then shadow and extension
-// rays from nearly the same point. Other tiles keep the row-major order per sample.
-// On 1080p x 128 spp over 1M triangles, one pixel x 64 samples took 147.3 ms per
-// frame, 4 x 4 x 4 148.1, 8 x 8 x 1 148.6 and row order 151.7. Only the queue is
-// reordered: a path's result slot (carried in its queue entry) stays row-major per
-// sample, so wf_resolve's loads stay coalesced across adjacent pixels, and every
-// pixel still adds its samples in sample order.
-struct PathGroup {
-    uint32_t lg;  // log2 of the block side g; kNone: row order
+// Path order within a tile. The tile's samples are cut into sections of m consecutive
+// samples: as many full ones as there are (m = 64, or all of fewer), then the rest. Within a
+// section the pixels come in order of position q, each with its m samples one after
+// another, so 64 consecutive paths (one wave's batch) are the m samples of about 64 / m
+// pixels. q runs through bands of g rows, column by column, with g near sqrt(64 / m):
+// those pixels are a block, whatever the image's size and sample count. At 128 spp a wave
+// traces 64 samples of one pixel: nearly the same primary ray in every lane, then shadow
+// and extension rays from nearly the same point. On 1080p x 128 spp over 1M triangles,
+// one pixel x 64 samples took 147.3 ms per frame, 4 x 4 x 4 148.1, 8 x 8 x 1 148.6 and row
+// order 151.7. (Blocks only where they divided the image and the sample count left every
+// other size in row order: packets of 64 pixels of a row; 12 views of odd
+// sizes, 8 to 64 spp: 2.43 -> 1.31 ms in the packet launch; 3840 x 2160 x 6 spp, which took
+// 8 x 8 x 1: 4.0 -> 2.55.)
+// A tile that does not cover whole rows is taken as one row. A path's result slot is its
+// position in this order; wf_resolve adds every pixel's samples in sample order.
+struct PathOrder {
+    uint32_t width, rows;  // of the tile (a tile of part of a row: its pixels, 1)
+    uint32_t pixels;
+    uint32_t m, full, rest;  // samples of a full section, full sections, samples of the last one (or 0)
+    uint32_t g;              // band height of the full sections
 };
-// force_lg (not kNone) asks for g = 2^force_lg; a tile it does not divide takes the
-// smallest g that does.
-__device__ __forceinline__ PathGroup tile_group(const WfTile& t, uint32_t width, uint32_t force_lg) {
-    const uint32_t w = t.p1 - t.p0, ns = t.s1 - t.s0;
-    if (t.p0 % width != 0u || w % width != 0u) return PathGroup{kNone};
-    const uint32_t rows = w / width;
-    auto fits = [&](uint32_t lg) {
-        const uint32_t g = 1u << lg, gs = 64u >> (2u * lg);
-        return ns % gs == 0u && width % g == 0u && rows % g == 0u;
-    };
-    if (force_lg <= 3u && fits(force_lg)) return PathGroup{force_lg};
-    for (uint32_t lg = 0; lg <= 3; ++lg)
-        if (fits(lg)) return PathGroup{lg};
-    return PathGroup{kNone};
+__device__ __forceinline__ uint32_t band_rows(uint32_t m) { return m >= 32u ? 1u : m >= 7u ? 2u : m >= 2u ? 4u : 8u; }
+// force_lg (not kNone) asks for bands of g = 2^force_lg rows and sections of 64 / g^2 samples.
+__device__ __forceinline__ PathOrder path_order(const WfTile& t, uint32_t width, uint32_t force_lg) {
+    PathOrder o;
+    o.pixels = t.p1 - t.p0;
+    const bool whole = t.p0 % width == 0u && o.pixels % width == 0u;
+    o.width = whole ? width : o.pixels;
+    o.rows = whole ? o.pixels / width : 1u;
+    const uint32_t ns = t.s1 - t.s0;
+    const bool force = force_lg <= 3u;
+    o.m = min(force ? 64u >> (2u * force_lg) : 64u, ns);
+    o.g = force ? 1u << force_lg : band_rows(o.m);
+    o.full = ns / o.m;
+    o.rest = ns - o.full * o.m;
+    return o;
 }
-// Position r of a grouped tile of w pixels -> (pixel offset from p0, sample offset from s0).
-__device__ __forceinline__ uint2 group_to_linear(uint32_t r, uint32_t w, uint32_t width, PathGroup pg) {
-    const uint32_t g = 1u << pg.lg, gs = 64u >> (2u * pg.lg);
-    const uint32_t per_sg = w * gs, sg = r / per_sg, rem = r % per_sg;
-    const uint32_t blk = rem >> 6, lane = rem & 63u, per_band = width >> pg.lg;
-    const uint32_t x = ((blk % per_band) << pg.lg) + (lane & (g - 1u));
-    const uint32_t y = ((blk / per_band) << pg.lg) + ((lane >> pg.lg) & (g - 1u));
-    return make_uint2(y * width + x, sg * gs + (lane >> (2u * pg.lg)));
+// Pixel offset from the tile's first pixel of position q in bands of g rows, and back.
+__device__ __forceinline__ uint32_t position_to_pixel(const PathOrder& o, uint32_t g, uint32_t q) {
+    if (g == 1u) return q;
+    const uint32_t per = o.width * g, band = q / per, in = q - band * per;
+    const uint32_t h = min(g, o.rows - band * g), x = in / h;
+    return (band * g + (in - x * h)) * o.width + x;
+}
+__device__ __forceinline__ uint32_t pixel_to_position(const PathOrder& o, uint32_t g, uint32_t pixel) {
+    if (g == 1u) return pixel;
+    const uint32_t y = pixel / o.width, x = pixel - y * o.width;
+    const uint32_t band = y / g, h = min(g, o.rows - band * g);
+    return band * g * o.width + x * h + (y - band * g);
 }
 
 __global__ __launch_bounds__(256) void wf_generate(WfArgs a) {
-    const WfChunk ch = a.chunks[a.ctr[kChunk]];
+    const WfChunk ch = current_chunk(a);
     for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < ch.paths; slot += gridDim.x * blockDim.x) {
         const WfTile t = a.tiles[find_tile(a.tiles, ch.tile0, ch.ntiles, slot, false)];
         const WfJob& j = a.jobs[t.job];
-        const uint32_t w = t.p1 - t.p0;
-        const uint32_t r = slot - t.slot0;
-        const PathGroup pg = tile_group(t, j.width, a.group_lg);
-        const uint2 ps = pg.lg != kNone ? group_to_linear(r, w, j.width, pg) : make_uint2(r % w, r / w);
-        const uint32_t pixel = t.p0 + ps.x, sample = t.s0 + ps.y;
+        const PathOrder o = path_order(t, j.width, a.group_lg);
+        const uint32_t r = slot - t.slot0, per = o.pixels * o.m;
+        const uint32_t sec = r / per, in = r - sec * per;
+        const bool last = sec == o.full;
+        const uint32_t m = last ? o.rest : o.m;
+        const uint32_t q = in / m;
+        const uint32_t pixel = t.p0 + position_to_pixel(o, last ? band_rows(m) : o.g, q);
+        const uint32_t sample = t.s0 + sec * o.m + (in - q * m);
         const int x = int(pixel % j.width), y = int(pixel / j.width);
         Rng rng{j.path.seed, j.path.view, pixel, sample};
         V3 ro, rd;
         camera_ray(j.cam, x, y, rng.block(0), ro, rd);
-        // C (throughput 1, previous bsdf 0) and D (colour 0, result slot) of a new path
-        // are not written: wf_shade(0) makes them from the tile (first_bounce_cd).
+        // C of a new path (throughput 1, no previous vertex, its slot) and its colour are
+        // made by wf_shade(0): the slot is the queue position.
         a.qa[0][slot] = make_float4(ro.x, ro.y, ro.z, __uint_as_float(pixel | (t.job << 24)));
         a.qb[0][slot] = make_float4(rd.x, rd.y, rd.z, __uint_as_float(sample));
     }
-}
-
-// The C and D entries of a new path (queue position i in the first extend queue of
-// chunk ch): throughput 1, previous bsdf 0, colour 0, and the path's result slot,
-// row-major per sample within its tile.
-__device__ __forceinline__ void first_bounce_cd(const WfArgs& a, const WfChunk& ch, uint32_t i, uint32_t pixel,
-                                                uint32_t sample, float4& C, float4& D) {
-    const WfTile t = a.tiles[find_tile(a.tiles, ch.tile0, ch.ntiles, i, false)];
-    C = make_float4(1.f, 1.f, 1.f, __int_as_float(0));
-    D = make_float4(0.f, 0.f, 0.f, __uint_as_float(t.slot0 + (sample - t.s0) * (t.p1 - t.p0) + (pixel - t.p0)));
 }
 
 // Runs f(job) with the job index made wave-uniform (scalar loads of the job
@@ -422,7 +442,7 @@ template <bool COUNT, bool ONE_SCENE>
 __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, uint32_t it) {
     __shared__ int s_stack[kStackLdsQueue * kBlock];
     const uint32_t q = it & 1u;
-    const uint32_t n = a.ctr[kExt0 + q];
+    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.ctr[kExt0 + (q ^ 1u)] = 0;  // the queue shade(it) fills
         a.ctr[kShadow] = 0;
@@ -523,15 +543,15 @@ template <bool COUNT, bool ONE_SCENE>
 __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend_packet(WfArgs a, uint32_t it) {
     __shared__ int s_pk[kPacketStack];
     const uint32_t q = it & 1u;
-    const uint32_t n = a.ctr[kExt0 + q];
+    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.ctr[kExt0 + (q ^ 1u)] = 0;  // the queue shade(it) fills
         a.ctr[kShadow] = 0;
     }
     Counts cnt = {0, 0, 0, 0, 0, 0};
     const uint32_t lane = threadIdx.x & 63u;
-    SpreadFetch fetch = make_fetch(&a.ctr[fetch_group(3 * it)], n);
-    uint32_t base = n ? fetch.resolve(fetch.issue()) : kNone;
+    WaveFetch fetch;
+    uint32_t base = fetch.start(&a.ctr[fetch_group(3 * it)], n);
     uint32_t pending = base != kNone ? fetch.issue() : kNone;
     while (base != kNone) {
         const uint32_t i = base + lane;
@@ -606,13 +626,20 @@ __device__ __forceinline__ uint2 block_append(bool more, bool nee, uint32_t* ctr
     return r;
 }
 
+// Channels of a throughput that are not finite, as bits: mask * 0 is then NaN, not 0.
+__device__ __forceinline__ uint32_t nonfinite(V3 m) {
+    return (fabsf(m.x) <= kFltMax ? 0u : 1u) | (fabsf(m.y) <= kFltMax ? 0u : 2u) | (fabsf(m.z) <= kFltMax ? 0u : 4u);
+}
+constexpr uint32_t kSlotMask = 0x7FFFFFFFu;   // a queue of 2^31 slots would not fit the memory
+constexpr uint32_t kLightIdMask = 0x0FFFFFFFu;  // triangle ids are below 2^28
+
+// Shades every hit of the queue, sets up the shadow rays of the light samples and
+// compacts the survivors. The colour the vertex adds starts at 0 (0 + x = x exactly) and
+// is added to the path's result; a visible light sample's part is added by wf_shadow.
 template <bool COUNT>
 __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a, uint32_t it) {
     const uint32_t q = it & 1u;
-    const uint32_t n = a.ctr[kExt0 + q];
-    // Read once, before this kernel's queue atomics start on the counters' cache line.
-    const uint32_t chunk = __builtin_amdgcn_readfirstlane(a.ctr[kChunk]);
-    const WfChunk ch = a.chunks[chunk];
+    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
     // Static, workgroup-uniform partition of the queue (shading cost varies little).
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
@@ -621,27 +648,24 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         bool more = false, want_nee = false;
         PathState ps;
         NeeSample ns;
-        float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A, Cc = A, D = A, hh = A;
+        ShadowReq sr;
+        float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A, hh = A;
+        float4 Cc = make_float4(1.f, 1.f, 1.f, __uint_as_float(i));  // a new path's
         uint32_t hm = 0;
         if (valid) {
             A = a.qa[q][i];
             B = a.qb[q][i];
-            if (it == 0) {
-                first_bounce_cd(a, ch, i, __float_as_uint(A.w) & 0xFFFFFFu, __float_as_uint(B.w), Cc, D);
-            } else {
-                Cc = a.qc[q][i];
-                D = a.qd[q][i];
-            }
+            if (it != 0) Cc = a.qc[q][i];
             hh = a.hits[i];
             hm = a.hmat[i];
         }
         const uint32_t pj = __float_as_uint(A.w);
-        const uint32_t slot = __float_as_uint(D.w);
+        const uint32_t slot = __float_as_uint(Cc.w) & kSlotMask;
         ps.ro = v3(A);
         ps.rd = v3(B);
         ps.mask = v3(Cc);
-        ps.color = v3(D);
-        ps.prev = __float_as_int(Cc.w);
+        ps.color = v3(0.f, 0.f, 0.f);
+        ps.prev = __float_as_uint(Cc.w) >> 31 ? 1 /*SPECULAR*/ : 0;
         ps.b = it;
         ps.input = it == 0 ? v3(0.f, 0.f, 0.f) : ps.rd;  // at b >= 1 the stale input is the ray direction
         with_job(valid, pj >> 24, [&](uint32_t jb) {
@@ -659,34 +683,56 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
                 h.mat = hm;
                 Rng rng{j.path.seed, j.path.view, pj & 0xFFFFFFu, __float_as_uint(B.w)};
                 more = shade_vertex<COUNT, true>(j.sc, j.path, rng, ps, h, &want_nee, ns, cnt);
+                if (want_nee && !(nee_prepare<COUNT>(j.sc, ns, sr, cnt) && can_hit(sr.sd))) {
+                    want_nee = false;  // the light sample cannot be seen: add mask * 0
+                    ps.color = add_direct(ps.color, ns.mask, sr.direct, false);
+                }
             }
         });
-        if (valid && !more) a.result[slot] = make_float4(ps.color.x, ps.color.y, ps.color.z, 0.f);
-        const uint2 pos = block_append(more, want_nee, &a.ctr[kExt0 + (q ^ 1u)], &a.ctr[kShadow]);
-        const uint32_t qi = pos.x;
-        if (more) {
-            a.qa[q ^ 1u][qi] = make_float4(ps.ro.x, ps.ro.y, ps.ro.z, A.w);
-            a.qb[q ^ 1u][qi] = make_float4(ps.rd.x, ps.rd.y, ps.rd.z, B.w);
-            a.qc[q ^ 1u][qi] = make_float4(ps.mask.x, ps.mask.y, ps.mask.z, __int_as_float(ps.prev));
-            a.qd[q ^ 1u][qi] = make_float4(ps.color.x, ps.color.y, ps.color.z, D.w);
+        if (valid) {
+            if (it == 0) {
+                a.result[slot] = make_float4(ps.color.x, ps.color.y, ps.color.z, 0.f);
+            } else if (ps.color.x != 0.f || ps.color.y != 0.f || ps.color.z != 0.f) {  // (NaN too)
+                const V3 c = v3(a.result[slot]) + ps.color;
+                a.result[slot] = make_float4(c.x, c.y, c.z, 0.f);
+            }
         }
-        const uint32_t si = pos.y;
+        const uint2 pos = block_append(more, want_nee, &a.ctr[kExt0 + (q ^ 1u)], &a.ctr[kShadow]);
+        if (more) {
+            const uint32_t special = ps.prev == 1 /*SPECULAR*/ || ps.prev == 4 /*REFRACTIVE*/ ? ~kSlotMask : 0u;
+            a.qa[q ^ 1u][pos.x] = make_float4(ps.ro.x, ps.ro.y, ps.ro.z, A.w);
+            a.qb[q ^ 1u][pos.x] = make_float4(ps.rd.x, ps.rd.y, ps.rd.z, B.w);
+            a.qc[q ^ 1u][pos.x] = make_float4(ps.mask.x, ps.mask.y, ps.mask.z, __uint_as_float(slot | special));
+        }
         if (want_nee) {
-            const uint32_t target = more ? qi : slot;
-            a.se[si] = make_float4(ns.position.x, ns.position.y, ns.position.z, __uint_as_float(target));
-            a.sf[si] = make_float4(ns.normal.x, ns.normal.y, ns.normal.z, ns.lu);
-            a.sg[si] = make_float4(ns.mask.x, ns.mask.y, ns.mask.z, __uint_as_float(ns.li));
-            a.sh[si] = make_float4(ns.lv, __uint_as_float(more ? 0u : 1u), __uint_as_float(pj >> 24), 0.f);
+            const V3 c = ns.mask * sr.direct;
+            const uint32_t id = sr.lid | nonfinite(ns.mask) << 28;
+            a.se[pos.y] = make_float4(sr.so.x, sr.so.y, sr.so.z, sr.tL);
+            a.sf[pos.y] = make_float4(sr.sd.x, sr.sd.y, sr.sd.z, __uint_as_float(id));
+            a.sg[pos.y] = make_float4(c.x, c.y, c.z, __uint_as_float(slot));
+            if (!a.one_scene) a.sj[pos.y] = pj >> 24;
         }
     }
-    if (COUNT) flush_stats<false>(a.ctr, cnt);
+    if (COUNT) {
+        flush_stats<false>(a.ctr, cnt);
+        // Each shadow ray's own light triangle counts among the any-hit triangles.
+        unsigned long long x = cnt.shadow;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        if ((threadIdx.x & 63) == 0 && x)
+            atomicAdd(reinterpret_cast<unsigned long long*>(a.ctr + kStats) + kCntAnyTris, x);
+    }
 }
 
+// Occlusion test of every shadow ray; a visible light sample's contribution is added to
+// the path's colour. As in wf_extend a finished ray's update waits for the next refill
+// point; it is read back from the entry there, so that a lane holds only the entry's index
+// meanwhile (with the light geometry set up here and throughput, light and destination held
+// per lane, the kernel took 72 VGPRs and 7 waves per SIMD).
 template <bool COUNT, bool ONE_SCENE>
 __global__ __launch_bounds__(kBlock) PRT_SHADOW_WAVES void wf_shadow(WfArgs a, uint32_t it) {
     __shared__ int s_stack[kStackLdsQueue * kBlock];
-    const uint32_t q1 = (it & 1u) ^ 1u;  // the queue shade(it) filled
-    const uint32_t n = a.ctr[kShadow];
+    const uint32_t n = uniform_u32(a.ctr[kShadow]);
     StackT<kStackLdsQueue> st;
     st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
     Counts cnt = {0, 0, 0, 0, 0, 0};
@@ -698,54 +744,41 @@ __global__ __launch_bounds__(kBlock) PRT_SHADOW_WAVES void wf_shadow(WfArgs a, u
     HitRec occ;
     const float4* nodes = ONE_SCENE ? wave_uniform(a.jobs[0].sc.nodes) : nullptr;
     const float4* tris = ONE_SCENE ? wave_uniform(a.jobs[0].sc.tris) : nullptr;
-    float4* dst = nullptr;  // the path's colour: next-queue entry or result slot
-    V3 mask = v3(0.f, 0.f, 0.f), direct = mask;
-    // As in wf_extend: a finished ray's colour update waits for the next refill point.
+    uint32_t i = 0;
     bool finished = false, lit = false;
     while (true) {
         const uint32_t idle = idle_lanes(active);
         if (idle >= kRefill) {
             if (finished) {
-                const float4 c = *dst;
-                const V3 s = add_direct(v3(c), mask, direct, lit);
-                *dst = make_float4(s.x, s.y, s.z, c.w);
+                const uint32_t odd = __float_as_uint(a.sf[i].w) >> 28;
+                if (lit || odd != 0u) {
+                    const float4 g = a.sg[i];
+                    float4* dst = a.result + __float_as_uint(g.w);
+                    const float4 c = *dst;
+                    const float nan = __builtin_nanf("");
+                    const V3 add = lit ? v3(g) : v3(odd & 1u ? nan : 0.f, odd & 2u ? nan : 0.f, odd & 4u ? nan : 0.f);
+                    const V3 s = v3(c) + add;
+                    *dst = make_float4(s.x, s.y, s.z, 0.f);
+                }
                 finished = false;
             }
             if (!feed.more()) {
                 if (idle == 64) break;
             } else if (const uint32_t got = feed.take(!active); got != kNone) {
-                const float4 e = a.se[got], f = a.sf[got], g = a.sg[got], hx = a.sh[got];
-                const SceneArgs& sc = a.jobs[__float_as_uint(hx.z)].sc;
-                NeeSample ns;
-                ns.position = v3(e);
-                ns.normal = v3(f);
-                ns.mask = v3(g);
-                ns.li = __float_as_uint(g.w);
-                ns.lu = f.w;
-                ns.lv = hx.x;
-                ShadowReq sr;
-                sr.direct = v3(0.f, 0.f, 0.f);
-                const bool reach = nee_prepare<COUNT>(sc, ns, sr, cnt);
-                const uint32_t target = __float_as_uint(e.w);
-                dst = __float_as_uint(hx.y) ? a.result + target : a.qd[q1] + target;
-                mask = ns.mask;
-                direct = sr.direct;
+                i = got;
+                const float4 e = a.se[i], f = a.sf[i];
                 if (!ONE_SCENE) {
+                    const SceneArgs& sc = a.jobs[a.sj[i]].sc;
                     nodes = sc.nodes;
                     tris = sc.tris;
                 }
-                occ.t = sr.tL;
-                occ.id = sr.lid;
+                occ.t = e.w;
+                occ.id = __float_as_uint(f.w) & kLightIdMask;
                 occ.rec = 0;
                 occ.mat = 0;
                 occ.u = occ.v = 0.f;
                 st.sp = 0;
-                active = reach && trav_begin(ray, sr.so, sr.sd);
-                if (!active) {  // the light sample cannot be seen: add mask * 0
-                    const float4 c = *dst;
-                    const V3 s = add_direct(v3(c), mask, direct, false);
-                    *dst = make_float4(s.x, s.y, s.z, c.w);
-                }
+                active = trav_begin(ray, v3(e), v3(f));  // true: wf_shade queues only rays that can hit
             }
         }
         const bool node_phase = node_phase_for<PRT_SHADOW_PHASE_MIN>(active && trav_wants_nodes(ray), active);
@@ -761,21 +794,41 @@ __global__ __launch_bounds__(kBlock) PRT_SHADOW_WAVES void wf_shadow(WfArgs a, u
     if (COUNT) flush_stats<true>(a.ctr, cnt);
 }
 
+// Adds each pixel's results to its running sum in sample order. A thread per pixel, in the
+// order of the full sections, so a wave reads one run of memory; a lane's samples of a
+// section lie one after another, and eight are read at once, the 128 bytes of a line.
 __global__ __launch_bounds__(256) void wf_resolve(WfArgs a) {
-    const WfChunk ch = a.chunks[a.ctr[kChunk]];
+    const WfChunk ch = current_chunk(a);
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < ch.pixels; k += gridDim.x * blockDim.x) {
         const WfTile t = a.tiles[find_tile(a.tiles, ch.tile0, ch.ntiles, k, true)];
-        const uint32_t w = t.p1 - t.p0;
-        const uint32_t p = t.p0 + (k - t.pix0);
-        float4* acc = a.jobs[t.job].accum + p;
-        float4 s = *acc;
-        V3 sum = v3(s.x, s.y, s.z);
         const WfJob& jb = a.jobs[t.job];
+        const PathOrder o = path_order(t, jb.width, a.group_lg);
+        const uint32_t q = k - t.pix0, off = position_to_pixel(o, o.g, q), p = t.p0 + off;
+        float4* acc = jb.accum + p;
+        const float4 s = *acc;
+        V3 sum = v3(s.x, s.y, s.z);
         const size_t npx = size_t(jb.width) * jb.height;
-        for (uint32_t smp = t.s0; smp < t.s1; ++smp) {
-            const float4 r = a.result[t.slot0 + (smp - t.s0) * w + (p - t.p0)];
+        uint32_t smp = t.s0;
+        auto add = [&](float4 r) {
             sum = sum + v3(r);
             if (jb.samples && smp < jb.samples_cap) jb.samples[size_t(smp) * npx + p] = make_float4(r.x, r.y, r.z, 0.f);
+            ++smp;
+        };
+        for (uint32_t sec = 0; sec <= o.full; ++sec) {
+            const bool last = sec == o.full;
+            const uint32_t m = last ? o.rest : o.m;
+            if (m == 0u) break;
+            const uint32_t at = last ? pixel_to_position(o, band_rows(m), off) : q;
+            const float4* r = a.result + t.slot0 + sec * (o.pixels * o.m) + at * m;
+            uint32_t j = 0;
+            for (; j + 8u <= m; j += 8u) {
+                float4 v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = r[j + e];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) add(v[e]);
+            }
+            for (; j < m; ++j) add(r[j]);
         }
         *acc = make_float4(sum.x, sum.y, sum.z, 0.f);
     }
@@ -868,7 +921,6 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
     w.mem = nullptr;
     w.spill = nullptr;
     w.ctr = nullptr;
-    // per slot: 2 queues x 64 B, hit 16 + 4, shadow 64, result 16
     w.bytes = kSlotBytes * size_t(capacity);
     WF_TRY(hipMalloc(&w.mem, w.bytes));
     WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
@@ -887,15 +939,14 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
         a.qa[k] = static_cast<float4*>(take(16 * C));
         a.qb[k] = static_cast<float4*>(take(16 * C));
         a.qc[k] = static_cast<float4*>(take(16 * C));
-        a.qd[k] = static_cast<float4*>(take(16 * C));
     }
     a.hits = static_cast<float4*>(take(16 * C));
     a.se = static_cast<float4*>(take(16 * C));
     a.sf = static_cast<float4*>(take(16 * C));
     a.sg = static_cast<float4*>(take(16 * C));
-    a.sh = static_cast<float4*>(take(16 * C));
     a.result = static_cast<float4*>(take(16 * C));
     a.hmat = static_cast<uint32_t*>(take(4 * C));
+    a.sj = static_cast<uint32_t*>(take(4 * C));
     a.ctr = w.ctr;
     a.spill = w.spill;
     a.spill_stride = persistent;
@@ -920,13 +971,12 @@ struct RunStats {
 };
 
 // Launches one chunk's kernels on `stream`: setup, generate, then per iteration
-// extend (wf_extend_packet at the first), shade and shadow, then resolve and
-// advance. With `ev` (4 per iteration) the extend / shade / shadow launches are
+// extend (wf_extend_packet at the first), shade and shadow, then resolve. With `ev` (4 per iteration) the extend / shade / shadow launches are
 // bracketed by events.
 template <bool COUNT, bool ONE_SCENE>
 void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int pblocks, int gblocks, int sblocks,
                   hipEvent_t* ev) {
-    hipLaunchKernelGGL(dev::wf_setup, dim3(1), dim3(64), 0, stream, a);
+    hipLaunchKernelGGL(dev::wf_setup, dim3((3 * max_depth * kSpread + 255) / 256), dim3(256), 0, stream, a);
     hipLaunchKernelGGL(dev::wf_generate, dim3(gblocks), dim3(256), 0, stream, a);
     for (uint32_t it = 0; it < max_depth; ++it) {
         if (ev) (void)hipEventRecord(ev[4 * it], stream);
@@ -942,7 +992,6 @@ void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int p
         if (ev) (void)hipEventRecord(ev[4 * it + 3], stream);
     }
     hipLaunchKernelGGL(dev::wf_resolve, dim3(gblocks), dim3(256), 0, stream, a);
-    hipLaunchKernelGGL(dev::wf_advance, dim3(1), dim3(64), 0, stream, a);
 }
 
 void launch_chunk_any(bool count, bool one_scene, const WfArgs& a, hipStream_t stream, uint32_t max_depth,
@@ -1027,7 +1076,8 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
                                           : reinterpret_cast<const void*>(dev::wf_extend<true, false>))
                              : (one_scene ? reinterpret_cast<const void*>(dev::wf_extend<false, true>)
                                           : reinterpret_cast<const void*>(dev::wf_extend<false, false>));
-    const int pblocks = persistent_blocks(kext, blocks_per_cu, device);
+    // No more waves than the largest queue has batches.
+    const int pblocks = std::min(persistent_blocks(kext, blocks_per_cu, device), int((need + kBatch - 1) / kBatch));
     int rc = ensure_state(w, device, need, uint32_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;
     rc = ensure_buffer(w.d_jobs, w.cap_jobs, jobs.size());
@@ -1037,13 +1087,14 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     WF_TRY(hipMemcpyAsync(w.d_jobs, jobs.data(), jobs.size() * sizeof(WfJob), hipMemcpyHostToDevice, stream));
     WF_TRY(hipMemcpyAsync(w.d_tiles, tiles.data(), tiles.size() * sizeof(WfTile), hipMemcpyHostToDevice, stream));
     WF_TRY(hipMemcpyAsync(w.d_chunks, chunks.data(), chunks.size() * sizeof(WfChunk), hipMemcpyHostToDevice, stream));
-    WF_TRY(hipMemsetAsync(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
+    WF_TRY(hipMemsetAsync(w.ctr, 0, kFetch * sizeof(uint32_t), stream));  // wf_setup clears the rest
     WfArgs a = w.args;
     a.jobs = w.d_jobs;
     a.tiles = w.d_tiles;
     a.chunks = w.d_chunks;
     a.max_depth = max_depth;
     a.group_lg = group_lg;
+    a.one_scene = one_scene ? 1u : 0u;
     a.spill_stride = uint32_t(pblocks) * kBlock;
 
     hipDeviceProp_t prop;

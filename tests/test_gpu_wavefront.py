@@ -121,3 +121,20 @@ def test_deep_stack_spill_equals_megakernel_and_oracle(gpu):
     np.testing.assert_allclose(wf, acc / np.float32(4), rtol=1e-5, atol=1e-6)
     assert cw == tuple(int(x) for x in cnt)
     assert float(wf.mean()) > 0.0
+
+
+# The order of a tile's camera paths: sample counts below, at and above a section of 64 with
+# every remainder class, images that no band height divides, tiles of part of a row (a queue
+# smaller than a row), sections cut by the queue size, and forced groups that divide nothing.
+@pytest.mark.parametrize("w,h,spp,queue,group", [
+    (1, 1, 1, 0, 0), (37, 1, 3, 0, 0), (1, 29, 65, 0, 0), (53, 41, 1, 0, 0), (53, 41, 2, 0, 0), (53, 41, 7, 0, 0),
+    (53, 41, 16, 0, 0), (31, 23, 33, 0, 0), (17, 13, 64, 0, 0), (17, 13, 130, 0, 0), (53, 41, 3, 40, 0),
+    (53, 41, 6, 53 * 41 * 4, 0), (53, 41, 5, 0, 1), (53, 41, 21, 0, 2), (53, 41, 9, 0, 4), (53, 41, 2, 0, 8)])
+def test_every_path_order_equals_megakernel(gpu, w, h, spp, queue, group):
+    scene = ca.Scene(W.spheres1m(w, h, instances=12).mesh)
+    cam = ca.camera_look_at((4.0, 12.0, 35.0), (0.0, 8.0, 0.0), (0.0, 1.0, 0.0), 45.0, w, h)
+    mk, cm = _render(scene, cam, w, h, spp, max_depth=5)
+    wf, cw = _render(scene, cam, w, h, spp, max_depth=5, integrator=ca.INTEGRATOR_WAVEFRONT, wavefront_queue=queue,
+                     wavefront_group=group)
+    assert np.array_equal(_bits(mk), _bits(wf))
+    assert cm == cw
