@@ -592,15 +592,12 @@ __device__ __forceinline__ void packet_traverse(const float4* nodes, const float
     }
 }
 
-// u, v and material of best.rec, by the intersection test that selected it
-// (identical inputs, so identical results).
-__device__ __forceinline__ void hit_details(const float4* tris, const TravRay& r, HitRec& best) {
+// t, u, v and material of the closest hit best.rec of the ray (o, d), by the intersection
+// test that selected it (identical inputs, so identical results).
+__device__ __forceinline__ void hit_details(const float4* tris, V3 o, V3 d, HitRec& best) {
     const size_t tb = size_t(best.rec) * 3;
     const float4 a = gload(tris, tb), b = gload(tris, tb + 1), c = gload(tris, tb + 2);
-    float t, u, v;
-    mt_intersect(a, b, c, r.o, r.d, t, u, v);
-    best.u = u;
-    best.v = v;
+    mt_intersect(a, b, c, o, d, best.t, best.u, best.v);
     best.mat = __float_as_uint(b.w);
 }
 

@@ -60,8 +60,8 @@ constexpr int kShadeBlock = PRT_SHADE_BLOCK;
 #define PRT_SHADE_GRID_WAVES 16
 #endif
 constexpr int kShadeGridWaves = PRT_SHADE_GRID_WAVES;
-// Bytes of queues and path state per slot: 2 queues x 48, hit 16 + 4, shadow 48 + 4, result 16.
-constexpr size_t kSlotBytes = 2 * 48 + 16 + 4 + 48 + 4 + 16;
+// Bytes of queues and path state per slot: 2 queues x 48, hit record 4, shadow 48 + 4, result 16.
+constexpr size_t kSlotBytes = 2 * 48 + 4 + 48 + 4 + 16;
 // Counter words per 128-byte cache line. Each queue counter and each fetch counter
 // has a line of its own: atomics on one line serialize in its L2 channel, and the
 // appends of wf_shade and the batch fetches of the traversal kernels would otherwise
@@ -125,8 +125,7 @@ struct WfArgs {
     float4* qa[2];
     float4* qb[2];
     float4* qc[2];
-    float4* hits;    // t, u, v, record (0xFFFFFFFF = miss)
-    uint32_t* hmat;  // material of the hit record
+    uint32_t* hits;  // record of the closest hit (0xFFFFFFFF = miss)
     float4* se;
     float4* sf;
     float4* sg;
@@ -468,9 +467,7 @@ __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, u
         const uint32_t idle = idle_lanes(active);
         if (idle >= kRefill) {
             if (finished) {
-                if (h.rec != 0xFFFFFFFFu) hit_details(tris, ray, h);
-                a.hits[i] = make_float4(h.t, h.u, h.v, __uint_as_float(h.rec));
-                a.hmat[i] = h.mat;
+                a.hits[i] = h.rec;
                 finished = false;
             }
             if (!feed.more()) {
@@ -494,8 +491,7 @@ __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, u
                 st.sp = 0;
                 active = trav_begin(ray, v3(o), v3(d));
                 if (!active) {  // zero direction: no triangle can be hit
-                    a.hits[i] = make_float4(h.t, h.u, h.v, __uint_as_float(0xFFFFFFFFu));
-                    a.hmat[i] = 0;
+                    a.hits[i] = 0xFFFFFFFFu;
                 }
             }
         }
@@ -580,8 +576,7 @@ __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend_packet(WfAr
             packet_traverse<false, COUNT>(nodes, tris, mine, ray, kEps, h, (lds_int*)s_pk, cnt, occ);
         });
         if (valid) {
-            a.hits[i] = make_float4(h.t, h.u, h.v, __uint_as_float(h.rec));
-            a.hmat[i] = h.mat;
+            a.hits[i] = h.rec;
         }
         base = fetch.resolve(pending);
         pending = base != kNone ? fetch.issue() : kNone;
@@ -649,15 +644,14 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         PathState ps;
         NeeSample ns;
         ShadowReq sr;
-        float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A, hh = A;
+        float4 A = make_float4(0.f, 0.f, 0.f, 0.f), B = A;
         float4 Cc = make_float4(1.f, 1.f, 1.f, __uint_as_float(i));  // a new path's
-        uint32_t hm = 0;
+        uint32_t rec = 0xFFFFFFFFu;
         if (valid) {
             A = a.qa[q][i];
             B = a.qb[q][i];
             if (it != 0) Cc = a.qc[q][i];
-            hh = a.hits[i];
-            hm = a.hmat[i];
+            rec = a.hits[i];
         }
         const uint32_t pj = __float_as_uint(A.w);
         const uint32_t slot = __float_as_uint(Cc.w) & kSlotMask;
@@ -670,17 +664,13 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         ps.input = it == 0 ? v3(0.f, 0.f, 0.f) : ps.rd;  // at b >= 1 the stale input is the ray direction
         with_job(valid, pj >> 24, [&](uint32_t jb) {
             const WfJob& j = a.jobs[jb];
-            const uint32_t rec = __float_as_uint(hh.w);
             if (rec == 0xFFFFFFFFu) {
                 path_miss(ps);
             } else {
                 HitRec h;
-                h.t = hh.x;
-                h.u = hh.y;
-                h.v = hh.z;
                 h.rec = rec;
                 h.id = 0;
-                h.mat = hm;
+                hit_details(j.sc.tris, ps.ro, ps.rd, h);
                 Rng rng{j.path.seed, j.path.view, pj & 0xFFFFFFu, __float_as_uint(B.w)};
                 more = shade_vertex<COUNT, true>(j.sc, j.path, rng, ps, h, &want_nee, ns, cnt);
                 if (want_nee && !(nee_prepare<COUNT>(j.sc, ns, sr, cnt) && can_hit(sr.sd))) {
@@ -940,12 +930,11 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
         a.qb[k] = static_cast<float4*>(take(16 * C));
         a.qc[k] = static_cast<float4*>(take(16 * C));
     }
-    a.hits = static_cast<float4*>(take(16 * C));
     a.se = static_cast<float4*>(take(16 * C));
     a.sf = static_cast<float4*>(take(16 * C));
     a.sg = static_cast<float4*>(take(16 * C));
     a.result = static_cast<float4*>(take(16 * C));
-    a.hmat = static_cast<uint32_t*>(take(4 * C));
+    a.hits = static_cast<uint32_t*>(take(4 * C));
     a.sj = static_cast<uint32_t*>(take(4 * C));
     a.ctr = w.ctr;
     a.spill = w.spill;
