@@ -71,18 +71,19 @@ constexpr size_t kSlotBytes = 2 * 48 + 4 + 48 + 4 + 16;
 #endif
 constexpr uint32_t kCtrLine = PRT_CTR_LINE;
 enum WfCounter : uint32_t {
-    kExt0 = 0,                 // ray count of queue 0
-    kExt1 = kCtrLine,          // ray count of queue 1
-    kShadow = 2 * kCtrLine,    // shadow ray count
-    kChunk = 3 * kCtrLine,     // number of the chunk being rendered, from 1
-    kStats = 4 * kCtrLine,     // kCntNum 64-bit counters (two words each)
-    kFetch = 8 * kCtrLine,     // per (kernel, iteration) fetch counters: 3 * kMaxIter groups of kSpread,
+    kChunk = 0,                // number of the chunk being rendered, from 1
+    kStats = kCtrLine,         // kCntNum 64-bit counters (two words each)
+    kQueue = 4 * kCtrLine,     // rays of each iteration's queues: extension at kQueue + 2 * it lines, shadow after it
+    kFetch = kQueue + 2 * (kMaxIter + 1) * kCtrLine,  // fetch counters: 2 * kMaxIter groups of kSpread,
                                // counter c of group g at kFetch + (g * kSpread + c) * kCtrLine
-    kNumCounters = kFetch + 3 * kMaxIter * kSpread * kCtrLine,
+    kNumCounters = kFetch + 2 * kMaxIter * kSpread * kCtrLine,
 };
-static_assert(kStats + 2 * kCntNum <= kFetch, "the statistics lie below the fetch counters");
-// First fetch counter of group g (3 * iteration + kernel: 0 extend, 2 shadow).
-constexpr uint32_t fetch_group(uint32_t g) { return kFetch + g * kSpread * kCtrLine; }
+static_assert(kStats + 2 * kCntNum <= kQueue, "the statistics lie below the queue counters");
+constexpr uint32_t ext_count(uint32_t it) { return kQueue + 2 * it * kCtrLine; }
+constexpr uint32_t shadow_count(uint32_t it) { return kQueue + (2 * it + 1) * kCtrLine; }
+// First fetch counter of an iteration's extension or shadow rays.
+constexpr uint32_t ext_fetch(uint32_t it) { return kFetch + 2 * it * kSpread * kCtrLine; }
+constexpr uint32_t shadow_fetch(uint32_t it) { return kFetch + (2 * it + 1) * kSpread * kCtrLine; }
 
 struct WfJob {
     SceneArgs sc;
@@ -117,6 +118,8 @@ struct WfChunk {
 // coalesce. (Carrying the colour in the queue entries, and the light sample's position,
 // normal, coordinates and throughput in the shadow entries, took 64 bytes each, and
 // wf_shade, whose first launch runs at the memory's rate, wrote them.)
+constexpr uint32_t kSlotMask = 0x7FFFFFFFu;   // a queue of 2^31 slots would not fit the memory
+constexpr uint32_t kLightIdMask = 0x0FFFFFFFu;  // triangle ids are below 2^28
 struct WfArgs {
     const WfJob* jobs;
     const WfTile* tiles;
@@ -198,14 +201,16 @@ struct WaveFetch {
         }
         return item(k, idx);
     }
-    // The wave's first batch; sets up the fetch of the others.
-    __device__ __forceinline__ uint32_t start(uint32_t* counters, uint32_t n) {
+    // The wave's first batch (counted from the last wave if `reversed`); sets up the fetch
+    // of the others.
+    __device__ __forceinline__ uint32_t start(uint32_t* counters, uint32_t n, bool reversed = false) {
         const uint32_t wave = uniform_u32(blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64);
         ctr = counters;
         k = wave % kSpread;
         nb = (n + kBatch - 1) / kBatch;
         waves = gridDim.x * (blockDim.x / 64);
-        return wave < nb ? wave * kBatch : kNone;
+        const uint32_t first = reversed ? waves - 1u - wave : wave;
+        return first < nb ? first * kBatch : kNone;
     }
 };
 // Hands single items of [0, n) to individual lanes: the wave holds one 64-item
@@ -216,9 +221,9 @@ struct WaveFetch {
 struct LaneFeeder {
     WaveFetch fetch;
     uint32_t n, base, used, pending;
-    __device__ __forceinline__ void start(uint32_t* ctr, uint32_t count) {
+    __device__ __forceinline__ void start(uint32_t* ctr, uint32_t count, bool reversed = false) {
         n = count;
-        base = fetch.start(ctr, count);
+        base = fetch.start(ctr, count, reversed);
         used = 0;
         pending = base != kNone ? fetch.issue() : kNone;
     }
@@ -287,11 +292,8 @@ static_assert(PRT_SHADOW_PHASE_MIN >= 0 && PRT_SHADOW_PHASE_MIN <= 64, "phase th
 // wf_extend fits 8 (64 VGPRs, 2 spilled on rarely taken paths) and wf_shadow too (54, with
 // its rays set up by wf_shade: 35.6 -> 31.6 ms per frame of 1080p x 128 spp over 1M
 // triangles, against 72 VGPRs, 7 waves and the set-up in its refill).
-#ifndef PRT_SHADOW_WAVES
-#define PRT_SHADOW_WAVES __attribute__((amdgpu_waves_per_eu(8)))
-#endif
-#ifndef PRT_EXTEND_WAVES
-#define PRT_EXTEND_WAVES __attribute__((amdgpu_waves_per_eu(8)))
+#ifndef PRT_TRACE_WAVES
+#define PRT_TRACE_WAVES __attribute__((amdgpu_waves_per_eu(8)))
 #endif
 // wf_shade keeps the compiler's occupancy (104 VGPRs, 4 waves per SIMD): forcing 5
 // or 6 waves spills 36 / 104 bytes per lane and measured 2% / 12% slower per frame;
@@ -331,17 +333,16 @@ __device__ __forceinline__ uint32_t find_tile(const WfTile* t, uint32_t first, u
     return lo;
 }
 
-// Goes on to the next chunk: its path count, empty queues, and the fetch counters of
-// the iterations it will run (one workgroup clearing all of them took 9 us).
+// Goes on to the next chunk: its path count, empty queues and fetch counters for the
+// iterations it will run, a thread each (one workgroup clearing all of them took 9 us).
 __global__ __launch_bounds__(256) void wf_setup(WfArgs a) {
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < 3 * a.max_depth * kSpread; k += gridDim.x * blockDim.x)
-        a.ctr[kFetch + k * kCtrLine] = 0;
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < 2 * a.max_depth * kSpread) a.ctr[kFetch + k * kCtrLine] = 0;
+    if (k >= 1 && k <= 2 * a.max_depth) a.ctr[kQueue + k * kCtrLine] = 0;
+    if (k != 0) return;
     const uint32_t c = a.ctr[kChunk];
     a.ctr[kChunk] = c + 1;
-    a.ctr[kExt0] = a.chunks[c].paths;
-    a.ctr[kExt1] = 0;
-    a.ctr[kShadow] = 0;
+    a.ctr[ext_count(0)] = a.chunks[c].paths;
 }
 // The chunk that wf_setup has gone on to.
 __device__ __forceinline__ WfChunk current_chunk(const WfArgs& a) {
@@ -435,27 +436,19 @@ __device__ __forceinline__ void with_job(bool valid, uint32_t job, F&& f) {
     }
 }
 
-// ONE_SCENE: every job of the batch traverses the same scene, so the node and
-// triangle arrays are wave-uniform (scalar registers).
+// Closest hit of every ray in the queue of iteration `it`. ONE_SCENE: every job of the
+// batch traverses the same scene, so the node and triangle arrays are wave-uniform
+// (scalar registers).
 template <bool COUNT, bool ONE_SCENE>
-__global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, uint32_t it) {
-    __shared__ int s_stack[kStackLdsQueue * kBlock];
+__device__ __forceinline__ void extend_rays(const WfArgs& a, uint32_t it, StackT<kStackLdsQueue>& st) {
     const uint32_t q = it & 1u;
-    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.ctr[kExt0 + (q ^ 1u)] = 0;  // the queue shade(it) fills
-        a.ctr[kShadow] = 0;
-    }
-    StackT<kStackLdsQueue> st;
-    st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
+    const uint32_t n = uniform_u32(a.ctr[ext_count(it)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
     LaneFeeder feed;
-    feed.start(&a.ctr[fetch_group(3 * it)], n);
+    feed.start(&a.ctr[ext_fetch(it)], n, true);
     bool active = false;
-    // A lane whose ray has finished keeps its hit in registers until the next refill
-    // point, where every such lane writes it at once: hit_details() (a triangle load
-    // and a full intersection) then runs with at least kRefill lanes instead of the
-    // few that finish in any one step.
+    // A lane whose ray has finished keeps its hit record in a register until the next
+    // refill point, where every such lane writes it at once.
     bool finished = false;
     uint32_t i = 0;
     TravRay ray;
@@ -490,9 +483,7 @@ __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, u
                 h.u = h.v = 0.f;
                 st.sp = 0;
                 active = trav_begin(ray, v3(o), v3(d));
-                if (!active) {  // zero direction: no triangle can be hit
-                    a.hits[i] = 0xFFFFFFFFu;
-                }
+                if (!active) a.hits[i] = 0xFFFFFFFFu;  // zero direction: no triangle can be hit
             }
         }
         // One node phase or leaf phase per step; a refill is considered every step.
@@ -505,6 +496,90 @@ __global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend(WfArgs a, u
         }
     }
     if (COUNT) flush_stats<false>(a.ctr, cnt);
+}
+
+// Occlusion test of every shadow ray of iteration `it`; a visible light sample's
+// contribution is added to the path's colour. A finished ray's update waits for the next
+// refill point too; it is read back from the entry there, so that a lane holds only the
+// entry's index meanwhile (with the light geometry set up here and throughput, light and
+// destination held per lane, this took 72 VGPRs and 7 waves per SIMD).
+template <bool COUNT, bool ONE_SCENE>
+__device__ __forceinline__ void shadow_rays(const WfArgs& a, uint32_t it, StackT<kStackLdsQueue>& st) {
+    const uint32_t n = uniform_u32(a.ctr[shadow_count(it)]);
+    Counts cnt = {0, 0, 0, 0, 0, 0};
+    LaneFeeder feed;
+    feed.start(&a.ctr[shadow_fetch(it)], n);
+    bool active = false;
+    TravRay ray;
+    ray.leaf = kNoChild;
+    HitRec occ;
+    const float4* nodes = ONE_SCENE ? wave_uniform(a.jobs[0].sc.nodes) : nullptr;
+    const float4* tris = ONE_SCENE ? wave_uniform(a.jobs[0].sc.tris) : nullptr;
+    uint32_t i = 0;
+    bool finished = false, lit = false;
+    while (true) {
+        const uint32_t idle = idle_lanes(active);
+        if (idle >= kRefill) {
+            if (finished) {
+                const uint32_t odd = __float_as_uint(a.sf[i].w) >> 28;
+                if (lit || odd != 0u) {
+                    const float4 g = a.sg[i];
+                    float4* dst = a.result + __float_as_uint(g.w);
+                    const float4 c = *dst;
+                    const float nan = __builtin_nanf("");
+                    const V3 add = lit ? v3(g) : v3(odd & 1u ? nan : 0.f, odd & 2u ? nan : 0.f, odd & 4u ? nan : 0.f);
+                    const V3 s = v3(c) + add;
+                    *dst = make_float4(s.x, s.y, s.z, 0.f);
+                }
+                finished = false;
+            }
+            if (!feed.more()) {
+                if (idle == 64) break;
+            } else if (const uint32_t got = feed.take(!active); got != kNone) {
+                i = got;
+                const float4 e = a.se[i], f = a.sf[i];
+                if (!ONE_SCENE) {
+                    const SceneArgs& sc = a.jobs[a.sj[i]].sc;
+                    nodes = sc.nodes;
+                    tris = sc.tris;
+                }
+                occ.t = e.w;
+                occ.id = __float_as_uint(f.w) & kLightIdMask;
+                occ.rec = 0;
+                occ.mat = 0;
+                occ.u = occ.v = 0.f;
+                st.sp = 0;
+                active = trav_begin(ray, v3(e), v3(f));  // true: wf_shade queues only rays that can hit
+            }
+        }
+        const bool node_phase = node_phase_for<PRT_SHADOW_PHASE_MIN>(active && trav_wants_nodes(ray), active);
+        if (active) {
+            const int r = trav_step<true, COUNT, true>(node_phase, nodes, tris, ray, kEps, occ, st, cnt);
+            if (r != kTravRunning) {
+                active = false;
+                finished = true;
+                lit = r == kTravDone;
+            }
+        }
+    }
+    if (COUNT) flush_stats<true>(a.ctr, cnt);
+}
+
+// The shadow rays of iteration it - 1 and the extension rays of iteration `it`, both made
+// by wf_shade(it - 1) and independent of each other, in one launch: a wave that finds no
+// more shadow rays goes on to extension rays, so the end of the one, where a few long rays
+// are left, is filled by the other, and in small queues (fewer batches than waves) the
+// first waves take the shadow rays while the last take the extension rays.(1280 x 720 x
+// 16 samples, 1M triangles, depth 8: wf_extend + wf_shadow 6.96 -> 6.13 ms per frame; 1080p x
+// 128: 73.9 -> 73.1; a 256 x 256 x 16 box: 376 -> 325 us.)
+enum : uint32_t { kTraceShadow = 1, kTraceExtend = 2 };
+template <bool COUNT, bool ONE_SCENE>
+__global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_trace(WfArgs a, uint32_t it, uint32_t parts) {
+    __shared__ int s_stack[kStackLdsQueue * kBlock];
+    StackT<kStackLdsQueue> st;
+    st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
+    if (parts & kTraceShadow) shadow_rays<COUNT, ONE_SCENE>(a, it - 1, st);
+    if (parts & kTraceExtend) extend_rays<COUNT, ONE_SCENE>(a, it, st);
 }
 
 // Runs f(lanes, job) once per distinct job among the wave's `live` lanes, with
@@ -536,30 +611,23 @@ __device__ __forceinline__ void per_scene_pass(bool live, uint32_t job, F&& f) {
 // lights, and later iterations' rays leave diffuse bounces in all directions.)
 static_assert(kBatch == 64 && kBlock == 64, "a packet is one fetch batch traced by one wave");
 template <bool COUNT, bool ONE_SCENE>
-__global__ __launch_bounds__(kBlock) PRT_EXTEND_WAVES void wf_extend_packet(WfArgs a, uint32_t it) {
+__global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_extend_packet(WfArgs a) {
     __shared__ int s_pk[kPacketStack];
-    const uint32_t q = it & 1u;
-    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.ctr[kExt0 + (q ^ 1u)] = 0;  // the queue shade(it) fills
-        a.ctr[kShadow] = 0;
-    }
+    const uint32_t n = uniform_u32(a.ctr[ext_count(0)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
     const uint32_t lane = threadIdx.x & 63u;
     WaveFetch fetch;
-    uint32_t base = fetch.start(&a.ctr[fetch_group(3 * it)], n);
+    uint32_t base = fetch.start(&a.ctr[ext_fetch(0)], n);
     uint32_t pending = base != kNone ? fetch.issue() : kNone;
     while (base != kNone) {
         const uint32_t i = base + lane;
         const bool valid = i < n;
         float4 o = make_float4(0.f, 0.f, 0.f, 0.f), d = o;
         if (valid) {
-            o = a.qa[q][i];
-            d = a.qb[q][i];
+            o = a.qa[0][i];
+            d = a.qb[0][i];
         }
-        if (COUNT && valid) {
-            if (it == 0) cnt.primary++; else cnt.extension++;
-        }
+        if (COUNT && valid) cnt.primary++;
         TravRay ray;
         const bool began = trav_begin(ray, v3(o), v3(d));  // false for the zero ray of an empty lane
         const bool live = valid && began;
@@ -625,8 +693,6 @@ __device__ __forceinline__ uint2 block_append(bool more, bool nee, uint32_t* ctr
 __device__ __forceinline__ uint32_t nonfinite(V3 m) {
     return (fabsf(m.x) <= kFltMax ? 0u : 1u) | (fabsf(m.y) <= kFltMax ? 0u : 2u) | (fabsf(m.z) <= kFltMax ? 0u : 4u);
 }
-constexpr uint32_t kSlotMask = 0x7FFFFFFFu;   // a queue of 2^31 slots would not fit the memory
-constexpr uint32_t kLightIdMask = 0x0FFFFFFFu;  // triangle ids are below 2^28
 
 // Shades every hit of the queue, sets up the shadow rays of the light samples and
 // compacts the survivors. The colour the vertex adds starts at 0 (0 + x = x exactly) and
@@ -634,7 +700,7 @@ constexpr uint32_t kLightIdMask = 0x0FFFFFFFu;  // triangle ids are below 2^28
 template <bool COUNT>
 __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a, uint32_t it) {
     const uint32_t q = it & 1u;
-    const uint32_t n = uniform_u32(a.ctr[kExt0 + q]);
+    const uint32_t n = uniform_u32(a.ctr[ext_count(it)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
     // Static, workgroup-uniform partition of the queue (shading cost varies little).
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
@@ -687,7 +753,7 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
                 a.result[slot] = make_float4(c.x, c.y, c.z, 0.f);
             }
         }
-        const uint2 pos = block_append(more, want_nee, &a.ctr[kExt0 + (q ^ 1u)], &a.ctr[kShadow]);
+        const uint2 pos = block_append(more, want_nee, &a.ctr[ext_count(it + 1)], &a.ctr[shadow_count(it)]);
         if (more) {
             const uint32_t special = ps.prev == 1 /*SPECULAR*/ || ps.prev == 4 /*REFRACTIVE*/ ? ~kSlotMask : 0u;
             a.qa[q ^ 1u][pos.x] = make_float4(ps.ro.x, ps.ro.y, ps.ro.z, A.w);
@@ -712,76 +778,6 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         if ((threadIdx.x & 63) == 0 && x)
             atomicAdd(reinterpret_cast<unsigned long long*>(a.ctr + kStats) + kCntAnyTris, x);
     }
-}
-
-// Occlusion test of every shadow ray; a visible light sample's contribution is added to
-// the path's colour. As in wf_extend a finished ray's update waits for the next refill
-// point; it is read back from the entry there, so that a lane holds only the entry's index
-// meanwhile (with the light geometry set up here and throughput, light and destination held
-// per lane, the kernel took 72 VGPRs and 7 waves per SIMD).
-template <bool COUNT, bool ONE_SCENE>
-__global__ __launch_bounds__(kBlock) PRT_SHADOW_WAVES void wf_shadow(WfArgs a, uint32_t it) {
-    __shared__ int s_stack[kStackLdsQueue * kBlock];
-    const uint32_t n = uniform_u32(a.ctr[kShadow]);
-    StackT<kStackLdsQueue> st;
-    st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
-    Counts cnt = {0, 0, 0, 0, 0, 0};
-    LaneFeeder feed;
-    feed.start(&a.ctr[fetch_group(3 * it + 2)], n);
-    bool active = false;
-    TravRay ray;
-    ray.leaf = kNoChild;
-    HitRec occ;
-    const float4* nodes = ONE_SCENE ? wave_uniform(a.jobs[0].sc.nodes) : nullptr;
-    const float4* tris = ONE_SCENE ? wave_uniform(a.jobs[0].sc.tris) : nullptr;
-    uint32_t i = 0;
-    bool finished = false, lit = false;
-    while (true) {
-        const uint32_t idle = idle_lanes(active);
-        if (idle >= kRefill) {
-            if (finished) {
-                const uint32_t odd = __float_as_uint(a.sf[i].w) >> 28;
-                if (lit || odd != 0u) {
-                    const float4 g = a.sg[i];
-                    float4* dst = a.result + __float_as_uint(g.w);
-                    const float4 c = *dst;
-                    const float nan = __builtin_nanf("");
-                    const V3 add = lit ? v3(g) : v3(odd & 1u ? nan : 0.f, odd & 2u ? nan : 0.f, odd & 4u ? nan : 0.f);
-                    const V3 s = v3(c) + add;
-                    *dst = make_float4(s.x, s.y, s.z, 0.f);
-                }
-                finished = false;
-            }
-            if (!feed.more()) {
-                if (idle == 64) break;
-            } else if (const uint32_t got = feed.take(!active); got != kNone) {
-                i = got;
-                const float4 e = a.se[i], f = a.sf[i];
-                if (!ONE_SCENE) {
-                    const SceneArgs& sc = a.jobs[a.sj[i]].sc;
-                    nodes = sc.nodes;
-                    tris = sc.tris;
-                }
-                occ.t = e.w;
-                occ.id = __float_as_uint(f.w) & kLightIdMask;
-                occ.rec = 0;
-                occ.mat = 0;
-                occ.u = occ.v = 0.f;
-                st.sp = 0;
-                active = trav_begin(ray, v3(e), v3(f));  // true: wf_shade queues only rays that can hit
-            }
-        }
-        const bool node_phase = node_phase_for<PRT_SHADOW_PHASE_MIN>(active && trav_wants_nodes(ray), active);
-        if (active) {
-            const int r = trav_step<true, COUNT, true>(node_phase, nodes, tris, ray, kEps, occ, st, cnt);
-            if (r != kTravRunning) {
-                active = false;
-                finished = true;
-                lit = r == kTravDone;
-            }
-        }
-    }
-    if (COUNT) flush_stats<true>(a.ctr, cnt);
 }
 
 // Adds each pixel's results to its running sum in sample order. A thread per pixel, in the
@@ -959,26 +955,34 @@ struct RunStats {
     uint32_t launches[3];
 };
 
-// Launches one chunk's kernels on `stream`: setup, generate, then per iteration
-// extend (wf_extend_packet at the first), shade and shadow, then resolve. With `ev` (4 per iteration) the extend / shade / shadow launches are
-// bracketed by events.
+// Launches one chunk's kernels on `stream`: setup, generate, the camera rays' extension
+// (wf_extend_packet), then per iteration shade and one launch that traces its shadow rays
+// and the next iteration's extension rays, then resolve. With `ev` (4 per iteration) those
+// two are launched one after the other, and each extend / shade / shadow part is bracketed
+// by events.
 template <bool COUNT, bool ONE_SCENE>
 void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int pblocks, int gblocks, int sblocks,
                   hipEvent_t* ev) {
-    hipLaunchKernelGGL(dev::wf_setup, dim3((3 * max_depth * kSpread + 255) / 256), dim3(256), 0, stream, a);
+    auto mark = [&](uint32_t k) {
+        if (ev) (void)hipEventRecord(ev[k], stream);
+    };
+    auto trace = [&](uint32_t it, uint32_t parts) {
+        hipLaunchKernelGGL((dev::wf_trace<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a, it, parts);
+    };
+    hipLaunchKernelGGL(dev::wf_setup, dim3((2 * max_depth * kSpread + 255) / 256), dim3(256), 0, stream, a);
     hipLaunchKernelGGL(dev::wf_generate, dim3(gblocks), dim3(256), 0, stream, a);
     for (uint32_t it = 0; it < max_depth; ++it) {
-        if (ev) (void)hipEventRecord(ev[4 * it], stream);
+        mark(4 * it);
         if (it == 0)
-            hipLaunchKernelGGL((dev::wf_extend_packet<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a,
-                               it);
-        else
-            hipLaunchKernelGGL((dev::wf_extend<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a, it);
-        if (ev) (void)hipEventRecord(ev[4 * it + 1], stream);
+            hipLaunchKernelGGL((dev::wf_extend_packet<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a);
+        else if (ev)
+            trace(it, dev::kTraceExtend);
+        mark(4 * it + 1);
         hipLaunchKernelGGL(dev::wf_shade<COUNT>, dim3(sblocks), dim3(kShadeBlock), 0, stream, a, it);
-        if (ev) (void)hipEventRecord(ev[4 * it + 2], stream);
-        hipLaunchKernelGGL((dev::wf_shadow<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a, it);
-        if (ev) (void)hipEventRecord(ev[4 * it + 3], stream);
+        mark(4 * it + 2);
+        // The last iteration leaves no extension rays.
+        trace(it + 1, ev || it + 1 == max_depth ? dev::kTraceShadow : dev::kTraceShadow | dev::kTraceExtend);
+        mark(4 * it + 3);
     }
     hipLaunchKernelGGL(dev::wf_resolve, dim3(gblocks), dim3(256), 0, stream, a);
 }
@@ -1061,12 +1065,12 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     bool one_scene = true;
     for (const WfJob& j : jobs)
         one_scene = one_scene && j.sc.nodes == jobs[0].sc.nodes && j.sc.tris == jobs[0].sc.tris;
-    const void* kext = count ? (one_scene ? reinterpret_cast<const void*>(dev::wf_extend<true, true>)
-                                          : reinterpret_cast<const void*>(dev::wf_extend<true, false>))
-                             : (one_scene ? reinterpret_cast<const void*>(dev::wf_extend<false, true>)
-                                          : reinterpret_cast<const void*>(dev::wf_extend<false, false>));
+    const void* ktrace = count ? (one_scene ? reinterpret_cast<const void*>(dev::wf_trace<true, true>)
+                                          : reinterpret_cast<const void*>(dev::wf_trace<true, false>))
+                             : (one_scene ? reinterpret_cast<const void*>(dev::wf_trace<false, true>)
+                                          : reinterpret_cast<const void*>(dev::wf_trace<false, false>));
     // No more waves than the largest queue has batches.
-    const int pblocks = std::min(persistent_blocks(kext, blocks_per_cu, device), int((need + kBatch - 1) / kBatch));
+    const int pblocks = std::min(persistent_blocks(ktrace, blocks_per_cu, device), int((need + kBatch - 1) / kBatch));
     int rc = ensure_state(w, device, need, uint32_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;
     rc = ensure_buffer(w.d_jobs, w.cap_jobs, jobs.size());
