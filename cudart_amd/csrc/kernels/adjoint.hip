@@ -7,7 +7,8 @@
 // takes L from the forward pass when the renderer kept it (keep_samples), or traces
 // the path once (primal, the megakernel's arithmetic) to get it, then replays the
 // path with the same Philox slots, keeping the radiance still to be collected,
-// rem = L - (what the path collected so far). Parameters:
+// rem = L - (what the path collected so far). With the path's vertices kept as well, the
+// replay traces no ray (adjoint_stored). Parameters:
 //   kd_m (RGB)  a diffuse vertex multiplies everything collected after it by
 //               kd_c, so it contributes delta_c * rem_c / kd_c (rem taken after
 //               that vertex's emission, before its next-event estimate);
@@ -46,7 +47,9 @@ struct AdjArgs {
     uint32_t tiles_x, tiles;
     uint32_t parts;       // workgroups per tile, each replaying a 1/parts range of its pixel-samples
     const float* grad;    // W*H*3 dLoss / dI
-    const float4* samples;  // nullptr, or each sample's radiance from the forward pass [s * W * H + p]
+    const float4* samples;  // nullptr, or each sample's radiance from the forward pass [p * sample_cap + s]
+    const uint32_t* vertices;  // nullptr, or its path's vertices [(b * W * H + p) * sample_cap + s]
+    uint32_t sample_cap;
     double norm;          // 1 / spp: dI / dL of one sample
     double half_hess;     // (d2 Loss / dI2) / (2 spp^2): loss curvature per sample radiance
     uint32_t num_params;  // 4 * materials: kd (M*3) then emission (M)
@@ -380,7 +383,7 @@ __global__ __launch_bounds__(kBlock) PRT_ADJOINT_WAVES void adjoint_kernel(AdjAr
                     const size_t pix = size_t(y) * a.width + size_t(x);
                     const D3 delta{a.norm * double(a.grad[pix * 3]), a.norm * double(a.grad[pix * 3 + 1]),
                                    a.norm * double(a.grad[pix * 3 + 2])};
-                    const V3 L = a.samples ? v3(a.samples[size_t(s) * a.width * a.height + pix])
+                    const V3 L = a.samples ? v3(a.samples[pix * a.sample_cap + s])
                                            : primal(a, x, y, s, st, cnt);
                     replay_begin(a, x, y, s, delta, L, r);
                     mode = start_ext(r, tr, h, st) ? kLaneExt : kLaneIdle;
@@ -405,6 +408,125 @@ __global__ __launch_bounds__(kBlock) PRT_ADJOINT_WAVES void adjoint_kernel(AdjAr
     __syncthreads();
     double* out = a.partial + size_t(blockIdx.x) * a.num_params;
     for (uint32_t k = threadIdx.x; k < a.num_params; k += kBlock) out[k] = s_g[k];
+}
+
+// The replay from kept vertices: each closest hit's record and each light sample's
+// visibility are known, so no ray is traced; the vertex's work is the one above.
+//
+// A lane replays one path, 64 consecutive samples of a pixel to a wave, with the bounces in
+// step (the vertices, [bounce][pixel][sample], are read coalesced). The tracing replay waited
+// for node fetches for 0.43 of its waves' time, had 0.39 of its lanes active and takes 167
+// VGPRs; on 512^2 x 64 samples of the 100k-triangle scene it took 35.6 ms, this 3.15, and the
+// forward pass pays for the vertices with 4 bytes written per vertex (within its run-to-run
+// spread). What is left is the vertices' arithmetic (122 VGPRs, 4 waves per SIMD; held at 5:
+// 3.31 ms). The fp64 sums in LDS are not what bounds it: 4 or 8 copies of them, a lane adding
+// to copy lane % 8, so that lanes meeting one material do not take turns, measured the same.
+//
+// Russian roulette: step j adds kappa_j (w_{j-1} - w_j) for every diffuse vertex before the
+// step and -kappa_j w_j for the step's own (replay_after_nee). The first is the same for all
+// of them, so with P the running sum of kappa (w_{j-1} - w_j), a vertex adds
+// -kappa_j w_j - P at its own step and P's last value when the path has ended: two adds per
+// vertex and channel instead of one per vertex, step and channel.
+// The vertex `word` of the path. Returns true when the path goes on.
+__device__ __forceinline__ bool stored_vertex(const AdjArgs& a, Replay& r, uint32_t word, D3& P, double* g,
+                                              Counts& cnt) {
+    const SceneArgs& sc = a.sc;
+    const uint32_t M = a.num_materials;
+    const double gain = 3.0 * double(sc.lights_area);  // d ka / d e
+    PathState& ps = r.ps;
+    HitRec h;
+    h.rec = word & kVertexMiss;
+    h.id = 0;
+    hit_details(sc.tris, ps.ro, ps.rd, h);
+    const float4 mkd = sc.mats[size_t(h.mat) * 4], mka = sc.mats[size_t(h.mat) * 4 + 1];
+    if (ps.b == 0 || ps.prev == 1 || ps.prev == 4) {
+        const V3 e = ps.mask * v3(mka) * sc.inv_lights_area;
+        atomicAdd(&g[3 * M + h.mat], ddot(r.delta, d3(ps.mask)) * gain * double(sc.inv_lights_area));
+        r.rem = dsub(r.rem, d3(e));
+    }
+    const uint32_t b = ps.b;
+    bool want_nee;
+    NeeSample ns;
+    RrInfo rr;
+    const bool more = shade_vertex<false, false>(sc, a.path, r.rng, ps, h, &want_nee, ns, cnt, &rr);
+    const bool diffuse = ps.prev == 0 /*DIFFUSE*/ && __float_as_int(mka.w) < 0;
+    D3 own{r.delta.x * r.rem.x, r.delta.y * r.rem.y, r.delta.z * r.rem.z};
+    if (want_nee) {
+        ShadowReq sr;
+        sr.direct = v3(0.f, 0.f, 0.f);
+        const bool reach = nee_prepare<false>(sc, ns, sr, cnt);
+        const bool visible = reach && ((word & kVertexLit) != 0u || !can_hit(sr.sd));
+        if (visible) {
+            r.rem = dsub(r.rem, d3(ns.mask * sr.direct));
+            atomicAdd(&g[3 * M + sr.lmat], ddot(r.delta, d3(ns.mask)) * gain * double(sr.wf));
+        }
+        ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
+    }
+    const bool survived = rr.p >= 0.f && ps.b == b + 1;
+    if (survived) {
+        const D3 R = dsub(d3(r.L), d3(ps.color));
+        const double kappa = rr.p >= 1.f ? ddot(r.delta, R) : a.half_hess * ddot(R, R);
+        const D3 w = rr_weight(rr.ties), wp = rr_weight(r.prev_ties);
+        if (wp.x != w.x) P.x += kappa * (wp.x - w.x);
+        if (wp.y != w.y) P.y += kappa * (wp.y - w.y);
+        if (wp.z != w.z) P.z += kappa * (wp.z - w.z);
+        own.x -= (w.x != 0.0 ? kappa * w.x : 0.0) + P.x;
+        own.y -= (w.y != 0.0 ? kappa * w.y : 0.0) + P.y;
+        own.z -= (w.z != 0.0 ? kappa * w.z : 0.0) + P.z;
+        r.prev_ties = rr.ties;
+    }
+    if (diffuse) {
+        if (mkd.x != 0.f) atomicAdd(&g[3 * h.mat], own.x / double(mkd.x));
+        if (mkd.y != 0.f) atomicAdd(&g[3 * h.mat + 1], own.y / double(mkd.y));
+        if (mkd.z != 0.f) atomicAdd(&g[3 * h.mat + 2], own.z / double(mkd.z));
+        // A vertex whose roulette step ended the path has no part in P.
+        if (survived || rr.p < 0.f) r.vl.push(h.mat);
+    }
+    return more;
+}
+
+__global__ __launch_bounds__(kBlock) void adjoint_stored(AdjArgs a) {
+    extern __shared__ double s_sums[];  // num_params
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t k = lane; k < a.num_params; k += kBlock) s_sums[k] = 0.0;
+    __syncthreads();
+    const uint32_t units = a.tiles * a.parts;
+    const uint32_t unit = xcd_tile(blockIdx.x, units);
+    if (unit < units) {
+        const uint32_t tile = unit / a.parts, part = unit - tile * a.parts;
+        const uint32_t tx = (tile % a.tiles_x) * 8, ty = (tile / a.tiles_x) * 8;
+        const uint32_t cols = min(8u, a.width - tx), rows = min(8u, a.height - ty);
+        const uint64_t items = uint64_t(cols) * rows * a.spp;
+        const uint32_t i0 = uint32_t(items * part / a.parts), i1 = uint32_t(items * (part + 1) / a.parts);
+        const size_t stride = size_t(a.width) * a.height * a.sample_cap;
+        Counts cnt = {0, 0, 0, 0, 0, 0};
+        for (uint32_t j = i0 + lane; j < i1; j += kBlock) {
+            const uint32_t p = j / a.spp, s = j - p * a.spp;
+            const int x = int(tx + p % cols), y = int(ty + p / cols);
+            const size_t pix = size_t(y) * a.width + size_t(x), path = pix * a.sample_cap + s;
+            const D3 delta{a.norm * double(a.grad[pix * 3]), a.norm * double(a.grad[pix * 3 + 1]),
+                           a.norm * double(a.grad[pix * 3 + 2])};
+            Replay r;
+            replay_begin(a, x, y, s, delta, v3(a.samples[path]), r);
+            D3 P{0.0, 0.0, 0.0};
+            const uint32_t* at = a.vertices + path;
+            for (bool more = true; more; at += stride) {
+                const uint32_t word = *at;
+                more = word != kVertexMiss && stored_vertex(a, r, word, P, s_sums, cnt);  // the sky carries no parameter
+            }
+            if (P.x != 0.0 || P.y != 0.0 || P.z != 0.0)
+                for (uint32_t i = 0; i < r.vl.n; ++i) {
+                    const uint32_t m = r.vl.at(i);
+                    const float4 kd = a.sc.mats[size_t(m) * 4];
+                    if (kd.x != 0.f) atomicAdd(&s_sums[3 * m], P.x / double(kd.x));
+                    if (kd.y != 0.f) atomicAdd(&s_sums[3 * m + 1], P.y / double(kd.y));
+                    if (kd.z != 0.f) atomicAdd(&s_sums[3 * m + 2], P.z / double(kd.z));
+                }
+        }
+    }
+    __syncthreads();
+    double* out = a.partial + size_t(blockIdx.x) * a.num_params;
+    for (uint32_t k = lane; k < a.num_params; k += kBlock) out[k] = s_sums[k];
 }
 
 // Sums the per-workgroup partials of parameter blockIdx.x in a fixed order: thread t
@@ -519,6 +641,8 @@ AdjArgs adjoint_args(const prt_renderer* r, const float* grad, float hess, uint3
                         r->samples_version == r->scene->mats_version
                     ? r->samples
                     : nullptr;
+    a.vertices = a.samples ? r->vertices : nullptr;
+    a.sample_cap = r->spp;
     a.norm = 1.0 / double(spp);
     a.half_hess = double(hess) / (2.0 * double(spp) * double(spp));
     a.num_params = 4 * r->scene->num_materials;
@@ -527,6 +651,16 @@ AdjArgs adjoint_args(const prt_renderer* r, const float* grad, float hess, uint3
     a.spill = r->spill;
     a.spill_stride = r->spill_threads;
     return a;
+}
+
+// The replay over `grid` workgroups: from kept vertices where there are any, else tracing
+// each path.
+hipError_t launch_adjoint(const AdjArgs& a, uint32_t grid, hipStream_t s) {
+    if (a.vertices)
+        hipLaunchKernelGGL(dev::adjoint_stored, dim3(grid), dim3(kBlock), a.num_params * sizeof(double), s, a);
+    else
+        hipLaunchKernelGGL(dev::adjoint_kernel, dim3(grid), dim3(kBlock), 0, s, a);
+    return hipGetLastError();
 }
 }  // namespace
 
@@ -553,6 +687,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     double* d_out = nullptr;
     float4* d_samp = nullptr;  // this call's per-sample radiance, when none was kept
     float4* d_acc = nullptr;
+    uint32_t* d_vert = nullptr;
     std::vector<double> g(P);
     float ms = 0.f;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -562,30 +697,36 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_out), P * sizeof(double)));
     ADJ_TRY(copy_wait(d_grad, grad_rgb, px * 3 * sizeof(float), hipMemcpyHostToDevice, r->stream));
     a = adjoint_args(r, d_grad, hess, spp, d_part);
-    // Without kept radiance, a wavefront forward pass first writes each sample's
-    // radiance to a buffer of this call (when that fits in a quarter of the free
-    // memory), and the replay kernel only replays; otherwise each lane traces its
-    // sample's primal path before replaying it. The radiance is the same bit for
-    // bit either way, and so are the gradients.
-    if (!a.samples && !primal_in_replay()) {
+    // Without kept vertices, a wavefront forward pass first writes each sample's radiance and
+    // path vertices to buffers of this call (when they fit in a quarter of the free memory),
+    // and the replay traces no ray. Where only the radiance fits it traces the path's rays
+    // again, and where that does not fit either each lane traces its sample's primal path
+    // before replaying it. Radiance and vertices are the same either way.
+    if (!a.vertices && !primal_in_replay()) {
         size_t free_b = 0, total_b = 0;
-        const size_t need = px * (size_t(spp) + 1) * sizeof(float4);
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= free_b / 4) {
-            ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_samp), px * spp * sizeof(float4)));
-            ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_acc), px * sizeof(float4)));
-            ADJ_TRY(hipMemsetAsync(d_acc, 0, px * sizeof(float4), r->stream));
+        const size_t radiance = px * (size_t(spp) + 1) * sizeof(float4);
+        const size_t vert = px * spp * r->cfg.max_depth * sizeof(uint32_t);
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
+            const bool with = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && radiance + vert <= free_b / 4;
+            if (with || (!a.samples && radiance <= free_b / 4)) {
+                ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_samp), px * spp * sizeof(float4)));
+                ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_acc), px * sizeof(float4)));
+                ADJ_TRY(hipMemsetAsync(d_acc, 0, px * sizeof(float4), r->stream));
+            }
+            if (with) ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_vert), vert));
         }
     }
     ADJ_TRY(hipEventCreate(&e0));
     ADJ_TRY(hipEventCreate(&e1));
     ADJ_TRY(hipEventRecord(e0, r->stream));
     if (d_samp) {
-        rc = wavefront_samples(r, spp, d_acc, d_samp);
+        rc = wavefront_samples(r, spp, d_acc, d_samp, d_vert);
         if (rc != PRT_OK) goto done;
         a.samples = d_samp;
+        a.vertices = d_vert;
+        a.sample_cap = spp;
     }
-    hipLaunchKernelGGL(dev::adjoint_kernel, dim3(grid), dim3(kBlock), 0, r->stream, a);
-    ADJ_TRY(hipGetLastError());
+    ADJ_TRY(launch_adjoint(a, grid, r->stream));
     hipLaunchKernelGGL(dev::adjoint_reduce, dim3(P), dim3(dev::kReduceBlock), 0, r->stream, d_part, grid, P, d_out);
     ADJ_TRY(hipGetLastError());
     ADJ_TRY(hipEventRecord(e1, r->stream));
@@ -598,7 +739,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
 done:
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
-    void* ptrs[] = {d_grad, d_part, d_out, d_samp, d_acc};
+    void* ptrs[] = {d_grad, d_part, d_out, d_samp, d_acc, d_vert};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     return rc;
@@ -639,8 +780,7 @@ extern "C" int prt_adjoint_grad_static(prt_renderer* r, const float* grad_rgb_de
     double g[4 * PRT_MAX_MATERIALS];
     float ms = 0.f;
     HIP_CHECK(hipEventRecord(r->ev0, r->stream));
-    hipLaunchKernelGGL(dev::adjoint_kernel, dim3(grid), dim3(kBlock), 0, r->stream, a);
-    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(launch_adjoint(a, grid, r->stream));
     hipLaunchKernelGGL(dev::adjoint_reduce, dim3(P), dim3(dev::kReduceBlock), 0, r->stream,
                        static_cast<const double*>(base), grid, P, d_out);
     HIP_CHECK(hipGetLastError());

@@ -216,6 +216,16 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     HIP_TRY(copy_wait(r->gamma_lut, lut, 256, hipMemcpyHostToDevice, r->stream));
     if (c.keep_samples && spp > 0)
         HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->samples), px * spp * sizeof(float4)));
+    if (r->samples && c.integrator == PRT_INTEGRATOR_WAVEFRONT && vertices_fit(w, h, spp, c.max_depth)) {
+        // Only where there is room for them (without, the adjoint traces the paths again).
+        size_t free_b = 0, total_b = 0;
+        const size_t need = px * spp * c.max_depth * sizeof(uint32_t);
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= free_b / 4 &&
+            hipMalloc(reinterpret_cast<void**>(&r->vertices), need) != hipSuccess) {
+            r->vertices = nullptr;
+            (void)hipGetLastError();
+        }
+    }
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
     rc = ensure_spill(r.get(), ((r->tiles + 7) / 8) * 8 * kBlock);
@@ -415,7 +425,7 @@ extern "C" int prt_renderer_destroy(prt_renderer* r) {
     (void)hipSetDevice(r->cfg.device);
     release_wavefront(r);
     if (r->stream) (void)hipStreamSynchronize(r->stream);
-    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples};
+    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (r->ev0) (void)hipEventDestroy(r->ev0);

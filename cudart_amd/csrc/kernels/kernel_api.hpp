@@ -47,6 +47,11 @@ struct PathArgs {
     uint32_t max_depth, rr_start;
 };
 
+// A path vertex as a forward pass keeps it: the record of the closest hit, whether the
+// vertex's light sample was visible, or kVertexMiss. Records are below 2^28 - 1.
+constexpr uint32_t kVertexLit = 0x80000000u;
+constexpr uint32_t kVertexMiss = 0x0FFFFFFFu;
+
 // Counter slots (unsigned long long each).
 enum CounterSlot {
     kCntPrimary = 0,
@@ -69,7 +74,7 @@ struct MegaArgs {
     uint32_t s0, nspp;
     uint32_t tiles_x, tiles;  // 8x8 tiles
     float4* accum;            // width*height, .xyz = running sum
-    float4* samples;          // nullptr, or each sample's radiance at [sample * width * height + pixel]
+    float4* samples;          // nullptr, or each sample's radiance at [pixel * samples_cap + sample]
     uint32_t samples_cap;     // samples stored per pixel
     unsigned long long* counters;  // kCntNum or nullptr
     int* spill;               // (kStackMax - kStackLds) * spill_stride ints

@@ -32,10 +32,12 @@ struct prt_renderer {
     double kernel_ms[3] = {0, 0, 0};  // profile_kernels: extend, shade, shadow of the last wavefront render
     uint32_t kernel_launches[3] = {0, 0, 0};
     prt::WavefrontState* wf = nullptr;
-    // keep_samples: radiance of pixel-sample (s, p) at samples[s * w * h + p], s < spp.
-    // Valid for the adjoint while every sample since the last reset was rendered with
+    // keep_samples: radiance of pixel-sample (p, s) at samples[p * spp + s], s < spp, and
+    // (wavefront, where it fits) its path's vertex at bounce b at
+    // vertices[(b * w * h + p) * spp + s]. Valid for the adjoint while every sample since the last reset was rendered with
     // the scene's current materials (samples_version).
     float4* samples = nullptr;
+    uint32_t* vertices = nullptr;
     bool samples_ok = false;
     uint64_t samples_version = 0;
 };
@@ -60,9 +62,15 @@ CamArgs cam_args(const prt_camera& c);
 int set_device(int device);
 int ensure_spill(prt_renderer* r, uint32_t threads);
 int render_wavefront(prt_renderer* r, uint32_t n);  // wavefront.hip
-// Samples 0..spp-1 of the renderer's view into `accum` (zeroed) and each sample's
-// radiance into `samples` ([sample * pixels + pixel]), without touching the
-// renderer's own accumulation or counters.
-int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples);  // wavefront.hip
+// Samples 0..spp-1 of the renderer's view into `accum` (zeroed), each sample's radiance
+// into `samples` ([pixel * spp + sample]) and, unless null, its path's vertices into
+// `vertices` ([(bounce * pixels + pixel) * spp + sample]), without touching the renderer's
+// own accumulation or counters.
+int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples,
+                      uint32_t* vertices);  // wavefront.hip
+// Whether path vertices of spp samples of this view can be kept (index and depth limits).
+inline bool vertices_fit(uint32_t w, uint32_t h, uint32_t spp, uint32_t max_depth) {
+    return max_depth <= 16 && uint64_t(w) * h <= (1u << 24) && uint64_t(w) * h * spp < (uint64_t(1) << 32);
+}
 void release_wavefront(prt_renderer* r);            // wavefront.hip
 }  // namespace prt

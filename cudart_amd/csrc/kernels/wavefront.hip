@@ -91,7 +91,7 @@ struct WfJob {
     PathArgs path;
     uint32_t width, height;
     float4* accum;
-    float4* samples;       // nullptr, or each sample's radiance at [sample * width * height + pixel]
+    float4* samples;       // nullptr, or each sample's radiance at [pixel * samples_cap + sample]
     uint32_t samples_cap;  // samples stored per pixel
 };
 
@@ -132,8 +132,13 @@ struct WfArgs {
     float4* se;
     float4* sf;
     float4* sg;
-    uint32_t* sj;    // job of the shadow entry
+    uint32_t* sj;    // the shadow entry's job or, with `vertices`, its pixel-sample
     float4* result;  // per slot colour
+    // One job only: nullptr, or every path's vertices, pixel-sample (p, s) at bounce b at
+    // vertices[b * vertex_stride + p * vertex_cap + s], s < vertex_cap.
+    uint32_t* vertices;
+    size_t vertex_stride;
+    uint32_t vertex_cap;
     int* spill;
     uint32_t spill_stride;
     uint32_t max_depth;
@@ -530,6 +535,10 @@ __device__ __forceinline__ void shadow_rays(const WfArgs& a, uint32_t it, StackT
                     const V3 add = lit ? v3(g) : v3(odd & 1u ? nan : 0.f, odd & 2u ? nan : 0.f, odd & 4u ? nan : 0.f);
                     const V3 s = v3(c) + add;
                     *dst = make_float4(s.x, s.y, s.z, 0.f);
+                    if (lit && a.vertices) {
+                        const uint32_t path = a.sj[i];
+                        if (path != kNone) atomicOr(a.vertices + it * a.vertex_stride + path, kVertexLit);
+                    }
                 }
                 finished = false;
             }
@@ -721,6 +730,10 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         }
         const uint32_t pj = __float_as_uint(A.w);
         const uint32_t slot = __float_as_uint(Cc.w) & kSlotMask;
+        const uint32_t sample = __float_as_uint(B.w);
+        const bool keep = a.vertices != nullptr && sample < a.vertex_cap;
+        const uint32_t path = keep ? (pj & 0xFFFFFFu) * a.vertex_cap + sample : kNone;
+        if (keep && valid) a.vertices[it * a.vertex_stride + path] = rec == 0xFFFFFFFFu ? kVertexMiss : rec;
         ps.ro = v3(A);
         ps.rd = v3(B);
         ps.mask = v3(Cc);
@@ -737,7 +750,7 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
                 h.rec = rec;
                 h.id = 0;
                 hit_details(j.sc.tris, ps.ro, ps.rd, h);
-                Rng rng{j.path.seed, j.path.view, pj & 0xFFFFFFu, __float_as_uint(B.w)};
+                Rng rng{j.path.seed, j.path.view, pj & 0xFFFFFFu, sample};
                 more = shade_vertex<COUNT, true>(j.sc, j.path, rng, ps, h, &want_nee, ns, cnt);
                 if (want_nee && !(nee_prepare<COUNT>(j.sc, ns, sr, cnt) && can_hit(sr.sd))) {
                     want_nee = false;  // the light sample cannot be seen: add mask * 0
@@ -766,7 +779,8 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
             a.se[pos.y] = make_float4(sr.so.x, sr.so.y, sr.so.z, sr.tL);
             a.sf[pos.y] = make_float4(sr.sd.x, sr.sd.y, sr.sd.z, __uint_as_float(id));
             a.sg[pos.y] = make_float4(c.x, c.y, c.z, __uint_as_float(slot));
-            if (!a.one_scene) a.sj[pos.y] = pj >> 24;
+            if (a.vertices) a.sj[pos.y] = path;
+            else if (!a.one_scene) a.sj[pos.y] = pj >> 24;
         }
     }
     if (COUNT) {
@@ -793,11 +807,10 @@ __global__ __launch_bounds__(256) void wf_resolve(WfArgs a) {
         float4* acc = jb.accum + p;
         const float4 s = *acc;
         V3 sum = v3(s.x, s.y, s.z);
-        const size_t npx = size_t(jb.width) * jb.height;
         uint32_t smp = t.s0;
         auto add = [&](float4 r) {
             sum = sum + v3(r);
-            if (jb.samples && smp < jb.samples_cap) jb.samples[size_t(smp) * npx + p] = make_float4(r.x, r.y, r.z, 0.f);
+            if (jb.samples && smp < jb.samples_cap) jb.samples[size_t(p) * jb.samples_cap + smp] = make_float4(r.x, r.y, r.z, 0.f);
             ++smp;
         };
         for (uint32_t sec = 0; sec <= o.full; ++sec) {
@@ -1044,7 +1057,8 @@ int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t m
 // group_side: camera-path block side g for wf_generate (1, 2, 4, 8; 0 = choose per tile).
 int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::vector<WfJob>& jobs,
                   const std::vector<PlanJob>& pjobs, uint32_t max_depth, uint32_t capacity, uint32_t blocks_per_cu,
-                  uint32_t group_side, bool count, RunStats* rs, bool profile = false) {
+                  uint32_t group_side, bool count, RunStats* rs, bool profile = false, uint32_t* vertices = nullptr,
+                  uint32_t vertex_cap = 0) {
     if (max_depth == 0 || max_depth > uint32_t(kMaxIter)) return fail(PRT_ERR_INVALID_ARG, "max_depth out of range");
     uint32_t group_lg = dev::kNone;
     if (group_side != 0) {
@@ -1089,6 +1103,9 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     a.group_lg = group_lg;
     a.one_scene = one_scene ? 1u : 0u;
     a.spill_stride = uint32_t(pblocks) * kBlock;
+    a.vertices = vertices;
+    a.vertex_cap = vertex_cap;
+    a.vertex_stride = size_t(pjobs[0].pixels) * vertex_cap;
 
     hipDeviceProp_t prop;
     WF_TRY(hipGetDeviceProperties(&prop, device));
@@ -1170,7 +1187,7 @@ int render_wavefront(prt_renderer* r, uint32_t n) {
     RunStats rs;
     int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
                            r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, r->cfg.count_rays != 0, &rs,
-                           r->cfg.profile_kernels != 0);
+                           r->cfg.profile_kernels != 0, r->vertices, r->spp);
     if (rc != PRT_OK) return rc;
     // Fold the wavefront's counters into the renderer's.
     unsigned long long host[kCntNum];
@@ -1187,7 +1204,7 @@ int render_wavefront(prt_renderer* r, uint32_t n) {
     return PRT_OK;
 }
 
-int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples) {
+int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples, uint32_t* vertices) {
     const bool had_state = r->wf != nullptr;
     if (!r->wf) r->wf = new WavefrontState();
     WfJob j;
@@ -1205,7 +1222,8 @@ int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samp
     const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(total);
     RunStats rs;
     const int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
-                                 r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, false, &rs);
+                                 r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, false, &rs, false, vertices,
+                                 spp);
     // A megakernel renderer does not keep the queues of a one-off forward pass.
     if (!had_state && r->cfg.integrator != PRT_INTEGRATOR_WAVEFRONT) release_wavefront(r);
     return rc;

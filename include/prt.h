@@ -127,7 +127,9 @@ typedef struct prt_render_config {
                                          (0 = as many as fit) */
     uint32_t keep_samples;  /* 1 = also store each pixel-sample's radiance (16 B per pixel-sample, for
                                the first `spp` samples), so the adjoint replays paths without
-                               tracing them first */
+                               tracing them first; the wavefront also stores each path's vertices
+                               (4 B per sample and max_depth, when that fits in a quarter of the
+                               free device memory), so the replay traces no ray */
 } prt_render_config;
 
 /* Counters accumulated since the renderer was created (or reset). */
@@ -311,7 +313,7 @@ int prt_autotune(prt_job *jobs, uint32_t num_jobs, const prt_render_config *cfg,
 /* Gradients of the image loss sum_px,c (I - target)^2 / (W*H*3) with respect to every
  * material's diffuse albedo kd (RGB) and emission scale e (MTL Ka = e*(1,1,1)).
  * The adjoint replays each path with the same Philox stream as the forward render
- * (path-replay backpropagation), so nothing per path is stored.
+ * (path-replay backpropagation); of a path at most its vertices (4 B each) are kept.
  * target_rgb: host W*H*3; image_rgb: host W*H*3 mean radiance of the forward pass
  * at the same seed and spp (NULL = render it here). d_albedo: num_materials*3,
  * d_emission: num_materials (host, overwritten). loss may be NULL. */
@@ -334,11 +336,12 @@ int prt_adjoint_grad(prt_renderer *r, const float *grad_rgb, float hess, uint32_
  * the caller's device memory on the renderer's device (W*H*3 floats, dLoss/dI), the
  * per-workgroup partial gradients live in a static 16 MiB device array (2^21
  * doubles) that each GPU holds until the process ends, and it never writes a
- * per-sample radiance buffer: without radiance kept by the forward pass
+ * per-sample buffer: without radiance kept by the forward pass
  * (keep_samples) each sample's primal path is traced inside the replay. Limit:
  * ceil8(ceil(W/8) * ceil(H/8)) * 4M + 4M <= 2^21 (e.g. 1920x1080 with 16 materials);
- * larger calls fail with PRT_ERR_LIMIT. The gradients equal prt_adjoint_grad's for
- * the same inputs. Calls that overlap on one GPU (several host threads) share its
+ * larger calls fail with PRT_ERR_LIMIT. The gradients are the sums of
+ * prt_adjoint_grad's fp64 terms for the same inputs (in another order where that call
+ * keeps path vertices and this one has none). Calls that overlap on one GPU (several host threads) share its
  * array and race; serialise them. d_albedo: M*3, d_emission: M (host, overwritten). */
 int prt_adjoint_grad_static(prt_renderer *r, const float *grad_rgb_device, float hess, uint32_t spp,
                             float *d_albedo, float *d_emission);
