@@ -10,7 +10,8 @@
 //            in groups of 64 that share a pixel (or a small pixel block)
 //   extend   closest hit of every ray in the current queue (traversal only, low
 //            register pressure, persistent waves fetching 64 rays at a time; the
-//            first iteration's camera rays are traced 64 at a time as packets)
+//            first iteration's camera rays are traced 64 at a time as packets where there
+//            are enough of them)
 //   shade    shade_vertex() of every hit; survivors are compacted into the next
 //            queue and shadow rays into the shadow queue (wave ballots + one atomic
 //            per workgroup and queue); what a vertex adds goes to the path's result slot
@@ -26,6 +27,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -968,14 +970,24 @@ struct RunStats {
     uint32_t launches[3];
 };
 
+// Whether a chunk's camera rays are traced as packets. A packet visits what any of its rays
+// would, one dependent step after another, so a launch lasts at least one packet: 0.012 ms
+// over 36 triangles, 0.1 over 20,000, 0.3 over 1M, 0.65 over 2.8M, about the triangles'
+// square root (their number across an image); from there on it is faster per ray. Per-lane
+// rays take 0.09 ms and 0.065 ns each. Measured, packets against rays, in us: 1M triangles,
+// 640 x 480 x 1 329 / 148, 1920 x 1080 x 2 340 / 370, x 16 1058 / 1833; 20,000 triangles,
+// 125 x 93 x 8 179 / 53, 640 x 480 x 4 82 / 93; 2.8M triangles, 1280 x 720 x 6 720 / 576,
+// 640 x 480 x 64 1405 / 1678; 36 triangles, 64 x 64 x 1 12 / 15.
+bool use_packets(uint32_t paths, uint32_t triangles) { return double(paths) >= 4096.0 * std::sqrt(double(triangles)); }
+
 // Launches one chunk's kernels on `stream`: setup, generate, the camera rays' extension
-// (wf_extend_packet), then per iteration shade and one launch that traces its shadow rays
+// (as packets or per lane), then per iteration shade and one launch that traces its shadow rays
 // and the next iteration's extension rays, then resolve. With `ev` (4 per iteration) those
 // two are launched one after the other, and each extend / shade / shadow part is bracketed
 // by events.
 template <bool COUNT, bool ONE_SCENE>
 void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int pblocks, int gblocks, int sblocks,
-                  hipEvent_t* ev) {
+                  bool packets, hipEvent_t* ev) {
     auto mark = [&](uint32_t k) {
         if (ev) (void)hipEventRecord(ev[k], stream);
     };
@@ -986,9 +998,9 @@ void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int p
     hipLaunchKernelGGL(dev::wf_generate, dim3(gblocks), dim3(256), 0, stream, a);
     for (uint32_t it = 0; it < max_depth; ++it) {
         mark(4 * it);
-        if (it == 0)
+        if (it == 0 && packets)
             hipLaunchKernelGGL((dev::wf_extend_packet<COUNT, ONE_SCENE>), dim3(pblocks), dim3(kBlock), 0, stream, a);
-        else if (ev)
+        else if (it == 0 || ev)
             trace(it, dev::kTraceExtend);
         mark(4 * it + 1);
         hipLaunchKernelGGL(dev::wf_shade<COUNT>, dim3(sblocks), dim3(kShadeBlock), 0, stream, a, it);
@@ -1001,17 +1013,16 @@ void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int p
 }
 
 void launch_chunk_any(bool count, bool one_scene, const WfArgs& a, hipStream_t stream, uint32_t max_depth,
-                      int pblocks, int gblocks, int sblocks, hipEvent_t* ev) {
-    if (count && one_scene) launch_chunk<true, true>(a, stream, max_depth, pblocks, gblocks, sblocks, ev);
-    else if (count) launch_chunk<true, false>(a, stream, max_depth, pblocks, gblocks, sblocks, ev);
-    else if (one_scene) launch_chunk<false, true>(a, stream, max_depth, pblocks, gblocks, sblocks, ev);
-    else launch_chunk<false, false>(a, stream, max_depth, pblocks, gblocks, sblocks, ev);
+                      int pblocks, int gblocks, int sblocks, bool packets, hipEvent_t* ev) {
+    auto go = count ? one_scene ? launch_chunk<true, true> : launch_chunk<true, false>
+                    : one_scene ? launch_chunk<false, true> : launch_chunk<false, false>;
+    go(a, stream, max_depth, pblocks, gblocks, sblocks, packets, ev);
 }
 
 // Profile mode: every chunk launched directly, each extend / shade / shadow launch
 // timed with events; per-kernel device time summed into rs.
 int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t max_depth, int pblocks, int gblocks,
-                 int sblocks, bool count, bool one_scene, RunStats* rs) {
+                 int sblocks, bool packets, bool count, bool one_scene, RunStats* rs) {
     std::vector<hipEvent_t> ev(4 * max_depth, nullptr);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = PRT_OK;
@@ -1025,7 +1036,7 @@ int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t m
     for (size_t c = 0; c < nchunks && e == hipSuccess; ++c) {
         e = hipEventRecord(e0, stream);
         if (e != hipSuccess) break;
-        launch_chunk_any(count, one_scene, a, stream, max_depth, pblocks, gblocks, sblocks, ev.data());
+        launch_chunk_any(count, one_scene, a, stream, max_depth, pblocks, gblocks, sblocks, packets, ev.data());
         e = hipGetLastError();
         if (e == hipSuccess) e = hipEventRecord(e1, stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
@@ -1112,8 +1123,13 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     const int gblocks = prop.multiProcessorCount * 8;
     const int sblocks = prop.multiProcessorCount * kShadeGridWaves * 64 / kShadeBlock;
 
+    uint32_t triangles = 0;
+    for (const WfJob& j : jobs) triangles = std::max(triangles, j.sc.num_records);
+    const bool packets = use_packets(need, triangles);
+
     if (profile) {
-        rc = run_profiled(a, stream, chunks.size(), max_depth, pblocks, gblocks, sblocks, count, one_scene, rs);
+        rc = run_profiled(a, stream, chunks.size(), max_depth, pblocks, gblocks, sblocks, packets, count, one_scene,
+                          rs);
         if (rc == PRT_OK && rs) WF_TRY(copy_wait(rs->c, w.ctr + kStats, sizeof rs->c, hipMemcpyDeviceToHost, stream));
         return rc;
     }
@@ -1121,7 +1137,7 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     WF_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    launch_chunk_any(count, one_scene, a, stream, max_depth, pblocks, gblocks, sblocks, nullptr);
+    launch_chunk_any(count, one_scene, a, stream, max_depth, pblocks, gblocks, sblocks, packets, nullptr);
     hipError_t e = hipStreamEndCapture(stream, &graph);
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
     e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);

@@ -138,3 +138,21 @@ def test_every_path_order_equals_megakernel(gpu, w, h, spp, queue, group):
                      wavefront_group=group)
     assert np.array_equal(_bits(mk), _bits(wf))
     assert cm == cw
+
+
+# Camera rays as packets, which a chunk of at least 4096 sqrt(triangles) paths takes (24,576
+# over the 36 triangles here): just below and above it, batches with idle lanes at the end,
+# blocks of one and of many pixels, and packets that hold rays of two scenes.
+@pytest.mark.parametrize("w,h,spp", [(64, 64, 6), (63, 65, 6), (157, 161, 1), (53, 41, 13), (13, 11, 200)])
+def test_packets_equal_megakernel(gpu, w, h, spp):
+    scene = ca.Scene(W.cornell().mesh)
+    cam = ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, w, h)
+    mk, cm = _render(scene, cam, w, h, spp, max_depth=4)
+    wf, cw = _render(scene, cam, w, h, spp, max_depth=4, integrator=ca.INTEGRATOR_WAVEFRONT)
+    assert np.array_equal(_bits(mk), _bits(wf))
+    assert cm == cw
+    other = ca.Scene(W.cornell().mesh)
+    imgs, _ = ca.render_batch([ca.BatchJob(scene, cam, spp, 1), ca.BatchJob(other, cam, spp, 2)], max_depth=4)
+    for view, img in enumerate(imgs, 1):
+        ref, _ = _render(scene, cam, w, h, spp, max_depth=4, view_id=view)
+        assert np.array_equal(_bits(img), _bits(ref))
