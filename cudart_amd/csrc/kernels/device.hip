@@ -133,6 +133,9 @@ int ensure_spill(prt_renderer* r, uint32_t threads) {
     return PRT_OK;
 }
 
+// Resident workgroups of the megakernel per compute unit (4 waves per SIMD).
+constexpr uint32_t kMegaWaves = 16;
+
 int set_device(int device) {
     int count = 0;
     hipError_t e = hipGetDeviceCount(&count);
@@ -208,8 +211,14 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     const size_t px = size_t(w) * h;
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->accum), px * sizeof(float4)));
     HIP_TRY(hipMemsetAsync(r->accum, 0, px * sizeof(float4), r->stream));  // F9: the reference never clears it
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->counters), kCntNum * sizeof(unsigned long long)));
-    HIP_TRY(hipMemsetAsync(r->counters, 0, kCntNum * sizeof(unsigned long long), r->stream));
+    const size_t ticket_bytes = size_t(kTicketSets) * kTicketWords * sizeof(uint32_t);
+    const size_t counter_bytes = (kCntNum * sizeof(unsigned long long) + 255) / 256 * 256;
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->counters), counter_bytes + ticket_bytes));
+    HIP_TRY(hipMemsetAsync(r->counters, 0, counter_bytes + ticket_bytes, r->stream));
+    r->tickets = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(r->counters) + counter_bytes);
+    int cus = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
+    r->compute_units = uint32_t(cus);
     uint8_t lut[256];
     gamma_table(lut);
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->gamma_lut), 256));
@@ -259,21 +268,40 @@ extern "C" int prt_render_spp(prt_renderer* r, uint32_t n) {
     a.path = PathArgs{r->cfg.seed, r->cfg.view_id, r->cfg.max_depth, r->cfg.rr_start};
     a.width = r->w;
     a.height = r->h;
-    a.tiles_x = r->tiles_x;
-    a.tiles = r->tiles;
     a.accum = r->accum;
     a.samples = r->samples;
     a.samples_cap = r->samples ? r->spp : 0;
     a.counters = r->counters;
-    a.spill = r->spill;
-    a.spill_stride = r->spill_threads;
-    const uint32_t per = r->cfg.spp_per_launch ? r->cfg.spp_per_launch : 1u;
     HIP_TRY(hipEventRecord(r->ev0, r->stream));
     for (uint32_t done = 0; done < n;) {
-        uint32_t k = std::min(per, n - done);
+        uint32_t k = n - done;
+        if (r->cfg.spp_per_launch) {
+            k = std::min(k, r->cfg.spp_per_launch);
+        } else {  // the largest power of two, up to a wave's lanes
+            uint32_t p = 1;
+            while (p < 64 && 2 * p <= k) p *= 2;
+            k = p;
+        }
         a.s0 = r->samples_done + done;
         a.nspp = k;
-        HIP_TRY(launch_megakernel(a, r->cfg.count_rays != 0, r->stream));
+        a.lanes_lg = 0;
+        while (a.lanes_lg < 6 && k % (2u << a.lanes_lg) == 0) ++a.lanes_lg;
+        const uint32_t bw = 1u << block_width_lg(a.lanes_lg), bh = 1u << block_height_lg(a.lanes_lg);
+        a.tiles_x = (r->w + bw - 1) / bw;
+        a.tiles = a.tiles_x * ((r->h + bh - 1) / bh);
+        if (r->ticket_sets_used == kTicketSets) {
+            HIP_TRY(hipMemsetAsync(r->tickets, 0, size_t(kTicketSets) * kTicketWords * sizeof(uint32_t), r->stream));
+            r->ticket_sets_used = 0;
+        }
+        a.tickets = r->tickets + size_t(r->ticket_sets_used++) * kTicketWords;
+        // 8x8 blocks: a workgroup each, which the spill area has room for; else the resident ones.
+        uint32_t grid = (a.tiles + 7) / 8 * 8;
+        if (a.lanes_lg != 0) grid = std::min(grid, r->compute_units * kMegaWaves);
+        rc = ensure_spill(r, grid * kBlock);
+        if (rc != PRT_OK) return rc;
+        a.spill = r->spill;
+        a.spill_stride = r->spill_threads;
+        HIP_TRY(launch_megakernel(a, grid, r->cfg.count_rays != 0, r->stream));
         done += k;
     }
     HIP_TRY(hipEventRecord(r->ev1, r->stream));

@@ -72,7 +72,9 @@ struct MegaArgs {
     PathArgs path;
     uint32_t width, height;
     uint32_t s0, nspp;
-    uint32_t tiles_x, tiles;  // 8x8 tiles
+    uint32_t lanes_lg;        // log2 of the lanes that share a pixel, each a sample of its own; nspp is a multiple of them
+    uint32_t tiles_x, tiles;  // pixel blocks of a wave
+    uint32_t* tickets;        // one per XCD, kTicketLine words apart: blocks of its band handed out beyond the first
     float4* accum;            // width*height, .xyz = running sum
     float4* samples;          // nullptr, or each sample's radiance at [pixel * samples_cap + sample]
     uint32_t samples_cap;     // samples stored per pixel
@@ -95,11 +97,18 @@ struct FirstHitArgs {
 };
 
 // Launchers (render.hip). Return hipError_t.
-hipError_t launch_megakernel(const MegaArgs& a, bool count, hipStream_t s);
+hipError_t launch_megakernel(const MegaArgs& a, uint32_t grid, bool count, hipStream_t s);
 hipError_t launch_first_hit(const FirstHitArgs& a, hipStream_t s);
 hipError_t launch_tonemap(const float4* accum, uint32_t n, float inv_unused, uint32_t samples, const uint8_t* gamma_lut,
                           uint8_t* out, hipStream_t s);
 hipError_t launch_mean(const float4* accum, uint32_t n, uint32_t samples, float* out_rgb, hipStream_t s);
+
+// Pixel block of a wave in which 2^lg lanes share a pixel: 8x8, 8x4, 4x4, 4x2, 2x2, 2x1, 1x1.
+__host__ __device__ inline uint32_t block_width_lg(uint32_t lg) { return (7u - lg) / 2u; }
+__host__ __device__ inline uint32_t block_height_lg(uint32_t lg) { return 6u - lg - block_width_lg(lg); }
+constexpr uint32_t kTicketLine = 32;             // words between tickets: a cache line each
+constexpr uint32_t kTicketSets = 32;             // launches between two clearings
+constexpr uint32_t kTicketWords = 8 * kTicketLine;  // of one launch
 
 // Workgroup order: consecutive workgroups land on different XCDs (round robin),
 // so tile k is given to workgroup (k % per) * 8 + k / per, making each XCD's L2

@@ -1,10 +1,10 @@
 // Megakernel path tracer, primary-hit kernel and output kernels for gfx950.
 //
-// One wave64 workgroup renders one 8x8 pixel tile; each lane follows one pixel's
-// paths for `nspp` consecutive sample indices and adds them to the running sum in
-// sample order, the order SequentialRenderer::renderOneSamplePerPixel
-// (src/renderer/sequential_renderer.cu:91-116) and renderKernel
-// (src/renderer/parallel_renderer.cu:318-342) accumulate in.
+// A wave64 workgroup renders blocks of pixels, one after another. With `nspp` samples per
+// pixel in the launch, the lanes that share a pixel take a sample each, and one of them adds
+// the results to the running sum in sample order, the order
+// SequentialRenderer::renderOneSamplePerPixel (src/renderer/sequential_renderer.cu:91-116)
+// and renderKernel (src/renderer/parallel_renderer.cu:318-342) accumulate in.
 #include "path.hpp"
 
 namespace prt {
@@ -69,28 +69,100 @@ __device__ __forceinline__ void flush_counts(unsigned long long* out, const Coun
     }
 }
 
+constexpr uint32_t kNoBlock = 0xFFFFFFFFu;
+
+// The blocks of pixels, handed out to the workgroups of a launch. XCD x has a band of
+// consecutive blocks (its L2 then sees one part of the image), workgroup w starts with block
+// w / 8 of band w % 8, and the rest of a band is handed out by its ticket; a workgroup whose
+// band is done helps with the next. Where lanes share pixels the grid is the resident
+// workgroups, not the blocks, so that the traversal stacks' spill area has one entry per
+// resident thread: a workgroup per 8x8 block takes 0.8 GB at 1080p, and per one-pixel block
+// it would take 64 times that. For 8x8 blocks a workgroup each it stays: with one sample
+// per pixel a launch lasts as long as its slowest block, and the tickets made 640 x 480 x 1
+// over 36 triangles 184 -> 200 us.
+struct BlockQueue {
+    uint32_t* tickets;
+    uint32_t blocks, per, x;
+    // Blocks of band b beyond the workgroups' first ones.
+    __device__ __forceinline__ uint32_t rest(uint32_t b) const {
+        const uint32_t all = b * per < blocks ? min(per, blocks - b * per) : 0u, first = gridDim.x >> 3;
+        return all > first ? all - first : 0u;
+    }
+    __device__ __forceinline__ uint32_t start(uint32_t* t, uint32_t n) {
+        tickets = t;
+        blocks = n;
+        per = (n + 7u) / 8u;
+        x = blockIdx.x & 7u;
+        const uint32_t first = blockIdx.x >> 3;
+        return first < per && x * per + first < n ? x * per + first : kNoBlock;
+    }
+    __device__ __forceinline__ uint32_t next() {
+        if (blocks <= gridDim.x) return kNoBlock;
+        const uint32_t lane = threadIdx.x;
+        unsigned long long left = 1ull << x;
+        while (true) {
+            if (rest(x) != 0u && left != 0ull) {
+                uint32_t idx = 0u;
+                if (lane == 0) idx = atomicAdd(tickets + x * kTicketLine, 1u);
+                idx = uniform_u32(idx);
+                if (idx < rest(x)) return x * per + (gridDim.x >> 3) + idx;
+            }
+            // The band is done: one load shows the tickets of all.
+            uint32_t seen = 0u;
+            if (lane < 8u)
+                seen = __hip_atomic_load(tickets + lane * kTicketLine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            left = __ballot(lane < 8u && seen < rest(lane));
+            if (left == 0ull) return kNoBlock;
+            do x = (x + 1u) & 7u;
+            while (((left >> x) & 1ull) == 0ull);
+        }
+    }
+};
+
+// What bounds it is the slowest lane: at every bounce a wave waits for its longest ray, and a
+// launch for its longest wave. With a launch per sample and a pixel per lane, 961 x 541 x 8
+// over 1M triangles took 13.0 ms. Lanes that share a pixel start from nearly the same ray and
+// meet the same surfaces, and a launch of 8 samples has 8 times the waves: 5.8 ms; 125 x 93 x 8
+// over 97,292 triangles (192 waves before) 5.3 -> 0.82. Held at 5 and 6 waves per SIMD it
+// spills 30 / 47 registers: 5.9 / 6.0 ms.
 template <bool COUNT>
 __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
     __shared__ int s_stack[kStackLds * kBlock];
-    const uint32_t tile = xcd_tile(blockIdx.x, a.tiles);
-    if (tile >= a.tiles) return;
-    const int lane = int(threadIdx.x);
-    const int x = int(tile % a.tiles_x) * 8 + (lane & 7);
-    const int y = int(tile / a.tiles_x) * 8 + (lane >> 3);
+    __shared__ float s_rgb[3][kBlock];
+    const uint32_t lane = threadIdx.x, share = 1u << a.lanes_lg, sub = lane & (share - 1u), px = lane >> a.lanes_lg;
+    const uint32_t wlg = block_width_lg(a.lanes_lg), hlg = block_height_lg(a.lanes_lg);
+    Stack st;
+    st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
     Counts cnt = {0, 0, 0, 0, 0, 0};
-    if (x < int(a.width) && y < int(a.height)) {
-        Stack st;
-        st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
-        const size_t idx = size_t(y) * a.width + size_t(x);
-        float4 acc = a.accum[idx];
-        V3 sum = v3(acc.x, acc.y, acc.z);
-        for (uint32_t k = 0; k < a.nspp; ++k) {
-            V3 L = sample_path<COUNT>(a.sc, a.cam, a.path, x, y, a.s0 + k, st, cnt);
-            sum = sum + L;
-            if (a.samples && a.s0 + k < a.samples_cap)
-                a.samples[idx * a.samples_cap + a.s0 + k] = make_float4(L.x, L.y, L.z, 0.f);
+    BlockQueue queue;
+    for (uint32_t block = queue.start(a.tickets, a.tiles); block != kNoBlock; block = queue.next()) {
+        const uint32_t x = ((block % a.tiles_x) << wlg) + (px & ((1u << wlg) - 1u));
+        const uint32_t y = ((block / a.tiles_x) << hlg) + (px >> wlg);
+        const bool inside = x < a.width && y < a.height;
+        const size_t idx = size_t(y) * a.width + x;
+        V3 sum = v3(0.f, 0.f, 0.f);
+        if (inside && sub == 0u) sum = v3(a.accum[idx]);
+        for (uint32_t k = 0; k < a.nspp; k += share) {
+            const uint32_t sample = a.s0 + k + sub;
+            V3 L = v3(0.f, 0.f, 0.f);
+            if (inside) {
+                L = sample_path<COUNT>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
+                if (a.samples && sample < a.samples_cap)
+                    a.samples[idx * a.samples_cap + sample] = make_float4(L.x, L.y, L.z, 0.f);
+            }
+            if (share == 1u) {
+                sum = sum + L;
+                continue;
+            }
+            s_rgb[0][lane] = L.x;
+            s_rgb[1][lane] = L.y;
+            s_rgb[2][lane] = L.z;
+            __syncthreads();
+            if (sub == 0u)
+                for (uint32_t j = lane; j < lane + share; ++j) sum = sum + v3(s_rgb[0][j], s_rgb[1][j], s_rgb[2][j]);
+            __syncthreads();
         }
-        a.accum[idx] = make_float4(sum.x, sum.y, sum.z, 0.f);
+        if (inside && sub == 0u) a.accum[idx] = make_float4(sum.x, sum.y, sum.z, 0.f);
     }
     if (COUNT) flush_counts<COUNT>(a.counters, cnt);
 }
@@ -153,8 +225,7 @@ __global__ void mean_kernel(const float4* accum, uint32_t n, uint32_t samples, f
 
 }  // namespace dev
 
-hipError_t launch_megakernel(const MegaArgs& a, bool count, hipStream_t s) {
-    const uint32_t grid = ((a.tiles + 7) / 8) * 8;
+hipError_t launch_megakernel(const MegaArgs& a, uint32_t grid, bool count, hipStream_t s) {
     if (count) hipLaunchKernelGGL(dev::megakernel<true>, dim3(grid), dim3(kBlock), 0, s, a);
     else hipLaunchKernelGGL(dev::megakernel<false>, dim3(grid), dim3(kBlock), 0, s, a);
     return hipGetLastError();

@@ -22,10 +22,13 @@ struct prt_renderer {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     float4* accum = nullptr;               // w*h running sums
     unsigned long long* counters = nullptr;
+    uint32_t* tickets = nullptr;   // kTicketSets x kTicketWords, behind the counters
+    uint32_t ticket_sets_used = 0;
     uint8_t* gamma_lut = nullptr;
     int* spill = nullptr;
     uint32_t spill_threads = 0;
-    uint32_t tiles_x = 0, tiles = 0;
+    uint32_t tiles_x = 0, tiles = 0;  // 8x8 pixel tiles
+    uint32_t compute_units = 0;
     uint32_t samples_done = 0;
     uint64_t samples_total = 0;
     double last_ms = 0.0;

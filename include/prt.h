@@ -115,7 +115,7 @@ typedef struct prt_render_config {
     uint32_t view_id;       /* Philox key word 1 */
     int32_t device;         /* HIP device ordinal; the reference picks device 1 when >1 (main.cpp:160-162) */
     uint32_t integrator;    /* PRT_INTEGRATOR_* */
-    uint32_t spp_per_launch;/* megakernel: samples per pixel per launch (0 = choose) */
+    uint32_t spp_per_launch;/* megakernel: samples per pixel per launch (0 = choose: powers of two up to 64) */
     uint32_t count_rays;    /* 1 = keep per-kind ray / node / triangle counters */
     uint32_t wavefront_group;   /* wavefront: side g (1, 2, 4 or 8) of the pixel block whose
                                    64 / g^2 consecutive samples make one wave's 64 camera paths

@@ -178,3 +178,23 @@ def test_radiance_textured_terrain_matches_oracle(gpu):
     tri, mat, _ = r.first_hit(0)
     textured = [i for i, m in enumerate(wl.mesh.materials) if m.tex_kd >= 0]
     assert np.isin(mat, textured).mean() > 0.05
+
+
+# The megakernel with 1 to 64 lanes to a pixel: every pixel block shape on images that it does
+# not divide, launches of several rounds, several launches, and more launches than there are
+# ticket sets, against one sample per pixel and launch.
+@pytest.mark.parametrize("w,h,spp,per", [(1, 1, 64, 0), (37, 21, 2, 0), (37, 21, 4, 0), (37, 21, 13, 0), (21, 37, 48, 48),
+                                         (19, 23, 127, 0), (19, 23, 96, 96), (33, 17, 40, 1), (300, 200, 32, 0)])
+def test_lanes_sharing_pixels_equal_one_per_pixel(gpu, w, h, spp, per):
+    scene = ca.Scene(W.spheres1m(w, h, instances=12).mesh)
+    cam = ca.camera_look_at((4.0, 12.0, 35.0), (0.0, 8.0, 0.0), (0.0, 1.0, 0.0), 45.0, w, h)
+    imgs = []
+    for single in (True, False):
+        r = ca.ParallelRenderer(scene, w, h, spp, camera=cam, max_depth=5, seed=3, count_rays=1,
+                                spp_per_launch=1 if single else per)
+        r.render(spp)
+        st = r.stats()
+        imgs.append((r.radiance().view(np.uint32), st.primary_rays, st.extension_rays, st.shadow_rays))
+        r.close()
+    assert np.array_equal(imgs[0][0], imgs[1][0])
+    assert imgs[0][1:] == imgs[1][1:]
