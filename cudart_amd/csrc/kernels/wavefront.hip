@@ -74,7 +74,7 @@ constexpr size_t kSlotBytes = 2 * 48 + 4 + 48 + 4 + 16;
 constexpr uint32_t kCtrLine = PRT_CTR_LINE;
 enum WfCounter : uint32_t {
     kChunk = 0,                // number of the chunk being rendered, from 1
-    kStats = kCtrLine,         // kCntNum 64-bit counters (two words each)
+    kStats = kCtrLine,         // kCntNum 64-bit counters (two words each) of a batch
     kQueue = 4 * kCtrLine,     // rays of each iteration's queues: extension at kQueue + 2 * it lines, shadow after it
     kFetch = kQueue + 2 * (kMaxIter + 1) * kCtrLine,  // fetch counters: 2 * kMaxIter groups of kSpread,
                                // counter c of group g at kFetch + (g * kSpread + c) * kCtrLine
@@ -127,6 +127,7 @@ struct WfArgs {
     const WfTile* tiles;
     const WfChunk* chunks;
     uint32_t* ctr;
+    unsigned long long* stats;  // kCntNum counters that the rays are added to
     float4* qa[2];
     float4* qb[2];
     float4* qc[2];
@@ -148,6 +149,14 @@ struct WfArgs {
     uint32_t group_lg;  // log2 of the forced camera-path block side, or kNone: choose per section
 };
 
+// What a captured launch sequence was made for.
+struct LaunchKey {
+    WfArgs args;
+    uint32_t max_depth;
+    int pblocks, gblocks, sblocks;
+    bool packets, count;
+};
+
 struct WavefrontState {
     int device = -1;
     uint32_t capacity = 0;       // slots
@@ -157,11 +166,16 @@ struct WavefrontState {
     int* spill = nullptr;
     uint32_t* ctr = nullptr;
     WfArgs args{};
-    // plan buffers
-    WfJob* d_jobs = nullptr;
-    WfTile* d_tiles = nullptr;
-    WfChunk* d_chunks = nullptr;
-    size_t cap_jobs = 0, cap_tiles = 0, cap_chunks = 0;
+    // jobs, tiles and chunks of the plan, one after another
+    char* d_plan = nullptr;
+    size_t cap_plan = 0;
+    std::vector<char> h_plan;
+    // The launch sequence of a chunk. Its kernels take their arguments by value, and what
+    // those point to are this state's buffers, so it stays good while the key does:
+    // capturing and instantiating it again on every call took about 0.1 ms.
+    hipGraphExec_t exec = nullptr;
+    LaunchKey key;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 
 namespace dev {
@@ -313,9 +327,8 @@ static_assert(PRT_SHADOW_PHASE_MIN >= 0 && PRT_SHADOW_PHASE_MIN <= 64, "phase th
 // Adds the wave's counts to the counter slots; ANYHIT also books nodes and
 // triangles as the shadow (any-hit) kernel's share.
 template <bool ANYHIT>
-__device__ __forceinline__ void flush_stats(uint32_t* ctr, const Counts& c) {
+__device__ __forceinline__ void flush_stats(unsigned long long* out, const Counts& c) {
     unsigned long long v[6] = {c.primary, c.extension, c.shadow, c.nodes, c.tris, c.hits};
-    unsigned long long* out = reinterpret_cast<unsigned long long*>(ctr + kStats);
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         unsigned long long x = v[k];
@@ -502,7 +515,7 @@ __device__ __forceinline__ void extend_rays(const WfArgs& a, uint32_t it, StackT
             }
         }
     }
-    if (COUNT) flush_stats<false>(a.ctr, cnt);
+    if (COUNT) flush_stats<false>(a.stats, cnt);
 }
 
 // Occlusion test of every shadow ray of iteration `it`; a visible light sample's
@@ -573,7 +586,7 @@ __device__ __forceinline__ void shadow_rays(const WfArgs& a, uint32_t it, StackT
             }
         }
     }
-    if (COUNT) flush_stats<true>(a.ctr, cnt);
+    if (COUNT) flush_stats<true>(a.stats, cnt);
 }
 
 // The shadow rays of iteration it - 1 and the extension rays of iteration `it`, both made
@@ -660,7 +673,7 @@ __global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_extend_packet(WfArg
         base = fetch.resolve(pending);
         pending = base != kNone ? fetch.issue() : kNone;
     }
-    if (COUNT) flush_stats<false>(a.ctr, cnt);
+    if (COUNT) flush_stats<false>(a.stats, cnt);
 }
 
 // Appends to two queues for a whole workgroup with one atomic per queue: lanes
@@ -786,13 +799,12 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         }
     }
     if (COUNT) {
-        flush_stats<false>(a.ctr, cnt);
+        flush_stats<false>(a.stats, cnt);
         // Each shadow ray's own light triangle counts among the any-hit triangles.
         unsigned long long x = cnt.shadow;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-        if ((threadIdx.x & 63) == 0 && x)
-            atomicAdd(reinterpret_cast<unsigned long long*>(a.ctr + kStats) + kCntAnyTris, x);
+        if ((threadIdx.x & 63) == 0 && x) atomicAdd(a.stats + kCntAnyTris, x);
     }
 }
 
@@ -894,24 +906,15 @@ void make_plan(const std::vector<PlanJob>& jobs, uint32_t cap, std::vector<WfTil
     if (cur.ntiles) chunks.push_back(cur);
 }
 
-int persistent_blocks(const void* kernel, uint32_t blocks_per_cu, int device) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) != hipSuccess) return 1024;
+// Resident workgroups of a kernel on the whole device, and the device's compute units.
+int persistent_blocks(const void* kernel, uint32_t blocks_per_cu, int device, int* compute_units) {
+    if (hipDeviceGetAttribute(compute_units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        *compute_units = 128;
     int occ = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kBlock, 0) != hipSuccess || occ <= 0) occ = 8;
-    uint32_t per = blocks_per_cu ? blocks_per_cu : uint32_t(occ);
-    return int(std::max<uint32_t>(1, per * uint32_t(prop.multiProcessorCount)));
-}
-
-template <class T>
-int ensure_buffer(T*& p, size_t& cap, size_t n) {
-    if (cap >= n && p) return PRT_OK;
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    size_t want = std::max<size_t>(n, 16);
-    WF_TRY(hipMalloc(reinterpret_cast<void**>(&p), want * sizeof(T)));
-    cap = want;
-    return PRT_OK;
+    if (!blocks_per_cu && (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kBlock, 0) != hipSuccess || occ <= 0))
+        occ = 8;
+    const uint32_t per = blocks_per_cu ? blocks_per_cu : uint32_t(occ);
+    return int(std::max<uint32_t>(1, per * uint32_t(*compute_units)));
 }
 
 int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t persistent, hipStream_t stream) {
@@ -920,10 +923,13 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
     if (w.spill) (void)hipFree(w.spill);
     if (w.ctr) (void)hipFree(w.ctr);
     w.mem = nullptr;
+    w.bytes = 0;
+    w.capacity = 0;  // until everything is there
     w.spill = nullptr;
     w.ctr = nullptr;
-    w.bytes = kSlotBytes * size_t(capacity);
-    WF_TRY(hipMalloc(&w.mem, w.bytes));
+    const size_t bytes = kSlotBytes * size_t(capacity);
+    WF_TRY(hipMalloc(&w.mem, bytes));
+    w.bytes = bytes;
     WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
     WF_TRY(fill_wait(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
     const size_t spill_entries = size_t(kStackMax - kStackLdsQueue) * persistent;
@@ -957,9 +963,12 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
 }
 
 void free_state(WavefrontState& w) {
-    void* ptrs[] = {w.mem, w.spill, w.ctr, w.d_jobs, w.d_tiles, w.d_chunks};
+    void* ptrs[] = {w.mem, w.spill, w.ctr, w.d_plan};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (w.exec) (void)hipGraphExecDestroy(w.exec);
+    if (w.e0) (void)hipEventDestroy(w.e0);
+    if (w.e1) (void)hipEventDestroy(w.e1);
     w = WavefrontState();
 }
 
@@ -1019,6 +1028,27 @@ void launch_chunk_any(bool count, bool one_scene, const WfArgs& a, hipStream_t s
     go(a, stream, max_depth, pblocks, gblocks, sblocks, packets, ev);
 }
 
+// The captured launch sequence for `k`: the state's own when it was made for the same.
+int chunk_graph(WavefrontState& w, hipStream_t stream, const LaunchKey& k) {
+    if (w.exec && std::memcmp(&w.key, &k, sizeof k) == 0) return PRT_OK;
+    if (w.exec) (void)hipGraphExecDestroy(w.exec);
+    w.exec = nullptr;
+    hipGraph_t graph = nullptr;
+    WF_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+    launch_chunk_any(k.count, k.args.one_scene != 0, k.args, stream, k.max_depth, k.pblocks, k.gblocks, k.sblocks,
+                     k.packets, nullptr);
+    hipError_t e = hipStreamEndCapture(stream, &graph);
+    if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
+    e = hipGraphInstantiate(&w.exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) {
+        w.exec = nullptr;
+        return hip_fail(e, "hipGraphInstantiate");
+    }
+    std::memcpy(&w.key, &k, sizeof k);
+    return PRT_OK;
+}
+
 // Profile mode: every chunk launched directly, each extend / shade / shadow launch
 // timed with events; per-kernel device time summed into rs.
 int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t max_depth, int pblocks, int gblocks,
@@ -1065,11 +1095,12 @@ int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t m
 }
 
 // Renders every job of the plan on `stream`. Returns PRT_OK or an error.
-// group_side: camera-path block side g for wf_generate (1, 2, 4, 8; 0 = choose per tile).
+// group_side: camera-path block side g for wf_generate (1, 2, 4, 8; 0 = choose per section).
+// stats: device counters that the rays are added to (else rs->c receives them).
 int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::vector<WfJob>& jobs,
                   const std::vector<PlanJob>& pjobs, uint32_t max_depth, uint32_t capacity, uint32_t blocks_per_cu,
                   uint32_t group_side, bool count, RunStats* rs, bool profile = false, uint32_t* vertices = nullptr,
-                  uint32_t vertex_cap = 0) {
+                  uint32_t vertex_cap = 0, unsigned long long* stats = nullptr) {
     if (max_depth == 0 || max_depth > uint32_t(kMaxIter)) return fail(PRT_ERR_INVALID_ARG, "max_depth out of range");
     uint32_t group_lg = dev::kNone;
     if (group_side != 0) {
@@ -1094,22 +1125,33 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
                                           : reinterpret_cast<const void*>(dev::wf_trace<true, false>))
                              : (one_scene ? reinterpret_cast<const void*>(dev::wf_trace<false, true>)
                                           : reinterpret_cast<const void*>(dev::wf_trace<false, false>));
+    int cus = 0;
     // No more waves than the largest queue has batches.
-    const int pblocks = std::min(persistent_blocks(ktrace, blocks_per_cu, device), int((need + kBatch - 1) / kBatch));
+    const int pblocks = std::min(persistent_blocks(ktrace, blocks_per_cu, device, &cus), int((need + kBatch - 1) / kBatch));
     int rc = ensure_state(w, device, need, uint32_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;
-    rc = ensure_buffer(w.d_jobs, w.cap_jobs, jobs.size());
-    if (rc == PRT_OK) rc = ensure_buffer(w.d_tiles, w.cap_tiles, tiles.size());
-    if (rc == PRT_OK) rc = ensure_buffer(w.d_chunks, w.cap_chunks, chunks.size());
-    if (rc != PRT_OK) return rc;
-    WF_TRY(hipMemcpyAsync(w.d_jobs, jobs.data(), jobs.size() * sizeof(WfJob), hipMemcpyHostToDevice, stream));
-    WF_TRY(hipMemcpyAsync(w.d_tiles, tiles.data(), tiles.size() * sizeof(WfTile), hipMemcpyHostToDevice, stream));
-    WF_TRY(hipMemcpyAsync(w.d_chunks, chunks.data(), chunks.size() * sizeof(WfChunk), hipMemcpyHostToDevice, stream));
-    WF_TRY(hipMemsetAsync(w.ctr, 0, kFetch * sizeof(uint32_t), stream));  // wf_setup clears the rest
+    // The plan in one upload. (Every part is a multiple of 16 bytes.)
+    const size_t at_tiles = jobs.size() * sizeof(WfJob), at_chunks = at_tiles + tiles.size() * sizeof(WfTile);
+    const size_t plan_bytes = at_chunks + chunks.size() * sizeof(WfChunk);
+    static_assert(sizeof(WfJob) % 8 == 0 && sizeof(WfTile) % 16 == 0 && sizeof(WfChunk) % 16 == 0, "plan alignment");
+    w.h_plan.resize(plan_bytes);
+    std::memcpy(w.h_plan.data(), jobs.data(), at_tiles);
+    std::memcpy(w.h_plan.data() + at_tiles, tiles.data(), at_chunks - at_tiles);
+    std::memcpy(w.h_plan.data() + at_chunks, chunks.data(), plan_bytes - at_chunks);
+    if (w.cap_plan < plan_bytes) {
+        if (w.d_plan) (void)hipFree(w.d_plan);
+        w.d_plan = nullptr;
+        w.cap_plan = 0;
+        WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.d_plan), std::max<size_t>(plan_bytes, 4096)));
+        w.cap_plan = std::max<size_t>(plan_bytes, 4096);
+    }
+    WF_TRY(hipMemcpyAsync(w.d_plan, w.h_plan.data(), plan_bytes, hipMemcpyHostToDevice, stream));
+    WF_TRY(hipMemsetAsync(w.ctr, 0, kQueue * sizeof(uint32_t), stream));  // wf_setup clears the rest
     WfArgs a = w.args;
-    a.jobs = w.d_jobs;
-    a.tiles = w.d_tiles;
-    a.chunks = w.d_chunks;
+    a.jobs = reinterpret_cast<const WfJob*>(w.d_plan);
+    a.tiles = reinterpret_cast<const WfTile*>(w.d_plan + at_tiles);
+    a.chunks = reinterpret_cast<const WfChunk*>(w.d_plan + at_chunks);
+    a.stats = stats ? stats : reinterpret_cast<unsigned long long*>(w.ctr + kStats);
     a.max_depth = max_depth;
     a.group_lg = group_lg;
     a.one_scene = one_scene ? 1u : 0u;
@@ -1118,46 +1160,44 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     a.vertex_cap = vertex_cap;
     a.vertex_stride = size_t(pjobs[0].pixels) * vertex_cap;
 
-    hipDeviceProp_t prop;
-    WF_TRY(hipGetDeviceProperties(&prop, device));
-    const int gblocks = prop.multiProcessorCount * 8;
-    const int sblocks = prop.multiProcessorCount * kShadeGridWaves * 64 / kShadeBlock;
+    const int gblocks = cus * 8;
+    const int sblocks = cus * kShadeGridWaves * 64 / kShadeBlock;
 
     uint32_t triangles = 0;
     for (const WfJob& j : jobs) triangles = std::max(triangles, j.sc.num_records);
     const bool packets = use_packets(need, triangles);
 
+    // The counters of a run that adds them to its own (a batch); a run that counts nothing
+    // leaves them 0.
+    auto read_stats = [&]() -> int {
+        std::memset(rs->c, 0, sizeof rs->c);
+        if (count && !stats) WF_TRY(copy_wait(rs->c, a.stats, sizeof rs->c, hipMemcpyDeviceToHost, stream));
+        return PRT_OK;
+    };
     if (profile) {
         rc = run_profiled(a, stream, chunks.size(), max_depth, pblocks, gblocks, sblocks, packets, count, one_scene,
                           rs);
-        if (rc == PRT_OK && rs) WF_TRY(copy_wait(rs->c, w.ctr + kStats, sizeof rs->c, hipMemcpyDeviceToHost, stream));
-        return rc;
+        return rc == PRT_OK && rs ? read_stats() : rc;
     }
-    // Capture one chunk's launch sequence.
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    WF_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    launch_chunk_any(count, one_scene, a, stream, max_depth, pblocks, gblocks, sblocks, packets, nullptr);
-    hipError_t e = hipStreamEndCapture(stream, &graph);
-    if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture");
-    e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(graph);
-        return hip_fail(e, "hipGraphInstantiate");
-    }
-    hipEvent_t e0, e1;
-    (void)hipEventCreate(&e0);
-    (void)hipEventCreate(&e1);
-    (void)hipEventRecord(e0, stream);
-    for (size_t c = 0; c < chunks.size() && e == hipSuccess; ++c) e = hipGraphLaunch(exec, stream);
-    (void)hipEventRecord(e1, stream);
-    if (e == hipSuccess) e = hipEventSynchronize(e1);
+    LaunchKey key;
+    std::memset(&key, 0, sizeof key);  // padding too: keys are compared as bytes
+    std::memcpy(&key.args, &a, sizeof a);
+    key.max_depth = max_depth;
+    key.pblocks = pblocks;
+    key.gblocks = gblocks;
+    key.sblocks = sblocks;
+    key.packets = packets;
+    key.count = count;
+    rc = chunk_graph(w, stream, key);
+    if (rc != PRT_OK) return rc;
+    if (!w.e0) WF_TRY(hipEventCreate(&w.e0));
+    if (!w.e1) WF_TRY(hipEventCreate(&w.e1));
+    hipError_t e = hipEventRecord(w.e0, stream);
+    for (size_t c = 0; c < chunks.size() && e == hipSuccess; ++c) e = hipGraphLaunch(w.exec, stream);
+    if (e == hipSuccess) e = hipEventRecord(w.e1, stream);
+    if (e == hipSuccess) e = hipEventSynchronize(w.e1);
     float ms = 0.f;
-    if (e == hipSuccess) (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms, w.e0, w.e1);
     if (e != hipSuccess) return hip_fail(e, "wavefront launch");
     if (rs) {
         rs->ms = ms;
@@ -1165,22 +1205,24 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
             rs->kernel_ms[k] = 0.0;
             rs->launches[k] = 0;
         }
-        WF_TRY(copy_wait(rs->c, w.ctr + kStats, sizeof rs->c, hipMemcpyDeviceToHost, stream));
+        return read_stats();
     }
     return PRT_OK;
 }
 
 // The most path slots worth holding: a quarter of the device's free memory (an
 // MI355X's 288 GB holds a whole 1080p x 128-spp frame, 265M paths, in one chunk),
-// at most 2^28. Fewer, larger chunks leave fewer nearly empty late iterations.
-uint64_t max_slots() {
+// at most 2^28. Fewer, larger chunks leave fewer nearly empty late iterations. What the
+// state already holds counts as free.
+uint64_t max_slots(const WavefrontState& w) {
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = size_t(8) << 30;
-    return std::max<uint64_t>(1u << 20, std::min<uint64_t>(1ull << 28, free_b / 4 / kSlotBytes));
+    return std::max<uint64_t>(1u << 20, std::min<uint64_t>(1ull << 28, (free_b + w.bytes) / 4 / kSlotBytes));
 }
 
-uint32_t default_capacity(uint64_t total_paths) {
-    return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(max_slots(), total_paths)));
+uint32_t default_capacity(const WavefrontState& w, uint64_t total_paths) {
+    if (w.mem && w.capacity >= total_paths && total_paths > 0) return uint32_t(total_paths);
+    return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(max_slots(w), total_paths)));
 }
 
 }  // namespace
@@ -1199,17 +1241,12 @@ int render_wavefront(prt_renderer* r, uint32_t n) {
     std::vector<WfJob> jobs = {j};
     std::vector<PlanJob> pj = {PlanJob{r->w * r->h, r->samples_done, r->samples_done + n}};
     const uint64_t total = uint64_t(r->w) * r->h * n;
-    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(total);
+    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*r->wf, total);
     RunStats rs;
     int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
                            r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, r->cfg.count_rays != 0, &rs,
-                           r->cfg.profile_kernels != 0, r->vertices, r->spp);
+                           r->cfg.profile_kernels != 0, r->vertices, r->spp, r->counters);
     if (rc != PRT_OK) return rc;
-    // Fold the wavefront's counters into the renderer's.
-    unsigned long long host[kCntNum];
-    WF_TRY(copy_wait(host, r->counters, sizeof host, hipMemcpyDeviceToHost, r->stream));
-    for (int k = 0; k < kCntNum; ++k) host[k] += rs.c[k];
-    WF_TRY(copy_wait(r->counters, host, sizeof host, hipMemcpyHostToDevice, r->stream));
     r->last_ms = rs.ms;
     for (int k = 0; k < 3; ++k) {
         r->kernel_ms[k] = rs.kernel_ms[k];
@@ -1235,7 +1272,7 @@ int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samp
     std::vector<WfJob> jobs = {j};
     std::vector<PlanJob> pj = {PlanJob{r->w * r->h, 0, spp}};
     const uint64_t total = uint64_t(r->w) * r->h * spp;
-    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(total);
+    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*r->wf, total);
     RunStats rs;
     const int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
                                  r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, false, &rs, false, vertices,
@@ -1329,7 +1366,7 @@ extern "C" int prt_render_batch(prt_job* jobs, uint32_t n, const prt_render_conf
         return rc;
     }
     WavefrontState w;
-    const uint32_t cap = tune && tune->queue_slots ? tune->queue_slots : default_capacity(b.total);
+    const uint32_t cap = tune && tune->queue_slots ? tune->queue_slots : default_capacity(w, b.total);
     RunStats rs;
     rc = run_wavefront(w, c.device, s, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
                        tune ? tune->group_side : c.wavefront_group, c.count_rays != 0, &rs);
@@ -1407,7 +1444,7 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
     // 28. Chunk counts: the fewest that fit the path slots (larger chunks were faster
     // at every size measured on one view, since every chunk ends in nearly empty
     // iterations), and twice and four times as many.
-    const uint64_t limit = max_slots();
+    const uint64_t limit = max_slots(w);
     const uint32_t full_cap = uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(full, limit)));
     // The trial's path slots for a full-run chunk size: the trial is cut into as many
     // chunks as the full run would take, so its queues drain like the full run's.

@@ -156,3 +156,24 @@ def test_packets_equal_megakernel(gpu, w, h, spp):
     for view, img in enumerate(imgs, 1):
         ref, _ = _render(scene, cam, w, h, spp, max_depth=4, view_id=view)
         assert np.array_equal(_bits(img), _bits(ref))
+
+
+# A renderer keeps the captured launch sequence of its last call: the same call again, larger
+# and smaller ones, changed materials and counters in between, each against a new renderer.
+def test_repeated_calls_equal_first_calls(gpu):
+    w, h = 72, 40
+    scene = ca.Scene(W.cornell().mesh)
+    cam = ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, w, h)
+    kw = dict(max_depth=5, integrator=ca.INTEGRATOR_WAVEFRONT)
+    kept = ca.ParallelRenderer(scene, w, h, 8, camera=cam, count_rays=1, **kw)
+    for step, spp in enumerate((4, 4, 1, 12, 4, 4, 300, 4)):
+        if step == 5:
+            scene.set_material_params(1, (0.2, 0.3, 0.4), 0.0)
+        kept.reset()
+        kept.reset_stats()
+        kept.render(spp)
+        img, st = kept.radiance(), kept.stats()
+        ref, cnt = _render(scene, cam, w, h, spp, **kw)
+        assert np.array_equal(_bits(img), _bits(ref)), (step, spp)
+        assert (st.primary_rays, st.extension_rays, st.shadow_rays) == cnt
+        kept.copyImageBytes()
