@@ -23,6 +23,7 @@ struct DeviceScene {
     void* texinfo = nullptr;
     void* lin = nullptr;
     uint64_t mats_version = 0;
+    bool counted = false;  // scene_uploaded() was called for it
 };
 
 void release_device_scene(DeviceScene& d);  // device.hip

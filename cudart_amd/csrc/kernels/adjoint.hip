@@ -682,44 +682,50 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     const uint32_t M = r->scene->num_materials;
     const uint32_t P = 4 * M;
     const uint32_t grid = ((r->tiles * adjoint_parts(r, spp) + 7) / 8) * 8;
-    float* d_grad = nullptr;
-    double* d_part = nullptr;
-    double* d_out = nullptr;
-    float4* d_samp = nullptr;  // this call's per-sample radiance, when none was kept
-    float4* d_acc = nullptr;
-    uint32_t* d_vert = nullptr;
-    std::vector<double> g(P);
+    // One block of the renderer's: gradient image, partials, results, and what a forward pass of
+    // this call keeps. It stays with the renderer unless it is large (at the end).
+    auto part = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t b_grad = part(px * 3 * sizeof(float)), b_part = part(size_t(grid) * P * sizeof(double));
+    const size_t b_out = part(P * sizeof(double)), b_acc = part(px * sizeof(float4));
+    const size_t b_samp = part(px * spp * sizeof(float4)), b_vert = part(px * spp * r->cfg.max_depth * sizeof(uint32_t));
+    std::vector<double> g;
+    try {
+        g.resize(P);
+    } catch (const std::bad_alloc&) {
+        return fail(PRT_ERR_OUT_OF_MEMORY, "host allocation failed");
+    }
     float ms = 0.f;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    AdjArgs a;
-    ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_grad), px * 3 * sizeof(float)));
-    ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_part), size_t(grid) * P * sizeof(double)));
-    ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_out), P * sizeof(double)));
-    ADJ_TRY(copy_wait(d_grad, grad_rgb, px * 3 * sizeof(float), hipMemcpyHostToDevice, r->stream));
-    a = adjoint_args(r, d_grad, hess, spp, d_part);
+    AdjArgs a = adjoint_args(r, nullptr, hess, spp, nullptr);
     // Without kept vertices, a wavefront forward pass first writes each sample's radiance and
     // path vertices to buffers of this call (when they fit in a quarter of the free memory),
     // and the replay traces no ray. Where only the radiance fits it traces the path's rays
     // again, and where that does not fit either each lane traces its sample's primal path
     // before replaying it. Radiance and vertices are the same either way.
+    bool forward = false, keep_vertices = false;
     if (!a.vertices && !primal_in_replay()) {
         size_t free_b = 0, total_b = 0;
-        const size_t radiance = px * (size_t(spp) + 1) * sizeof(float4);
-        const size_t vert = px * spp * r->cfg.max_depth * sizeof(uint32_t);
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
-            const bool with = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && radiance + vert <= free_b / 4;
-            if (with || (!a.samples && radiance <= free_b / 4)) {
-                ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_samp), px * spp * sizeof(float4)));
-                ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_acc), px * sizeof(float4)));
-                ADJ_TRY(hipMemsetAsync(d_acc, 0, px * sizeof(float4), r->stream));
-            }
-            if (with) ADJ_TRY(hipMalloc(reinterpret_cast<void**>(&d_vert), vert));
+            free_b += r->adjoint_bytes;
+            keep_vertices = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && b_acc + b_samp + b_vert <= free_b / 4;
+            forward = keep_vertices || (!a.samples && b_acc + b_samp <= free_b / 4);
         }
     }
-    ADJ_TRY(hipEventCreate(&e0));
-    ADJ_TRY(hipEventCreate(&e1));
-    ADJ_TRY(hipEventRecord(e0, r->stream));
-    if (d_samp) {
+    const size_t bytes = b_grad + b_part + b_out + (forward ? b_acc + b_samp : 0) + (keep_vertices ? b_vert : 0);
+    rc = scratch_for(r->adjoint, r->adjoint_bytes, bytes);
+    if (rc != PRT_OK) return rc;
+    char* at = static_cast<char*>(r->adjoint);
+    float* d_grad = reinterpret_cast<float*>(at);
+    double* d_part = reinterpret_cast<double*>(at += b_grad);
+    double* d_out = reinterpret_cast<double*>(at += b_part);
+    float4* d_acc = reinterpret_cast<float4*>(at += b_out);
+    float4* d_samp = reinterpret_cast<float4*>(at += b_acc);
+    uint32_t* d_vert = keep_vertices ? reinterpret_cast<uint32_t*>(at += b_samp) : nullptr;
+    a.grad = d_grad;
+    a.partial = d_part;
+    ADJ_TRY(hipMemcpyAsync(d_grad, grad_rgb, px * 3 * sizeof(float), hipMemcpyHostToDevice, r->stream));
+    ADJ_TRY(hipEventRecord(r->ev0, r->stream));
+    if (forward) {
+        ADJ_TRY(hipMemsetAsync(d_acc, 0, px * sizeof(float4), r->stream));
         rc = wavefront_samples(r, spp, d_acc, d_samp, d_vert);
         if (rc != PRT_OK) goto done;
         a.samples = d_samp;
@@ -729,19 +735,23 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     ADJ_TRY(launch_adjoint(a, grid, r->stream));
     hipLaunchKernelGGL(dev::adjoint_reduce, dim3(P), dim3(dev::kReduceBlock), 0, r->stream, d_part, grid, P, d_out);
     ADJ_TRY(hipGetLastError());
-    ADJ_TRY(hipEventRecord(e1, r->stream));
-    ADJ_TRY(hipEventSynchronize(e1));
-    ADJ_TRY(hipEventElapsedTime(&ms, e0, e1));
+    ADJ_TRY(hipEventRecord(r->ev1, r->stream));
     ADJ_TRY(copy_wait(g.data(), d_out, P * sizeof(double), hipMemcpyDeviceToHost, r->stream));
+    ADJ_TRY(hipEventElapsedTime(&ms, r->ev0, r->ev1));
     for (uint32_t k = 0; k < 3 * M; ++k) d_albedo[k] = float(g[k]);
     for (uint32_t k = 0; k < M; ++k) d_emission[k] = float(g[3 * M + k]);
     r->last_ms = ms;
 done:
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    void* ptrs[] = {d_grad, d_part, d_out, d_samp, d_acc, d_vert};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
+    if (rc != PRT_OK) (void)hipStreamSynchronize(r->stream);
+    {
+        size_t free_b = 0, total_b = 0;
+        if (r->adjoint_bytes > (size_t(64) << 20) &&
+            (hipMemGetInfo(&free_b, &total_b) != hipSuccess || r->adjoint_bytes > total_b / 16)) {
+            (void)hipFree(r->adjoint);
+            r->adjoint = nullptr;
+            r->adjoint_bytes = 0;
+        }
+    }
     return rc;
 }
 
@@ -785,9 +795,8 @@ extern "C" int prt_adjoint_grad_static(prt_renderer* r, const float* grad_rgb_de
                        static_cast<const double*>(base), grid, P, d_out);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipEventRecord(r->ev1, r->stream));
-    HIP_CHECK(hipEventSynchronize(r->ev1));
-    HIP_CHECK(hipEventElapsedTime(&ms, r->ev0, r->ev1));
     HIP_CHECK(copy_wait(g, d_out, P * sizeof(double), hipMemcpyDeviceToHost, r->stream));
+    HIP_CHECK(hipEventElapsedTime(&ms, r->ev0, r->ev1));
     for (uint32_t k = 0; k < 3 * M; ++k) d_albedo[k] = float(g[k]);
     for (uint32_t k = 0; k < M; ++k) d_emission[k] = float(g[3 * M + k]);
     r->last_ms = ms;

@@ -28,12 +28,14 @@ int hip_fail(hipError_t e, const char* what) {
 
 void release_device_scene(DeviceScene& d) {
     if (d.device < 0) return;
+    const bool counted = d.counted;
     int prev = 0;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(d.device);
     void* ptrs[] = {d.nodes, d.tris, d.shade, d.mats, d.lights, d.texels, d.texinfo, d.lin};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (counted) scene_released();
     (void)hipSetDevice(prev);
     d = DeviceScene();
 }
@@ -42,7 +44,7 @@ namespace {
 template <class T>
 hipError_t upload(void** dst, const std::vector<T>& v, hipStream_t stream) {
     size_t bytes = std::max<size_t>(v.size() * sizeof(T), 16);
-    hipError_t e = hipMalloc(dst, bytes);
+    hipError_t e = device_alloc(dst, bytes);
     if (e != hipSuccess) return e;
     if (!v.empty()) e = copy_wait(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, stream);
     return e;
@@ -67,7 +69,7 @@ int device_scene(prt_scene* s, int device, SceneArgs& out, hipStream_t stream) {
         if (e == hipSuccess) e = upload(&n.lights, s->lights, stream);
         if (e == hipSuccess) e = upload(&n.texels, s->texels, stream);
         if (e == hipSuccess) e = upload(&n.texinfo, s->texinfo, stream);
-        if (e == hipSuccess) e = hipMalloc(&n.lin, 256 * sizeof(float));
+        if (e == hipSuccess) e = device_alloc(&n.lin, 256 * sizeof(float));
         if (e == hipSuccess) e = copy_wait(n.lin, s->lin, 256 * sizeof(float), hipMemcpyHostToDevice, stream);
         n.mats_version = s->mats_version;
         if (e != hipSuccess) {
@@ -75,6 +77,8 @@ int device_scene(prt_scene* s, int device, SceneArgs& out, hipStream_t stream) {
             return hip_fail(e, "uploading scene");
         }
         s->devices.push_back(n);
+        s->devices.back().counted = true;
+        scene_uploaded();
         d = &s->devices.back();
     } else if (d->mats_version != s->mats_version) {
         HIP_TRY(copy_wait(d->mats, s->mats.data(), s->mats.size() * sizeof(float), hipMemcpyHostToDevice, stream));
@@ -128,8 +132,19 @@ int ensure_spill(prt_renderer* r, uint32_t threads) {
     if (r->spill && r->spill_threads >= threads) return PRT_OK;
     if (r->spill) (void)hipFree(r->spill);
     r->spill = nullptr;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->spill), bytes));
+    r->spill_threads = 0;
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), bytes));
     r->spill_threads = threads;
+    return PRT_OK;
+}
+
+int scratch_for(void*& p, size_t& have, size_t bytes) {
+    if (have >= bytes) return PRT_OK;
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    have = 0;
+    HIP_TRY(device_alloc(&p, bytes));
+    have = bytes;
     return PRT_OK;
 }
 
@@ -209,7 +224,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     HIP_TRY(hipEventCreate(&r->ev0));
     HIP_TRY(hipEventCreate(&r->ev1));
     const size_t px = size_t(w) * h;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->accum), px * sizeof(float4)));
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->accum), px * sizeof(float4)));
     HIP_TRY(hipMemsetAsync(r->accum, 0, px * sizeof(float4), r->stream));  // F9: the reference never clears it
     const size_t ticket_bytes = size_t(kTicketSets) * kTicketWords * sizeof(uint32_t);
     const size_t counter_bytes = (kCntNum * sizeof(unsigned long long) + 255) / 256 * 256;
@@ -224,7 +239,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->gamma_lut), 256));
     HIP_TRY(copy_wait(r->gamma_lut, lut, 256, hipMemcpyHostToDevice, r->stream));
     if (c.keep_samples && spp > 0)
-        HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->samples), px * spp * sizeof(float4)));
+        HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->samples), px * spp * sizeof(float4)));
     if (r->samples && c.integrator == PRT_INTEGRATOR_WAVEFRONT && vertices_fit(w, h, spp, c.max_depth)) {
         // Only where there is room for them (without, the adjoint traces the paths again).
         size_t free_b = 0, total_b = 0;
@@ -326,17 +341,17 @@ extern "C" int prt_renderer_reset(prt_renderer* r) {
     if (!r) return fail(PRT_ERR_INVALID_ARG, "null argument");
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
+    // Every other use of the accumulators is on this stream too.
     HIP_TRY(hipMemsetAsync(r->accum, 0, size_t(r->w) * r->h * sizeof(float4), r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
     r->samples_done = 0;
     r->samples_ok = false;
     return PRT_OK;
 }
 
+// Launches the mean of the samples so far into dst_device.
 static int mean_to(prt_renderer* r, float* dst_device) {
     if (r->samples_done == 0) return fail(PRT_ERR_INVALID_ARG, "no samples rendered yet");
     HIP_TRY(launch_mean(r->accum, r->w * r->h, r->samples_done, dst_device, r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
     return PRT_OK;
 }
 
@@ -346,15 +361,12 @@ extern "C" int prt_get_radiance(prt_renderer* r, float* rgb) {
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     const size_t bytes = size_t(r->w) * r->h * 3 * sizeof(float);
-    float* tmp = nullptr;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&tmp), bytes));
-    rc = mean_to(r, tmp);
-    if (rc == PRT_OK) {
-        hipError_t e = copy_wait(rgb, tmp, bytes, hipMemcpyDeviceToHost, r->stream);
-        if (e != hipSuccess) rc = hip_fail(e, "copying radiance");
-    }
-    (void)hipFree(tmp);
-    return rc;
+    rc = scratch_for(r->out, r->out_bytes, bytes);
+    if (rc == PRT_OK) rc = mean_to(r, static_cast<float*>(r->out));
+    if (rc != PRT_OK) return rc;
+    const CopyOut c{rgb, r->out, bytes};
+    HIP_TRY(copy_out(&c, 1, r->cfg.device, r->stream));
+    return PRT_OK;
 }
 
 extern "C" int prt_get_radiance_device(prt_renderer* r, void* device_rgb) {
@@ -362,7 +374,10 @@ extern "C" int prt_get_radiance_device(prt_renderer* r, void* device_rgb) {
     if (!r || !device_rgb) return fail(PRT_ERR_INVALID_ARG, "null argument");
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
-    return mean_to(r, static_cast<float*>(device_rgb));
+    rc = mean_to(r, static_cast<float*>(device_rgb));
+    if (rc != PRT_OK) return rc;
+    HIP_TRY(hipStreamSynchronize(r->stream));
+    return PRT_OK;
 }
 
 extern "C" int prt_copy_image_bytes(prt_renderer* r, uint8_t* rgba) {
@@ -372,13 +387,12 @@ extern "C" int prt_copy_image_bytes(prt_renderer* r, uint8_t* rgba) {
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     const size_t n = size_t(r->w) * r->h;
-    uint8_t* tmp = nullptr;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&tmp), n * 4));
-    hipError_t e = launch_tonemap(r->accum, uint32_t(n), 0.f, r->samples_done, r->gamma_lut, tmp, r->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-    if (e == hipSuccess) e = copy_wait(rgba, tmp, n * 4, hipMemcpyDeviceToHost, r->stream);
-    (void)hipFree(tmp);
-    if (e != hipSuccess) return hip_fail(e, "tonemap");
+    rc = scratch_for(r->out, r->out_bytes, n * 4);
+    if (rc != PRT_OK) return rc;
+    HIP_TRY(launch_tonemap(r->accum, uint32_t(n), 0.f, r->samples_done, r->gamma_lut, static_cast<uint8_t*>(r->out),
+                           r->stream));
+    const CopyOut c{rgba, r->out, n * 4};
+    HIP_TRY(copy_out(&c, 1, r->cfg.device, r->stream));
     return PRT_OK;
 }
 
@@ -388,8 +402,9 @@ extern "C" int prt_first_hit(prt_renderer* r, uint32_t sample, int32_t* tri, int
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     const size_t n = size_t(r->w) * r->h;
-    char* buf = nullptr;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&buf), n * 12));
+    rc = scratch_for(r->out, r->out_bytes, n * 12);
+    if (rc != PRT_OK) return rc;
+    char* buf = static_cast<char*>(r->out);
     FirstHitArgs a;
     a.sc = r->sc;
     a.cam = cam_args(r->cam);
@@ -404,13 +419,13 @@ extern "C" int prt_first_hit(prt_renderer* r, uint32_t sample, int32_t* tri, int
     a.t = reinterpret_cast<float*>(buf + n * 8);
     a.spill = r->spill;
     a.spill_stride = r->spill_threads;
-    hipError_t e = launch_first_hit(a, r->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-    if (e == hipSuccess && tri) e = copy_wait(tri, a.tri, n * 4, hipMemcpyDeviceToHost, r->stream);
-    if (e == hipSuccess && mat) e = copy_wait(mat, a.mat, n * 4, hipMemcpyDeviceToHost, r->stream);
-    if (e == hipSuccess && t) e = copy_wait(t, a.t, n * 4, hipMemcpyDeviceToHost, r->stream);
-    (void)hipFree(buf);
-    if (e != hipSuccess) return hip_fail(e, "first hit");
+    HIP_TRY(launch_first_hit(a, r->stream));
+    CopyOut c[3];
+    size_t parts = 0;
+    if (tri) c[parts++] = CopyOut{tri, a.tri, n * 4};
+    if (mat) c[parts++] = CopyOut{mat, a.mat, n * 4};
+    if (t) c[parts++] = CopyOut{t, a.t, n * 4};
+    HIP_TRY(copy_out(c, parts, r->cfg.device, r->stream));
     return PRT_OK;
 }
 
@@ -453,7 +468,7 @@ extern "C" int prt_renderer_destroy(prt_renderer* r) {
     (void)hipSetDevice(r->cfg.device);
     release_wavefront(r);
     if (r->stream) (void)hipStreamSynchronize(r->stream);
-    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices};
+    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices, r->out, r->adjoint};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (r->ev0) (void)hipEventDestroy(r->ev0);

@@ -42,6 +42,12 @@ struct prt_renderer {
     float4* samples = nullptr;
     uint32_t* vertices = nullptr;
     bool samples_ok = false;
+    // Device memory of the calls that hand results out, kept until the renderer goes (at most
+    // 12 bytes per pixel), and of the adjoint (scratch_for).
+    void* out = nullptr;
+    size_t out_bytes = 0;
+    void* adjoint = nullptr;
+    size_t adjoint_bytes = 0;
     uint64_t samples_version = 0;
 };
 
@@ -59,6 +65,23 @@ inline hipError_t fill_wait(void* dst, int value, size_t bytes, hipStream_t s) {
     hipError_t e = hipMemsetAsync(dst, value, bytes, s);
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
+// buffers.hip.
+// hipMalloc, after idle memory has been given back if there is no room.
+hipError_t device_alloc(void** p, size_t bytes);
+// Device memory to the caller's host buffers, ordered on `stream` and waited for.
+struct CopyOut {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+hipError_t copy_out(const CopyOut* c, size_t n, int device, hipStream_t stream);
+// While a scene is on a device, idle memory is kept for the next call.
+void scene_uploaded();
+void scene_released();
+bool scenes_on_devices();
+void release_idle_queues();  // wavefront.hip
+// At least `bytes` of the renderer's scratch memory p (of `have` bytes), grown as needed.
+int scratch_for(void*& p, size_t& have, size_t bytes);
 // Uploads the scene to `device` on first use (copies ordered on `stream`).
 int device_scene(prt_scene* s, int device, SceneArgs& out, hipStream_t stream);
 CamArgs cam_args(const prt_camera& c);

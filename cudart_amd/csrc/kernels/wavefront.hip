@@ -30,6 +30,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -928,12 +929,12 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
     w.spill = nullptr;
     w.ctr = nullptr;
     const size_t bytes = kSlotBytes * size_t(capacity);
-    WF_TRY(hipMalloc(&w.mem, bytes));
+    WF_TRY(device_alloc(&w.mem, bytes));
     w.bytes = bytes;
-    WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
+    WF_TRY(device_alloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
     WF_TRY(fill_wait(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
     const size_t spill_entries = size_t(kStackMax - kStackLdsQueue) * persistent;
-    WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.spill), spill_entries * sizeof(int)));
+    WF_TRY(device_alloc(reinterpret_cast<void**>(&w.spill), spill_entries * sizeof(int)));
     char* p = static_cast<char*>(w.mem);
     auto take = [&](size_t bytes) {
         void* r = p;
@@ -1142,7 +1143,7 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
         if (w.d_plan) (void)hipFree(w.d_plan);
         w.d_plan = nullptr;
         w.cap_plan = 0;
-        WF_TRY(hipMalloc(reinterpret_cast<void**>(&w.d_plan), std::max<size_t>(plan_bytes, 4096)));
+        WF_TRY(device_alloc(reinterpret_cast<void**>(&w.d_plan), std::max<size_t>(plan_bytes, 4096)));
         w.cap_plan = std::max<size_t>(plan_bytes, 4096);
     }
     WF_TRY(hipMemcpyAsync(w.d_plan, w.h_plan.data(), plan_bytes, hipMemcpyHostToDevice, stream));
@@ -1225,9 +1226,88 @@ uint32_t default_capacity(const WavefrontState& w, uint64_t total_paths) {
     return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(max_slots(w), total_paths)));
 }
 
+// What a call without a renderer needs: queues, its views' accumulators and images, a
+// stream. One call uses it at a time, and waits for its stream before it gives it back.
+struct CallSpace {
+    int device = -1;
+    WavefrontState w;
+    void* accum = nullptr;
+    size_t accum_bytes = 0;
+    void* rgb = nullptr;
+    size_t rgb_bytes = 0;
+    hipStream_t stream = nullptr;
+    size_t bytes() const { return w.bytes + accum_bytes + rgb_bytes; }
+};
+
+void free_space(CallSpace* c) {
+    int prev = 0;
+    (void)hipGetDevice(&prev);
+    (void)hipSetDevice(c->device);
+    free_state(c->w);
+    if (c->accum) (void)hipFree(c->accum);
+    if (c->rgb) (void)hipFree(c->rgb);
+    if (c->stream) (void)hipStreamDestroy(c->stream);
+    (void)hipSetDevice(prev);
+    delete c;
+}
+
+std::mutex g_space_mutex;
+constexpr int kSpaceDevices = 64;
+CallSpace* g_idle_space[kSpaceDevices] = {};  // one per device (none kept beyond these)
+
+// Takes the device's idle space or makes a new one; the destructor gives it back, or frees
+// it when it holds more than a sixteenth of the device's memory, another one is there, or
+// the call has failed. (Allocating and freeing the queues on every call: 12 views, 42M paths,
+// 7 GB took 278 ms a call, of which 10 ms were kernels; once a process has used as much
+// memory as the device has, the driver clears every page that it hands out again.)
+class CallSpaceLease {
+public:
+    int take(int device) {
+        {
+            std::lock_guard<std::mutex> g(g_space_mutex);
+            if (device < kSpaceDevices) std::swap(c_, g_idle_space[device]);
+        }
+        if (c_) return PRT_OK;
+        c_ = new CallSpace;
+        c_->device = device;
+        WF_TRY(hipStreamCreateWithFlags(&c_->stream, hipStreamNonBlocking));
+        return PRT_OK;
+    }
+    void done() { ok_ = true; }
+    CallSpace* operator->() const { return c_; }
+    ~CallSpaceLease() {
+        if (!c_) return;
+        size_t free_b = 0, total_b = 0;
+        if (ok_ && scenes_on_devices() && hipMemGetInfo(&free_b, &total_b) == hipSuccess && c_->bytes() <= total_b / 16) {
+            std::lock_guard<std::mutex> g(g_space_mutex);
+            if (c_->device < kSpaceDevices && !g_idle_space[c_->device]) {
+                g_idle_space[c_->device] = c_;
+                return;
+            }
+        }
+        if (c_->stream) (void)hipStreamSynchronize(c_->stream);
+        free_space(c_);
+    }
+
+private:
+    CallSpace* c_ = nullptr;
+    bool ok_ = false;
+};
+
 }  // namespace
 
+void release_idle_queues() {
+    CallSpace* all[kSpaceDevices] = {};
+    {
+        std::lock_guard<std::mutex> g(g_space_mutex);
+        for (int k = 0; k < kSpaceDevices; ++k) std::swap(all[k], g_idle_space[k]);
+    }
+    for (CallSpace* c : all)
+        if (c) free_space(c);
+}
+
 int render_wavefront(prt_renderer* r, uint32_t n) {
+    PRT_TRY_BEGIN
     if (!r->wf) r->wf = new WavefrontState();
     WfJob j;
     j.sc = r->sc;
@@ -1255,11 +1335,20 @@ int render_wavefront(prt_renderer* r, uint32_t n) {
     r->samples_done += n;
     r->samples_total += total;
     return PRT_OK;
+    PRT_TRY_END
 }
 
 int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples, uint32_t* vertices) {
-    const bool had_state = r->wf != nullptr;
-    if (!r->wf) r->wf = new WavefrontState();
+    PRT_TRY_BEGIN
+    // A megakernel renderer does not keep the queues of a one-off forward pass.
+    CallSpaceLease space;
+    WavefrontState* w = r->wf;
+    if (!w && r->cfg.integrator == PRT_INTEGRATOR_WAVEFRONT) w = r->wf = new WavefrontState();
+    if (!w) {
+        const int rc = space.take(r->cfg.device);
+        if (rc != PRT_OK) return rc;
+        w = &space->w;
+    }
     WfJob j;
     j.sc = r->sc;
     j.cam = cam_args(r->cam);
@@ -1272,14 +1361,16 @@ int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samp
     std::vector<WfJob> jobs = {j};
     std::vector<PlanJob> pj = {PlanJob{r->w * r->h, 0, spp}};
     const uint64_t total = uint64_t(r->w) * r->h * spp;
-    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*r->wf, total);
+    const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*w, total);
     RunStats rs;
-    const int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
+    // On the renderer's stream, and waited for: the queues are idle when the call returns.
+    const int rc = run_wavefront(*w, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
                                  r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, false, &rs, false, vertices,
                                  spp);
-    // A megakernel renderer does not keep the queues of a one-off forward pass.
-    if (!had_state && r->cfg.integrator != PRT_INTEGRATOR_WAVEFRONT) release_wavefront(r);
+    if (rc == PRT_OK) space.done();
+    else (void)hipStreamSynchronize(r->stream);
     return rc;
+    PRT_TRY_END
 }
 
 void release_wavefront(prt_renderer* r) {
@@ -1294,12 +1385,15 @@ namespace {
 struct BatchCtx {
     std::vector<WfJob> jobs;
     std::vector<PlanJob> pjobs;
-    std::vector<float4*> accum;
+    std::vector<size_t> pixel0;  // each view's first pixel in the accumulators
+    size_t pixels = 0;
     uint32_t max_depth = 0;
     uint64_t total = 0;
 };
 
-int batch_prepare(prt_job* jobs, uint32_t n, const prt_render_config& c, BatchCtx& b, hipStream_t stream) {
+// Checks the jobs, uploads their scenes and clears accumulators for all of them.
+int batch_prepare(prt_job* jobs, uint32_t n, const prt_render_config& c, BatchCtx& b, CallSpace& space) {
+    hipStream_t stream = space.stream;
     if (!jobs || n == 0) return fail(PRT_ERR_INVALID_ARG, "no jobs");
     b.max_depth = c.max_depth;
     for (uint32_t i = 0; i < n; ++i) {
@@ -1318,24 +1412,20 @@ int batch_prepare(prt_job* jobs, uint32_t n, const prt_render_config& c, BatchCt
         w.width = uint32_t(jb.camera.xpixels);
         w.height = uint32_t(jb.camera.ypixels);
         const size_t px = size_t(w.width) * w.height;
-        float4* acc = nullptr;
-        WF_TRY(hipMalloc(reinterpret_cast<void**>(&acc), px * sizeof(float4)));
-        b.accum.push_back(acc);
-        WF_TRY(fill_wait(acc, 0, px * sizeof(float4), stream));
-        w.accum = acc;
+        w.accum = nullptr;
+        b.pixel0.push_back(b.pixels);
+        b.pixels += px;
         w.samples = nullptr;
         w.samples_cap = 0;
         b.jobs.push_back(w);
         b.pjobs.push_back(PlanJob{uint32_t(px), 0, jb.spp});
         b.total += uint64_t(px) * jb.spp;
     }
+    const int rc = scratch_for(space.accum, space.accum_bytes, b.pixels * sizeof(float4));
+    if (rc != PRT_OK) return rc;
+    for (uint32_t i = 0; i < n; ++i) b.jobs[i].accum = static_cast<float4*>(space.accum) + b.pixel0[i];
+    WF_TRY(hipMemsetAsync(space.accum, 0, b.pixels * sizeof(float4), stream));
     return PRT_OK;
-}
-
-void batch_release(BatchCtx& b) {
-    for (float4* p : b.accum)
-        if (p) (void)hipFree(p);
-    b.accum.clear();
 }
 
 }  // namespace
@@ -1356,33 +1446,28 @@ extern "C" int prt_render_batch(prt_job* jobs, uint32_t n, const prt_render_conf
     if (rc != PRT_OK) return rc;
     PRT_TRY_BEGIN
     BatchCtx b;
-    hipStream_t s;
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e != hipSuccess) return hip_fail(e, "stream");
-    rc = batch_prepare(jobs, n, c, b, s);
-    if (rc != PRT_OK) {
-        batch_release(b);
-        (void)hipStreamDestroy(s);
-        return rc;
-    }
-    WavefrontState w;
-    const uint32_t cap = tune && tune->queue_slots ? tune->queue_slots : default_capacity(w, b.total);
+    CallSpaceLease space;
+    rc = space.take(c.device);
+    if (rc == PRT_OK) rc = batch_prepare(jobs, n, c, b, *space.operator->());
+    if (rc != PRT_OK) return rc;
+    hipStream_t s = space->stream;
+    const uint32_t cap = tune && tune->queue_slots ? tune->queue_slots : default_capacity(space->w, b.total);
     RunStats rs;
-    rc = run_wavefront(w, c.device, s, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
+    rc = run_wavefront(space->w, c.device, s, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
                        tune ? tune->group_side : c.wavefront_group, c.count_rays != 0, &rs);
-    if (rc == PRT_OK) {
-        for (uint32_t i = 0; i < n && rc == PRT_OK; ++i) {
-            if (!jobs[i].out_rgb) continue;
-            const size_t px = size_t(b.jobs[i].width) * b.jobs[i].height;
-            float* tmp = nullptr;
-            e = hipMalloc(reinterpret_cast<void**>(&tmp), px * 3 * sizeof(float));
-            if (e == hipSuccess) e = launch_mean(b.accum[i], uint32_t(px), jobs[i].spp, tmp, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e == hipSuccess) e = copy_wait(jobs[i].out_rgb, tmp, px * 3 * sizeof(float), hipMemcpyDeviceToHost, s);
-            if (tmp) (void)hipFree(tmp);
-            if (e != hipSuccess) rc = hip_fail(e, "batch readback");
-        }
+    // Every image's mean, then all copies in one run.
+    if (rc == PRT_OK) rc = scratch_for(space->rgb, space->rgb_bytes, b.pixels * 3 * sizeof(float));
+    std::vector<CopyOut> out;
+    hipError_t e = hipSuccess;
+    for (uint32_t i = 0; i < n && rc == PRT_OK && e == hipSuccess; ++i) {
+        if (!jobs[i].out_rgb) continue;
+        const size_t px = size_t(b.jobs[i].width) * b.jobs[i].height;
+        float* rgb = static_cast<float*>(space->rgb) + b.pixel0[i] * 3;
+        e = launch_mean(b.jobs[i].accum, uint32_t(px), jobs[i].spp, rgb, s);
+        out.push_back(CopyOut{jobs[i].out_rgb, rgb, px * 3 * sizeof(float)});
     }
+    if (rc == PRT_OK && e == hipSuccess) e = copy_out(out.data(), out.size(), c.device, s);
+    if (e != hipSuccess) rc = hip_fail(e, "batch readback");
     if (rc == PRT_OK && stats) {
         stats->primary_rays = rs.c[kCntPrimary];
         stats->extension_rays = rs.c[kCntExtension];
@@ -1393,9 +1478,7 @@ extern "C" int prt_render_batch(prt_job* jobs, uint32_t n, const prt_render_conf
         stats->samples = b.total;
         stats->last_render_ms = rs.ms;
     }
-    free_state(w);
-    (void)hipStreamDestroy(s);
-    batch_release(b);
+    if (rc == PRT_OK) space.done();
     return rc;
     PRT_TRY_END
 }
@@ -1425,17 +1508,14 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
         paths += uint64_t(t.camera.xpixels) * t.camera.ypixels * t.spp;
     }
     BatchCtx b;
-    hipStream_t s;
-    WF_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    rc = batch_prepare(trial.data(), n, c, b, s);
-    if (rc != PRT_OK) {
-        batch_release(b);
-        (void)hipStreamDestroy(s);
-        return rc;
-    }
+    CallSpaceLease space;
+    rc = space.take(c.device);
+    if (rc == PRT_OK) rc = batch_prepare(trial.data(), n, c, b, *space.operator->());
+    if (rc != PRT_OK) return rc;
+    hipStream_t s = space->stream;
+    WavefrontState& w = space->w;
     uint64_t full = 0;
     for (uint32_t i = 0; i < n; ++i) full += uint64_t(jobs[i].camera.xpixels) * jobs[i].camera.ypixels * jobs[i].spp;
-    WavefrontState w;
     double bms = 1e30;
     prt_tune bt{};
     // Every candidate is timed (best of two) on the trial cut into as many chunks as
@@ -1493,10 +1573,8 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
         t.queue_slots = std::max<uint32_t>(1u << 16, full_cap / div);
         if (t.queue_slots < full_cap && rc == PRT_OK) consider(t);
     }
-    free_state(w);
-    (void)hipStreamDestroy(s);
-    batch_release(b);
     if (rc != PRT_OK) return rc;
+    space.done();
     *best = bt;
     if (best_ms) *best_ms = bms;
     return PRT_OK;

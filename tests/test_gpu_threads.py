@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import cudart_amd as ca
+import oracle as O
 from cudart_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +86,57 @@ def test_two_threads_batch_as_one_after_the_other(gpu):
     for w, g in zip(want, got):
         for x, y in zip(w, g):
             assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+
+
+# Results larger and smaller than the staging block's segments, whole and partial segments,
+# several destinations to a segment, from several threads at once (each takes its own block).
+@pytest.mark.parametrize("w,h", [(300, 200), (512, 342), (600, 437), (1100, 960)])
+def test_results_of_any_size_from_several_threads(gpu, w, h):
+    scene = ca.Scene(W.cornell().mesh)
+    cam = ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, w, h)
+
+    def results(seed, out):
+        r = ca.ParallelRenderer(scene, w, h, 1, camera=cam, max_depth=2, seed=seed)
+        r.render(1)
+        out[seed] = [r.radiance(), r.copyImageBytes(), *r.first_hit(0)]
+        r.close()
+
+    alone, together = {}, {}
+    for seed in (1, 2, 3, 4):
+        results(seed, alone)
+    threads = [threading.Thread(target=results, args=(seed, together)) for seed in (1, 2, 3, 4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for seed in alone:
+        for a, b in zip(alone[seed], together[seed]):
+            assert np.array_equal(a, b)
+        orc, cfg = O.OracleScene(scene._src.desc()), O.cfg(max_depth=2, seed=seed)
+        acc, _ = orc.render(cam, w, h, 0, 1, cfg)
+        np.testing.assert_allclose(alone[seed][0], acc, rtol=1e-5, atol=1e-6)
+        for a, b in zip(alone[seed][2:], orc.first_hit(cam, w, h, 0, cfg)):
+            assert np.array_equal(a, b)
+
+
+# A batch call leaves its queues for the next: calls of other sizes and scenes, calls from two
+# threads at once, and calls after every scene on the device has gone.
+def test_batch_calls_share_no_results(gpu):
+    def images(side, spp, seed):
+        scene = ca.Scene(W.cornell().mesh)
+        cam = ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, side, side)
+        out, _ = ca.render_batch([ca.BatchJob(scene, cam, spp, v) for v in (1, 2)], max_depth=4, seed=seed)
+        scene.close()
+        return out
+
+    sizes = [(40, 3, 1), (90, 9, 2), (17, 1, 3), (40, 3, 1)]
+    first = [images(*s) for s in sizes]
+    assert np.array_equal(first[0], first[3])
+    got = {}
+    threads = [threading.Thread(target=lambda k: got.update({k: images(*sizes[k])}), args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(4):
+        assert np.array_equal(first[k], got[k])
