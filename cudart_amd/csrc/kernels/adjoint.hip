@@ -612,6 +612,7 @@ bool primal_in_replay() {
 // The partials (ceil8(tiles x parts) x 4 x materials doubles) must also fit the
 // allocation-free entry point's scratch, so both entry points pick the same split and
 // give the same sums.
+}  // namespace
 uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp) {
     constexpr uint64_t kTargetUnits = 8ull * 3 * 4 * 256;  // 8 x (3 waves x 4 SIMDs x 256 CUs)
     const uint64_t tiles = std::max<uint32_t>(1, r->tiles);
@@ -619,8 +620,13 @@ uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp) {
     uint64_t parts = std::max<uint64_t>(1, (kTargetUnits + tiles - 1) / tiles);
     parts = std::min<uint64_t>(parts, std::max<uint32_t>(1, spp));
     while (parts > 1 && ((tiles * parts + 7) / 8) * 8 * P + P > kStaticScratchDoubles) --parts;
+    // The tracing replay's workgroups each need their threads' columns of the spill area, made
+    // for the renderer's own sample count. (Where there were fewer columns than threads,
+    // workgroups of different parts wrote each other's entries.)
+    while (parts > 1 && r->spill && ((tiles * parts + 7) / 8) * 8 * kBlock > r->spill_threads) --parts;
     return uint32_t(parts);
 }
+namespace {
 
 AdjArgs adjoint_args(const prt_renderer* r, const float* grad, float hess, uint32_t spp, double* partial) {
     AdjArgs a;

@@ -124,16 +124,13 @@ void gamma_table(uint8_t lut[256]) {
 }
 
 int ensure_spill(prt_renderer* r, uint32_t threads) {
-    // Entries the deepest walk of this BVH can hold: a node visit pushes at most its
-    // three farther children, once per level 0..max_depth.
-    const uint32_t need_entries = 3 * (r->scene->bvh.max_depth + 1);
-    if (need_entries <= uint32_t(kStackLds)) return PRT_OK;
-    size_t bytes = size_t(kStackMax - kStackLds) * threads * sizeof(int);
+    const uint32_t entries = stack_entries(r->scene);
+    if (entries <= uint32_t(kStackLds)) return PRT_OK;
     if (r->spill && r->spill_threads >= threads) return PRT_OK;
     if (r->spill) (void)hipFree(r->spill);
     r->spill = nullptr;
     r->spill_threads = 0;
-    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), bytes));
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), size_t(entries - kStackLds) * threads * sizeof(int)));
     r->spill_threads = threads;
     return PRT_OK;
 }
@@ -252,7 +249,9 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     }
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
-    rc = ensure_spill(r.get(), ((r->tiles + 7) / 8) * 8 * kBlock);
+    // Room for the first-hit and the one-sample launch (a workgroup per tile) and for the
+    // adjoint's.
+    rc = ensure_spill(r.get(), (r->tiles * adjoint_parts(r.get(), std::max(1u, spp)) + 7) / 8 * 8 * kBlock);
     if (rc != PRT_OK) return rc;
     HIP_TRY(hipStreamSynchronize(r->stream));
     *out = r.release();

@@ -14,7 +14,7 @@ constexpr int kStackLds = 32;    // traversal stack entries per lane in LDS (meg
 #define PRT_QUEUE_STACK_LDS 16
 #endif
 constexpr int kStackLdsQueue = PRT_QUEUE_STACK_LDS;  // LDS entries of the queue-based traversal kernels
-constexpr int kStackMax = 128;   // total entries (the rest in the global spill area)
+constexpr int kStackMax = 128;   // total entries (those of the deepest scene; the rest in the global spill area)
 
 // Device view of a built scene. Layouts:
 //   nodes   4 x float4 per four-wide node (64 B, quantized child boxes)
@@ -79,7 +79,7 @@ struct MegaArgs {
     float4* samples;          // nullptr, or each sample's radiance at [pixel * samples_cap + sample]
     uint32_t samples_cap;     // samples stored per pixel
     unsigned long long* counters;  // kCntNum or nullptr
-    int* spill;               // (kStackMax - kStackLds) * spill_stride ints
+    int* spill;               // a row of spill_stride ints per stack entry beyond the LDS ones
     uint32_t spill_stride;
 };
 

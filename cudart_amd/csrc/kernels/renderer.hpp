@@ -86,7 +86,14 @@ int scratch_for(void*& p, size_t& have, size_t bytes);
 int device_scene(prt_scene* s, int device, SceneArgs& out, hipStream_t stream);
 CamArgs cam_args(const prt_camera& c);
 int set_device(int device);
+// Entries the deepest walk of the scene's BVH can hold: a node visit pushes at most its
+// three farther children, once per level 0..max_depth. (At most kStackMax.) What does not
+// fit a kernel's LDS stack goes to a spill area of that many rows, a column per thread; with
+// kStackMax rows it took 235 MB for the wavefront's resident threads, 0.8 GB for a 1080p
+// megakernel.
+inline uint32_t stack_entries(const prt_scene* s) { return 3 * (s->bvh.max_depth + 1); }
 int ensure_spill(prt_renderer* r, uint32_t threads);
+uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp);  // adjoint.hip
 int render_wavefront(prt_renderer* r, uint32_t n);  // wavefront.hip
 // Samples 0..spp-1 of the renderer's view into `accum` (zeroed), each sample's radiance
 // into `samples` ([pixel * spp + sample]) and, unless null, its path's vertices into

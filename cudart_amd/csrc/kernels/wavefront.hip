@@ -161,7 +161,7 @@ struct LaunchKey {
 struct WavefrontState {
     int device = -1;
     uint32_t capacity = 0;       // slots
-    uint32_t persistent = 0;     // threads of the persistent kernels (spill stride)
+    size_t spill_ints = 0;
     void* mem = nullptr;
     size_t bytes = 0;
     int* spill = nullptr;
@@ -918,8 +918,9 @@ int persistent_blocks(const void* kernel, uint32_t blocks_per_cu, int device, in
     return int(std::max<uint32_t>(1, per * uint32_t(*compute_units)));
 }
 
-int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t persistent, hipStream_t stream) {
-    if (w.mem && w.capacity >= capacity && w.persistent >= persistent && w.device == device) return PRT_OK;
+// Queues of `capacity` slots and a spill area of `spill_ints`.
+int ensure_state(WavefrontState& w, int device, uint32_t capacity, size_t spill_ints, hipStream_t stream) {
+    if (w.mem && w.capacity >= capacity && w.spill_ints >= spill_ints && w.device == device) return PRT_OK;
     if (w.mem) (void)hipFree(w.mem);
     if (w.spill) (void)hipFree(w.spill);
     if (w.ctr) (void)hipFree(w.ctr);
@@ -933,8 +934,7 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
     w.bytes = bytes;
     WF_TRY(device_alloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
     WF_TRY(fill_wait(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
-    const size_t spill_entries = size_t(kStackMax - kStackLdsQueue) * persistent;
-    WF_TRY(device_alloc(reinterpret_cast<void**>(&w.spill), spill_entries * sizeof(int)));
+    if (spill_ints) WF_TRY(device_alloc(reinterpret_cast<void**>(&w.spill), spill_ints * sizeof(int)));
     char* p = static_cast<char*>(w.mem);
     auto take = [&](size_t bytes) {
         void* r = p;
@@ -956,9 +956,8 @@ int ensure_state(WavefrontState& w, int device, uint32_t capacity, uint32_t pers
     a.sj = static_cast<uint32_t*>(take(4 * C));
     a.ctr = w.ctr;
     a.spill = w.spill;
-    a.spill_stride = persistent;
     w.capacity = capacity;
-    w.persistent = persistent;
+    w.spill_ints = spill_ints;
     w.device = device;
     return PRT_OK;
 }
@@ -1096,9 +1095,10 @@ int run_profiled(const WfArgs& a, hipStream_t stream, size_t nchunks, uint32_t m
 }
 
 // Renders every job of the plan on `stream`. Returns PRT_OK or an error.
+// entries: traversal stack entries that the scenes need (stack_entries).
 // group_side: camera-path block side g for wf_generate (1, 2, 4, 8; 0 = choose per section).
 // stats: device counters that the rays are added to (else rs->c receives them).
-int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::vector<WfJob>& jobs,
+int run_wavefront(WavefrontState& w, int device, hipStream_t stream, uint32_t entries, const std::vector<WfJob>& jobs,
                   const std::vector<PlanJob>& pjobs, uint32_t max_depth, uint32_t capacity, uint32_t blocks_per_cu,
                   uint32_t group_side, bool count, RunStats* rs, bool profile = false, uint32_t* vertices = nullptr,
                   uint32_t vertex_cap = 0, unsigned long long* stats = nullptr) {
@@ -1129,7 +1129,8 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, const std::
     int cus = 0;
     // No more waves than the largest queue has batches.
     const int pblocks = std::min(persistent_blocks(ktrace, blocks_per_cu, device, &cus), int((need + kBatch - 1) / kBatch));
-    int rc = ensure_state(w, device, need, uint32_t(pblocks) * kBlock, stream);
+    const size_t rows = entries > uint32_t(kStackLdsQueue) ? entries - kStackLdsQueue : 0;
+    int rc = ensure_state(w, device, need, rows * size_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;
     // The plan in one upload. (Every part is a multiple of 16 bytes.)
     const size_t at_tiles = jobs.size() * sizeof(WfJob), at_chunks = at_tiles + tiles.size() * sizeof(WfTile);
@@ -1323,7 +1324,7 @@ int render_wavefront(prt_renderer* r, uint32_t n) {
     const uint64_t total = uint64_t(r->w) * r->h * n;
     const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*r->wf, total);
     RunStats rs;
-    int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
+    int rc = run_wavefront(*r->wf, r->cfg.device, r->stream, stack_entries(r->scene), jobs, pj, r->cfg.max_depth, cap,
                            r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, r->cfg.count_rays != 0, &rs,
                            r->cfg.profile_kernels != 0, r->vertices, r->spp, r->counters);
     if (rc != PRT_OK) return rc;
@@ -1364,7 +1365,7 @@ int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samp
     const uint32_t cap = r->cfg.wavefront_queue ? r->cfg.wavefront_queue : default_capacity(*w, total);
     RunStats rs;
     // On the renderer's stream, and waited for: the queues are idle when the call returns.
-    const int rc = run_wavefront(*w, r->cfg.device, r->stream, jobs, pj, r->cfg.max_depth, cap,
+    const int rc = run_wavefront(*w, r->cfg.device, r->stream, stack_entries(r->scene), jobs, pj, r->cfg.max_depth, cap,
                                  r->cfg.wavefront_blocks_per_cu, r->cfg.wavefront_group, false, &rs, false, vertices,
                                  spp);
     if (rc == PRT_OK) space.done();
@@ -1388,6 +1389,7 @@ struct BatchCtx {
     std::vector<size_t> pixel0;  // each view's first pixel in the accumulators
     size_t pixels = 0;
     uint32_t max_depth = 0;
+    uint32_t entries = 0;  // traversal stack entries that the scenes need
     uint64_t total = 0;
 };
 
@@ -1407,6 +1409,7 @@ int batch_prepare(prt_job* jobs, uint32_t n, const prt_render_config& c, BatchCt
         WfJob w;
         int rc = device_scene(jb.scene, c.device, w.sc, stream);
         if (rc != PRT_OK) return rc;
+        b.entries = std::max(b.entries, stack_entries(jb.scene));
         w.cam = cam_args(jb.camera);
         w.path = PathArgs{c.seed, jb.view_id, c.max_depth, c.rr_start};
         w.width = uint32_t(jb.camera.xpixels);
@@ -1453,7 +1456,7 @@ extern "C" int prt_render_batch(prt_job* jobs, uint32_t n, const prt_render_conf
     hipStream_t s = space->stream;
     const uint32_t cap = tune && tune->queue_slots ? tune->queue_slots : default_capacity(space->w, b.total);
     RunStats rs;
-    rc = run_wavefront(space->w, c.device, s, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
+    rc = run_wavefront(space->w, c.device, s, b.entries, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
                        tune ? tune->group_side : c.wavefront_group, c.count_rays != 0, &rs);
     // Every image's mean, then all copies in one run.
     if (rc == PRT_OK) rc = scratch_for(space->rgb, space->rgb_bytes, b.pixels * 3 * sizeof(float));
@@ -1536,7 +1539,7 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
         double best_t = 1e30;
         for (int rep = 0; rep < 2 && rc == PRT_OK; ++rep) {  // best of two
             RunStats rs;
-            rc = run_wavefront(w, c.device, s, b.jobs, b.pjobs, c.max_depth, trial_cap_for(t.queue_slots),
+            rc = run_wavefront(w, c.device, s, b.entries, b.jobs, b.pjobs, c.max_depth, trial_cap_for(t.queue_slots),
                                t.blocks_per_cu, t.group_side, false, &rs);
             best_t = std::min(best_t, rs.ms);
         }
