@@ -215,11 +215,14 @@ __device__ __forceinline__ bool mt_intersect(float4 a, float4 b, float4 c, V3 o,
     return t > kEps;
 }
 
-// One four-wide node (64 bytes, quantized child boxes): decodes each child plane as
-// fmaf(q, 2^e, origin) (exactly as the builder bounded it; with FOLD the decode is
-// folded into the slab FMA), slab-tests the four boxes against [tmin, tfar], and
-// orders the children hit nearest first. Pushes the farther ones (farthest first,
-// so the nearest of them is popped next) and returns the nearest, or kNoChild.
+// One four-wide node (64 bytes, quantized child boxes): slab-tests the four boxes against
+// [tmin, tfar], and orders the children hit nearest first. Pushes the farther ones (farthest
+// first, so the nearest of them is popped next) and returns the nearest, or kNoChild. A
+// child plane is fmaf(q, 2^e, origin), and its decode is folded into the slab FMA,
+// t = q (2^e i) + (origin i - o i), the two factors made once per node: 6 FMAs instead of 12
+// per child (see packet_traverse for why culling stays conservative). An empty slot's box is
+// the point at the origin corner; a ray through it finds kNoChild there, which is neither
+// pushed nor entered.
 //
 // The near and far plane of each axis are picked once per node from the sign of
 // the inverse direction, instead of a min and a max per child and axis: for i > 0,
@@ -237,11 +240,10 @@ __device__ __forceinline__ void cswap(float& ka, int& wa, float& kb, int& wb) {
     wa = w;
 }
 __device__ __forceinline__ float qbyte(uint32_t w, int c) { return float((w >> (8 * c)) & 0xFFu); }
-// FOLD: each plane's decode folded into its slab FMA, t = q (2^e i) + (origin i - o i),
-// the two factors made once per node (6 FMAs instead of 12 per child; see
-// packet_traverse for why culling stays conservative). Occlusion rays use it
-// (wf_shadow 2 % faster); closest-hit rays do not (wf_extend 3 % slower with it).
-template <bool FOLD, class StackType>
+// On 1080p x 128 spp over 1M triangles wf_trace took 72.3 ms with the decode apart for
+// closest-hit rays and slots tested for kNoChild here, 71.4 without; terrain at 4K 10.86 and
+// 10.62.
+template <class StackType>
 __device__ __forceinline__ int visit_node(const float4* nodes, int node, float ix, float iy, float iz, float ox,
                                           float oy, float oz, float tmin, float tfar, StackType& st) {
     const size_t nb = size_t(node) * 4;
@@ -261,26 +263,15 @@ __device__ __forceinline__ int visit_node(const float4* nodes, int node, float i
     const float bx = __builtin_fmaf(org.x, ix, -ox), by = __builtin_fmaf(org.y, iy, -oy), bz = __builtin_fmaf(org.z, iz, -oz);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-        float tn, tf;
-        if (FOLD) {
-            tn = fmaxf(fmaxf(__builtin_fmaf(qbyte(nqx, c), ax, bx), __builtin_fmaf(qbyte(nqy, c), ay, by)),
-                       fmaxf(__builtin_fmaf(qbyte(nqz, c), az, bz), tmin));
-            tf = fminf(fminf(__builtin_fmaf(qbyte(fqx, c), ax, bx), __builtin_fmaf(qbyte(fqy, c), ay, by)),
-                       fminf(__builtin_fmaf(qbyte(fqz, c), az, bz), tfar));
-        } else {
-            const float nx = __builtin_fmaf(qbyte(nqx, c), sx, org.x), fx_ = __builtin_fmaf(qbyte(fqx, c), sx, org.x);
-            const float ny = __builtin_fmaf(qbyte(nqy, c), sy, org.y), fy_ = __builtin_fmaf(qbyte(fqy, c), sy, org.y);
-            const float nz = __builtin_fmaf(qbyte(nqz, c), sz, org.z), fz_ = __builtin_fmaf(qbyte(fqz, c), sz, org.z);
-            tn = fmaxf(fmaxf(__builtin_fmaf(nx, ix, -ox), __builtin_fmaf(ny, iy, -oy)),
-                       fmaxf(__builtin_fmaf(nz, iz, -oz), tmin));
-            tf = fminf(fminf(__builtin_fmaf(fx_, ix, -ox), __builtin_fmaf(fy_, iy, -oy)),
-                       fminf(__builtin_fmaf(fz_, iz, -oz), tfar));
-        }
-        const bool hit = tn <= tf && word[c] != kNoChild;
+        const float tn = fmaxf(fmaxf(__builtin_fmaf(qbyte(nqx, c), ax, bx), __builtin_fmaf(qbyte(nqy, c), ay, by)),
+                               fmaxf(__builtin_fmaf(qbyte(nqz, c), az, bz), tmin));
+        const float tf = fminf(fminf(__builtin_fmaf(qbyte(fqx, c), ax, bx), __builtin_fmaf(qbyte(fqy, c), ay, by)),
+                               fminf(__builtin_fmaf(qbyte(fqz, c), az, bz), tfar));
+        const bool hit = tn <= tf;
         key[c] = hit ? tn : __builtin_inff();
         word[c] = hit ? word[c] : kNoChild;
-        // One child at a time: interleaving the four decodes would hold all 24
-        // decoded planes live (register pressure, hence occupancy).
+        // One child at a time: interleaving the four tests would hold all 24 planes live
+        // (register pressure, hence occupancy).
         __builtin_amdgcn_sched_barrier(0);
     }
     // Occlusion rays use the same order: the nearest boxes hold occluders most often.
@@ -358,15 +349,13 @@ __device__ __forceinline__ bool trav_wants_nodes(const TravRay& r) { return r.le
 // written; hit_details() recomputes them from the record afterwards).
 // `any` (default ANY) may also be set per lane at run time, for kernels whose lanes
 // trace closest-hit and occlusion rays in the same steps.
-// FOLD: the box test visit_node<FOLD> uses (by default the folded one for occlusion
-// rays only).
-template <bool ANY, bool COUNT, bool LEAN, bool FOLD = ANY, class StackType>
+template <bool ANY, bool COUNT, bool LEAN, class StackType>
 __device__ __forceinline__ int trav_step(bool node_phase, const float4* nodes, const float4* tris, TravRay& r,
                                          float tmin, HitRec& best, StackType& st, Counts& cnt, bool any = ANY) {
     if (node_phase) {
         if (uint32_t(r.node) < uint32_t(kNoChild)) {  // an inner node
             if (COUNT) cnt.nodes++;
-            int next = visit_node<FOLD>(nodes, r.node, r.ix, r.iy, r.iz, r.o.x * r.ix, r.o.y * r.iy, r.o.z * r.iz,
+            int next = visit_node(nodes, r.node, r.ix, r.iy, r.iz, r.o.x * r.ix, r.o.y * r.iy, r.o.z * r.iz,
                                         tmin, best.t, st);
             if (next == kNoChild && st.sp != 0) next = st.pop();
             r.node = next;
