@@ -125,12 +125,12 @@ void gamma_table(uint8_t lut[256]) {
 
 int ensure_spill(prt_renderer* r, uint32_t threads) {
     const uint32_t entries = stack_entries(r->scene);
-    if (entries <= uint32_t(kStackLds)) return PRT_OK;
+    if (entries <= uint32_t(kStackLdsQueue)) return PRT_OK;  // the smallest LDS stack of the kernels that use it
     if (r->spill && r->spill_threads >= threads) return PRT_OK;
     if (r->spill) (void)hipFree(r->spill);
     r->spill = nullptr;
     r->spill_threads = 0;
-    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), size_t(entries - kStackLds) * threads * sizeof(int)));
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), size_t(entries - kStackLdsQueue) * threads * sizeof(int)));
     r->spill_threads = threads;
     return PRT_OK;
 }

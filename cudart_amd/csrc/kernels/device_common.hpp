@@ -425,8 +425,9 @@ static_assert(PRT_LOOP_PHASE_MIN >= 0 && PRT_LOOP_PHASE_MIN <= 64, "phase thresh
 // (tmin, best.t) or t == best.t with a lower original id: the closest hit is the
 // lexicographic minimum of (t, original id), independent of tree shape and
 // visiting order. Returns true when best changed (closest) or when an occluder was
-// found (any). The stack must be empty on entry, and is empty on return.
-template <bool ANY, bool COUNT, class StackType>
+// found (any). The stack must be empty on entry, and is empty on return. LEAN as trav_step's,
+// PHASE_MIN as node_phase_for's.
+template <bool ANY, bool COUNT, bool LEAN = false, uint32_t PHASE_MIN = PRT_LOOP_PHASE_MIN, class StackType>
 __device__ __forceinline__ bool traverse(const SceneArgs& sc, V3 o, V3 d, float tmin, HitRec& best, StackType& st,
                                          Counts& cnt) {
     TravRay r;
@@ -434,8 +435,8 @@ __device__ __forceinline__ bool traverse(const SceneArgs& sc, V3 o, V3 d, float 
     const float t0 = best.t;
     const uint32_t id0 = best.id;
     while (true) {
-        const bool node_phase = node_phase_for<PRT_LOOP_PHASE_MIN>(trav_wants_nodes(r), true);
-        const int s = trav_step<ANY, COUNT, false>(node_phase, sc.nodes, sc.tris, r, tmin, best, st, cnt);
+        const bool node_phase = node_phase_for<PHASE_MIN>(trav_wants_nodes(r), true);
+        const int s = trav_step<ANY, COUNT, LEAN>(node_phase, sc.nodes, sc.tris, r, tmin, best, st, cnt);
         if (s == kTravOccluded) return true;
         if (s == kTravDone) break;
     }

@@ -167,15 +167,22 @@ __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
     if (COUNT) flush_counts<COUNT>(a.counters, cnt);
 }
 
+// An 8x8 tile per workgroup. What bounds it is the waves in flight: a tile lasts as long as its
+// longest ray, a dependent load per step. With 32 stack entries in LDS per lane 5 waves fitted a
+// SIMD; with 16, and only the hit's record held through the traversal, 8 do. The lanes' rays are
+// alike and reach leaves together, so a leaf phase with fewer than 16 lanes wanting nodes pays
+// (the megakernel's lanes, at different bounces of different rays, wait best for the last).
+// 1271 x 713 over 1M triangles: 232 -> 207 -> 161 us (a threshold of 8: 155, 24: 165); 1920 x
+// 1080 over 2.8M 559 -> 437 -> 362; 3840 x 2160 over 1M 981 -> 790 -> 652.
 __global__ __launch_bounds__(kBlock) void first_hit_kernel(FirstHitArgs a) {
-    __shared__ int s_stack[kStackLds * kBlock];
+    __shared__ int s_stack[kStackLdsQueue * kBlock];
     const uint32_t tile = xcd_tile(blockIdx.x, a.tiles);
     if (tile >= a.tiles) return;
     const int lane = int(threadIdx.x);
     const int x = int(tile % a.tiles_x) * 8 + (lane & 7);
     const int y = int(tile / a.tiles_x) * 8 + (lane >> 3);
     if (x >= int(a.width) || y >= int(a.height)) return;
-    Stack st;
+    StackT<kStackLdsQueue> st;
     st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
     Rng rng{a.path.seed, a.path.view, uint32_t(y) * uint32_t(a.cam.xpixels) + uint32_t(x), a.sample};
     V3 ro, rd;
@@ -184,13 +191,11 @@ __global__ __launch_bounds__(kBlock) void first_hit_kernel(FirstHitArgs a) {
     h.t = kFltMax;
     h.id = 0;
     h.rec = 0;
-    h.mat = 0;
-    h.u = h.v = 0.f;
     Counts cnt;
-    bool hit = traverse<false, false>(a.sc, ro, rd, kEps, h, st, cnt);
+    const bool hit = traverse<false, false, true, 16>(a.sc, ro, rd, kEps, h, st, cnt);
     const size_t idx = size_t(y) * a.width + size_t(x);
     if (a.tri) a.tri[idx] = hit ? int32_t(h.id) : -1;
-    if (a.mat) a.mat[idx] = hit ? int32_t(h.mat) : -1;
+    if (a.mat) a.mat[idx] = hit ? int32_t(__float_as_uint(gload(a.sc.tris, size_t(h.rec) * 3 + 1).w)) : -1;
     if (a.t) a.t[idx] = hit ? h.t : kFltMax;
 }
 
