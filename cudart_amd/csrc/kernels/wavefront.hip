@@ -683,35 +683,40 @@ __global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_extend_packet(WfArg
 // batches mostly share a light, measured 2% slower per frame on the 1M-triangle
 // scene with its two lights 10 units apart: the queue order of shade, pixel by
 // pixel, is the better one for the L2.)
-__device__ __forceinline__ uint2 block_append(bool more, bool nee, uint32_t* ctr_next, uint32_t* ctr_shadow) {
-    __shared__ uint32_t s_off[2][kShadeBlock / 64];
-    __shared__ uint32_t s_base[2];
+// Every wave of the workgroup waits here for the atomics' round trip, so what comes before and
+// after it is kept short: 8 lanes per queue add up the waves' counts, both atomics go out in
+// one instruction, and the LDS slots alternate (`turn`), so that two barriers a turn are
+// enough. 1080p x 128 spp over 1M triangles: wf_shade 25.4 ms with one thread adding up and
+// three barriers, 24.7 so; 256 x 256 x 16 over 36 155 and 151 us. (The counters themselves are
+// not what bounds it: with eight counters and queue segments, one per XCD, 24.7 too.)
+constexpr uint32_t kShadeWaves = kShadeBlock / 64;
+static_assert(kShadeWaves <= 32 && (kShadeWaves & (kShadeWaves - 1)) == 0, "a wave holds both queues' counts");
+__device__ __forceinline__ uint2 block_append(bool more, bool nee, uint32_t* ctr_next, uint32_t* ctr_shadow,
+                                              uint32_t turn) {
+    __shared__ uint32_t s_off[2][2 * kShadeWaves];
+    uint32_t* off = s_off[turn & 1u];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x / 64;
     const unsigned long long m0 = __ballot(more), m1 = __ballot(nee);
     if (lane == 0) {
-        s_off[0][wave] = uint32_t(__popcll(m0));
-        s_off[1][wave] = uint32_t(__popcll(m1));
+        off[wave] = uint32_t(__popcll(m0));
+        off[kShadeWaves + wave] = uint32_t(__popcll(m1));
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t t0 = 0, t1 = 0;
-        for (int w = 0; w < kShadeBlock / 64; ++w) {
-            uint32_t c0 = s_off[0][w], c1 = s_off[1][w];
-            s_off[0][w] = t0;
-            s_off[1][w] = t1;
-            t0 += c0;
-            t1 += c1;
+    if (wave == 0 && lane < 2 * kShadeWaves) {
+        const uint32_t count = off[lane], w = lane & (kShadeWaves - 1u);
+        uint32_t sum = count;  // of the queue's waves up to this one
+#pragma unroll
+        for (uint32_t d = 1; d < kShadeWaves; d <<= 1) {
+            const uint32_t below = __shfl_up(sum, d, kShadeWaves);
+            if (w >= d) sum += below;
         }
-        s_base[0] = t0 ? atomicAdd(ctr_next, t0) : 0u;
-        s_base[1] = t1 ? atomicAdd(ctr_shadow, t1) : 0u;
+        uint32_t base = 0;
+        if (w == kShadeWaves - 1u && sum != 0u) base = atomicAdd(lane < kShadeWaves ? ctr_next : ctr_shadow, sum);
+        off[lane] = __shfl(base, kShadeWaves - 1, kShadeWaves) + sum - count;
     }
     __syncthreads();
     const unsigned long long lt = (1ull << lane) - 1ull;
-    uint2 r;
-    r.x = s_base[0] + s_off[0][wave] + uint32_t(__popcll(m0 & lt));
-    r.y = s_base[1] + s_off[1][wave] + uint32_t(__popcll(m1 & lt));
-    __syncthreads();  // s_off / s_base are reused by the next iteration
-    return r;
+    return make_uint2(off[wave] + uint32_t(__popcll(m0 & lt)), off[kShadeWaves + wave] + uint32_t(__popcll(m1 & lt)));
 }
 
 // Channels of a throughput that are not finite, as bits: mask * 0 is then NaN, not 0.
@@ -728,6 +733,7 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
     const uint32_t n = uniform_u32(a.ctr[ext_count(it)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
     // Static, workgroup-uniform partition of the queue (shading cost varies little).
+    uint32_t turn = 0;
     for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
         const uint32_t i = base + threadIdx.x;
         const bool valid = i < n;
@@ -782,7 +788,7 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
                 a.result[slot] = make_float4(c.x, c.y, c.z, 0.f);
             }
         }
-        const uint2 pos = block_append(more, want_nee, &a.ctr[ext_count(it + 1)], &a.ctr[shadow_count(it)]);
+        const uint2 pos = block_append(more, want_nee, &a.ctr[ext_count(it + 1)], &a.ctr[shadow_count(it)], turn++);
         if (more) {
             const uint32_t special = ps.prev == 1 /*SPECULAR*/ || ps.prev == 4 /*REFRACTIVE*/ ? ~kSlotMask : 0u;
             a.qa[q ^ 1u][pos.x] = make_float4(ps.ro.x, ps.ro.y, ps.ro.z, A.w);
