@@ -219,7 +219,7 @@ __device__ __forceinline__ bool mt_intersect(float4 a, float4 b, float4 c, V3 o,
 // [tmin, tfar], and orders the children hit nearest first. Pushes the farther ones (farthest
 // first, so the nearest of them is popped next) and returns the nearest, or kNoChild. A
 // child plane is fmaf(q, 2^e, origin), and its decode is folded into the slab FMA,
-// t = q (2^e i) + (origin i - o i), the two factors made once per node: 6 FMAs instead of 12
+// t = q (2^e i) + (origin - o) i, the two factors made once per node: 6 FMAs instead of 12
 // per child (see packet_traverse for why culling stays conservative). An empty slot's box is
 // the point at the origin corner; a ray through it finds kNoChild there, which is neither
 // pushed nor entered.
@@ -229,23 +229,35 @@ __device__ __forceinline__ bool mt_intersect(float4 a, float4 b, float4 c, V3 o,
 // q_lo <= q_hi gives t(q_lo) <= t(q_hi) (each rounding is monotonic), so the picked
 // planes are the values min / max would give. i is finite and nonzero
 // (slab_inverse), so no plane is NaN for a finite origin.
+//
+// A child is sorted as one double, its distance's bits above its word: a distance is at
+// least tmin > 0 and at most infinity, whose bits begin an ordinary finite double, so
+// v_min_f64 / v_max_f64 (full rate here) swap both in two instructions, where a compare and
+// four selects were needed; the selects also stood next to each other, and measured back to
+// back, v_cndmask from VCC issues every 22 cycles instead of every 4. With the planes picked
+// by sign masks instead of selects a visit has about 25 of 150 VALU instructions fewer. It
+// mostly waits for loads all the same: wf_trace 71.4 -> 70.7 ms on 1080p x 128 spp over 1M
+// triangles, 10.7 -> 10.5 on a 4K terrain, the megakernel 5.20 -> 5.15 on 961 x 541 x 8.
 constexpr int kNoChild = 0x7FFFFFFF;  // also the word of an empty slot
-__device__ __forceinline__ void cswap(float& ka, int& wa, float& kb, int& wb) {
-    const bool sw = kb < ka;
-    const float k = sw ? kb : ka;
-    kb = sw ? ka : kb;
-    ka = k;
-    const int w = sw ? wb : wa;
-    wb = sw ? wa : wb;
-    wa = w;
+__device__ __forceinline__ uint32_t sign_mask(float x) { return uint32_t(int(__float_as_uint(x)) >> 31); }
+__device__ __forceinline__ double keyed(uint32_t key, uint32_t word) {
+    return __longlong_as_double((long long)((uint64_t(key) << 32) | word));
+}
+__device__ __forceinline__ int key_word(double k) { return int(uint32_t(uint64_t(__double_as_longlong(k)))); }
+__device__ __forceinline__ double key_min(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double key_max(double a, double b) {
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
 __device__ __forceinline__ float qbyte(uint32_t w, int c) { return float((w >> (8 * c)) & 0xFFu); }
-// On 1080p x 128 spp over 1M triangles wf_trace took 72.3 ms with the decode apart for
-// closest-hit rays and slots tested for kNoChild here, 71.4 without; terrain at 4K 10.86 and
-// 10.62.
 template <class StackType>
-__device__ __forceinline__ int visit_node(const float4* nodes, int node, float ix, float iy, float iz, float ox,
-                                          float oy, float oz, float tmin, float tfar, StackType& st) {
+__device__ __forceinline__ int visit_node(const float4* nodes, int node, float ix, float iy, float iz, V3 o, float tmin,
+                                          float tfar, StackType& st) {
     const size_t nb = size_t(node) * 4;
     const uint4* un = reinterpret_cast<const uint4*>(nodes);
     const float4 org = gload(nodes, nb);
@@ -253,14 +265,15 @@ __device__ __forceinline__ int visit_node(const float4* nodes, int node, float i
     const uint32_t ex = __float_as_uint(org.w);
     const float sx = __uint_as_float((ex & 0xFFu) << 23), sy = __uint_as_float(((ex >> 8) & 0xFFu) << 23),
                 sz = __uint_as_float(((ex >> 16) & 0xFFu) << 23);
-    float key[4];
-    int word[4] = {int(w.x), int(w.y), int(w.z), int(w.w)};
-    const bool fx = ix < 0.f, fy = iy < 0.f, fz = iz < 0.f;  // the hi plane is the near one
-    const uint32_t nqx = fx ? qxy.y : qxy.x, fqx = fx ? qxy.x : qxy.y;
-    const uint32_t nqy = fy ? qxy.w : qxy.z, fqy = fy ? qxy.z : qxy.w;
-    const uint32_t nqz = fz ? qz.y : qz.x, fqz = fz ? qz.x : qz.y;
+    const uint32_t mx = sign_mask(ix), my = sign_mask(iy), mz = sign_mask(iz);  // all ones: the hi plane is the near one
+    const uint32_t dqx = qxy.x ^ qxy.y, dqy = qxy.z ^ qxy.w, dqz = qz.x ^ qz.y;
+    const uint32_t nqx = qxy.x ^ (dqx & mx), fqx = nqx ^ dqx;
+    const uint32_t nqy = qxy.z ^ (dqy & my), fqy = nqy ^ dqy;
+    const uint32_t nqz = qz.x ^ (dqz & mz), fqz = nqz ^ dqz;
     const float ax = sx * ix, ay = sy * iy, az = sz * iz;
-    const float bx = __builtin_fmaf(org.x, ix, -ox), by = __builtin_fmaf(org.y, iy, -oy), bz = __builtin_fmaf(org.z, iz, -oz);
+    const float bx = (org.x - o.x) * ix, by = (org.y - o.y) * iy, bz = (org.z - o.z) * iz;
+    const uint32_t cw[4] = {w.x, w.y, w.z, w.w};
+    double child[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const float tn = fmaxf(fmaxf(__builtin_fmaf(qbyte(nqx, c), ax, bx), __builtin_fmaf(qbyte(nqy, c), ay, by)),
@@ -268,22 +281,20 @@ __device__ __forceinline__ int visit_node(const float4* nodes, int node, float i
         const float tf = fminf(fminf(__builtin_fmaf(qbyte(fqx, c), ax, bx), __builtin_fmaf(qbyte(fqy, c), ay, by)),
                                fminf(__builtin_fmaf(qbyte(fqz, c), az, bz), tfar));
         const bool hit = tn <= tf;
-        key[c] = hit ? tn : __builtin_inff();
-        word[c] = hit ? word[c] : kNoChild;
+        child[c] = keyed(hit ? __float_as_uint(tn) : 0x7F800000u, hit ? cw[c] : uint32_t(kNoChild));
         // One child at a time: interleaving the four tests would hold all 24 planes live
         // (register pressure, hence occupancy).
         __builtin_amdgcn_sched_barrier(0);
     }
     // Occlusion rays use the same order: the nearest boxes hold occluders most often.
-    cswap(key[0], word[0], key[1], word[1]);
-    cswap(key[2], word[2], key[3], word[3]);
-    cswap(key[0], word[0], key[2], word[2]);
-    cswap(key[1], word[1], key[3], word[3]);
-    cswap(key[1], word[1], key[2], word[2]);
-    if (word[3] != kNoChild) st.push(word[3]);
-    if (word[2] != kNoChild) st.push(word[2]);
-    if (word[1] != kNoChild) st.push(word[1]);
-    return word[0];
+    const double a = key_min(child[0], child[1]), b = key_max(child[0], child[1]);
+    const double c = key_min(child[2], child[3]), d = key_max(child[2], child[3]);
+    const double e = key_max(a, c), f = key_min(b, d);
+    const int w3 = key_word(key_max(b, d)), w2 = key_word(key_max(e, f)), w1 = key_word(key_min(e, f));
+    if (w3 != kNoChild) st.push(w3);
+    if (w2 != kNoChild) st.push(w2);
+    if (w1 != kNoChild) st.push(w1);
+    return key_word(key_min(a, c));
 }
 
 // Resumable form of traverse() for kernels that refill finished lanes with new
@@ -305,7 +316,7 @@ __device__ __forceinline__ int visit_node(const float4* nodes, int node, float i
 // (any-hit only).
 struct TravRay {
     V3 o, d;
-    float ix, iy, iz;  // o * i is recomputed per node (the same fp32 products as traverse's)
+    float ix, iy, iz;
     int node;          // the inner node to visit next, a second leaf, or kNoChild
     int leaf;          // the leaf set aside for the next leaf phase, or kNoChild
 };
@@ -355,8 +366,7 @@ __device__ __forceinline__ int trav_step(bool node_phase, const float4* nodes, c
     if (node_phase) {
         if (uint32_t(r.node) < uint32_t(kNoChild)) {  // an inner node
             if (COUNT) cnt.nodes++;
-            int next = visit_node(nodes, r.node, r.ix, r.iy, r.iz, r.o.x * r.ix, r.o.y * r.iy, r.o.z * r.iz,
-                                        tmin, best.t, st);
+            int next = visit_node(nodes, r.node, r.ix, r.iy, r.iz, r.o, tmin, best.t, st);
             if (next == kNoChild && st.sp != 0) next = st.pop();
             r.node = next;
         }
