@@ -24,7 +24,11 @@ struct V3 {
     float x, y, z;
 };
 __device__ __forceinline__ V3 v3(float x, float y, float z) { return V3{x, y, z}; }
+struct alignas(16) Float3 {  // the first three floats of a float4
+    float x, y, z;
+};
 __device__ __forceinline__ V3 v3(float4 a) { return V3{a.x, a.y, a.z}; }
+__device__ __forceinline__ V3 v3(Float3 a) { return V3{a.x, a.y, a.z}; }
 __device__ __forceinline__ V3 operator+(V3 a, V3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
 __device__ __forceinline__ V3 operator-(V3 a, V3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 __device__ __forceinline__ V3 operator*(V3 a, V3 b) { return {a.x * b.x, a.y * b.y, a.z * b.z}; }
@@ -199,7 +203,8 @@ struct HitRec {
 };
 
 // Moller-Trumbore exactly as Triangle::intersect (src/geometry/geometry.cu:38-65).
-__device__ __forceinline__ bool mt_intersect(float4 a, float4 b, float4 c, V3 o, V3 d, float& t, float& u, float& v) {
+template <class Edge>
+__device__ __forceinline__ bool mt_intersect(float4 a, Edge b, Edge c, V3 o, V3 d, float& t, float& u, float& v) {
     V3 v1 = v3(a), e1 = v3(b), e2 = v3(c);
     V3 P = cross(d, e2);
     float det = dot(e1, P);
@@ -375,9 +380,22 @@ __device__ __forceinline__ int trav_step(bool node_phase, const float4* nodes, c
         const uint32_t first = w & 0x0FFFFFFFu;
         const uint32_t count = ((w >> 28) & 7u) + 1u;
         r.leaf = kNoChild;
+        // The next record is fetched while one is tested: a leaf's two or three records waited
+        // for memory one after the other (wf_trace 70.7 -> 67.5 ms on 1080p x 128 spp over 1M
+        // triangles, 10.5 -> 10.1 on a 4K terrain; the megakernel 63.2 -> 60.7 ms on
+        // 1280 x 720 x 64 over 1M triangles). The edges are read without their fourth float,
+        // which saves registers in flight.
+        const Float3* tv = reinterpret_cast<const Float3*>(tris);
+        size_t tb = size_t(first) * 3;
+        float4 na = gload(tris, tb);
+        Float3 nb = gload(tv, tb + 1), nc = gload(tv, tb + 2);
         for (uint32_t k = 0; k < count; ++k) {
-            const size_t tb = size_t(first + k) * 3;
-            float4 a = gload(tris, tb), b = gload(tris, tb + 1), c = gload(tris, tb + 2);
+            const float4 a = na;
+            const Float3 b = nb, c = nc;
+            if (k + 1 < count) {
+                tb += 3;
+                na = gload(tris, tb), nb = gload(tv, tb + 1), nc = gload(tv, tb + 2);
+            }
             if (COUNT) cnt.tris++;
             float t, u, v;
             if (!mt_intersect(a, b, c, r.o, r.d, t, u, v)) continue;
@@ -395,7 +413,7 @@ __device__ __forceinline__ int trav_step(bool node_phase, const float4* nodes, c
                 if (!LEAN) {
                     best.u = u;
                     best.v = v;
-                    best.mat = __float_as_uint(b.w);
+                    best.mat = __float_as_uint(gload(tris, size_t(first + k) * 3 + 1).w);
                 }
             }
         }

@@ -310,12 +310,13 @@ __device__ __forceinline__ const T* wave_uniform(const T* p) {
 static_assert(PRT_EXTEND_PHASE_MIN >= 0 && PRT_EXTEND_PHASE_MIN <= 64, "phase threshold out of range");
 static_assert(PRT_SHADOW_PHASE_MIN >= 0 && PRT_SHADOW_PHASE_MIN <= 64, "phase threshold out of range");
 
-// Waves per SIMD of the traversal kernels: with the scene bases and the feeder in SGPRs,
-// wf_extend fits 8 (64 VGPRs, 2 spilled on rarely taken paths) and wf_shadow too (54, with
-// its rays set up by wf_shade: 35.6 -> 31.6 ms per frame of 1080p x 128 spp over 1M
-// triangles, against 72 VGPRs, 7 waves and the set-up in its refill).
-#ifndef PRT_TRACE_WAVES
-#define PRT_TRACE_WAVES __attribute__((amdgpu_waves_per_eu(8)))
+// Waves per SIMD of the traversal kernels: 8 with the scene bases and the feeder in SGPRs.
+// wf_trace then has 4 VGPRs too few and spills on rarely taken paths (7 waves, no spill:
+// 66.9 instead of 66.4 ms on 1080p x 128 spp over 1M triangles). Rays of several scenes hold
+// their bases in VGPRs too; at 8 waves that spills 8 in the loop (5.25 instead of 4.23 ms on
+// 12 views of several scenes), so there wf_trace keeps 7.
+#ifndef PRT_PACKET_WAVES
+#define PRT_PACKET_WAVES __attribute__((amdgpu_waves_per_eu(8)))
 #endif
 // wf_shade keeps the compiler's occupancy (104 VGPRs, 4 waves per SIMD): forcing 5
 // or 6 waves spills 36 / 104 bytes per lane and measured 2% / 12% slower per frame;
@@ -594,12 +595,13 @@ __device__ __forceinline__ void shadow_rays(const WfArgs& a, uint32_t it, StackT
 // by wf_shade(it - 1) and independent of each other, in one launch: a wave that finds no
 // more shadow rays goes on to extension rays, so the end of the one, where a few long rays
 // are left, is filled by the other, and in small queues (fewer batches than waves) the
-// first waves take the shadow rays while the last take the extension rays.(1280 x 720 x
-// 16 samples, 1M triangles, depth 8: wf_extend + wf_shadow 6.96 -> 6.13 ms per frame; 1080p x
+// first waves take the shadow rays while the last take the extension rays. (1280 x 720 x
+// 16 samples, 1M triangles, depth 8: 6.96 -> 6.13 ms per frame for the two together; 1080p x
 // 128: 73.9 -> 73.1; a 256 x 256 x 16 box: 376 -> 325 us.)
 enum : uint32_t { kTraceShadow = 1, kTraceExtend = 2 };
 template <bool COUNT, bool ONE_SCENE>
-__global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_trace(WfArgs a, uint32_t it, uint32_t parts) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(ONE_SCENE ? 8 : 7)))
+void wf_trace(WfArgs a, uint32_t it, uint32_t parts) {
     __shared__ int s_stack[kStackLdsQueue * kBlock];
     StackT<kStackLdsQueue> st;
     st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
@@ -636,7 +638,7 @@ __device__ __forceinline__ void per_scene_pass(bool live, uint32_t job, F&& f) {
 // lights, and later iterations' rays leave diffuse bounces in all directions.)
 static_assert(kBatch == 64 && kBlock == 64, "a packet is one fetch batch traced by one wave");
 template <bool COUNT, bool ONE_SCENE>
-__global__ __launch_bounds__(kBlock) PRT_TRACE_WAVES void wf_extend_packet(WfArgs a) {
+__global__ __launch_bounds__(kBlock) PRT_PACKET_WAVES void wf_extend_packet(WfArgs a) {
     __shared__ int s_pk[kPacketStack];
     const uint32_t n = uniform_u32(a.ctr[ext_count(0)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
