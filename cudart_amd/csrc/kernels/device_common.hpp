@@ -610,12 +610,19 @@ __device__ __forceinline__ void packet_traverse(const float4* nodes, const float
     }
 }
 
-// t, u, v and material of the closest hit best.rec of the ray (o, d), by the intersection
-// test that selected it (identical inputs, so identical results).
+// t, u, v and material of the closest hit best.rec of the ray (o, d), by the arithmetic of the
+// intersection test that selected it (mt_intersect; identical inputs, so identical results).
+// Without that test's branches the loads that follow can be sent out with these.
 __device__ __forceinline__ void hit_details(const float4* tris, V3 o, V3 d, HitRec& best) {
     const size_t tb = size_t(best.rec) * 3;
     const float4 a = gload(tris, tb), b = gload(tris, tb + 1), c = gload(tris, tb + 2);
-    mt_intersect(a, b, c, o, d, best.t, best.u, best.v);
+    const V3 v1 = v3(a), e1 = v3(b), e2 = v3(c);
+    const V3 P = cross(d, e2);
+    const float inv = 1.f / dot(e1, P);
+    const V3 T = o - v1, Q = cross(T, e1);
+    best.u = dot(T, P) * inv;
+    best.v = dot(d, Q) * inv;
+    best.t = dot(e2, Q) * inv;
     best.mat = __float_as_uint(b.w);
 }
 
@@ -629,8 +636,7 @@ __device__ __forceinline__ V3 shading_normal(float4 s0, float4 s1, float4 s2, fl
 
 // Software bilinear texture with wrap on linearised RGBA8 texels.
 __device__ __forceinline__ V3 tex_sample(const SceneArgs& sc, int tex, float u, float v) {
-    const uint4 info = sc.texinfo[tex];  // offset (texels), width, height
-    const uint8_t* px = sc.texels + size_t(info.x) * 4;
+    const uint4 info = gload(sc.texinfo, size_t(tex));  // offset (texels), width, height
     const int W = int(info.y), H = int(info.z);
     u = u - floorf(u);
     v = v - floorf(v);
@@ -646,8 +652,9 @@ __device__ __forceinline__ V3 tex_sample(const SceneArgs& sc, int tex, float u, 
     if (i0 < 0) i0 += W;
     if (j0 < 0) j0 += H;
     auto texel = [&](int i, int j) {
-        const uint8_t* p = px + (size_t(j) * W + i) * 4;
-        return V3{sc.lin[p[0]], sc.lin[p[1]], sc.lin[p[2]]};
+        const size_t p = (info.x + size_t(j) * W + i) * 4;
+        return V3{gload(sc.lin, gload(sc.texels, p)), gload(sc.lin, gload(sc.texels, p + 1)),
+                  gload(sc.lin, gload(sc.texels, p + 2))};
     };
     V3 a = texel(i0, j0) * (1.f - ax) + texel(i1, j0) * ax;
     V3 b = texel(i0, j1) * (1.f - ax) + texel(i1, j1) * ax;

@@ -71,14 +71,15 @@ struct RrInfo {
 // Shades the hit `h` of the current ray. Returns true when the path continues
 // (next ray in ps.ro / ps.rd, bounce incremented); sets *want_nee and fills `ns`
 // at a diffuse vertex whose chosen light is another triangle.
-// EAGER evaluates both Philox blocks of the bounce up front, independent of any
-// load (latency hiding in the shade kernel); otherwise only the blocks the
+// EAGER evaluates both Philox blocks of the bounce up front, independent of any load,
+// and reads the light's index (latency hiding in wf_shade); otherwise only the blocks the
 // material needs are evaluated (fewer registers in the megakernel). The values
-// are the same either way: a block depends only on (pixel, sample, bounce).
+// are the same either way: a block depends only on (pixel, sample, bounce). `normals` may
+// hold the hit's shading normals (three float4s), read by the caller.
 template <bool COUNT, bool EAGER, class RngType>
 __device__ __forceinline__ bool shade_vertex(const SceneArgs& sc, const PathArgs& pa, const RngType& rng, PathState& ps,
                                              const HitRec& h, bool* want_nee, NeeSample& ns, Counts& cnt,
-                                             RrInfo* rr = nullptr) {
+                                             RrInfo* rr = nullptr, const float4* normals = nullptr) {
     *want_nee = false;
     if (rr) rr->p = -1.f;
     const uint32_t b = ps.b;
@@ -88,10 +89,16 @@ __device__ __forceinline__ bool shade_vertex(const SceneArgs& sc, const PathArgs
         rb = rng.block(2u + 2u * b);
     }
     if (COUNT) cnt.hits++;
-    const float4* mp = sc.mats + size_t(h.mat) * 4;
-    const float4* shp = sc.shade + size_t(h.rec) * 4;
-    const float4 mkd = mp[0], mka = mp[1], mks = mp[2], maux = mp[3];
-    const float4 s0 = shp[0], s1 = shp[1], s2 = shp[2];
+    const size_t mp = size_t(h.mat) * 4, shp = size_t(h.rec) * 4;
+    const float4 mkd = gload(sc.mats, mp), mka = gload(sc.mats, mp + 1), mks = gload(sc.mats, mp + 2),
+                 maux = gload(sc.mats, mp + 3);
+    const float4 s0 = normals ? normals[0] : gload(sc.shade, shp), s1 = normals ? normals[1] : gload(sc.shade, shp + 1),
+                 s2 = normals ? normals[2] : gload(sc.shade, shp + 2);
+    uint32_t li = 0;
+    if (EAGER) {
+        const float pick = u01(ra.w) * (float(sc.num_lights) - .00001f);
+        li = gload(sc.lights, uint32_t(truncf(pick)));
+    }
     if (!EAGER) {
         const int k = __float_as_int(mkd.w);
         if (k == 0 || k == 2 || k == 4) ra = rng.block(1u + 2u * b);
@@ -173,7 +180,7 @@ __device__ __forceinline__ bool shade_vertex(const SceneArgs& sc, const PathArgs
         V3 kd = v3(mkd);
         const int tex = __float_as_int(mka.w);
         if (tex >= 0) {
-            const float4 s3 = shp[3];
+            const float4 s3 = gload(sc.shade, shp + 3);
             float bu = h.u, bv = h.v, bw = 1.f - bu - bv;
             // uv1 = (s2.y, s2.z), uv2 = (s2.w, s3.x), uv3 = (s3.y, s3.z)
             float tu = s2.y * bw + s2.w * bu + s3.y * bv;
@@ -184,8 +191,10 @@ __device__ __forceinline__ bool shade_vertex(const SceneArgs& sc, const PathArgs
 
         // Light choice (renderer.cu:218-221); estimateDirectLighting returns 0 when the
         // shading triangle is the chosen light (:421-423).
-        float pick = u01(ra.w) * (float(sc.num_lights) - .00001f);
-        const uint32_t li = sc.lights[uint32_t(truncf(pick))];
+        if (!EAGER) {
+            const float pick = u01(ra.w) * (float(sc.num_lights) - .00001f);
+            li = gload(sc.lights, uint32_t(truncf(pick)));
+        }
         if (h.rec != li) {
             float lu = u01(rb.x), lv = u01(rb.y);
             if (lu + lv >= 1.0f) {
@@ -230,8 +239,8 @@ __device__ __forceinline__ bool shade_vertex(const SceneArgs& sc, const PathArgs
 // visible iff nothing has (t, id) below (tL, light id) along the ray.
 template <bool COUNT>
 __device__ __forceinline__ bool nee_prepare(const SceneArgs& sc, const NeeSample& ns, ShadowReq& sr, Counts& cnt) {
-    const float4* lp = sc.tris + size_t(ns.li) * 3;
-    const float4 la = lp[0], lb = lp[1], lc = lp[2];
+    const size_t lp = size_t(ns.li) * 3, lsp = size_t(ns.li) * 4;
+    const float4 la = gload(sc.tris, lp), lb = gload(sc.tris, lp + 1), lc = gload(sc.tris, lp + 2);
     V3 pt = v3(la) + v3(lb) * ns.lu + v3(lc) * ns.lv;
     sr.so = ns.position + ns.normal * kEps;
     sr.sd = normalize(pt - ns.position);
@@ -240,15 +249,15 @@ __device__ __forceinline__ bool nee_prepare(const SceneArgs& sc, const NeeSample
         cnt.tris++;
     }
     float tL, uL, vL;
+    const float4 l0 = gload(sc.shade, lsp), l1 = gload(sc.shade, lsp + 1), l2 = gload(sc.shade, lsp + 2),
+                 l3 = gload(sc.shade, lsp + 3);
+    const float4 lka = gload(sc.mats, size_t(__float_as_uint(lb.w)) * 4 + 1);
     if (!mt_intersect(la, lb, lc, sr.so, sr.sd, tL, uL, vL)) return false;
-    const float4* lsp = sc.shade + size_t(ns.li) * 4;
-    const float4 l0 = lsp[0], l1 = lsp[1], l2 = lsp[2], l3 = lsp[3];
     if (COUNT) cnt.hits++;
     float sa = l3.w;
     float d2 = tL * tL;
     float cosT = fabsf(dot(shading_normal(l0, l1, l2, uL, vL), sr.sd * -1.0f));
     float wf = sa / (d2 * sc.lights_area) * cosT;
-    const float4 lka = sc.mats[size_t(__float_as_uint(lb.w)) * 4 + 1];
     sr.tL = tL;
     sr.lid = __float_as_uint(la.w);
     sr.direct = v3(0.f, 0.f, 0.f) + v3(lka) * wf;

@@ -194,7 +194,7 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 // flight is wave-uniform and stays in scalar registers.
 // What bounds small queues is this ending: with every wave asking all other counters one
 // after the other, each launch ended in 63 dependent loads, about 45 us (256 x 256 x 16 samples
-// of a 36-triangle box, depth 5: wf_extend and wf_shadow 632 -> 400 us per frame);
+// of a 36-triangle box, depth 5: the traversal launches 632 -> 400 us per frame);
 // one vector load of all 64 counters per wave still read each of their lines once
 // per wave, and cost a 0.9 ms packet launch 70 us.
 struct WaveFetch {
@@ -298,8 +298,27 @@ __device__ __forceinline__ const T* wave_uniform(const T* p) {
     return reinterpret_cast<const T*>((uint64_t(hi) << 32) | lo);
 }
 
-// Phase thresholds of the two traversal kernels (node_phase_for). On 1080p x 128
-// spp over 1M triangles, 24 measured best for both (extend 109 -> 92 ms, shadow
+// The first job's scene, by scalar loads.
+__device__ __forceinline__ SceneArgs uniform_scene(const WfJob* jobs) {
+    const SceneArgs& j = jobs->sc;
+    SceneArgs s;
+    s.nodes = sload(&j.nodes, 0);
+    s.tris = sload(&j.tris, 0);
+    s.shade = sload(&j.shade, 0);
+    s.mats = sload(&j.mats, 0);
+    s.lights = sload(&j.lights, 0);
+    s.texels = sload(&j.texels, 0);
+    s.texinfo = sload(&j.texinfo, 0);
+    s.lin = sload(&j.lin, 0);
+    s.lights_area = sload(&j.lights_area, 0);
+    s.inv_lights_area = sload(&j.inv_lights_area, 0);
+    s.num_lights = sload(&j.num_lights, 0);
+    s.num_records = sload(&j.num_records, 0);
+    return s;
+}
+
+// Phase thresholds of wf_trace's extension and shadow rays (node_phase_for). On 1080p x 128
+// spp over 1M triangles, 24 measured best for both (extension 109 -> 92 ms, shadow
 // 54 -> 43 ms per frame against no phases; 8 and 32 to 48 were slower).
 #ifndef PRT_EXTEND_PHASE_MIN
 #define PRT_EXTEND_PHASE_MIN 24
@@ -318,14 +337,6 @@ static_assert(PRT_SHADOW_PHASE_MIN >= 0 && PRT_SHADOW_PHASE_MIN <= 64, "phase th
 #ifndef PRT_PACKET_WAVES
 #define PRT_PACKET_WAVES __attribute__((amdgpu_waves_per_eu(8)))
 #endif
-// wf_shade keeps the compiler's occupancy (104 VGPRs, 4 waves per SIMD): forcing 5
-// or 6 waves spills 36 / 104 bytes per lane and measured 2% / 12% slower per frame;
-// with 256-thread workgroups at 5 waves (24 bytes spilled) and 128-thread ones at 6,
-// each with a grid of 20 / 24 waves per compute unit, 4% and 25% slower.
-#ifndef PRT_SHADE_WAVES
-#define PRT_SHADE_WAVES
-#endif
-
 // Adds the wave's counts to the counter slots; ANYHIT also books nodes and
 // triangles as the shadow (any-hit) kernel's share.
 template <bool ANYHIT>
@@ -443,18 +454,6 @@ __global__ __launch_bounds__(256) void wf_generate(WfArgs a) {
         // made by wf_shade(0): the slot is the queue position.
         a.qa[0][slot] = make_float4(ro.x, ro.y, ro.z, __uint_as_float(pixel | (t.job << 24)));
         a.qb[0][slot] = make_float4(rd.x, rd.y, rd.z, __uint_as_float(sample));
-    }
-}
-
-// Runs f(job) with the job index made wave-uniform (scalar loads of the job
-// descriptor) when every valid lane of the wave belongs to the same job.
-template <class F>
-__device__ __forceinline__ void with_job(bool valid, uint32_t job, F&& f) {
-    const uint32_t j0 = __builtin_amdgcn_readfirstlane(job);
-    if (__ballot(valid && job != j0) == 0ull) {
-        if (valid) f(j0);
-    } else {
-        if (valid) f(job);
     }
 }
 
@@ -629,7 +628,7 @@ __device__ __forceinline__ void per_scene_pass(bool live, uint32_t job, F&& f) {
     }
 }
 
-// wf_extend for the first iteration, whose queue holds the camera rays in 64-ray
+// The first iteration's extension rays, whose queue holds the camera rays in 64-ray
 // batches of 64 samples of a pixel or pixel block (wf_generate): nearly the same
 // ray in every lane. Each wave takes one batch at a time and traces it as a packet
 // (packet_traverse). On the 1080p 128-spp frame over 1M triangles this launch took
@@ -728,9 +727,23 @@ __device__ __forceinline__ uint32_t nonfinite(V3 m) {
 
 // Shades every hit of the queue, sets up the shadow rays of the light samples and
 // compacts the survivors. The colour the vertex adds starts at 0 (0 + x = x exactly) and
-// is added to the path's result; a visible light sample's part is added by wf_shadow.
-template <bool COUNT>
-__global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a, uint32_t it) {
+// is added to the path's result; a visible light sample's part is added by wf_trace.
+//
+// A path's loads are a chain (its entry and hit, the triangle, the material, the light), and
+// 16 waves per compute unit hide little of it, so the chain is kept short. With ONE_SCENE the
+// scene's arrays come from scalar registers: read through the job they took vector loads of
+// the descriptor before every other load (the compiler reads memory that the kernel may have
+// written, and the queues might be that, by vector loads), 23.05 -> 21.15 ms on 1080p x 128
+// spp over 1M triangles. The triangle's loads go out before the Philox blocks (-> 20.25),
+// the light's index, the light's records and its material before they are known to be needed
+// (24.8 -> 23.3 with hit_details without branches), all as global instead of flat loads
+// (-> 23.05). The launches now move 4.6 TB/s, the rate of a copy. 512-thread workgroups, 128
+// VGPRs: 5 or 6 waves per SIMD spilled and took 2 % and 12 % longer, 256- and 128-thread
+// workgroups at 5 and 6 waves 4 % and 25 %.
+template <bool COUNT, bool ONE_SCENE>
+__global__ __launch_bounds__(kShadeBlock) __attribute__((amdgpu_waves_per_eu(4)))
+void wf_shade(WfArgs a, uint32_t it) {
+    const SceneArgs shared = uniform_scene(a.jobs);
     const uint32_t q = it & 1u;
     const uint32_t n = uniform_u32(a.ctr[ext_count(it)]);
     Counts cnt = {0, 0, 0, 0, 0, 0};
@@ -765,23 +778,30 @@ __global__ __launch_bounds__(kShadeBlock) PRT_SHADE_WAVES void wf_shade(WfArgs a
         ps.prev = __float_as_uint(Cc.w) >> 31 ? 1 /*SPECULAR*/ : 0;
         ps.b = it;
         ps.input = it == 0 ? v3(0.f, 0.f, 0.f) : ps.rd;  // at b >= 1 the stale input is the ray direction
-        with_job(valid, pj >> 24, [&](uint32_t jb) {
-            const WfJob& j = a.jobs[jb];
-            if (rec == 0xFFFFFFFFu) {
-                path_miss(ps);
-            } else {
-                HitRec h;
-                h.rec = rec;
-                h.id = 0;
-                hit_details(j.sc.tris, ps.ro, ps.rd, h);
-                Rng rng{j.path.seed, j.path.view, pj & 0xFFFFFFu, sample};
-                more = shade_vertex<COUNT, true>(j.sc, j.path, rng, ps, h, &want_nee, ns, cnt);
-                if (want_nee && !(nee_prepare<COUNT>(j.sc, ns, sr, cnt) && can_hit(sr.sd))) {
-                    want_nee = false;  // the light sample cannot be seen: add mask * 0
-                    ps.color = add_direct(ps.color, ns.mask, sr.direct, false);
-                }
+        if (valid && rec == 0xFFFFFFFFu) {
+            path_miss(ps);
+        } else if (valid) {
+            const WfJob& j = a.jobs[pj >> 24];
+            const SceneArgs& sc = ONE_SCENE ? shared : j.sc;
+            const PathArgs path_args = j.path;
+            HitRec h;
+            h.rec = rec;
+            h.id = 0;
+            // With several scenes the normals' loads go out first as well (2.67 -> 2.49 ms on 12
+            // views); with one, 20.2 ms become 20.8 on 1080p x 128 spp.
+            float4 normals[3] = {};
+            if (!ONE_SCENE)
+                for (uint32_t k = 0; k < 3; ++k) normals[k] = gload(sc.shade, size_t(rec) * 4 + k);
+            __builtin_amdgcn_sched_barrier(0);
+            hit_details(sc.tris, ps.ro, ps.rd, h);
+            Rng rng{path_args.seed, path_args.view, pj & 0xFFFFFFu, sample};
+            more = shade_vertex<COUNT, true>(sc, path_args, rng, ps, h, &want_nee, ns, cnt, nullptr,
+                                             ONE_SCENE ? nullptr : normals);
+            if (want_nee && !(nee_prepare<COUNT>(sc, ns, sr, cnt) && can_hit(sr.sd))) {
+                want_nee = false;  // the light sample cannot be seen: add mask * 0
+                ps.color = add_direct(ps.color, ns.mask, sr.direct, false);
             }
-        });
+        }
         if (valid) {
             if (it == 0) {
                 a.result[slot] = make_float4(ps.color.x, ps.color.y, ps.color.z, 0.f);
@@ -1020,7 +1040,7 @@ void launch_chunk(const WfArgs& a, hipStream_t stream, uint32_t max_depth, int p
         else if (it == 0 || ev)
             trace(it, dev::kTraceExtend);
         mark(4 * it + 1);
-        hipLaunchKernelGGL(dev::wf_shade<COUNT>, dim3(sblocks), dim3(kShadeBlock), 0, stream, a, it);
+        hipLaunchKernelGGL((dev::wf_shade<COUNT, ONE_SCENE>), dim3(sblocks), dim3(kShadeBlock), 0, stream, a, it);
         mark(4 * it + 2);
         // The last iteration leaves no extension rays.
         trace(it + 1, ev || it + 1 == max_depth ? dev::kTraceShadow : dev::kTraceShadow | dev::kTraceExtend);
@@ -1531,8 +1551,8 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
     prt_tune bt{};
     // Every candidate is timed (best of two) on the trial cut into as many chunks as
     // the full run at that chunk size would take. Occupancy candidates stay near full
-    // occupancy: wf_extend fits 32 one-wave workgroups per CU (8 per SIMD), wf_shadow
-    // 28. Chunk counts: the fewest that fit the path slots (larger chunks were faster
+    // occupancy: wf_trace fits 32 one-wave workgroups per CU (8 per SIMD), 28 with several
+    // scenes. Chunk counts: the fewest that fit the path slots (larger chunks were faster
     // at every size measured on one view, since every chunk ends in nearly empty
     // iterations), and twice and four times as many.
     const uint64_t limit = max_slots(w);
