@@ -419,12 +419,16 @@ __device__ __forceinline__ PathOrder path_order(const WfTile& t, uint32_t width,
     o.rest = ns - o.full * o.m;
     return o;
 }
-// Pixel offset from the tile's first pixel of position q in bands of g rows, and back.
-__device__ __forceinline__ uint32_t position_to_pixel(const PathOrder& o, uint32_t g, uint32_t q) {
+// Pixel offset from the tile's first pixel of position q, in band `band` of bands of g rows
+// (a power of two), and back.
+__device__ __forceinline__ uint32_t position_to_pixel(const PathOrder& o, uint32_t g, uint32_t band, uint32_t q) {
     if (g == 1u) return q;
-    const uint32_t per = o.width * g, band = q / per, in = q - band * per;
-    const uint32_t h = min(g, o.rows - band * g), x = in / h;
+    const uint32_t in = q - band * (o.width * g), h = min(g, o.rows - band * g);
+    const uint32_t x = h == g ? in >> (31 - __builtin_clz(g)) : in / h;
     return (band * g + (in - x * h)) * o.width + x;
+}
+__device__ __forceinline__ uint32_t position_to_pixel(const PathOrder& o, uint32_t g, uint32_t q) {
+    return position_to_pixel(o, g, g == 1u ? 0u : q / (o.width * g), q);
 }
 __device__ __forceinline__ uint32_t pixel_to_position(const PathOrder& o, uint32_t g, uint32_t pixel) {
     if (g == 1u) return pixel;
@@ -433,23 +437,50 @@ __device__ __forceinline__ uint32_t pixel_to_position(const PathOrder& o, uint32
     return band * g * o.width + x * h + (y - band * g);
 }
 
+// n / d for inv = 1.0 / d, any 32-bit n and d >= 1: (n + 1/2) / d is at least 1 / (2d) from a
+// whole number, and the roundings of inv and of the product move it by less than 2^-20 / d.
+__device__ __forceinline__ uint32_t quotient(uint32_t n, double inv) { return uint32_t((double(n) + 0.5) * inv); }
+
+// The camera rays of the chunk's paths, one thread each, striding over the slots. Bound by
+// VALU issue: of about 400 instructions a path 200 were the divisions that find its tile's
+// order, pixel and sample. A thread now keeps its tile, the tile's order and the reciprocals
+// of its divisors until its slot leaves the tile, which hundreds of its slots share.
+// (2.70 -> 2.02 ms on 1080p x 128 spp, 0.55 -> 0.37 at 4K x 6 spp; 32 bytes a path are
+// written, 4.2 TB/s.)
 __global__ __launch_bounds__(256) void wf_generate(WfArgs a) {
     const WfChunk ch = current_chunk(a);
+    WfTile t;
+    PathOrder o;
+    uint32_t paths = 0, g_rest = 1, width = 1;  // `paths` slots from t.slot0 on are the tile's
+    double by_section = 0, by_m = 0, by_rest = 0, by_band = 0, by_band_rest = 0, by_width = 0;
+    t.slot0 = 0;
     for (uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x; slot < ch.paths; slot += gridDim.x * blockDim.x) {
-        const WfTile t = a.tiles[find_tile(a.tiles, ch.tile0, ch.ntiles, slot, false)];
+        if (slot - t.slot0 >= paths) {
+            t = a.tiles[find_tile(a.tiles, ch.tile0, ch.ntiles, slot, false)];
+            width = a.jobs[t.job].width;
+            o = path_order(t, width, a.group_lg);
+            paths = o.pixels * (t.s1 - t.s0);
+            g_rest = band_rows(o.rest);
+            by_section = 1.0 / double(o.pixels * o.m);
+            by_m = 1.0 / double(o.m);
+            by_rest = 1.0 / double(max(o.rest, 1u));
+            by_band = 1.0 / double(o.width * o.g);
+            by_band_rest = 1.0 / double(o.width * g_rest);
+            by_width = 1.0 / double(width);
+        }
         const WfJob& j = a.jobs[t.job];
-        const PathOrder o = path_order(t, j.width, a.group_lg);
-        const uint32_t r = slot - t.slot0, per = o.pixels * o.m;
-        const uint32_t sec = r / per, in = r - sec * per;
+        const uint32_t r = slot - t.slot0;
+        const uint32_t sec = quotient(r, by_section), in = r - sec * (o.pixels * o.m);
         const bool last = sec == o.full;
-        const uint32_t m = last ? o.rest : o.m;
-        const uint32_t q = in / m;
-        const uint32_t pixel = t.p0 + position_to_pixel(o, last ? band_rows(m) : o.g, q);
-        const uint32_t sample = t.s0 + sec * o.m + (in - q * m);
-        const int x = int(pixel % j.width), y = int(pixel / j.width);
+        const uint32_t q = quotient(in, last ? by_rest : by_m);
+        const uint32_t g = last ? g_rest : o.g;
+        const uint32_t band = g == 1u ? 0u : quotient(q, last ? by_band_rest : by_band);
+        const uint32_t pixel = t.p0 + position_to_pixel(o, g, band, q);
+        const uint32_t sample = t.s0 + sec * o.m + (in - q * (last ? o.rest : o.m));
+        const uint32_t row = quotient(pixel, by_width);
         Rng rng{j.path.seed, j.path.view, pixel, sample};
         V3 ro, rd;
-        camera_ray(j.cam, x, y, rng.block(0), ro, rd);
+        camera_ray(j.cam, int(pixel - row * width), int(row), rng.block(0), ro, rd);
         // C of a new path (throughput 1, no previous vertex, its slot) and its colour are
         // made by wf_shade(0): the slot is the queue position.
         a.qa[0][slot] = make_float4(ro.x, ro.y, ro.z, __uint_as_float(pixel | (t.job << 24)));
