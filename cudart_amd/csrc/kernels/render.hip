@@ -11,7 +11,7 @@ namespace prt {
 namespace dev {
 
 // samplePixel (src/renderer/renderer.cu:119-262) for one pixel-sample.
-template <bool COUNT>
+template <bool COUNT, uint32_t PHASE_MIN>
 __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArgs& pa, int x, int y, uint32_t sample,
                           Stack& st, Counts& cnt) {
     Rng rng{pa.seed, pa.view, uint32_t(y) * uint32_t(cam.xpixels) + uint32_t(x), sample};
@@ -29,7 +29,7 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
         h.rec = 0;
         h.mat = 0;
         h.u = h.v = 0.f;
-        if (!traverse<false, COUNT>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
+        if (!traverse<false, COUNT, false, PHASE_MIN>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
             path_miss(ps);
             break;
         }
@@ -47,7 +47,7 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
                 occ.rec = 0;
                 occ.mat = 0;
                 occ.u = occ.v = 0.f;
-                visible = !traverse<true, COUNT>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
+                visible = !traverse<true, COUNT, false, PHASE_MIN>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
             }
             ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
         }
@@ -125,12 +125,19 @@ struct BlockQueue {
 // meet the same surfaces, and a launch of 8 samples has 8 times the waves: 5.8 ms; 125 x 93 x 8
 // over 97,292 triangles (192 waves before) 5.3 -> 0.82. Held at 5 and 6 waves per SIMD it
 // spills 30 / 47 registers: 5.9 / 6.0 ms.
-template <bool COUNT>
+//
+// SHARED: lanes share pixels (lanes_lg != 0). Such a wave's lanes trace nearly the same
+// camera ray and reach their leaves together, so a leaf phase begins when fewer than 4 lanes
+// want nodes (961 x 541 x 8 over 1M triangles 4.92 -> 4.77 ms, 512 x 512 x 16 over 100k
+// 8.20 -> 7.86, 125 x 93 x 8 0.69 -> 0.63; thresholds 2 and 6 are 1 % behind). A wave of 64
+// pixels waits for the last lane (4: 640 x 480 x 1 186 -> 206 us, 1280 x 720 x 1 522 -> 560).
+template <bool COUNT, bool SHARED>
 __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
     __shared__ int s_stack[kStackLds * kBlock];
     __shared__ float s_rgb[3][kBlock];
-    const uint32_t lane = threadIdx.x, share = 1u << a.lanes_lg, sub = lane & (share - 1u), px = lane >> a.lanes_lg;
-    const uint32_t wlg = block_width_lg(a.lanes_lg), hlg = block_height_lg(a.lanes_lg);
+    const uint32_t lanes_lg = SHARED ? a.lanes_lg : 0u;
+    const uint32_t lane = threadIdx.x, share = 1u << lanes_lg, sub = lane & (share - 1u), px = lane >> lanes_lg;
+    const uint32_t wlg = block_width_lg(lanes_lg), hlg = block_height_lg(lanes_lg);
     Stack st;
     st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
     Counts cnt = {0, 0, 0, 0, 0, 0};
@@ -146,7 +153,7 @@ __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
             const uint32_t sample = a.s0 + k + sub;
             V3 L = v3(0.f, 0.f, 0.f);
             if (inside) {
-                L = sample_path<COUNT>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
+                L = sample_path<COUNT, SHARED ? 4u : 1u>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
                 if (a.samples && sample < a.samples_cap)
                     a.samples[idx * a.samples_cap + sample] = make_float4(L.x, L.y, L.z, 0.f);
             }
@@ -231,8 +238,9 @@ __global__ void mean_kernel(const float4* accum, uint32_t n, uint32_t samples, f
 }  // namespace dev
 
 hipError_t launch_megakernel(const MegaArgs& a, uint32_t grid, bool count, hipStream_t s) {
-    if (count) hipLaunchKernelGGL(dev::megakernel<true>, dim3(grid), dim3(kBlock), 0, s, a);
-    else hipLaunchKernelGGL(dev::megakernel<false>, dim3(grid), dim3(kBlock), 0, s, a);
+    auto kernel = a.lanes_lg != 0 ? count ? dev::megakernel<true, true> : dev::megakernel<false, true>
+                                  : count ? dev::megakernel<true, false> : dev::megakernel<false, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, a);
     return hipGetLastError();
 }
 
