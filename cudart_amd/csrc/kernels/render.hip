@@ -11,9 +11,10 @@ namespace prt {
 namespace dev {
 
 // samplePixel (src/renderer/renderer.cu:119-262) for one pixel-sample.
-template <bool COUNT, uint32_t PHASE_MIN>
+template <bool COUNT, bool SHARED>
 __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArgs& pa, int x, int y, uint32_t sample,
                           Stack& st, Counts& cnt) {
+    constexpr uint32_t kPhase = SHARED ? 4 : 1;
     Rng rng{pa.seed, pa.view, uint32_t(y) * uint32_t(cam.xpixels) + uint32_t(x), sample};
     V3 ro, rd;
     camera_ray(cam, x, y, rng.block(0), ro, rd);
@@ -29,10 +30,11 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
         h.rec = 0;
         h.mat = 0;
         h.u = h.v = 0.f;
-        if (!traverse<false, COUNT, false, PHASE_MIN>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
+        if (!traverse<false, COUNT, SHARED, kPhase, SHARED>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
             path_miss(ps);
             break;
         }
+        if (SHARED) hit_details(sc.tris, ps.ro, ps.rd, h);
         bool want_nee;
         NeeSample ns;
         const bool more = shade_vertex<COUNT, false>(sc, pa, rng, ps, h, &want_nee, ns, cnt);
@@ -47,7 +49,7 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
                 occ.rec = 0;
                 occ.mat = 0;
                 occ.u = occ.v = 0.f;
-                visible = !traverse<true, COUNT, false, PHASE_MIN>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
+                visible = !traverse<true, COUNT, false, kPhase, SHARED>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
             }
             ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
         }
@@ -131,6 +133,9 @@ struct BlockQueue {
 // want nodes (961 x 541 x 8 over 1M triangles 4.92 -> 4.77 ms, 512 x 512 x 16 over 100k
 // 8.20 -> 7.86, 125 x 93 x 8 0.69 -> 0.63; thresholds 2 and 6 are 1 % behind). A wave of 64
 // pixels waits for the last lane (4: 640 x 480 x 1 186 -> 206 us, 1280 x 720 x 1 522 -> 560).
+// It also fetches nodes a step ahead and keeps only the record of its best hit (4.76 -> 4.52,
+// 7.86 -> 7.59 and, 1280 x 720 x 64 over 1M triangles, 59.0 -> 56.1 ms); with 64 pixels, where
+// the leaf phases wait for every lane, fetching ahead takes 186 -> 191 us at 640 x 480 x 1.
 template <bool COUNT, bool SHARED>
 __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
     __shared__ int s_stack[kStackLds * kBlock];
@@ -153,7 +158,7 @@ __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
             const uint32_t sample = a.s0 + k + sub;
             V3 L = v3(0.f, 0.f, 0.f);
             if (inside) {
-                L = sample_path<COUNT, SHARED ? 4u : 1u>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
+                L = sample_path<COUNT, SHARED>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
                 if (a.samples && sample < a.samples_cap)
                     a.samples[idx * a.samples_cap + sample] = make_float4(L.x, L.y, L.z, 0.f);
             }
