@@ -17,7 +17,7 @@ is the same), and the ratio of the two rates is reported.
 
 Roofline of the dominant kernel: the extend launches (closest-hit traversal of
 every primary and extension ray; wf_extend_packet traces the first iteration's
-camera rays 64 at a time as packets, wf_extend the other iterations' rays one per
+camera rays 64 at a time as packets, wf_trace the other iterations' rays one per
 lane). The traversal is irregular pointer chasing with no dense
 contraction, so the roofline is HBM's (peak 8 TB/s). `achieved` = measured HBM
 bytes per extend launch (rocprofv3 FETCH_SIZE and WRITE_SIZE passes, each scaled
@@ -513,7 +513,7 @@ def main():
         ext_bytes = (nb * (st.nodes_visited - st.anyhit_nodes) + 48 * (st.tris_tested - st.anyhit_tris)
                      + 48 * st.hits + 52 * ext_rays)
         bytes_per_launch = ext_bytes / launches
-        kernel = "extend launches (wf_extend_packet + wf_extend)"
+        kernel = "extend launches (wf_extend_packet + wf_trace)"
         kernel_times = {"extend": round(sp.kernel_ms[0], 2), "shade": round(sp.kernel_ms[1], 2),
                         "shadow": round(sp.kernel_ms[2], 2), "launches_each": launches,
                         "profiled_frame_ms": round(sp.last_render_ms, 2)}

@@ -396,8 +396,8 @@ void write_node(float* o, const float* const boxes[4], const int32_t words[4]) {
 
 // Writes the four-wide layout depth first from the binary build tree. A node's
 // inner children get consecutive indices (siblings share cache lines and DRAM
-// pages): on the 1080p 1M-triangle frame wf_extend ran 0.7 %, wf_shadow 1.2 % and
-// the camera packets 0.9 % faster than with each child placed just before its
+// pages): on the 1080p 1M-triangle frame extension rays ran 0.7 %, shadow rays 1.2 %
+// and the camera packets 0.9 % faster than with each child placed just before its
 // own subtree (kernel traces, two interleaved runs).
 struct Emitter {
     const BNode* bn;
