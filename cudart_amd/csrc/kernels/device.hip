@@ -237,7 +237,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     HIP_TRY(copy_wait(r->gamma_lut, lut, 256, hipMemcpyHostToDevice, r->stream));
     if (c.keep_samples && spp > 0)
         HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->samples), px * spp * sizeof(float4)));
-    if (r->samples && c.integrator == PRT_INTEGRATOR_WAVEFRONT && vertices_fit(w, h, spp, c.max_depth)) {
+    if (r->samples && vertices_fit(w, h, spp, c.max_depth)) {
         // Only where there is room for them (without, the adjoint traces the paths again).
         size_t free_b = 0, total_b = 0;
         const size_t need = px * spp * c.max_depth * sizeof(uint32_t);
@@ -259,6 +259,62 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     PRT_TRY_END
 }
 
+namespace prt {
+// Results added to `accum`; the first `cap` samples of a pixel to `samples` and their paths'
+// vertices to `vertices`, unless null.
+MegaArgs megakernel_args(prt_renderer* r, float4* accum, float4* samples, uint32_t* vertices, uint32_t cap) {
+    MegaArgs a;
+    a.sc = r->sc;
+    a.cam = cam_args(r->cam);
+    a.path = PathArgs{r->cfg.seed, r->cfg.view_id, r->cfg.max_depth, r->cfg.rr_start};
+    a.width = r->w;
+    a.height = r->h;
+    a.accum = accum;
+    a.samples = samples;
+    a.vertices = vertices;
+    a.samples_cap = samples ? cap : 0;
+    a.counters = r->counters;
+    return a;
+}
+
+// Samples first .. first + n - 1 of every pixel by the megakernel, in launches of
+// spp_per_launch (0: powers of two).
+int megakernel_samples(prt_renderer* r, MegaArgs& a, uint32_t first, uint32_t n, uint32_t spp_per_launch, bool count) {
+    for (uint32_t done = 0; done < n;) {
+        uint32_t k = n - done;
+        if (spp_per_launch) {
+            k = std::min(k, spp_per_launch);
+        } else {  // the largest power of two, up to a wave's lanes
+            uint32_t p = 1;
+            while (p < 64 && 2 * p <= k) p *= 2;
+            k = p;
+        }
+        a.s0 = first + done;
+        a.nspp = k;
+        a.lanes_lg = 0;
+        while (a.lanes_lg < 6 && k % (2u << a.lanes_lg) == 0) ++a.lanes_lg;
+        const uint32_t bw = 1u << block_width_lg(a.lanes_lg), bh = 1u << block_height_lg(a.lanes_lg);
+        a.tiles_x = (r->w + bw - 1) / bw;
+        a.tiles = a.tiles_x * ((r->h + bh - 1) / bh);
+        if (r->ticket_sets_used == kTicketSets) {
+            HIP_TRY(hipMemsetAsync(r->tickets, 0, size_t(kTicketSets) * kTicketWords * sizeof(uint32_t), r->stream));
+            r->ticket_sets_used = 0;
+        }
+        a.tickets = r->tickets + size_t(r->ticket_sets_used++) * kTicketWords;
+        // 8x8 blocks: a workgroup each, which the spill area has room for; else the resident ones.
+        uint32_t grid = (a.tiles + 7) / 8 * 8;
+        if (a.lanes_lg != 0) grid = std::min(grid, r->compute_units * kMegaWaves);
+        int rc = ensure_spill(r, grid * kBlock);
+        if (rc != PRT_OK) return rc;
+        a.spill = r->spill;
+        a.spill_stride = r->spill_threads;
+        HIP_TRY(launch_megakernel(a, grid, count, r->stream));
+        done += k;
+    }
+    return PRT_OK;
+}
+}  // namespace prt
+
 extern "C" int prt_render_spp(prt_renderer* r, uint32_t n) {
     clear_error();
     if (!r) return fail(PRT_ERR_INVALID_ARG, "null argument");
@@ -276,48 +332,10 @@ extern "C" int prt_render_spp(prt_renderer* r, uint32_t n) {
         }
     }
     if (r->cfg.integrator == PRT_INTEGRATOR_WAVEFRONT) return render_wavefront(r, n);
-    MegaArgs a;
-    a.sc = r->sc;
-    a.cam = cam_args(r->cam);
-    a.path = PathArgs{r->cfg.seed, r->cfg.view_id, r->cfg.max_depth, r->cfg.rr_start};
-    a.width = r->w;
-    a.height = r->h;
-    a.accum = r->accum;
-    a.samples = r->samples;
-    a.samples_cap = r->samples ? r->spp : 0;
-    a.counters = r->counters;
+    MegaArgs a = megakernel_args(r, r->accum, r->samples, r->vertices, r->spp);
     HIP_TRY(hipEventRecord(r->ev0, r->stream));
-    for (uint32_t done = 0; done < n;) {
-        uint32_t k = n - done;
-        if (r->cfg.spp_per_launch) {
-            k = std::min(k, r->cfg.spp_per_launch);
-        } else {  // the largest power of two, up to a wave's lanes
-            uint32_t p = 1;
-            while (p < 64 && 2 * p <= k) p *= 2;
-            k = p;
-        }
-        a.s0 = r->samples_done + done;
-        a.nspp = k;
-        a.lanes_lg = 0;
-        while (a.lanes_lg < 6 && k % (2u << a.lanes_lg) == 0) ++a.lanes_lg;
-        const uint32_t bw = 1u << block_width_lg(a.lanes_lg), bh = 1u << block_height_lg(a.lanes_lg);
-        a.tiles_x = (r->w + bw - 1) / bw;
-        a.tiles = a.tiles_x * ((r->h + bh - 1) / bh);
-        if (r->ticket_sets_used == kTicketSets) {
-            HIP_TRY(hipMemsetAsync(r->tickets, 0, size_t(kTicketSets) * kTicketWords * sizeof(uint32_t), r->stream));
-            r->ticket_sets_used = 0;
-        }
-        a.tickets = r->tickets + size_t(r->ticket_sets_used++) * kTicketWords;
-        // 8x8 blocks: a workgroup each, which the spill area has room for; else the resident ones.
-        uint32_t grid = (a.tiles + 7) / 8 * 8;
-        if (a.lanes_lg != 0) grid = std::min(grid, r->compute_units * kMegaWaves);
-        rc = ensure_spill(r, grid * kBlock);
-        if (rc != PRT_OK) return rc;
-        a.spill = r->spill;
-        a.spill_stride = r->spill_threads;
-        HIP_TRY(launch_megakernel(a, grid, r->cfg.count_rays != 0, r->stream));
-        done += k;
-    }
+    rc = megakernel_samples(r, a, r->samples_done, n, r->cfg.spp_per_launch, r->cfg.count_rays != 0);
+    if (rc != PRT_OK) return rc;
     HIP_TRY(hipEventRecord(r->ev1, r->stream));
     HIP_TRY(hipEventSynchronize(r->ev1));
     float ms = 0.f;

@@ -77,6 +77,7 @@ struct MegaArgs {
     uint32_t* tickets;        // one per XCD, kTicketLine words apart: blocks of its band handed out beyond the first
     float4* accum;            // width*height, .xyz = running sum
     float4* samples;          // nullptr, or each sample's radiance at [pixel * samples_cap + sample]
+    uint32_t* vertices;       // nullptr, or with `samples`: its path's vertices, [(b * width * height + pixel) * samples_cap + sample]
     uint32_t samples_cap;     // samples stored per pixel
     unsigned long long* counters;  // kCntNum or nullptr
     int* spill;               // a row of spill_stride ints per stack entry beyond the LDS ones

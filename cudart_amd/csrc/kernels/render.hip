@@ -7,13 +7,16 @@
 // and renderKernel (src/renderer/parallel_renderer.cu:318-342) accumulate in.
 #include "path.hpp"
 
+#include <type_traits>
+
 namespace prt {
 namespace dev {
 
-// samplePixel (src/renderer/renderer.cu:119-262) for one pixel-sample.
-template <bool COUNT, bool SHARED>
+// samplePixel (src/renderer/renderer.cu:119-262) for one pixel-sample. With KEEP its vertices
+// go to vertex[b * stride], unless that is null.
+template <bool COUNT, bool SHARED, bool KEEP>
 __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArgs& pa, int x, int y, uint32_t sample,
-                          Stack& st, Counts& cnt) {
+                          uint32_t* vertex, size_t stride, Stack& st, Counts& cnt) {
     constexpr uint32_t kPhase = SHARED ? 4 : 1;
     Rng rng{pa.seed, pa.view, uint32_t(y) * uint32_t(cam.xpixels) + uint32_t(x), sample};
     V3 ro, rd;
@@ -32,10 +35,13 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
         h.u = h.v = 0.f;
         if (!traverse<false, COUNT, SHARED, kPhase, SHARED>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
             path_miss(ps);
+            if (KEEP && vertex) vertex[ps.b * stride] = kVertexMiss;
             break;
         }
         if (SHARED) hit_details(sc.tris, ps.ro, ps.rd, h);
         bool want_nee;
+        uint32_t word = h.rec;
+        uint32_t* at = vertex + ps.b * stride;
         NeeSample ns;
         const bool more = shade_vertex<COUNT, false>(sc, pa, rng, ps, h, &want_nee, ns, cnt);
         if (want_nee) {
@@ -52,7 +58,9 @@ __device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArg
                 visible = !traverse<true, COUNT, false, kPhase, SHARED>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
             }
             ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
+            if (visible) word |= kVertexLit;
         }
+        if (KEEP && vertex) *at = word;
         if (!more) break;
     }
     return ps.color;
@@ -136,7 +144,10 @@ struct BlockQueue {
 // It also fetches nodes a step ahead and keeps only the record of its best hit (4.76 -> 4.52,
 // 7.86 -> 7.59 and, 1280 x 720 x 64 over 1M triangles, 59.0 -> 56.1 ms); with 64 pixels, where
 // the leaf phases wait for every lane, fetching ahead takes 186 -> 191 us at 640 x 480 x 1.
-template <bool COUNT, bool SHARED>
+//
+// KEEP: a.vertices is given (an instantiation of its own: the 15 instead of 11 registers spilled
+// make the others 1 % slower).
+template <bool COUNT, bool SHARED, bool KEEP>
 __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
     __shared__ int s_stack[kStackLds * kBlock];
     __shared__ float s_rgb[3][kBlock];
@@ -158,9 +169,12 @@ __global__ __launch_bounds__(kBlock, 4) void megakernel(MegaArgs a) {
             const uint32_t sample = a.s0 + k + sub;
             V3 L = v3(0.f, 0.f, 0.f);
             if (inside) {
-                L = sample_path<COUNT, SHARED>(a.sc, a.cam, a.path, int(x), int(y), sample, st, cnt);
-                if (a.samples && sample < a.samples_cap)
-                    a.samples[idx * a.samples_cap + sample] = make_float4(L.x, L.y, L.z, 0.f);
+                const size_t path = idx * a.samples_cap + sample;
+                const bool keep = a.samples && sample < a.samples_cap;
+                L = sample_path<COUNT, SHARED, KEEP>(a.sc, a.cam, a.path, int(x), int(y), sample,
+                                               KEEP && keep ? a.vertices + path : nullptr,
+                                               size_t(a.width) * a.height * a.samples_cap, st, cnt);
+                if (keep) a.samples[path] = make_float4(L.x, L.y, L.z, 0.f);
             }
             if (share == 1u) {
                 sum = sum + L;
@@ -243,8 +257,12 @@ __global__ void mean_kernel(const float4* accum, uint32_t n, uint32_t samples, f
 }  // namespace dev
 
 hipError_t launch_megakernel(const MegaArgs& a, uint32_t grid, bool count, hipStream_t s) {
-    auto kernel = a.lanes_lg != 0 ? count ? dev::megakernel<true, true> : dev::megakernel<false, true>
-                                  : count ? dev::megakernel<true, false> : dev::megakernel<false, false>;
+    auto pick = [&](auto keep) {
+        constexpr bool kKeep = decltype(keep)::value;
+        return a.lanes_lg != 0 ? count ? dev::megakernel<true, true, kKeep> : dev::megakernel<false, true, kKeep>
+                               : count ? dev::megakernel<true, false, kKeep> : dev::megakernel<false, false, kKeep>;
+    };
+    auto kernel = a.vertices ? pick(std::true_type{}) : pick(std::false_type{});
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s, a);
     return hipGetLastError();
 }

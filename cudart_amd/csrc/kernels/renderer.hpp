@@ -36,7 +36,7 @@ struct prt_renderer {
     uint32_t kernel_launches[3] = {0, 0, 0};
     prt::WavefrontState* wf = nullptr;
     // keep_samples: radiance of pixel-sample (p, s) at samples[p * spp + s], s < spp, and
-    // (wavefront, where it fits) its path's vertex at bounce b at
+    // (where it fits) its path's vertex at bounce b at
     // vertices[(b * w * h + p) * spp + s]. Valid for the adjoint while every sample since the last reset was rendered with
     // the scene's current materials (samples_version).
     float4* samples = nullptr;
@@ -101,6 +101,8 @@ int render_wavefront(prt_renderer* r, uint32_t n);  // wavefront.hip
 // own accumulation or counters.
 int wavefront_samples(prt_renderer* r, uint32_t spp, float4* accum, float4* samples,
                       uint32_t* vertices);  // wavefront.hip
+MegaArgs megakernel_args(prt_renderer* r, float4* accum, float4* samples, uint32_t* vertices, uint32_t cap);  // device.hip
+int megakernel_samples(prt_renderer* r, MegaArgs& a, uint32_t first, uint32_t n, uint32_t spp_per_launch, bool count);
 // Whether path vertices of spp samples of this view can be kept (index and depth limits).
 inline bool vertices_fit(uint32_t w, uint32_t h, uint32_t spp, uint32_t max_depth) {
     return max_depth <= 16 && uint64_t(w) * h <= (1u << 24) && uint64_t(w) * h * spp < (uint64_t(1) << 32);

@@ -7,8 +7,7 @@ dLoss/dImage. Russian-roulette decisions are differentiated through their surviv
 probability; the loss change of such a decision is taken to second order with the
 curvature `hess` (d2Loss/dI2 per element: 2/(H*W*3) for the mean squared error, 0 for
 a first-order estimate). A renderer created with keep_samples=1 stores each sample's
-radiance and, with the wavefront integrator, its path's vertices in the forward pass,
-and backward then replays the paths without tracing them.
+radiance and its path's vertices in the forward pass, and backward then replays the paths without tracing them.
 """
 from __future__ import annotations
 

@@ -127,9 +127,9 @@ typedef struct prt_render_config {
                                          (0 = as many as fit) */
     uint32_t keep_samples;  /* 1 = also store each pixel-sample's radiance (16 B per pixel-sample, for
                                the first `spp` samples), so the adjoint replays paths without
-                               tracing them first; the wavefront also stores each path's vertices
-                               (4 B per sample and max_depth, when that fits in a quarter of the
-                               free device memory), so the replay traces no ray */
+                               tracing them first, and each path's vertices (4 B per sample and
+                               max_depth, when that fits in a quarter of the free device
+                               memory), so the replay traces no ray */
 } prt_render_config;
 
 /* Counters accumulated since the renderer was created (or reset). */

@@ -279,3 +279,26 @@ def test_replay_from_vertices_equals_traced_replay(gpu, monkeypatch, kind, w, h,
     for a, b, c in zip(from_kept, from_own, traced):
         np.testing.assert_array_equal(a, b)
         np.testing.assert_allclose(a, c, rtol=2.0 ** -22, atol=1e-9 * np.abs(c).max())
+
+
+# Vertices kept by either integrator's render, and those of the adjoint's own forward pass (by
+# the megakernel up to 2^20 paths, by the wavefront above): the same paths, so the same bits.
+# One pixel, ragged blocks, lanes sharing a pixel and not, both sides of the line.
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (17, 9, 5), (125, 93, 8), (128, 128, 64), (128, 128, 65)])
+def test_vertices_of_both_integrators_are_the_same(gpu, w, h, spp):
+    mesh = W.cornell100k(w, h).mesh
+    scene = ca.Scene(mesh)
+    grad = np.random.default_rng(6).standard_normal((h, w, 3)).astype(np.float32)
+    kw = dict(camera=mesh.camera, max_depth=7, rr_start=2, seed=12)
+    results = []
+    for integrator in (ca.INTEGRATOR_MEGAKERNEL, ca.INTEGRATOR_WAVEFRONT):
+        r = ca.ParallelRenderer(scene, w, h, spp, keep_samples=1, integrator=integrator, **kw)
+        r.render(spp)
+        results.append(r.adjoint_grad(grad, spp, hess=0.25))
+        r.close()
+    r = ca.ParallelRenderer(scene, w, h, spp, **kw)
+    results.append(r.adjoint_grad(grad, spp, hess=0.25))
+    r.close()
+    for other in results[1:]:
+        for a, b in zip(results[0], other):
+            np.testing.assert_array_equal(a, b)
