@@ -414,9 +414,9 @@ __global__ __launch_bounds__(kBlock) PRT_ADJOINT_WAVES void adjoint_kernel(AdjAr
 // A lane replays one path, 64 consecutive samples of a pixel to a wave, with the bounces in
 // step (the vertices, [bounce][pixel][sample], are read coalesced). The tracing replay waited
 // for node fetches for 0.43 of its waves' time, had 0.39 of its lanes active and takes 167
-// VGPRs; on 512^2 x 64 samples of the 100k-triangle scene it took 35.6 ms, this 3.15, and the
+// VGPRs; on 512^2 x 64 samples of the 100k-triangle scene it took 35.6 ms, this 3.01, and the
 // forward pass pays for the vertices with 4 bytes written per vertex (within its run-to-run
-// spread). What is left is the vertices' arithmetic (122 VGPRs, 4 waves per SIMD; held at 5:
+// spread). What is left is the vertices' arithmetic (127 VGPRs, 4 waves per SIMD; held at 5:
 // 3.31 ms). The fp64 sums in LDS are not what bounds it: 4 or 8 copies of them, a lane adding
 // to copy lane % 8, so that lanes meeting one material do not take turns, measured the same.
 //
