@@ -4,11 +4,10 @@
 //
 // Given dLoss/dI for every pixel (I = mean of `spp` samples), each sample's
 // radiance L has adjoint delta = dLoss/dI / spp. For each pixel-sample the kernel
-// takes L from the forward pass when the renderer kept it (keep_samples), or traces
-// the path once (primal, the megakernel's arithmetic) to get it, then replays the
-// path with the same Philox slots, keeping the radiance still to be collected,
-// rem = L - (what the path collected so far). With the path's vertices kept as well, the
-// replay traces no ray (adjoint_stored). Parameters:
+// takes L and the path's vertices from a forward pass that kept them (adjoint_stored), or
+// traces the path once (the megakernel's arithmetic) to get them (adjoint_traced), then
+// replays the path with the same Philox slots, tracing no ray, keeping the radiance still to
+// be collected, rem = L - (what the path collected so far). Parameters:
 //   kd_m (RGB)  a diffuse vertex multiplies everything collected after it by
 //               kd_c, so it contributes delta_c * rem_c / kd_c (rem taken after
 //               that vertex's emission, before its next-event estimate);
@@ -55,18 +54,10 @@ struct AdjArgs {
     uint32_t num_params;  // 4 * materials: kd (M*3) then emission (M)
     uint32_t num_materials;
     double* partial;      // grid x num_params (grid: tiles x parts rounded up to 8)
-    int* spill;
-    uint32_t spill_stride;
+    uint32_t stack_rows;  // entries of a traversal stack
 };
 
 namespace dev {
-
-// The replay's RNG: Philox with each product's low and high halves taken by
-// separate instructions. The 64-bit-product form takes this kernel from 167 to 172
-// VGPRs, 2 waves per SIMD instead of 3 (45.2 against 34.1 ms on 512^2 x 64 samples
-// of the 100k-triangle scene), or, held at 3 waves, spills two VGPRs to scratch
-// memory, which the allocation-free entry point should not need. Same bits.
-using AdjRng = RngT<false>;
 
 struct D3 {
     double x, y, z;
@@ -83,54 +74,6 @@ __device__ __forceinline__ D3 rr_weight(uint32_t ties) {
     return D3{(ties & 1u) ? w : 0.0, (ties & 2u) ? w : 0.0, (ties & 4u) ? w : 0.0};
 }
 
-// Traces the shadow ray of a next-event sample; true when the light is visible.
-template <class StackType>
-__device__ __forceinline__ bool shadow_visible(const SceneArgs& sc, const NeeSample& ns, ShadowReq& sr, StackType& st,
-                                               Counts& cnt) {
-    sr.direct = v3(0.f, 0.f, 0.f);
-    if (!nee_prepare<false>(sc, ns, sr, cnt)) return false;
-    HitRec occ;
-    occ.t = sr.tL;
-    occ.id = sr.lid;
-    occ.rec = 0;
-    occ.mat = 0;
-    occ.u = occ.v = 0.f;
-    return !traverse<true, false>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
-}
-
-// samplePixel's radiance (the megakernel's arithmetic).
-template <class StackType>
-__device__ V3 primal(const AdjArgs& a, int x, int y, uint32_t sample, StackType& st, Counts& cnt) {
-    const SceneArgs& sc = a.sc;
-    AdjRng rng{a.path.seed, a.path.view, uint32_t(y) * uint32_t(a.cam.xpixels) + uint32_t(x), sample};
-    V3 ro, rd;
-    camera_ray(a.cam, x, y, rng.block(0), ro, rd);
-    PathState ps;
-    path_init(ps, ro, rd);
-    while (true) {
-        HitRec h;
-        h.t = kFltMax;
-        h.id = 0;
-        h.rec = 0;
-        h.mat = 0;
-        h.u = h.v = 0.f;
-        if (!traverse<false, false>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
-            path_miss(ps);
-            break;
-        }
-        bool want_nee;
-        NeeSample ns;
-        const bool more = shade_vertex<false, false>(sc, a.path, rng, ps, h, &want_nee, ns, cnt);
-        if (want_nee) {
-            ShadowReq sr;
-            const bool visible = shadow_visible(sc, ns, sr, st, cnt);
-            ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
-        }
-        if (!more) break;
-    }
-    return ps.color;
-}
-
 // Materials of the path's untextured diffuse vertices, 8 bits each (at most 16).
 struct VertexList {
     uint64_t lo = 0, hi = 0;
@@ -145,12 +88,10 @@ struct VertexList {
     }
 };
 
-// The replay state of one pixel-sample, advanced a vertex at a time (replay_hit,
-// replay_after_nee) so that a lane whose path has ended can start the next sample
-// while the others go on. L comes from the primal pass of the same sample.
+// The replay state of one pixel-sample. L is its radiance.
 struct Replay {
     PathState ps;
-    AdjRng rng;
+    Rng rng;
     D3 rem, delta;
     V3 L;
     VertexList vl;
@@ -164,265 +105,22 @@ __device__ __forceinline__ void replay_begin(const AdjArgs& a, int x, int y, uin
     r.L = L;
     r.vl = VertexList();
     r.prev_ties = 0;
-    r.rng = AdjRng{a.path.seed, a.path.view, uint32_t(y) * uint32_t(a.cam.xpixels) + uint32_t(x), sample};
+    r.rng = Rng{a.path.seed, a.path.view, uint32_t(y) * uint32_t(a.cam.xpixels) + uint32_t(x), sample};
     V3 ro, rd;
     camera_ray(a.cam, x, y, r.rng.block(0), ro, rd);
     path_init(r.ps, ro, rd);
 }
 
-// A lane of the replay kernel traces either its path's extension ray or the shadow
-// ray of the vertex it has just shaded; the vertex's work is split at the shadow
-// ray: replay_hit() once the extension ray's closest hit is known, replay_after_nee()
-// once the shadow ray's visibility is known (or at once when there is none).
-// The *Done modes hold a lane whose traversal has ended until its vertex's work runs.
-enum : int { kLaneIdle = 0, kLaneExt = 1, kLaneShadow = 2, kLaneExtDone = 3, kLaneShadowDone = 4 };
-
-// What replay_after_nee() needs of the vertex that replay_hit() shaded.
-struct Pending {
-    V3 mask;         // the light sample's throughput
-    V3 direct;       // the light's contribution if visible
-    float wf;        // its geometric weight
-    uint32_t lmat;   // the light triangle's material
-    RrInfo rr;
-    uint32_t b, before;  // bounce index and diffuse vertices ahead of the vertex
-    bool more, want_nee;
-};
-
-__device__ __forceinline__ void ray_reset(HitRec& h, float t, uint32_t id) {
-    h.t = t;
-    h.id = id;
-    h.rec = 0;
-    h.mat = 0;
-    h.u = h.v = 0.f;
-}
-
-// Starts the closest-hit traversal of the path's current ray; false when its
-// direction cannot hit any triangle (the path then ends, as at a miss).
-template <class StackType>
-__device__ __forceinline__ bool start_ext(const Replay& r, TravRay& tr, HitRec& h, StackType& st) {
-    ray_reset(h, kFltMax, 0);
-    st.sp = 0;
-    return trav_begin(tr, r.ps.ro, r.ps.rd);
-}
-
-// The light term and the roulette terms of the vertex; then the next ray. Returns
-// the lane's next mode.
-template <class StackType>
-__device__ int replay_after_nee(const AdjArgs& a, Replay& r, const Pending& pd, bool visible, TravRay& tr, HitRec& h,
-                                double* g, StackType& st) {
-    const SceneArgs& sc = a.sc;
-    const double gain = 3.0 * double(sc.lights_area);  // d ka / d e
-    PathState& ps = r.ps;
-    if (pd.want_nee) {
-        if (visible) {
-            r.rem = dsub(r.rem, d3(pd.mask * pd.direct));
-            atomicAdd(&g[3 * a.num_materials + pd.lmat], ddot(r.delta, d3(pd.mask)) * gain * double(pd.wf));
-        }
-        ps.color = add_direct(ps.color, pd.mask, pd.direct, visible);
-    }
-    if (pd.rr.p >= 0.f && ps.b == pd.b + 1) {
-        // Survived roulette step j. Everything collected after it, R_j = L - C_j,
-        // carries 1/p_j, and with S_k[c] = sum over diffuse vertices v <= k of
-        // d log kd_{m_v,c}: d log p_j = w_j . S_j - w_{j-1} . S_{j-1}. The step adds
-        // -kappa_j d log p_j, with kappa_j = delta . R_j where p_j >= 1 (the path
-        // always survives; mask /= p_j is a deterministic rescale), and where
-        // p_j < 1 kappa_j = (hess / 2) |R_j / spp|^2: the score term of the survival
-        // probability times the loss change of that decision, delta . R_j -
-        // (hess / 2) |R_j / spp|^2, less the derivative of 1/p_j.
-        const D3 R = dsub(d3(r.L), d3(ps.color));
-        const double kappa = pd.rr.p >= 1.f ? ddot(r.delta, R) : a.half_hess * ddot(R, R);
-        if (kappa != 0.0) {
-            const D3 w = rr_weight(pd.rr.ties), wp = rr_weight(r.prev_ties);
-            for (uint32_t i = 0; i < r.vl.n; ++i) {
-                const uint32_t m = r.vl.at(i);
-                const float4 k4 = sc.mats[size_t(m) * 4];
-                const double kd[3] = {k4.x, k4.y, k4.z};
-                const double cf[3] = {i < pd.before ? wp.x - w.x : -w.x, i < pd.before ? wp.y - w.y : -w.y,
-                                      i < pd.before ? wp.z - w.z : -w.z};
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    if (cf[c] != 0.0 && kd[c] != 0.0) atomicAdd(&g[3 * m + c], kappa * cf[c] / kd[c]);
-            }
-        }
-        r.prev_ties = pd.rr.ties;
-    }
-    if (!pd.more) return kLaneIdle;
-    return start_ext(r, tr, h, st) ? kLaneExt : kLaneIdle;
-}
-
-// The vertex at the extension ray's closest hit h (hit = false: the sky, which
-// carries no parameter): emission and diffuse terms, shade_vertex and the light
-// sample, whose shadow ray the lane then traces. Returns the lane's next mode.
-template <class StackType>
-__device__ int replay_hit(const AdjArgs& a, Replay& r, HitRec& h, bool hit, Pending& pd, TravRay& tr, double* g,
-                          StackType& st, Counts& cnt) {
-    if (!hit) return kLaneIdle;
-    const SceneArgs& sc = a.sc;
-    const uint32_t M = a.num_materials;
-    const double gain = 3.0 * double(sc.lights_area);  // d ka / d e
-    PathState& ps = r.ps;
-    const float4 mkd = sc.mats[size_t(h.mat) * 4], mka = sc.mats[size_t(h.mat) * 4 + 1];
-    if (ps.b == 0 || ps.prev == 1 || ps.prev == 4) {
-        // the emission term shade_vertex is about to add
-        const V3 e = ps.mask * v3(mka) * sc.inv_lights_area;
-        atomicAdd(&g[3 * M + h.mat], ddot(r.delta, d3(ps.mask)) * gain * double(sc.inv_lights_area));
-        r.rem = dsub(r.rem, d3(e));
-    }
-    NeeSample ns;
-    pd.b = ps.b;
-    pd.more = shade_vertex<false, false>(sc, a.path, r.rng, ps, h, &pd.want_nee, ns, cnt, &pd.rr);
-    pd.before = r.vl.n;
-    if (ps.prev == 0 /*DIFFUSE*/ && __float_as_int(mka.w) < 0) {
-        const double kd[3] = {mkd.x, mkd.y, mkd.z};
-        const double rc[3] = {r.rem.x, r.rem.y, r.rem.z};
-        const double dc[3] = {r.delta.x, r.delta.y, r.delta.z};
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-            if (kd[c] != 0.0) atomicAdd(&g[3 * h.mat + c], dc[c] * rc[c] / kd[c]);
-        r.vl.push(h.mat);
-    }
-    if (pd.want_nee) {
-        ShadowReq sr;
-        sr.direct = v3(0.f, 0.f, 0.f);
-        const bool reach = nee_prepare<false>(sc, ns, sr, cnt);
-        pd.mask = ns.mask;
-        pd.direct = sr.direct;
-        pd.wf = sr.wf;
-        pd.lmat = sr.lmat;
-        if (reach) {
-            // The occlusion bound: the light sample itself, (t, id) as the closest hit.
-            ray_reset(h, sr.tL, sr.lid);
-            st.sp = 0;
-            if (trav_begin(tr, sr.so, sr.sd)) return kLaneShadow;
-            return replay_after_nee(a, r, pd, true, tr, h, g, st);  // no triangle can occlude it
-        }
-        return replay_after_nee(a, r, pd, false, tr, h, g, st);
-    }
-    return replay_after_nee(a, r, pd, false, tr, h, g, st);
-}
-
-// Occupancy of the replay kernel (empty: the compiler's choice, 3 waves per SIMD).
-#ifndef PRT_ADJOINT_WAVES
-#define PRT_ADJOINT_WAVES
-#endif
-// Idle lanes that make the wave start new pixel-samples. On 512^2 x 64 samples of
-// the 100k-triangle scene, one workgroup per tile: 1 lane 71.7 / 73.1 ms, 8: 72.7 /
-// 74.6, 16: 72.5 / 72.9, 32: 79.8 / 79.0 (two runs each); 6 workgroups per tile:
-// 1 lane 34.31 / 34.29 ms, 8: 34.04 / 34.11 (interleaved).
-#ifndef PRT_ADJOINT_REFILL
-#define PRT_ADJOINT_REFILL 8
-#endif
-constexpr uint32_t kAdjRefill = PRT_ADJOINT_REFILL;
-// Lanes whose traversal has ended wait until this many have (or none is still
-// traversing), then do their vertices' work together (512^2 x 64 samples of the
-// 100k-triangle scene: 16 lanes 73.8 ms, 32: 66.3, 48: 68.8; each vertex's work at
-// the step its traversal ended: 77.9; with 6 workgroups per tile 16: 37.7, 32: 34.3,
-// 48: 36.8).
-#ifndef PRT_ADJOINT_BATCH
-#define PRT_ADJOINT_BATCH 32
-#endif
-constexpr uint32_t kAdjBatch = PRT_ADJOINT_BATCH;
-// Lanes still wanting nodes below which the wave's step is a leaf phase. With the
-// lanes tracing independently most of them are mid-traversal at any step (512^2 x
-// 64 samples: 1 lane 66.7 ms, 8: 55.1, 12: 54.1, 16: 52.6, 20: 52.8, 24: 53.9; with
-// 6 workgroups per tile 8: 34.6, 16: 34.3, 24: 35.4).
-#ifndef PRT_ADJOINT_PHASE_MIN
-#define PRT_ADJOINT_PHASE_MIN 16
-#endif
-static_assert(kAdjRefill >= 1 && kAdjRefill <= 64, "refill threshold out of range");
-__global__ __launch_bounds__(kBlock) PRT_ADJOINT_WAVES void adjoint_kernel(AdjArgs a) {
-    __shared__ int s_stack[kStackLds * kBlock];
-    __shared__ double s_g[4 * PRT_MAX_MATERIALS];
-    for (uint32_t k = threadIdx.x; k < a.num_params; k += kBlock) s_g[k] = 0.0;
-    __syncthreads();
-    const uint32_t units = a.tiles * a.parts;
-    const uint32_t unit = xcd_tile(blockIdx.x, units);
-    const int lane = int(threadIdx.x);
-    if (unit < units) {
-        const uint32_t tile = unit / a.parts, part = unit - tile * a.parts;
-        Stack st;
-        st.bind(s_stack, a.spill + size_t(blockIdx.x) * kBlock, a.spill_stride);
-        Counts cnt = {0, 0, 0, 0, 0, 0};
-        // The wave works through its tile's pixel-samples in pixel-major order (64
-        // consecutive samples of one pixel are 64 nearly equal camera rays). A lane
-        // whose path has ended takes the next item, so the wave does not wait for
-        // each group's longest path (512^2 x 64 samples: 77.9 ms with one sample per
-        // lane per pixel and whole traversals in lockstep).
-        const uint32_t tx = (tile % a.tiles_x) * 8, ty = (tile / a.tiles_x) * 8;
-        const uint32_t cols = min(8u, a.width - tx), rows = min(8u, a.height - ty);
-        // This workgroup's share: items [i0, i1) of the tile's pixel-samples.
-        const uint64_t items = uint64_t(cols) * rows * a.spp;
-        const uint32_t i0 = uint32_t(items * part / a.parts), i1 = uint32_t(items * (part + 1) / a.parts);
-        const unsigned long long below = (1ull << lane) - 1ull;
-        uint32_t next = i0;  // the first item not yet taken (the same in every lane)
-        int mode = kLaneIdle;
-        Replay r;
-        TravRay tr;
-        tr.leaf = kNoChild;
-        HitRec h;
-        Pending pd;
-        // Each step advances every busy lane's traversal by one node or leaf phase;
-        // a lane whose traversal ends does that vertex's work and starts its next ray
-        // (shadow or extension) at once, so lanes do not wait for one another's
-        // traversals, and a lane whose path has ended takes the next pixel-sample.
-        bool found = false;  // the ended traversal's result: a hit (extension) or visibility (shadow)
-        while (true) {
-            const unsigned long long done = __ballot(mode >= kLaneExtDone);
-            if (done != 0ull && (uint32_t(__popcll(done)) >= kAdjBatch ||
-                                 __ballot(mode == kLaneExt || mode == kLaneShadow) == 0ull)) {
-                if (mode == kLaneExtDone) mode = replay_hit(a, r, h, found, pd, tr, s_g, st, cnt);
-                else if (mode == kLaneShadowDone) mode = replay_after_nee(a, r, pd, found, tr, h, s_g, st);
-            }
-            const unsigned long long idle = __ballot(mode == kLaneIdle);
-            const uint32_t nidle = uint32_t(__popcll(idle));
-            if ((nidle >= kAdjRefill || nidle == 64u) && next < i1) {
-                const uint32_t j = next + uint32_t(__popcll(idle & below));
-                if (mode == kLaneIdle && j < i1) {
-                    const uint32_t p = j / a.spp, s = j - p * a.spp;
-                    const int x = int(tx + p % cols), y = int(ty + p / cols);
-                    const size_t pix = size_t(y) * a.width + size_t(x);
-                    const D3 delta{a.norm * double(a.grad[pix * 3]), a.norm * double(a.grad[pix * 3 + 1]),
-                                   a.norm * double(a.grad[pix * 3 + 2])};
-                    const V3 L = a.samples ? v3(a.samples[pix * a.sample_cap + s])
-                                           : primal(a, x, y, s, st, cnt);
-                    replay_begin(a, x, y, s, delta, L, r);
-                    mode = start_ext(r, tr, h, st) ? kLaneExt : kLaneIdle;
-                }
-                next += nidle;
-            }
-            if (__ballot(mode != kLaneIdle) == 0ull && next >= i1) break;
-            const bool busy = mode == kLaneExt || mode == kLaneShadow;
-            const bool node_phase = node_phase_for<PRT_ADJOINT_PHASE_MIN>(busy && trav_wants_nodes(tr), busy);
-            if (busy) {
-                const int res = trav_step<false, false, false>(node_phase, a.sc.nodes, a.sc.tris, tr, kEps, h,
-                                                                     st, cnt, mode == kLaneShadow);
-                if (res != kTravRunning) {
-                    found = mode == kLaneExt ? (h.t != kFltMax || h.id != 0u) : res != kTravOccluded;
-                    mode = mode == kLaneExt ? kLaneExtDone : kLaneShadowDone;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    double* out = a.partial + size_t(blockIdx.x) * a.num_params;
-    for (uint32_t k = threadIdx.x; k < a.num_params; k += kBlock) out[k] = s_g[k];
-}
-
-// The replay from kept vertices: each closest hit's record and each light sample's
-// visibility are known, so no ray is traced; the vertex's work is the one above.
-//
-// A lane replays one path, 64 consecutive samples of a pixel to a wave, with the bounces in
-// step (the vertices, [bounce][pixel][sample], are read coalesced). The tracing replay waited
-// for node fetches for 0.43 of its waves' time, had 0.39 of its lanes active and takes 167
-// VGPRs; on 512^2 x 64 samples of the 100k-triangle scene it took 35.6 ms, this 3.01, and the
-// forward pass pays for the vertices with 4 bytes written per vertex (within its run-to-run
-// spread). What is left is the vertices' arithmetic (127 VGPRs, 4 waves per SIMD; held at 5:
-// 3.31 ms). The fp64 sums in LDS are not what bounds it: 4 or 8 copies of them, a lane adding
-// to copy lane % 8, so that lanes meeting one material do not take turns, measured the same.
-//
-// Russian roulette: step j adds kappa_j (w_{j-1} - w_j) for every diffuse vertex before the
-// step and -kappa_j w_j for the step's own (replay_after_nee). The first is the same for all
-// of them, so with P the running sum of kappa (w_{j-1} - w_j), a vertex adds
+// Russian roulette: everything collected after survived step j, R_j = L - C_j, carries 1/p_j,
+// and with S_k[c] = sum over diffuse vertices v <= k of d log kd_{m_v,c}:
+// d log p_j = w_j . S_j - w_{j-1} . S_{j-1}. The step adds -kappa_j d log p_j, with
+// kappa_j = delta . R_j where p_j >= 1 (the path always survives; mask /= p_j is a
+// deterministic rescale), and where p_j < 1 kappa_j = (hess / 2) |R_j / spp|^2: the score term
+// of the survival probability times the loss change of that decision, delta . R_j -
+// (hess / 2) |R_j / spp|^2, less the derivative of 1/p_j.
+// So it adds kappa_j (w_{j-1} - w_j) for every diffuse vertex before the step and
+// -kappa_j w_j for the step's own. The first is the same for all of them, so with P the
+// running sum of kappa (w_{j-1} - w_j), a vertex adds
 // -kappa_j w_j - P at its own step and P's last value when the path has ended: two adds per
 // vertex and channel instead of one per vertex, step and channel.
 // The vertex `word` of the path. Returns true when the path goes on.
@@ -483,10 +181,23 @@ __device__ __forceinline__ bool stored_vertex(const AdjArgs& a, Replay& r, uint3
     return more;
 }
 
-__global__ __launch_bounds__(kBlock) void adjoint_stored(AdjArgs a) {
-    extern __shared__ double s_sums[];  // num_params
+// A traversal stack with all its entries in LDS: AdjArgs::stack_rows rows of kBlock ints.
+struct LdsStack {
+    lds_int* lds;
+    int sp;
+    __device__ __forceinline__ void push(int v) { lds[sp++ * kBlock + threadIdx.x] = v; }
+    __device__ __forceinline__ int pop() { return lds[--sp * kBlock + threadIdx.x]; }
+};
+
+// A workgroup's share of the pixel-samples: their terms into its LDS sums, then into its
+// partials. Each closest hit's record and each light sample's visibility are known before a
+// path is replayed, kept by a forward pass or (TRACE) found by tracing the path just before.
+// The terms and the order in which they are added are the same either way, so the sums are
+// too, bit for bit.
+template <bool TRACE>
+__device__ __forceinline__ void replay_unit(const AdjArgs& a, double* sums, uint32_t* words, LdsStack& st) {
     const uint32_t lane = threadIdx.x;
-    for (uint32_t k = lane; k < a.num_params; k += kBlock) s_sums[k] = 0.0;
+    for (uint32_t k = lane; k < a.num_params; k += kBlock) sums[k] = 0.0;
     __syncthreads();
     const uint32_t units = a.tiles * a.parts;
     const uint32_t unit = xcd_tile(blockIdx.x, units);
@@ -496,35 +207,67 @@ __global__ __launch_bounds__(kBlock) void adjoint_stored(AdjArgs a) {
         const uint32_t cols = min(8u, a.width - tx), rows = min(8u, a.height - ty);
         const uint64_t items = uint64_t(cols) * rows * a.spp;
         const uint32_t i0 = uint32_t(items * part / a.parts), i1 = uint32_t(items * (part + 1) / a.parts);
-        const size_t stride = size_t(a.width) * a.height * a.sample_cap;
+        const size_t stride = TRACE ? kBlock : size_t(a.width) * a.height * a.sample_cap;
         Counts cnt = {0, 0, 0, 0, 0, 0};
         for (uint32_t j = i0 + lane; j < i1; j += kBlock) {
             const uint32_t p = j / a.spp, s = j - p * a.spp;
             const int x = int(tx + p % cols), y = int(ty + p / cols);
             const size_t pix = size_t(y) * a.width + size_t(x), path = pix * a.sample_cap + s;
+            const uint32_t* at = TRACE ? words + lane : a.vertices + path;
+            const V3 L = TRACE ? sample_path<false, true, true>(a.sc, a.cam, a.path, x, y, s, words + lane, stride,
+                                                                st, cnt)
+                               : v3(a.samples[path]);
             const D3 delta{a.norm * double(a.grad[pix * 3]), a.norm * double(a.grad[pix * 3 + 1]),
                            a.norm * double(a.grad[pix * 3 + 2])};
             Replay r;
-            replay_begin(a, x, y, s, delta, v3(a.samples[path]), r);
+            replay_begin(a, x, y, s, delta, L, r);
             D3 P{0.0, 0.0, 0.0};
-            const uint32_t* at = a.vertices + path;
             for (bool more = true; more; at += stride) {
                 const uint32_t word = *at;
-                more = word != kVertexMiss && stored_vertex(a, r, word, P, s_sums, cnt);  // the sky carries no parameter
+                more = word != kVertexMiss && stored_vertex(a, r, word, P, sums, cnt);  // the sky carries no parameter
             }
             if (P.x != 0.0 || P.y != 0.0 || P.z != 0.0)
                 for (uint32_t i = 0; i < r.vl.n; ++i) {
                     const uint32_t m = r.vl.at(i);
                     const float4 kd = a.sc.mats[size_t(m) * 4];
-                    if (kd.x != 0.f) atomicAdd(&s_sums[3 * m], P.x / double(kd.x));
-                    if (kd.y != 0.f) atomicAdd(&s_sums[3 * m + 1], P.y / double(kd.y));
-                    if (kd.z != 0.f) atomicAdd(&s_sums[3 * m + 2], P.z / double(kd.z));
+                    if (kd.x != 0.f) atomicAdd(&sums[3 * m], P.x / double(kd.x));
+                    if (kd.y != 0.f) atomicAdd(&sums[3 * m + 1], P.y / double(kd.y));
+                    if (kd.z != 0.f) atomicAdd(&sums[3 * m + 2], P.z / double(kd.z));
                 }
         }
     }
     __syncthreads();
     double* out = a.partial + size_t(blockIdx.x) * a.num_params;
-    for (uint32_t k = lane; k < a.num_params; k += kBlock) out[k] = s_sums[k];
+    for (uint32_t k = lane; k < a.num_params; k += kBlock) out[k] = sums[k];
+}
+
+// The replay from kept vertices: no ray is traced.
+//
+// A lane replays one path, 64 consecutive samples of a pixel to a wave, with the bounces in
+// step (the vertices, [bounce][pixel][sample], are read coalesced). A replay that traced the
+// rays itself waited for node fetches for 0.43 of its waves' time, had 0.39 of its lanes active
+// and took 167 VGPRs; on 512^2 x 64 samples of the 100k-triangle scene it took 35.6 ms, this
+// 3.01, and the forward pass pays for the vertices with 4 bytes written per vertex (within its
+// run-to-run spread). What is left is the vertices' arithmetic (127 VGPRs, 4 waves per SIMD;
+// held at 5: 3.31 ms). The fp64 sums in LDS are not what bounds it: 4 or 8 copies of them, a
+// lane adding to copy lane % 8, so that lanes meeting one material do not take turns, measured
+// the same.
+__global__ __launch_bounds__(kBlock) void adjoint_stored(AdjArgs a) {
+    extern __shared__ double s_sums[];  // num_params
+    LdsStack st{nullptr, 0};
+    replay_unit<false>(a, s_sums, nullptr, st);
+}
+
+// The replay where no vertices are kept: each wave traces its 64 paths as the megakernel
+// does, leaves their vertices in LDS (max_depth x 64 words) and replays them from there.
+// It allocates nothing and uses no scratch or spill memory: the traversal stacks, as deep as
+// the scene needs, are in LDS as well (9 KB for the 100k-triangle scene; 12 waves per compute
+// unit, what the registers allow, fit up to about 44 entries).
+__global__ __launch_bounds__(kBlock) void adjoint_traced(AdjArgs a) {
+    extern __shared__ double s_sums[];  // num_params, then the words and the stacks
+    uint32_t* words = reinterpret_cast<uint32_t*>(s_sums + a.num_params);
+    LdsStack st{(lds_int*)(words + a.path.max_depth * kBlock), 0};
+    replay_unit<true>(a, s_sums, words, st);
 }
 
 // Sums the per-workgroup partials of parameter blockIdx.x in a fixed order: thread t
@@ -587,8 +330,8 @@ namespace {
             goto done;                                          \
         }                                                       \
     } while (0)
-// PRT_ADJOINT_PRIMAL_IN_REPLAY=1: without kept radiance, trace each sample's primal
-// path inside the replay kernel even where the per-sample buffer would fit (tests).
+// PRT_ADJOINT_PRIMAL_IN_REPLAY=1: without kept vertices, trace each sample's
+// path inside the replay kernel even where the per-sample buffers would fit (tests).
 #define HIP_CHECK(expr)                                    \
     do {                                                   \
         hipError_t e_ = (expr);                            \
@@ -618,9 +361,6 @@ uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp) {
     uint64_t parts = std::max<uint64_t>(1, (kTargetUnits + tiles - 1) / tiles);
     parts = std::min<uint64_t>(parts, std::max<uint32_t>(1, spp));
     while (parts > 1 && ((tiles * parts + 7) / 8) * 8 * P + P > kStaticScratchDoubles) --parts;
-    // The tracing replay's workgroups each need their threads' columns of the spill area, made
-    // for the renderer's own sample count. (Where there were fewer columns than threads,
-    // workgroups of different parts wrote each other's entries.)
     while (parts > 1 && r->spill && ((tiles * parts + 7) / 8) * 8 * kBlock > r->spill_threads) --parts;
     return uint32_t(parts);
 }
@@ -652,18 +392,19 @@ AdjArgs adjoint_args(const prt_renderer* r, const float* grad, float hess, uint3
     a.num_params = 4 * r->scene->num_materials;
     a.num_materials = r->scene->num_materials;
     a.partial = partial;
-    a.spill = r->spill;
-    a.spill_stride = r->spill_threads;
+    a.stack_rows = stack_entries(r->scene);
     return a;
 }
 
-// The replay over `grid` workgroups: from kept vertices where there are any, else tracing
-// each path.
+// The replay over `grid` workgroups.
 hipError_t launch_adjoint(const AdjArgs& a, uint32_t grid, hipStream_t s) {
+    const size_t sums = a.num_params * sizeof(double);
+    // At most 4 + 4 + 32 KB.
+    const size_t rows = a.path.max_depth + a.stack_rows;
     if (a.vertices)
-        hipLaunchKernelGGL(dev::adjoint_stored, dim3(grid), dim3(kBlock), a.num_params * sizeof(double), s, a);
+        hipLaunchKernelGGL(dev::adjoint_stored, dim3(grid), dim3(kBlock), sums, s, a);
     else
-        hipLaunchKernelGGL(dev::adjoint_kernel, dim3(grid), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL(dev::adjoint_traced, dim3(grid), dim3(kBlock), sums + rows * kBlock * sizeof(int), s, a);
     return hipGetLastError();
 }
 }  // namespace
@@ -702,19 +443,19 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     AdjArgs a = adjoint_args(r, nullptr, hess, spp, nullptr);
     // Without kept vertices, a forward pass first writes each sample's radiance and
     // path vertices to buffers of this call (when they fit in a quarter of the free memory),
-    // and the replay traces no ray. Where only the radiance fits it traces the path's rays
-    // again, and where that does not fit either each lane traces its sample's primal path
-    // before replaying it. Radiance and vertices are the same either way.
-    bool forward = false, keep_vertices = false;
+    // and the replay traces no ray. Otherwise each lane traces its sample's path before
+    // replaying it. Radiance and vertices are the same either way, and so are the gradients.
+    bool forward = false;
     if (!a.vertices && !primal_in_replay()) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
             free_b += r->adjoint_bytes;
-            keep_vertices = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && b_acc + b_samp + b_vert <= free_b / 4;
-            forward = keep_vertices || (!a.samples && b_acc + b_samp <= free_b / 4);
+            forward = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && b_acc + b_samp + b_vert <= free_b / 4;
+            if (!forward && !a.samples && px > (size_t(1) << 24) && b_acc + b_samp <= free_b / 4)
+                return fail(PRT_ERR_LIMIT, "a view with more than 2^24 pixels");
         }
     }
-    const size_t bytes = b_grad + b_part + b_out + (forward ? b_acc + b_samp : 0) + (keep_vertices ? b_vert : 0);
+    const size_t bytes = b_grad + b_part + b_out + (forward ? b_acc + b_samp + b_vert : 0);
     rc = scratch_for(r->adjoint, r->adjoint_bytes, bytes);
     if (rc != PRT_OK) return rc;
     char* at = static_cast<char*>(r->adjoint);
@@ -723,7 +464,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     double* d_out = reinterpret_cast<double*>(at += b_part);
     float4* d_acc = reinterpret_cast<float4*>(at += b_out);
     float4* d_samp = reinterpret_cast<float4*>(at += b_acc);
-    uint32_t* d_vert = keep_vertices ? reinterpret_cast<uint32_t*>(at += b_samp) : nullptr;
+    uint32_t* d_vert = reinterpret_cast<uint32_t*>(at += b_samp);
     a.grad = d_grad;
     a.partial = d_part;
     ADJ_TRY(hipMemcpyAsync(d_grad, grad_rgb, px * 3 * sizeof(float), hipMemcpyHostToDevice, r->stream));
@@ -740,8 +481,6 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
             rc = wavefront_samples(r, spp, d_acc, d_samp, d_vert);
         }
         if (rc != PRT_OK) goto done;
-        a.spill = r->spill;  // the pass may have made it larger
-        a.spill_stride = r->spill_threads;
         a.samples = d_samp;
         a.vertices = d_vert;
         a.sample_cap = spp;

@@ -12,60 +12,6 @@
 namespace prt {
 namespace dev {
 
-// samplePixel (src/renderer/renderer.cu:119-262) for one pixel-sample. With KEEP its vertices
-// go to vertex[b * stride], unless that is null.
-template <bool COUNT, bool SHARED, bool KEEP>
-__device__ V3 sample_path(const SceneArgs& sc, const CamArgs& cam, const PathArgs& pa, int x, int y, uint32_t sample,
-                          uint32_t* vertex, size_t stride, Stack& st, Counts& cnt) {
-    constexpr uint32_t kPhase = SHARED ? 4 : 1;
-    Rng rng{pa.seed, pa.view, uint32_t(y) * uint32_t(cam.xpixels) + uint32_t(x), sample};
-    V3 ro, rd;
-    camera_ray(cam, x, y, rng.block(0), ro, rd);
-    PathState ps;
-    path_init(ps, ro, rd);
-    while (true) {
-        if (COUNT) {
-            if (ps.b == 0) cnt.primary++; else cnt.extension++;
-        }
-        HitRec h;
-        h.t = kFltMax;
-        h.id = 0;
-        h.rec = 0;
-        h.mat = 0;
-        h.u = h.v = 0.f;
-        if (!traverse<false, COUNT, SHARED, kPhase, SHARED>(sc, ps.ro, ps.rd, kEps, h, st, cnt)) {
-            path_miss(ps);
-            if (KEEP && vertex) vertex[ps.b * stride] = kVertexMiss;
-            break;
-        }
-        if (SHARED) hit_details(sc.tris, ps.ro, ps.rd, h);
-        bool want_nee;
-        uint32_t word = h.rec;
-        uint32_t* at = vertex + ps.b * stride;
-        NeeSample ns;
-        const bool more = shade_vertex<COUNT, false>(sc, pa, rng, ps, h, &want_nee, ns, cnt);
-        if (want_nee) {
-            ShadowReq sr;
-            sr.direct = v3(0.f, 0.f, 0.f);
-            bool visible = false;
-            if (nee_prepare<COUNT>(sc, ns, sr, cnt)) {
-                HitRec occ;
-                occ.t = sr.tL;
-                occ.id = sr.lid;
-                occ.rec = 0;
-                occ.mat = 0;
-                occ.u = occ.v = 0.f;
-                visible = !traverse<true, COUNT, false, kPhase, SHARED>(sc, sr.so, sr.sd, kEps, occ, st, cnt);
-            }
-            ps.color = add_direct(ps.color, ns.mask, sr.direct, visible);
-            if (visible) word |= kVertexLit;
-        }
-        if (KEEP && vertex) *at = word;
-        if (!more) break;
-    }
-    return ps.color;
-}
-
 template <bool COUNT>
 __device__ __forceinline__ void flush_counts(unsigned long long* out, const Counts& c) {
     // Wave-level sums, one atomic per wave and slot.

@@ -338,12 +338,11 @@ int prt_adjoint_grad(prt_renderer *r, const float *grad_rgb, float hess, uint32_
  * the caller's device memory on the renderer's device (W*H*3 floats, dLoss/dI), the
  * per-workgroup partial gradients live in a static 16 MiB device array (2^21
  * doubles) that each GPU holds until the process ends, and it never writes a
- * per-sample buffer: without radiance kept by the forward pass
- * (keep_samples) each sample's primal path is traced inside the replay. Limit:
+ * per-sample buffer: without path vertices kept by the forward pass
+ * (keep_samples) each sample's path is traced inside the replay. Limit:
  * ceil8(ceil(W/8) * ceil(H/8)) * 4M + 4M <= 2^21 (e.g. 1920x1080 with 16 materials);
- * larger calls fail with PRT_ERR_LIMIT. The gradients are the sums of
- * prt_adjoint_grad's fp64 terms for the same inputs (in another order where that call
- * keeps path vertices and this one has none). Calls that overlap on one GPU (several host threads) share its
+ * larger calls fail with PRT_ERR_LIMIT. The gradients equal prt_adjoint_grad's for
+ * the same inputs. Calls that overlap on one GPU (several host threads) share its
  * array and race; serialise them. d_albedo: M*3, d_emission: M (host, overwritten). */
 int prt_adjoint_grad_static(prt_renderer *r, const float *grad_rgb_device, float hess, uint32_t spp,
                             float *d_albedo, float *d_emission);

@@ -154,3 +154,37 @@ def stack_at_first_leaf(nodes: np.ndarray, origin, direction) -> int:
         node = hits[0][1]
         if node < 0:
             return depth
+
+
+def nested_quads(scales: int = 32, ratio: float = 1.6, per: int = 32):
+    """`per` quads at each of `scales` sizes, each size `ratio` times the last and as much
+    farther down the -z axis, and an emissive quad above at z = 3. A builder that splits off
+    the large ones first makes a deep tree, and a ray along -z meets every box on its way
+    down: it holds more than 32 stack entries at its first leaf."""
+    ps, ns, mids = [], [], []
+    for i in range(scales):
+        r = ratio ** i
+        for e in range(per):
+            z = -r * (1 + 0.1 * e / per)
+            p, n = quad([-r, -r, z], [r, -r, z], [r, r, z], [-r, r, z])
+            ps.append(p)
+            ns.append(n)
+            mids += [0, 0]
+    p, n = quad([-0.5, -0.5, 3], [-0.5, 0.5, 3], [0.5, 0.5, 3], [0.5, -0.5, 3])
+    ps.append(p)
+    ns.append(n)
+    mids += [1, 1]
+    return np.concatenate(ps), np.concatenate(ns), mids, [material(0), material(5, ka=(1, 1, 1))]
+
+
+def cancelling_grad(emission_grad, w: int, h: int, light: int, seed: int = 7) -> np.ndarray:
+    """A gradient image whose derivative with respect to material `light`'s emission cancels to
+    the rounding of its fp64 sum, so that the derivative's bits show the order of the sum.
+    emission_grad(image) gives the derivatives, which are linear in the image."""
+    grad = np.zeros((h, w, 3), np.float32)
+    grad[: h - 3] = np.random.default_rng(seed).standard_normal((h - 3, w, 3))
+    for row in range(h - 3, h):  # each row takes away what is left, to 24 bits of it
+        one = np.zeros_like(grad)
+        one[row] = 1
+        grad[row] = -emission_grad(grad)[light] / emission_grad(one)[light]
+    return grad

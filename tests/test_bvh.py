@@ -269,3 +269,15 @@ def test_stacked_quads_walk_deeper_than_the_lds_stack():
     down = [stack_at_first_leaf(nodes, (x, y, 2.0), (0.0, 0.0, -1.0)) for x, y in grid]
     shadow = [stack_at_first_leaf(nodes, (x, y, 1e-5), (-x / 401, -y / 401, -1.0)) for x, y in grid]
     assert min(down) > 16 and min(shadow) > 16, (down, shadow)
+
+
+def test_nested_quads_walk_deeper_than_every_lds_stack():
+    """The scene of the deep-stack tests: more than the megakernel's 32 LDS entries are held
+    when a ray along -z first reaches a leaf."""
+    from tests.helpers import OwnedDesc, nested_quads, stack_at_first_leaf
+    p, n, m, mats = nested_quads()
+    cam = ca.camera_look_at((0, 0, 2), (0, 0, 0), (0, 1, 0), 40, 64, 48)
+    od = OwnedDesc(p, n, m, mats, cam)
+    nodes, _, _ = ca.Scene(od.desc).export_bvh()
+    held = [stack_at_first_leaf(nodes, (x, y, 2.0), (0.0, 0.0, -1.0)) for x in (-0.4, 0.0, 0.3) for y in (-0.2, 0.1)]
+    assert min(held) > 32, held

@@ -302,3 +302,42 @@ def test_vertices_of_both_integrators_are_the_same(gpu, w, h, spp):
     for other in results[1:]:
         for a, b in zip(results[0], other):
             np.testing.assert_array_equal(a, b)
+
+
+def _deep_scene(w, h):
+    from tests.helpers import OwnedDesc, nested_quads
+    p, n, m, mats = nested_quads()
+    cam = ca.camera_look_at((0, 0, 2), (0, 0, 0), (0, 1, 0), 40, w, h)
+    od = OwnedDesc(p, n, m, mats, cam)
+    return ca.Scene(od.desc), cam, 1
+
+
+def _box_scene(w, h):
+    mesh = W.cornell100k(w, h).mesh
+    return ca.Scene(mesh), mesh.camera, next(i for i, m in enumerate(mesh.materials) if m.ka[0] > 0)
+
+
+# The replay from vertices that a forward pass left and the one that finds them by tracing add
+# the same terms in the same order: equal bits, also where the sum cancels to its rounding.
+# Ragged tiles, a tile's samples in one and in several workgroups, and stacks beyond 32 entries.
+@pytest.mark.parametrize("kind,w,h,spp,depth,rr_start", [
+    ("box", 17, 9, 5, 16, 0), ("box", 9, 23, 70, 6, 3), ("box", 96, 80, 8, 6, 3), ("deep", 33, 18, 1, 3, 3),
+    ("deep", 40, 31, 12, 4, 1)])
+def test_traced_replay_adds_in_the_order_of_the_stored_one(gpu, monkeypatch, kind, w, h, spp, depth, rr_start):
+    from tests.helpers import cancelling_grad
+    scene, cam, light = {"box": _box_scene, "deep": _deep_scene}[kind](w, h)
+    kw = dict(camera=cam, max_depth=depth, rr_start=rr_start, seed=11)
+    r = ca.ParallelRenderer(scene, w, h, spp, **kw)
+    kept = ca.ParallelRenderer(scene, w, h, spp, keep_samples=1, integrator=ca.INTEGRATOR_WAVEFRONT, **kw)
+    kept.render(spp)
+    cancel = cancelling_grad(lambda g: r.adjoint_grad(g, spp, hess=0.0)[1].astype(np.float64), w, h, light)
+    noisy = np.random.default_rng(5).standard_normal((h, w, 3)).astype(np.float32)
+    for grad, hess in ((cancel, 0.0), (noisy, 0.25)):
+        stored = r.adjoint_grad(grad, spp, hess=hess)
+        from_kept = kept.adjoint_grad(grad, spp, hess=hess)
+        with monkeypatch.context() as m:
+            m.setenv("PRT_ADJOINT_PRIMAL_IN_REPLAY", "1")
+            traced = r.adjoint_grad(grad, spp, hess=hess)
+        for a, b, c in zip(stored, from_kept, traced):
+            np.testing.assert_array_equal(a, b)
+            np.testing.assert_array_equal(a, c)

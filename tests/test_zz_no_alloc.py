@@ -97,3 +97,16 @@ def test_static_scratch_adjoint_refuses_bad_input(gpu):
     dev.close()
     assert rc == -9 and "static scratch" in _err()
     big.close()
+
+
+# Nothing kept: the two entry points add the same terms in the same order, so the bits agree
+# also where the light's derivative cancels to the rounding of its sum.
+@pytest.mark.parametrize("w,h,spp", [(17, 11, 3), (96, 64, 4), (64, 40, 33)])
+def test_static_scratch_adjoint_adds_in_the_same_order(gpu, w, h, spp):
+    from tests.helpers import cancelling_grad
+    scene, r, _, _ = _case(w, h, spp, False)
+    light = next(i for i, m in enumerate(W.cornell100k(w, h).mesh.materials) if m.ka[0] > 0)
+    grad = cancelling_grad(lambda g: r.adjoint_grad(g, spp, hess=0.0)[1].astype(np.float64), w, h, light)
+    (ra, re), (sa, se) = _grads(r, scene, grad, spp, 0.0)
+    assert np.array_equal(ra, sa) and np.array_equal(re, se), (np.abs(ra - sa).max(), re[light], se[light])
+    r.close()
