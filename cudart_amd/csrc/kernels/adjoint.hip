@@ -342,8 +342,6 @@ bool primal_in_replay() {
     return v && v[0] == '1';
 }
 
-// The replay's arguments for the renderer's view: seed, view, depth and the scene
-// as the renderer holds them; grad = W*H*3 dLoss/dI on the device.
 // Workgroups per 8x8 tile of the replay. One workgroup per tile left most of the GPU
 // idle for the second half of the kernel: 512^2 x 64 samples of the 100k-triangle
 // scene is 4,096 tiles against 3,072 resident waves (3 per SIMD), and the tiles'
@@ -352,8 +350,8 @@ bool primal_in_replay() {
 // pixel-samples into `parts` ranges gives about 8 workgroups per resident wave slot.
 // The partials (ceil8(tiles x parts) x 4 x materials doubles) must also fit the
 // allocation-free entry point's scratch, so both entry points pick the same split and
-// give the same sums.
-}  // namespace
+// give the same sums. Nothing that a call may change takes part: the same call gives the
+// same bits whatever came before it.
 uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp) {
     constexpr uint64_t kTargetUnits = 8ull * 3 * 4 * 256;  // 8 x (3 waves x 4 SIMDs x 256 CUs)
     const uint64_t tiles = std::max<uint32_t>(1, r->tiles);
@@ -361,11 +359,11 @@ uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp) {
     uint64_t parts = std::max<uint64_t>(1, (kTargetUnits + tiles - 1) / tiles);
     parts = std::min<uint64_t>(parts, std::max<uint32_t>(1, spp));
     while (parts > 1 && ((tiles * parts + 7) / 8) * 8 * P + P > kStaticScratchDoubles) --parts;
-    while (parts > 1 && r->spill && ((tiles * parts + 7) / 8) * 8 * kBlock > r->spill_threads) --parts;
     return uint32_t(parts);
 }
-namespace {
 
+// The replay's arguments for the renderer's view: seed, view, depth and the scene
+// as the renderer holds them; grad = W*H*3 dLoss/dI on the device.
 AdjArgs adjoint_args(const prt_renderer* r, const float* grad, float hess, uint32_t spp, double* partial) {
     AdjArgs a;
     a.sc = r->sc;

@@ -249,9 +249,8 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     }
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
-    // Room for the first-hit and the one-sample launch (a workgroup per tile) and for the
-    // adjoint's.
-    rc = ensure_spill(r.get(), (r->tiles * adjoint_parts(r.get(), std::max(1u, spp)) + 7) / 8 * 8 * kBlock);
+    // Room for the first-hit and the one-sample launch (a workgroup per tile).
+    rc = ensure_spill(r.get(), (r->tiles + 7) / 8 * 8 * kBlock);
     if (rc != PRT_OK) return rc;
     HIP_TRY(hipStreamSynchronize(r->stream));
     *out = r.release();

@@ -93,7 +93,6 @@ int set_device(int device);
 // megakernel.
 inline uint32_t stack_entries(const prt_scene* s) { return 3 * (s->bvh.max_depth + 1); }
 int ensure_spill(prt_renderer* r, uint32_t threads);
-uint32_t adjoint_parts(const prt_renderer* r, uint32_t spp);  // adjoint.hip
 int render_wavefront(prt_renderer* r, uint32_t n);  // wavefront.hip
 // Samples 0..spp-1 of the renderer's view into `accum` (zeroed), each sample's radiance
 // into `samples` ([pixel * spp + sample]) and, unless null, its path's vertices into

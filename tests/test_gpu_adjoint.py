@@ -341,3 +341,22 @@ def test_traced_replay_adds_in_the_order_of_the_stored_one(gpu, monkeypatch, kin
         for a, b, c in zip(stored, from_kept, traced):
             np.testing.assert_array_equal(a, b)
             np.testing.assert_array_equal(a, c)
+
+
+# The split of the sums depends on the call alone: not on the sample count that the renderer
+# was made for, nor on what earlier calls made it allocate.
+def test_repeated_gradients_have_the_same_bits(gpu):
+    from tests.helpers import cancelling_grad
+    w, h, spp = 96, 80, 16
+    scene, cam, light = _box_scene(w, h)
+    kw = dict(camera=cam, max_depth=6, seed=11)
+    made_for = ca.ParallelRenderer(scene, w, h, spp, **kw)
+    grad = cancelling_grad(lambda g: made_for.adjoint_grad(g, spp, hess=0.0)[1].astype(np.float64), w, h, light)
+    want = made_for.adjoint_grad(grad, spp, hess=0.0)
+    for integrator in (ca.INTEGRATOR_MEGAKERNEL, ca.INTEGRATOR_WAVEFRONT):
+        r = ca.ParallelRenderer(scene, w, h, 1, integrator=integrator, **kw)
+        for call in range(3):
+            if call == 2:
+                r.render(64)
+            for a, b in zip(r.adjoint_grad(grad, spp, hess=0.0), want):
+                np.testing.assert_array_equal(a, b)
