@@ -123,16 +123,23 @@ void gamma_table(uint8_t lut[256]) {
     }
 }
 
-int ensure_spill(prt_renderer* r, uint32_t threads) {
+// Resident workgroups of the megakernel (4 waves per SIMD).
+static uint32_t mega_resident(const prt_renderer* r) { return r->compute_units * 16; }
+
+int ensure_spill(prt_renderer* r, uint64_t columns) {
     const uint32_t entries = stack_entries(r->scene);
     if (entries <= uint32_t(kStackLdsQueue)) return PRT_OK;  // the smallest LDS stack of the kernels that use it
-    if (r->spill && r->spill_threads >= threads) return PRT_OK;
-    if (r->spill) (void)hipFree(r->spill);
-    r->spill = nullptr;
-    r->spill_threads = 0;
-    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->spill), size_t(entries - kStackLdsQueue) * threads * sizeof(int)));
-    r->spill_threads = threads;
-    return PRT_OK;
+    if (columns > UINT32_MAX) return fail(PRT_ERR_LIMIT, "image too large for the traversal stacks");
+    hipError_t e = hipSuccess;
+    const bool ok = grow(
+        r->spill, r->spill_columns, columns,
+        [&](uint64_t n) {
+            void* p = nullptr;
+            e = device_alloc(&p, size_t(entries - kStackLdsQueue) * n * sizeof(int));
+            return static_cast<int*>(e == hipSuccess ? p : nullptr);
+        },
+        [](int* p) { (void)hipFree(p); });
+    return ok ? PRT_OK : hip_fail(e, "traversal-stack spill area");
 }
 
 int scratch_for(void*& p, size_t& have, size_t bytes) {
@@ -144,9 +151,6 @@ int scratch_for(void*& p, size_t& have, size_t bytes) {
     have = bytes;
     return PRT_OK;
 }
-
-// Resident workgroups of the megakernel per compute unit (4 waves per SIMD).
-constexpr uint32_t kMegaWaves = 16;
 
 int set_device(int device) {
     int count = 0;
@@ -249,8 +253,11 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     }
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
-    // Room for the first-hit and the one-sample launch (a workgroup per tile).
-    rc = ensure_spill(r.get(), (r->tiles + 7) / 8 * 8 * kBlock);
+    // What the renderer was made for needs no allocation later. (A wavefront renderer's queues
+    // have a spill area of their own; this one is made if first hits are asked for.)
+    if (c.integrator == PRT_INTEGRATOR_MEGAKERNEL)
+        rc = ensure_spill(r.get(), std::max(first_hit_columns(w, h), mega_columns(w, h, std::max(1u, spp), c.spp_per_launch,
+                                                                                  mega_resident(r.get()))));
     if (rc != PRT_OK) return rc;
     HIP_TRY(hipStreamSynchronize(r->stream));
     *out = r.release();
@@ -279,36 +286,25 @@ MegaArgs megakernel_args(prt_renderer* r, float4* accum, float4* samples, uint32
 // Samples first .. first + n - 1 of every pixel by the megakernel, in launches of
 // spp_per_launch (0: powers of two).
 int megakernel_samples(prt_renderer* r, MegaArgs& a, uint32_t first, uint32_t n, uint32_t spp_per_launch, bool count) {
+    // Before the first launch: a failure leaves the accumulators as they were.
+    const int rc = ensure_spill(r, mega_columns(r->w, r->h, n, spp_per_launch, mega_resident(r)));
+    if (rc != PRT_OK) return rc;
+    a.spill = r->spill;
+    a.spill_stride = uint32_t(r->spill_columns);
     for (uint32_t done = 0; done < n;) {
-        uint32_t k = n - done;
-        if (spp_per_launch) {
-            k = std::min(k, spp_per_launch);
-        } else {  // the largest power of two, up to a wave's lanes
-            uint32_t p = 1;
-            while (p < 64 && 2 * p <= k) p *= 2;
-            k = p;
-        }
+        const MegaShape s = mega_shape(r->w, r->h, n - done, spp_per_launch, mega_resident(r));
         a.s0 = first + done;
-        a.nspp = k;
-        a.lanes_lg = 0;
-        while (a.lanes_lg < 6 && k % (2u << a.lanes_lg) == 0) ++a.lanes_lg;
-        const uint32_t bw = 1u << block_width_lg(a.lanes_lg), bh = 1u << block_height_lg(a.lanes_lg);
-        a.tiles_x = (r->w + bw - 1) / bw;
-        a.tiles = a.tiles_x * ((r->h + bh - 1) / bh);
+        a.nspp = s.samples;
+        a.lanes_lg = s.lanes_lg;
+        a.tiles_x = s.tiles_x;
+        a.tiles = s.tiles;
         if (r->ticket_sets_used == kTicketSets) {
             HIP_TRY(hipMemsetAsync(r->tickets, 0, size_t(kTicketSets) * kTicketWords * sizeof(uint32_t), r->stream));
             r->ticket_sets_used = 0;
         }
         a.tickets = r->tickets + size_t(r->ticket_sets_used++) * kTicketWords;
-        // 8x8 blocks: a workgroup each, which the spill area has room for; else the resident ones.
-        uint32_t grid = (a.tiles + 7) / 8 * 8;
-        if (a.lanes_lg != 0) grid = std::min(grid, r->compute_units * kMegaWaves);
-        int rc = ensure_spill(r, grid * kBlock);
-        if (rc != PRT_OK) return rc;
-        a.spill = r->spill;
-        a.spill_stride = r->spill_threads;
-        HIP_TRY(launch_megakernel(a, grid, count, r->stream));
-        done += k;
+        HIP_TRY(launch_megakernel(a, s.grid, count, r->stream));
+        done += s.samples;
     }
     return PRT_OK;
 }
@@ -419,6 +415,7 @@ extern "C" int prt_first_hit(prt_renderer* r, uint32_t sample, int32_t* tri, int
     if (rc != PRT_OK) return rc;
     const size_t n = size_t(r->w) * r->h;
     rc = scratch_for(r->out, r->out_bytes, n * 12);
+    if (rc == PRT_OK) rc = ensure_spill(r, first_hit_columns(r->w, r->h));
     if (rc != PRT_OK) return rc;
     char* buf = static_cast<char*>(r->out);
     FirstHitArgs a;
@@ -434,7 +431,7 @@ extern "C" int prt_first_hit(prt_renderer* r, uint32_t sample, int32_t* tri, int
     a.mat = reinterpret_cast<int32_t*>(buf + n * 4);
     a.t = reinterpret_cast<float*>(buf + n * 8);
     a.spill = r->spill;
-    a.spill_stride = r->spill_threads;
+    a.spill_stride = uint32_t(r->spill_columns);
     HIP_TRY(launch_first_hit(a, r->stream));
     CopyOut c[3];
     size_t parts = 0;

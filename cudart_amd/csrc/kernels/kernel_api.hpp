@@ -6,9 +6,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include "launch_shape.hpp"
+
 namespace prt {
 
-constexpr int kBlock = 64;       // one wave64 per workgroup: an 8x8 pixel tile
 constexpr int kStackLds = 32;    // traversal stack entries per lane in LDS (megakernel)
 #ifndef PRT_QUEUE_STACK_LDS
 #define PRT_QUEUE_STACK_LDS 16
@@ -104,21 +105,8 @@ hipError_t launch_tonemap(const float4* accum, uint32_t n, float inv_unused, uin
                           uint8_t* out, hipStream_t s);
 hipError_t launch_mean(const float4* accum, uint32_t n, uint32_t samples, float* out_rgb, hipStream_t s);
 
-// Pixel block of a wave in which 2^lg lanes share a pixel: 8x8, 8x4, 4x4, 4x2, 2x2, 2x1, 1x1.
-__host__ __device__ inline uint32_t block_width_lg(uint32_t lg) { return (7u - lg) / 2u; }
-__host__ __device__ inline uint32_t block_height_lg(uint32_t lg) { return 6u - lg - block_width_lg(lg); }
 constexpr uint32_t kTicketLine = 32;             // words between tickets: a cache line each
 constexpr uint32_t kTicketSets = 32;             // launches between two clearings
 constexpr uint32_t kTicketWords = 8 * kTicketLine;  // of one launch
-
-// Workgroup order: consecutive workgroups land on different XCDs (round robin),
-// so tile k is given to workgroup (k % per) * 8 + k / per, making each XCD's L2
-// see a contiguous band of tiles.
-__host__ __device__ inline uint32_t xcd_tile(uint32_t wg, uint32_t tiles) {
-    const uint32_t per = (tiles + 7) / 8;
-    uint32_t xcd = wg % 8, slot = wg / 8;
-    uint32_t t = xcd * per + slot;
-    return t;
-}
 
 }  // namespace prt

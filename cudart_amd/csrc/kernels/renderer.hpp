@@ -26,7 +26,7 @@ struct prt_renderer {
     uint32_t ticket_sets_used = 0;
     uint8_t* gamma_lut = nullptr;
     int* spill = nullptr;
-    uint32_t spill_threads = 0;
+    uint64_t spill_columns = 0;  // one per thread of a launch (ensure_spill)
     uint32_t tiles_x = 0, tiles = 0;  // 8x8 pixel tiles
     uint32_t compute_units = 0;
     uint32_t samples_done = 0;
@@ -92,7 +92,9 @@ int set_device(int device);
 // kStackMax rows it took 235 MB for the wavefront's resident threads, 0.8 GB for a 1080p
 // megakernel.
 inline uint32_t stack_entries(const prt_scene* s) { return 3 * (s->bvh.max_depth + 1); }
-int ensure_spill(prt_renderer* r, uint32_t threads);
+// At least `columns` columns of the renderer's spill area, where its scene needs one. Every launch
+// that uses the area calls this first, with its own threads.
+int ensure_spill(prt_renderer* r, uint64_t columns);
 int render_wavefront(prt_renderer* r, uint32_t n);  // wavefront.hip
 // Samples 0..spp-1 of the renderer's view into `accum` (zeroed), each sample's radiance
 // into `samples` ([pixel * spp + sample]) and, unless null, its path's vertices into

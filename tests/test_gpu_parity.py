@@ -198,3 +198,28 @@ def test_lanes_sharing_pixels_equal_one_per_pixel(gpu, w, h, spp, per):
         r.close()
     assert np.array_equal(imgs[0][0], imgs[1][0])
     assert imgs[0][1:] == imgs[1][1:]
+
+
+# Traversal stacks beyond every kernel's LDS entries (test_bvh.py walks the scene): first hits,
+# one lane to a pixel and several, launches of more samples than the renderer was made for, and a
+# renderer of the other integrator, whose stack area is made when it is first needed.
+@pytest.mark.parametrize("w,h", [(40, 31), (300, 200)])
+def test_deep_stacks_on_every_path(gpu, w, h):
+    from tests.helpers import OwnedDesc, nested_quads
+    p, n, m, mats = nested_quads()
+    cam = ca.camera_look_at((0, 0, 2), (0, 0, 0), (0, 1, 0), 40, w, h)
+    od = OwnedDesc(p, n, m, mats, cam)
+    scene = ca.Scene(od.desc)
+    orc, cfg = O.OracleScene(od.desc), O.cfg(max_depth=3, seed=5)
+    want = orc.first_hit(cam, w, h, 0, cfg)
+    acc, _ = orc.render(cam, w, h, 0, 8, cfg)
+    kw = dict(camera=cam, max_depth=3, seed=5)
+    for integrator in (ca.INTEGRATOR_MEGAKERNEL, ca.INTEGRATOR_WAVEFRONT):
+        r = ca.ParallelRenderer(scene, w, h, 1, integrator=integrator, **kw)
+        for _ in range(2):
+            for a, b in zip(r.first_hit(0), want):
+                assert np.array_equal(a, b)
+            r.reset()
+            r.render(8)
+            np.testing.assert_allclose(r.radiance(), acc / np.float32(8), rtol=1e-5, atol=1e-6)
+        r.close()
