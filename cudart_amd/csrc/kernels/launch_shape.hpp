@@ -61,6 +61,29 @@ constexpr uint64_t mega_columns(uint32_t w, uint32_t h, uint32_t n, uint32_t spp
     return most * kBlock;
 }
 
+// How a launch's waves share the 64-item batches of a queue (WaveFetch): wave w's first batch is
+// batch w, the batches from `waves` on belong to kSpread counters in turn, and a wave draws from
+// counter w % kSpread, then from kSteal others, 21 apart.
+#ifndef PRT_FETCH_BATCH
+#define PRT_FETCH_BATCH 64
+#endif
+constexpr uint32_t kSpread = 64;
+constexpr uint32_t kSteal = 2;  // other counters a wave tries when its own is exhausted
+constexpr uint32_t kBatch = PRT_FETCH_BATCH;  // items per fetch atomic
+// Batches of counter c, and the batch that its idx-th draw gives.
+constexpr uint32_t fetch_limit(uint32_t batches, uint32_t waves, uint32_t c) {
+    return batches > waves + c ? (batches - waves - c + kSpread - 1) / kSpread : 0u;
+}
+constexpr uint32_t fetch_batch(uint32_t waves, uint32_t c, uint32_t idx) { return waves + idx * kSpread + c; }
+constexpr uint32_t next_counter(uint32_t c) { return (c + 21u) % kSpread; }
+// Waves of a launch over `batches`: the resident ones, no more than there are batches, and at
+// least one for every counter: one that is no wave's own might not be among those tried, and its
+// rays would not be traced. (20 waves leave out batches of 41 to 62, more waves of none.)
+constexpr uint32_t trace_waves(uint32_t resident, uint32_t batches) {
+    const uint32_t waves = resident < kSpread ? kSpread : resident;
+    return batches < waves ? batches : waves;
+}
+
 // Makes an area of `have` units one of at least `need`. The old one goes only when the new one is
 // there: a failure leaves it, and the launches that it was large enough for, as they were.
 template <class T, class Make, class Release>

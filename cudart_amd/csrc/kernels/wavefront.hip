@@ -44,19 +44,13 @@ constexpr int kMaxIter = 64;
 // Same-address atomics serialise (about 11 ns each on MI355X), so work beyond each
 // wave's first batch is handed out by kSpread counters, one kBatch-item batch per
 // atomic, and appends to a queue are aggregated per workgroup.
-// Fetch counters per (kernel, iteration), items per fetch atomic, and shade
+// Fetch counters per (kernel, iteration), items per fetch atomic (launch_shape.hpp), and shade
 // workgroup size. With every counter on its own line, 1080p x 128 spp measured
 // within noise of 64 / 512 for batch 128 and 1024-thread shade workgroups;
 // 256-thread shade workgroups were 2-4 % slower.
-#ifndef PRT_FETCH_BATCH
-#define PRT_FETCH_BATCH 64
-#endif
 #ifndef PRT_SHADE_BLOCK
 #define PRT_SHADE_BLOCK 512
 #endif
-constexpr uint32_t kSpread = 64;
-constexpr uint32_t kSteal = 2;  // other counters a wave tries when its own is exhausted
-constexpr uint32_t kBatch = PRT_FETCH_BATCH;  // items per fetch atomic
 constexpr int kShadeBlock = PRT_SHADE_BLOCK;
 // Waves of wf_shade per compute unit in its grid (its occupancy limit, 4 waves per SIMD).
 #ifndef PRT_SHADE_GRID_WAVES
@@ -187,7 +181,8 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 // is batch w, with no atomic; the batches from `waves` on belong to kSpread counters
 // in turn, and a wave draws from counter (wave % kSpread): issue() sends the atomic
 // for its next batch before the current batch is processed, so the round trip
-// overlaps the traversal. When its counter is exhausted the wave tries kSteal others:
+// overlaps the traversal. When its counter is exhausted the wave tries kSteal others (every
+// counter is some wave's own, trace_waves, so none is left out):
 // neighbouring batches belong to different counters, so these run out at about the same
 // time and there is little to take over. A queue of at most `waves` batches costs no
 // atomic. resolve() returns the batch's first item or kNone. All of it but the atomic in
@@ -200,12 +195,6 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 struct WaveFetch {
     uint32_t* ctr;
     uint32_t k, nb, waves;
-    __device__ __forceinline__ uint32_t limit(uint32_t c) const {
-        return nb > waves + c ? (nb - waves - c + kSpread - 1) / kSpread : 0u;
-    }
-    __device__ __forceinline__ uint32_t item(uint32_t c, uint32_t idx) const {
-        return (waves + idx * kSpread + c) * kBatch;
-    }
     __device__ __forceinline__ uint32_t issue() const {
         uint32_t idx = kNone;
         if (nb > waves && (threadIdx.x & 63) == 0) idx = atomicAdd(ctr + k * kCtrLine, 1u);
@@ -214,14 +203,14 @@ struct WaveFetch {
     __device__ __forceinline__ uint32_t resolve(uint32_t raw) {
         if (nb <= waves) return kNone;
         uint32_t idx = uniform_u32(raw);
-        for (uint32_t tries = 0; idx >= limit(k); ++tries) {
+        for (uint32_t tries = 0; idx >= fetch_limit(nb, waves, k); ++tries) {
             if (tries == kSteal) return kNone;
-            k = (k + 21u) % kSpread;
+            k = next_counter(k);
             idx = kNone;
             if ((threadIdx.x & 63) == 0) idx = atomicAdd(ctr + k * kCtrLine, 1u);
             idx = uniform_u32(idx);
         }
-        return item(k, idx);
+        return fetch_batch(waves, k, idx) * kBatch;
     }
     // The wave's first batch (counted from the last wave if `reversed`); sets up the fetch
     // of the others.
@@ -1186,8 +1175,8 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, uint32_t en
                              : (one_scene ? reinterpret_cast<const void*>(dev::wf_trace<false, true>)
                                           : reinterpret_cast<const void*>(dev::wf_trace<false, false>));
     int cus = 0;
-    // No more waves than the largest queue has batches.
-    const int pblocks = std::min(persistent_blocks(ktrace, blocks_per_cu, device, &cus), int((need + kBatch - 1) / kBatch));
+    const int resident = persistent_blocks(ktrace, blocks_per_cu, device, &cus);
+    const int pblocks = int(trace_waves(uint32_t(resident), (need + kBatch - 1) / kBatch));
     const size_t rows = entries > uint32_t(kStackLdsQueue) ? entries - kStackLdsQueue : 0;
     int rc = ensure_state(w, device, need, rows * size_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;

@@ -2,6 +2,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <initializer_list>
+#include <vector>
 
 #include "launch_shape.hpp"
 
@@ -64,7 +65,48 @@ static void failed_growth_leaves_the_area() {
           "%d", freed);
 }
 
+// Batches that the waves of a launch hand out, each at most once; every wave in turn draws until
+// it finds nothing.
+static uint32_t handed_out(uint32_t batches, uint32_t waves) {
+    std::vector<uint32_t> counter(kSpread, 0), given(batches, 0);
+    for (uint32_t w = 0; w < waves; ++w) {
+        if (w >= batches) continue;
+        ++given[w];
+        if (batches <= waves) continue;
+        uint32_t k = w % kSpread;
+        while (true) {
+            uint32_t idx = counter[k]++, tries = 0;
+            for (; idx >= fetch_limit(batches, waves, k) && tries < kSteal; ++tries) {
+                k = next_counter(k);
+                idx = counter[k]++;
+            }
+            if (idx >= fetch_limit(batches, waves, k)) break;
+            const uint32_t b = fetch_batch(waves, k, idx);
+            CHECK(b < batches, "batch %u of %u", b, batches);
+            ++given[b];
+        }
+    }
+    uint32_t n = 0;
+    for (uint32_t g : given) {
+        CHECK(g <= 1, "a batch given %u times", g);
+        n += g;
+    }
+    return n;
+}
+
+static void every_batch_is_handed_out() {
+    for (uint32_t resident : {1u, 7u, 16u, 20u, 32u, 63u, 64u, 65u, 100u, 8192u})
+        for (uint32_t batches : {1u, 2u, 19u, 20u, 21u, 63u, 64u, 65u, 129u, 1000u, 20000u}) {
+            const uint32_t waves = trace_waves(resident, batches);
+            CHECK(waves >= 1 && waves <= batches, "%u waves, %u batches", waves, batches);
+            CHECK(handed_out(batches, waves) == batches, "%u waves, %u batches", waves, batches);
+        }
+    // What trace_waves is for: fewer waves than counters may leave batches.
+    CHECK(handed_out(50, 20) < 50, "%u", handed_out(50, 20));
+}
+
 int main() {
+    every_batch_is_handed_out();
     spill_fits_every_launch();
     failed_growth_leaves_the_area();
     std::puts("ok");
