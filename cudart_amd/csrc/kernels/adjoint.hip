@@ -425,8 +425,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     const uint32_t M = r->scene->num_materials;
     const uint32_t P = 4 * M;
     const uint32_t grid = ((r->tiles * adjoint_parts(r, spp) + 7) / 8) * 8;
-    // One block of the renderer's: gradient image, partials, results, and what a forward pass of
-    // this call keeps. It stays with the renderer unless it is large (at the end).
+    // One block: gradient image, partials, results, and what a forward pass of this call keeps.
     auto part = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     const size_t b_grad = part(px * 3 * sizeof(float)), b_part = part(size_t(grid) * P * sizeof(double));
     const size_t b_out = part(P * sizeof(double)), b_acc = part(px * sizeof(float4));
@@ -437,6 +436,10 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     } catch (const std::bad_alloc&) {
         return fail(PRT_ERR_OUT_OF_MEMORY, "host allocation failed");
     }
+    struct Lease {
+        Scratch s;
+        ~Lease() { give_scratch(s); }
+    } scratch{take_scratch(r->cfg.device, b_grad + b_part + b_out + b_acc + b_samp + b_vert)};
     float ms = 0.f;
     AdjArgs a = adjoint_args(r, nullptr, hess, spp, nullptr);
     // Without kept vertices, a forward pass first writes each sample's radiance and
@@ -447,16 +450,16 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     if (!a.vertices && !primal_in_replay()) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess) {
-            free_b += r->adjoint_bytes;
+            free_b += scratch.s.bytes;
             forward = vertices_fit(r->w, r->h, spp, r->cfg.max_depth) && b_acc + b_samp + b_vert <= free_b / 4;
             if (!forward && !a.samples && px > (size_t(1) << 24) && b_acc + b_samp <= free_b / 4)
                 return fail(PRT_ERR_LIMIT, "a view with more than 2^24 pixels");
         }
     }
     const size_t bytes = b_grad + b_part + b_out + (forward ? b_acc + b_samp + b_vert : 0);
-    rc = scratch_for(r->adjoint, r->adjoint_bytes, bytes);
+    rc = scratch_for(scratch.s.mem, scratch.s.bytes, bytes);
     if (rc != PRT_OK) return rc;
-    char* at = static_cast<char*>(r->adjoint);
+    char* at = static_cast<char*>(scratch.s.mem);
     float* d_grad = reinterpret_cast<float*>(at);
     double* d_part = reinterpret_cast<double*>(at += b_grad);
     double* d_out = reinterpret_cast<double*>(at += b_part);
@@ -493,16 +496,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     for (uint32_t k = 0; k < M; ++k) d_emission[k] = float(g[3 * M + k]);
     r->last_ms = ms;
 done:
-    if (rc != PRT_OK) (void)hipStreamSynchronize(r->stream);
-    {
-        size_t free_b = 0, total_b = 0;
-        if (r->adjoint_bytes > (size_t(64) << 20) &&
-            (hipMemGetInfo(&free_b, &total_b) != hipSuccess || r->adjoint_bytes > total_b / 16)) {
-            (void)hipFree(r->adjoint);
-            r->adjoint = nullptr;
-            r->adjoint_bytes = 0;
-        }
-    }
+    if (rc != PRT_OK) (void)hipStreamSynchronize(r->stream);  // nothing in flight uses the block
     return rc;
 }
 

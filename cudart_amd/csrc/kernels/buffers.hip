@@ -1,8 +1,9 @@
 // Memory that calls share or leave for the next one, and copies to the caller's buffers.
 //
-// Idle memory is bounded (two staging blocks, and one set of queues per device of at most
-// a sixteenth of its memory), is taken by one call at a time, and is given back when no
-// scene is on a device any more or when an allocation of the library finds no room.
+// Idle memory is bounded (two staging blocks, and per device one set of queues of at most a
+// sixteenth of its memory and as much in blocks of scratch memory), is taken by one call at a
+// time, and is given back when no scene is on a device any more or when an allocation of the
+// library finds no room.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,8 +35,13 @@ struct Stage {
     hipEvent_t done[kSegments] = {};
 };
 
+// Scratch blocks are few: a call takes one, so several are only left by several threads.
+constexpr int kMaxIdleScratch = 4;
+constexpr size_t kSmallScratch = size_t(64) << 20;  // kept without asking for the device's memory
+
 std::mutex g_mutex;
 Stage g_idle[kMaxIdleStages];  // device < 0: none
+Scratch g_idle_scratch[kMaxIdleScratch];  // mem == nullptr: none
 std::atomic<int> g_scenes{0};
 
 void free_stage(Stage& s) {
@@ -79,11 +85,15 @@ void give_stage(Stage& s) {
 
 void release_idle() {
     Stage all[kMaxIdleStages];
+    Scratch scratch[kMaxIdleScratch];
     {
         std::lock_guard<std::mutex> g(g_mutex);
         for (int k = 0; k < kMaxIdleStages; ++k) std::swap(all[k], g_idle[k]);
+        for (int k = 0; k < kMaxIdleScratch; ++k) std::swap(scratch[k], g_idle_scratch[k]);
     }
     for (Stage& s : all) free_stage(s);
+    for (Scratch& s : scratch)
+        if (s.mem) (void)hipFree(s.mem);
     release_idle_queues();
 }
 
@@ -103,6 +113,41 @@ hipError_t device_alloc(void** p, size_t bytes) {
         e = hipMalloc(p, bytes);
     }
     return e;
+}
+
+Scratch take_scratch(int device, size_t bytes) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    Scratch* best = nullptr;  // the smallest that is large enough, else the largest
+    for (Scratch& o : g_idle_scratch) {
+        if (!o.mem || o.device != device) continue;
+        if (!best || (best->bytes < bytes ? o.bytes > best->bytes : o.bytes >= bytes && o.bytes < best->bytes)) best = &o;
+    }
+    Scratch s;
+    if (best) std::swap(s, *best);
+    s.device = device;
+    return s;
+}
+
+void give_scratch(Scratch& s) {
+    if (!s.mem) return;
+    size_t free_b = 0, total_b = 0;
+    if (s.bytes > kSmallScratch && hipMemGetInfo(&free_b, &total_b) != hipSuccess) total_b = 0;
+    {
+        std::lock_guard<std::mutex> g(g_mutex);
+        Scratch* slot = nullptr;
+        size_t idle = s.bytes;
+        for (Scratch& o : g_idle_scratch) {
+            if (!o.mem) slot = &o;
+            else if (o.device == s.device) idle += o.bytes;
+        }
+        if (slot && g_scenes.load() > 0 && (s.bytes <= kSmallScratch || idle <= total_b / 16)) {
+            *slot = s;
+            s = Scratch();
+            return;
+        }
+    }
+    (void)hipFree(s.mem);
+    s = Scratch();
 }
 
 hipError_t copy_out(const CopyOut* c, size_t n, int device, hipStream_t stream) {

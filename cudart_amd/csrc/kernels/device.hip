@@ -481,7 +481,7 @@ extern "C" int prt_renderer_destroy(prt_renderer* r) {
     (void)hipSetDevice(r->cfg.device);
     release_wavefront(r);
     if (r->stream) (void)hipStreamSynchronize(r->stream);
-    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices, r->out, r->adjoint};
+    void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices, r->out};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (r->ev0) (void)hipEventDestroy(r->ev0);

@@ -42,12 +42,10 @@ struct prt_renderer {
     float4* samples = nullptr;
     uint32_t* vertices = nullptr;
     bool samples_ok = false;
-    // Device memory of the calls that hand results out, kept until the renderer goes (at most
-    // 12 bytes per pixel), and of the adjoint (scratch_for).
+    // Device memory of the calls that hand results out, kept until the renderer goes: at most
+    // 12 bytes per pixel (scratch_for).
     void* out = nullptr;
     size_t out_bytes = 0;
-    void* adjoint = nullptr;
-    size_t adjoint_bytes = 0;
     uint64_t samples_version = 0;
 };
 
@@ -75,12 +73,22 @@ struct CopyOut {
     size_t bytes;
 };
 hipError_t copy_out(const CopyOut* c, size_t n, int device, hipStream_t stream);
+// Device memory of one call (scratch_for makes it large enough). take_scratch gives an idle block of
+// the device, if possible of at least `bytes`, or an empty one; give_scratch takes it back, once no
+// launch uses it any more, and keeps or frees it.
+struct Scratch {
+    int device = -1;
+    void* mem = nullptr;
+    size_t bytes = 0;
+};
+Scratch take_scratch(int device, size_t bytes);
+void give_scratch(Scratch& s);
 // While a scene is on a device, idle memory is kept for the next call.
 void scene_uploaded();
 void scene_released();
 bool scenes_on_devices();
 void release_idle_queues();  // wavefront.hip
-// At least `bytes` of the renderer's scratch memory p (of `have` bytes), grown as needed.
+// At least `bytes` of scratch memory p (of `have` bytes), grown as needed; its contents are lost.
 int scratch_for(void*& p, size_t& have, size_t bytes);
 // Uploads the scene to `device` on first use (copies ordered on `stream`).
 int device_scene(prt_scene* s, int device, SceneArgs& out, hipStream_t stream);

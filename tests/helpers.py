@@ -188,3 +188,13 @@ def cancelling_grad(emission_grad, w: int, h: int, light: int, seed: int = 7) ->
         one[row] = 1
         grad[row] = -emission_grad(grad)[light] / emission_grad(one)[light]
     return grad
+
+
+def device_free_bytes() -> int:
+    """Free memory of the current device, from the HIP runtime that libprt.so uses."""
+    import cudart_amd as ca
+    ca.lib()
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64.so" in l and "torch" not in l)
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL(path).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value

@@ -360,3 +360,23 @@ def test_repeated_gradients_have_the_same_bits(gpu):
                 r.render(64)
             for a, b in zip(r.adjoint_grad(grad, spp, hess=0.0), want):
                 np.testing.assert_array_equal(a, b)
+
+
+# The memory of a gradient call is one block for all renderers, not one each.
+def test_gradients_of_several_renderers_share_their_memory(gpu):
+    from tests.helpers import device_free_bytes
+    w, h, spp = 512, 256, 64
+    scene, cam, _ = _box_scene(w, h)
+    grad = np.random.default_rng(9).standard_normal((h, w, 3)).astype(np.float32)
+    block = w * h * spp * (16 + 4 * 6)  # radiance and vertices
+    left, renderers, results = [], [], []
+    for seed in (1, 2, 3, 1):
+        renderers.append(ca.ParallelRenderer(scene, w, h, spp, camera=cam, max_depth=6, seed=seed))
+        results.append(renderers[-1].adjoint_grad(grad, spp, hess=0.25))
+        left.append(device_free_bytes())
+    assert left[0] - left[-1] < block, left
+    for a, b in zip(results[0], results[-1]):
+        np.testing.assert_array_equal(a, b)
+    for r in renderers:
+        r.close()
+    scene.close()

@@ -140,3 +140,31 @@ def test_batch_calls_share_no_results(gpu):
         t.join()
     for k in range(4):
         assert np.array_equal(first[k], got[k])
+
+
+# Gradients from more threads than scratch blocks are kept, of sizes that share blocks in any
+# order: each call has its block to itself.
+def test_gradients_from_several_threads(gpu):
+    scene = ca.Scene(W.cornell100k(64, 48).mesh)
+    cam = W.cornell100k(64, 48).camera
+
+    def gradients(seed, out):
+        w, h, spp = 64, 48, 1 + 7 * seed
+        r = ca.ParallelRenderer(scene, w, h, spp, camera=cam, max_depth=5, seed=seed)
+        grad = np.random.default_rng(seed).standard_normal((h, w, 3)).astype(np.float32)
+        out[seed] = [r.adjoint_grad(grad, spp, hess=0.25) for _ in range(4)]
+        r.close()
+
+    alone, together = {}, {}
+    for seed in range(6):
+        gradients(seed, alone)
+    threads = [threading.Thread(target=gradients, args=(seed, together)) for seed in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for seed in range(6):
+        for one, other in zip(alone[seed], together[seed]):
+            for a, b, c in zip(one, other, alone[seed][0]):
+                np.testing.assert_array_equal(a, b)
+                np.testing.assert_array_equal(a, c)
