@@ -153,11 +153,9 @@ struct LaunchKey {
 };
 
 struct WavefrontState {
-    int device = -1;
     uint32_t capacity = 0;       // slots
     size_t spill_ints = 0;
-    void* mem = nullptr;
-    size_t bytes = 0;
+    void* mem = nullptr;  // the queues
     int* spill = nullptr;
     uint32_t* ctr = nullptr;
     WfArgs args{};
@@ -966,47 +964,48 @@ int persistent_blocks(const void* kernel, uint32_t blocks_per_cu, int device, in
     return int(std::max<uint32_t>(1, per * uint32_t(*compute_units)));
 }
 
-// Queues of `capacity` slots and a spill area of `spill_ints`.
-int ensure_state(WavefrontState& w, int device, uint32_t capacity, size_t spill_ints, hipStream_t stream) {
-    if (w.mem && w.capacity >= capacity && w.spill_ints >= spill_ints && w.device == device) return PRT_OK;
-    if (w.mem) (void)hipFree(w.mem);
-    if (w.spill) (void)hipFree(w.spill);
-    if (w.ctr) (void)hipFree(w.ctr);
-    w.mem = nullptr;
-    w.bytes = 0;
-    w.capacity = 0;  // until everything is there
-    w.spill = nullptr;
-    w.ctr = nullptr;
-    const size_t bytes = kSlotBytes * size_t(capacity);
-    WF_TRY(device_alloc(&w.mem, bytes));
-    w.bytes = bytes;
-    WF_TRY(device_alloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
-    WF_TRY(fill_wait(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
-    if (spill_ints) WF_TRY(device_alloc(reinterpret_cast<void**>(&w.spill), spill_ints * sizeof(int)));
-    char* p = static_cast<char*>(w.mem);
-    auto take = [&](size_t bytes) {
-        void* r = p;
-        p += bytes;
-        return r;
-    };
-    const size_t C = capacity;
+// Queues of at least `capacity` slots and a spill area of at least `spill_ints`. Each grows by
+// itself: calls of few paths over a deep scene and of many over a shallow one leave each other's.
+int ensure_state(WavefrontState& w, uint32_t capacity, size_t spill_ints, hipStream_t stream) {
     WfArgs& a = w.args;
-    for (int k = 0; k < 2; ++k) {
-        a.qa[k] = static_cast<float4*>(take(16 * C));
-        a.qb[k] = static_cast<float4*>(take(16 * C));
-        a.qc[k] = static_cast<float4*>(take(16 * C));
+    if (!w.ctr) {
+        WF_TRY(device_alloc(reinterpret_cast<void**>(&w.ctr), kNumCounters * sizeof(uint32_t)));
+        a.ctr = w.ctr;
+        WF_TRY(fill_wait(w.ctr, 0, kNumCounters * sizeof(uint32_t), stream));
     }
-    a.se = static_cast<float4*>(take(16 * C));
-    a.sf = static_cast<float4*>(take(16 * C));
-    a.sg = static_cast<float4*>(take(16 * C));
-    a.result = static_cast<float4*>(take(16 * C));
-    a.hits = static_cast<uint32_t*>(take(4 * C));
-    a.sj = static_cast<uint32_t*>(take(4 * C));
-    a.ctr = w.ctr;
-    a.spill = w.spill;
-    w.capacity = capacity;
-    w.spill_ints = spill_ints;
-    w.device = device;
+    if (w.spill_ints < spill_ints) {
+        if (w.spill) (void)hipFree(w.spill);
+        a.spill = w.spill = nullptr;
+        w.spill_ints = 0;
+        WF_TRY(device_alloc(reinterpret_cast<void**>(&w.spill), spill_ints * sizeof(int)));
+        a.spill = w.spill;
+        w.spill_ints = spill_ints;
+    }
+    if (w.capacity < capacity) {
+        if (w.mem) (void)hipFree(w.mem);
+        w.mem = nullptr;
+        w.capacity = 0;
+        const size_t C = capacity;
+        WF_TRY(device_alloc(&w.mem, kSlotBytes * C));
+        w.capacity = capacity;
+        char* p = static_cast<char*>(w.mem);
+        auto take = [&](size_t bytes) {
+            void* r = p;
+            p += bytes;
+            return r;
+        };
+        for (int k = 0; k < 2; ++k) {
+            a.qa[k] = static_cast<float4*>(take(16 * C));
+            a.qb[k] = static_cast<float4*>(take(16 * C));
+            a.qc[k] = static_cast<float4*>(take(16 * C));
+        }
+        a.se = static_cast<float4*>(take(16 * C));
+        a.sf = static_cast<float4*>(take(16 * C));
+        a.sg = static_cast<float4*>(take(16 * C));
+        a.result = static_cast<float4*>(take(16 * C));
+        a.hits = static_cast<uint32_t*>(take(4 * C));
+        a.sj = static_cast<uint32_t*>(take(4 * C));
+    }
     return PRT_OK;
 }
 
@@ -1178,7 +1177,7 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, uint32_t en
     const int resident = persistent_blocks(ktrace, blocks_per_cu, device, &cus);
     const int pblocks = int(trace_waves(uint32_t(resident), (need + kBatch - 1) / kBatch));
     const size_t rows = entries > uint32_t(kStackLdsQueue) ? entries - kStackLdsQueue : 0;
-    int rc = ensure_state(w, device, need, rows * size_t(pblocks) * kBlock, stream);
+    int rc = ensure_state(w, need, rows * size_t(pblocks) * kBlock, stream);
     if (rc != PRT_OK) return rc;
     // The plan in one upload. (Every part is a multiple of 16 bytes.)
     const size_t at_tiles = jobs.size() * sizeof(WfJob), at_chunks = at_tiles + tiles.size() * sizeof(WfTile);
@@ -1267,7 +1266,7 @@ int run_wavefront(WavefrontState& w, int device, hipStream_t stream, uint32_t en
 uint64_t max_slots(const WavefrontState& w) {
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = size_t(8) << 30;
-    return std::max<uint64_t>(1u << 20, std::min<uint64_t>(1ull << 28, (free_b + w.bytes) / 4 / kSlotBytes));
+    return std::max<uint64_t>(1u << 20, std::min<uint64_t>(1ull << 28, (free_b + kSlotBytes * w.capacity) / 4 / kSlotBytes));
 }
 
 uint32_t default_capacity(const WavefrontState& w, uint64_t total_paths) {
@@ -1285,7 +1284,9 @@ struct CallSpace {
     void* rgb = nullptr;
     size_t rgb_bytes = 0;
     hipStream_t stream = nullptr;
-    size_t bytes() const { return w.bytes + accum_bytes + rgb_bytes; }
+    size_t bytes() const {
+        return kSlotBytes * w.capacity + w.spill_ints * sizeof(int) + w.cap_plan + accum_bytes + rgb_bytes;
+    }
 };
 
 void free_space(CallSpace* c) {

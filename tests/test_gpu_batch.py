@@ -71,3 +71,29 @@ def test_full_batch_equals_per_view_megakernel(gpu):
         ref = r.radiance()
         r.close()
         assert np.array_equal(imgs[i].view(np.uint32), ref.view(np.uint32)), f"view {i}"
+
+
+# Calls of few paths over a deep scene (a larger stack area) and of many over a shallow one
+# (larger queues) in turn: the images are the megakernel's, and neither call frees what the
+# other will need again.
+def test_calls_of_other_shapes_leave_each_others_memory(gpu):
+    from tests.helpers import OwnedDesc, device_free_bytes, nested_quads
+    p, n, m, mats = nested_quads()
+    deep_cam = ca.camera_look_at((0, 0, 2), (0, 0, 0), (0, 1, 0), 40, 240, 160)
+    od = OwnedDesc(p, n, m, mats, deep_cam)
+    deep, shallow = ca.Scene(od.desc), ca.Scene(W.cornell().mesh)
+    cam = ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, 400, 300)
+    calls = [(deep, deep_cam, 240, 160, 4), (shallow, cam, 400, 300, 64)]
+    want = []
+    for scene, c, w, h, spp in calls:
+        r = ca.ParallelRenderer(scene, w, h, spp, camera=c, max_depth=3, seed=4, view_id=1)
+        r.render(spp)
+        want.append(r.radiance())
+        r.close()
+    left = []
+    for k in (1, 0, 1, 0, 1, 0):
+        scene, c, w, h, spp = calls[k]
+        images, _ = ca.render_batch([ca.BatchJob(scene, c, spp, 1)], max_depth=3, seed=4)
+        assert np.array_equal(images[0], want[k])
+        left.append(device_free_bytes())
+    assert len(set(left[2:])) == 1, left
