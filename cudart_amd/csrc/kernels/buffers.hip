@@ -1,7 +1,8 @@
 // Memory that calls share or leave for the next one, and copies to the caller's buffers.
 //
 // Idle memory is bounded (two staging blocks, and per device one set of queues of at most a
-// sixteenth of its memory and as much in blocks of scratch memory), is taken by one call at a
+// sixteenth of its memory and a quarter of what is free beside it, and as much in blocks of
+// scratch memory), is taken by one call at a
 // time, and is given back when no scene is on a device any more or when an allocation of the
 // library finds no room.
 #include <hip/hip_runtime.h>
@@ -131,7 +132,7 @@ Scratch take_scratch(int device, size_t bytes) {
 void give_scratch(Scratch& s) {
     if (!s.mem) return;
     size_t free_b = 0, total_b = 0;
-    if (s.bytes > kSmallScratch && hipMemGetInfo(&free_b, &total_b) != hipSuccess) total_b = 0;
+    if (s.bytes > kSmallScratch && hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = total_b = 0;
     {
         std::lock_guard<std::mutex> g(g_mutex);
         Scratch* slot = nullptr;
@@ -140,7 +141,7 @@ void give_scratch(Scratch& s) {
             if (!o.mem) slot = &o;
             else if (o.device == s.device) idle += o.bytes;
         }
-        if (slot && g_scenes.load() > 0 && (s.bytes <= kSmallScratch || idle <= total_b / 16)) {
+        if (slot && g_scenes.load() > 0 && (s.bytes <= kSmallScratch || may_stay_idle(idle, free_b, total_b))) {
             *slot = s;
             s = Scratch();
             return;

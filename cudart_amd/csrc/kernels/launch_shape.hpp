@@ -84,6 +84,13 @@ constexpr uint32_t trace_waves(uint32_t resident, uint32_t batches) {
     return batches < waves ? batches : waves;
 }
 
+// Whether `bytes` of idle memory of a device may stay for the next call: at most a sixteenth of the
+// device's, and at most a quarter of what is free beside it. Other allocators of the process
+// cannot take it back, so where they have left little, none is kept.
+constexpr bool may_stay_idle(uint64_t bytes, uint64_t free_bytes, uint64_t device_bytes) {
+    return bytes <= device_bytes / 16 && bytes <= free_bytes / 4;
+}
+
 // Makes an area of `have` units one of at least `need`. The old one goes only when the new one is
 // there: a failure leaves it, and the launches that it was large enough for, as they were.
 template <class T, class Make, class Release>

@@ -1306,8 +1306,8 @@ constexpr int kSpaceDevices = 64;
 CallSpace* g_idle_space[kSpaceDevices] = {};  // one per device (none kept beyond these)
 
 // Takes the device's idle space or makes a new one; the destructor gives it back, or frees
-// it when it holds more than a sixteenth of the device's memory, another one is there, or
-// the call has failed. (Allocating and freeing the queues on every call: 12 views, 42M paths,
+// it when it holds too much to stay (may_stay_idle), another one is there, or the call has
+// failed. (Allocating and freeing the queues on every call: 12 views, 42M paths,
 // 7 GB took 278 ms a call, of which 10 ms were kernels; once a process has used as much
 // memory as the device has, the driver clears every page that it hands out again.)
 class CallSpaceLease {
@@ -1328,7 +1328,8 @@ public:
     ~CallSpaceLease() {
         if (!c_) return;
         size_t free_b = 0, total_b = 0;
-        if (ok_ && scenes_on_devices() && hipMemGetInfo(&free_b, &total_b) == hipSuccess && c_->bytes() <= total_b / 16) {
+        if (ok_ && scenes_on_devices() && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+            may_stay_idle(c_->bytes(), free_b, total_b)) {
             std::lock_guard<std::mutex> g(g_space_mutex);
             if (c_->device < kSpaceDevices && !g_idle_space[c_->device]) {
                 g_idle_space[c_->device] = c_;

@@ -296,8 +296,9 @@ typedef struct prt_tune {
 /* Renders every job in one persistent wavefront launch sequence (a captured HIP
  * graph replayed until all work drains). Per-job images equal the megakernel's for
  * the same seed/view_id/depth. stats may be NULL. The call's device memory stays for the
- * next one when it is at most a sixteenth of the device's (one set per device; freed when
- * the last scene on the devices is destroyed, or when an allocation finds no room). */
+ * next one when it is at most a sixteenth of the device's and a quarter of what is free
+ * beside it (one set per device; freed when the last scene on the devices is destroyed, or
+ * when an allocation of the library finds no room). */
 int prt_render_batch(prt_job *jobs, uint32_t num_jobs, const prt_render_config *cfg,
                      const prt_tune *tune, prt_stats *stats);
 

@@ -105,7 +105,15 @@ static void every_batch_is_handed_out() {
     CHECK(handed_out(50, 20) < 50, "%u", handed_out(50, 20));
 }
 
+static void idle_memory_is_bounded() {
+    const uint64_t GB = 1ull << 30, device = 288 * GB;
+    CHECK(may_stay_idle(7 * GB, 270 * GB, device) && may_stay_idle(18 * GB, 72 * GB, device), "%d", 0);
+    CHECK(!may_stay_idle(19 * GB, 270 * GB, device), "%d", 0);
+    CHECK(!may_stay_idle(7 * GB, 27 * GB, device) && !may_stay_idle(1, 0, device) && !may_stay_idle(1, 0, 0), "%d", 0);
+}
+
 int main() {
+    idle_memory_is_bounded();
     every_batch_is_handed_out();
     spill_fits_every_launch();
     failed_growth_leaves_the_area();

@@ -1,8 +1,8 @@
 """Rules of cudart_amd/csrc/kernels/launch_shape.hpp, compiled for the CPU
 (tests/host_launch_shape.cpp): the spill columns asked for are enough for every thread of every
 launch of a call, whatever the image, the sample count and the launch size, an allocation
-that fails leaves the area that was there, and a launch of any number of resident waves hands
-out every batch of its queue."""
+that fails leaves the area that was there, a launch of any number of resident waves hands out
+every batch of its queue, and idle memory is bounded by the device's and by what is free."""
 import subprocess
 from pathlib import Path
 
