@@ -417,6 +417,7 @@ extern "C" int prt_adjoint_grad(prt_renderer* r, const float* grad_rgb, float he
     if (!r || !grad_rgb || !d_albedo || !d_emission || spp == 0 || !(hess >= 0.f))
         return fail(PRT_ERR_INVALID_ARG, "bad argument");
     if (r->cfg.max_depth > 16) return fail(PRT_ERR_LIMIT, "the adjoint supports max_depth <= 16");
+    const VertexUse use(r);
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     rc = device_scene(r->scene, r->cfg.device, r->sc, r->stream);
@@ -506,6 +507,7 @@ extern "C" int prt_adjoint_grad_static(prt_renderer* r, const float* grad_rgb_de
     if (!r || !grad_rgb_device || !d_albedo || !d_emission || spp == 0 || !(hess >= 0.f))
         return fail(PRT_ERR_INVALID_ARG, "bad argument");
     if (r->cfg.max_depth > 16) return fail(PRT_ERR_LIMIT, "the adjoint supports max_depth <= 16");
+    const VertexUse use(r);
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     {

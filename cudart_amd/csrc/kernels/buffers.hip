@@ -2,9 +2,8 @@
 //
 // Idle memory is bounded (two staging blocks, and per device one set of queues of at most a
 // sixteenth of its memory and a quarter of what is free beside it, and as much in blocks of
-// scratch memory), is taken by one call at a
-// time, and is given back when no scene is on a device any more or when an allocation of the
-// library finds no room.
+// scratch memory), is taken by one call at a time, and is given back when no scene is on a
+// device any more or when an allocation of the library finds no room.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,6 +42,7 @@ constexpr size_t kSmallScratch = size_t(64) << 20;  // kept without asking for t
 std::mutex g_mutex;
 Stage g_idle[kMaxIdleStages];  // device < 0: none
 Scratch g_idle_scratch[kMaxIdleScratch];  // mem == nullptr: none
+prt_renderer* g_keepers = nullptr;        // renderers that keep vertices
 std::atomic<int> g_scenes{0};
 
 void free_stage(Stage& s) {
@@ -98,7 +98,39 @@ void release_idle() {
     release_idle_queues();
 }
 
+// The vertices of `device`'s renderers that no call is using.
+void release_vertices(int device) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    for (prt_renderer* r = g_keepers; r; r = r->next_keeper) {
+        if (!r->vertices || r->vertex_users != 0 || r->cfg.device != device) continue;
+        (void)hipFree(r->vertices);
+        r->vertices = nullptr;
+    }
+}
+
 }  // namespace
+
+void offer_vertices(prt_renderer* r) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    r->next_keeper = g_keepers;
+    g_keepers = r;
+}
+void withdraw_vertices(prt_renderer* r) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    for (prt_renderer** p = &g_keepers; *p; p = &(*p)->next_keeper)
+        if (*p == r) {
+            *p = r->next_keeper;
+            return;
+        }
+}
+VertexUse::VertexUse(prt_renderer* r) : r_(r) {
+    std::lock_guard<std::mutex> g(g_mutex);
+    ++r->vertex_users;
+}
+VertexUse::~VertexUse() {
+    std::lock_guard<std::mutex> g(g_mutex);
+    --r_->vertex_users;
+}
 
 void scene_uploaded() { ++g_scenes; }
 void scene_released() {
@@ -111,6 +143,13 @@ hipError_t device_alloc(void** p, size_t bytes) {
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
         release_idle();
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int device = -1;
+        (void)hipGetDevice(&device);
+        release_vertices(device);
         e = hipMalloc(p, bytes);
     }
     return e;

@@ -229,7 +229,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     HIP_TRY(hipMemsetAsync(r->accum, 0, px * sizeof(float4), r->stream));  // F9: the reference never clears it
     const size_t ticket_bytes = size_t(kTicketSets) * kTicketWords * sizeof(uint32_t);
     const size_t counter_bytes = (kCntNum * sizeof(unsigned long long) + 255) / 256 * 256;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->counters), counter_bytes + ticket_bytes));
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->counters), counter_bytes + ticket_bytes));
     HIP_TRY(hipMemsetAsync(r->counters, 0, counter_bytes + ticket_bytes, r->stream));
     r->tickets = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(r->counters) + counter_bytes);
     int cus = 0;
@@ -237,7 +237,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     r->compute_units = uint32_t(cus);
     uint8_t lut[256];
     gamma_table(lut);
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&r->gamma_lut), 256));
+    HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->gamma_lut), 256));
     HIP_TRY(copy_wait(r->gamma_lut, lut, 256, hipMemcpyHostToDevice, r->stream));
     if (c.keep_samples && spp > 0)
         HIP_TRY(device_alloc(reinterpret_cast<void**>(&r->samples), px * spp * sizeof(float4)));
@@ -250,6 +250,7 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
             r->vertices = nullptr;
             (void)hipGetLastError();
         }
+        if (r->vertices) offer_vertices(r.get());
     }
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
@@ -314,6 +315,7 @@ extern "C" int prt_render_spp(prt_renderer* r, uint32_t n) {
     clear_error();
     if (!r) return fail(PRT_ERR_INVALID_ARG, "null argument");
     if (n == 0) return PRT_OK;
+    const VertexUse use(r);
     int rc = set_device(r->cfg.device);
     if (rc != PRT_OK) return rc;
     rc = device_scene(r->scene, r->cfg.device, r->sc, r->stream);
@@ -479,6 +481,7 @@ extern "C" int prt_reset_stats(prt_renderer* r) {
 extern "C" int prt_renderer_destroy(prt_renderer* r) {
     if (!r) return PRT_OK;
     (void)hipSetDevice(r->cfg.device);
+    withdraw_vertices(r);
     release_wavefront(r);
     if (r->stream) (void)hipStreamSynchronize(r->stream);
     void* ptrs[] = {r->accum, r->counters, r->gamma_lut, r->spill, r->samples, r->vertices, r->out};

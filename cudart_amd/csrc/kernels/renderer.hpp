@@ -41,6 +41,8 @@ struct prt_renderer {
     // the scene's current materials (samples_version).
     float4* samples = nullptr;
     uint32_t* vertices = nullptr;
+    uint32_t vertex_users = 0;              // VertexUse
+    prt_renderer* next_keeper = nullptr;    // of the renderers that keep vertices
     bool samples_ok = false;
     // Device memory of the calls that hand results out, kept until the renderer goes: at most
     // 12 bytes per pixel (scratch_for).
@@ -64,8 +66,24 @@ inline hipError_t fill_wait(void* dst, int value, size_t bytes, hipStream_t s) {
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
 // buffers.hip.
-// hipMalloc, after idle memory has been given back if there is no room.
+// hipMalloc; if there is no room, after idle memory has been given back, and then the vertices kept
+// by renderers that no call is using.
 hipError_t device_alloc(void** p, size_t bytes);
+// Kept vertices save an adjoint its forward pass, and it can do without: a renderer that has them
+// offers them (until it withdraws), and a call that reads or writes r->vertices holds a VertexUse
+// meanwhile. Every such call waits for its launches.
+void offer_vertices(prt_renderer* r);
+void withdraw_vertices(prt_renderer* r);
+class VertexUse {
+public:
+    explicit VertexUse(prt_renderer* r);
+    ~VertexUse();
+    VertexUse(const VertexUse&) = delete;
+    VertexUse& operator=(const VertexUse&) = delete;
+
+private:
+    prt_renderer* r_;
+};
 // Device memory to the caller's host buffers, ordered on `stream` and waited for.
 struct CopyOut {
     void* dst;

@@ -129,7 +129,8 @@ typedef struct prt_render_config {
                                the first `spp` samples), so the adjoint replays paths without
                                tracing them first, and each path's vertices (4 B per sample and
                                max_depth, when that fits in a quarter of the free device
-                               memory), so the replay traces no ray */
+                               memory; given up when an allocation of the library finds no
+                               room), so the replay traces no ray */
 } prt_render_config;
 
 /* Counters accumulated since the renderer was created (or reset). */

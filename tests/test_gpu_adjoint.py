@@ -380,3 +380,51 @@ def test_gradients_of_several_renderers_share_their_memory(gpu):
     for r in renderers:
         r.close()
     scene.close()
+
+
+# Run by itself below: the driver clears the pages of a process that has used most of the memory.
+_FULL_DEVICE = """
+import ctypes as C
+import numpy as np
+import cudart_amd as ca
+from cudart_amd import workloads as W
+from tests.helpers import device_free_bytes
+
+w = h = 512
+scene = ca.Scene(W.cornell100k(w, h).mesh)
+cam = W.cornell100k(w, h).camera
+kw = dict(camera=cam, max_depth=16, keep_samples=1, integrator=ca.INTEGRATOR_WAVEFRONT)
+grad = np.random.default_rng(9).standard_normal((h, w, 3)).astype(np.float32)
+before = device_free_bytes()
+first = ca.ParallelRenderer(scene, w, h, 128, seed=1, **kw)
+kept = 128 * w * h * (16 + 4 * 16)
+assert before - device_free_bytes() >= kept, (before, device_free_bytes())
+first.render(8)
+want = first.adjoint_grad(grad, 8, hess=0.25)
+hip = C.CDLL(next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64.so" in l))
+filler = C.c_void_p()
+left = device_free_bytes()
+samples = 192 * w * h * 16  # of the second renderer: more than is left free, less than with the vertices
+assert hip.hipMalloc(C.byref(filler), C.c_size_t(left - samples // 2)) == 0
+print("filled", flush=True)
+second = ca.ParallelRenderer(scene, w, h, 192, seed=1, **kw)
+hip.hipFree(filler)
+for r in (first, second):
+    r.reset()
+    r.render(8)
+    for a, b in zip(r.adjoint_grad(grad, 8, hess=0.25), want):
+        assert np.array_equal(a, b)
+    r.close()
+print("ok")
+"""
+
+
+def test_kept_vertices_give_way_to_a_renderer_that_needs_the_room(gpu):
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    root = Path(__file__).resolve().parent.parent
+    out = subprocess.run([sys.executable, "-u", "-c", _FULL_DEVICE], cwd=root, capture_output=True, text=True,
+                         timeout=100, env={**os.environ, "PYTHONPATH": str(root)})
+    assert out.returncode == 0 and out.stdout.split()[-1] == "ok", out.stdout + out.stderr
