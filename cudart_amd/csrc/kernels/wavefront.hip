@@ -1605,7 +1605,7 @@ extern "C" int prt_autotune(prt_job* jobs, uint32_t n, const prt_render_config* 
             bt = t;
         }
     };
-    // Coordinate search from the defaults (fewest chunks, smallest dividing group):
+    // Coordinate search from the defaults (fewest chunks, groups chosen per section):
     // occupancy, then the camera-path grouping, then the chunk count.
     bt = prt_tune{full_cap, 0, kBlock, 0};
     consider(bt);

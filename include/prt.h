@@ -119,7 +119,8 @@ typedef struct prt_render_config {
     uint32_t count_rays;    /* 1 = keep per-kind ray / node / triangle counters */
     uint32_t wavefront_group;   /* wavefront: side g (1, 2, 4 or 8) of the pixel block whose
                                    64 / g^2 consecutive samples make one wave's 64 camera paths
-                                   (0 = the smallest g that divides the tile) */
+                                   (0 = chosen from the sample count: sections of 64 samples
+                                   are a pixel each, the rest blocks of pixels) */
     uint32_t wavefront_queue;   /* wavefront: path slots in flight (0 = choose) */
     uint32_t profile_kernels;   /* wavefront: 1 = launch each chunk's kernels without a graph and
                                    time every extend / shade / shadow launch with events */
