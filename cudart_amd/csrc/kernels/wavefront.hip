@@ -1433,6 +1433,9 @@ void release_wavefront(prt_renderer* r) {
 
 namespace {
 
+// Device memory for a batch's images (CallSpace::rgb) at most.
+constexpr size_t kImageBytes = size_t(256) << 20;
+
 struct BatchCtx {
     std::vector<WfJob> jobs;
     std::vector<PlanJob> pjobs;
@@ -1508,16 +1511,27 @@ extern "C" int prt_render_batch(prt_job* jobs, uint32_t n, const prt_render_conf
     RunStats rs;
     rc = run_wavefront(space->w, c.device, s, b.entries, b.jobs, b.pjobs, c.max_depth, cap, tune ? tune->blocks_per_cu : 0,
                        tune ? tune->group_side : c.wavefront_group, c.count_rays != 0, &rs);
-    // Every image's mean, then all copies in one run.
-    if (rc == PRT_OK) rc = scratch_for(space->rgb, space->rgb_bytes, b.pixels * 3 * sizeof(float));
+    // The images' means, then their copies in one run, as many as fit kImageBytes (an image always
+    // does) at a time: the accumulators of a large batch leave little room.
+    static_assert((size_t(1) << 24) * 3 * sizeof(float) <= kImageBytes, "the largest view's image");
+    size_t images = 0, at = 0;
+    for (uint32_t i = 0; i < n; ++i)
+        if (jobs[i].out_rgb) images += size_t(b.jobs[i].width) * b.jobs[i].height * 3 * sizeof(float);
+    if (rc == PRT_OK && images) rc = scratch_for(space->rgb, space->rgb_bytes, std::min(images, kImageBytes));
     std::vector<CopyOut> out;
     hipError_t e = hipSuccess;
     for (uint32_t i = 0; i < n && rc == PRT_OK && e == hipSuccess; ++i) {
         if (!jobs[i].out_rgb) continue;
-        const size_t px = size_t(b.jobs[i].width) * b.jobs[i].height;
-        float* rgb = static_cast<float*>(space->rgb) + b.pixel0[i] * 3;
-        e = launch_mean(b.jobs[i].accum, uint32_t(px), jobs[i].spp, rgb, s);
-        out.push_back(CopyOut{jobs[i].out_rgb, rgb, px * 3 * sizeof(float)});
+        const size_t px = size_t(b.jobs[i].width) * b.jobs[i].height, bytes = px * 3 * sizeof(float);
+        if (at + bytes > space->rgb_bytes) {
+            e = copy_out(out.data(), out.size(), c.device, s);
+            out.clear();
+            at = 0;
+        }
+        float* rgb = reinterpret_cast<float*>(static_cast<char*>(space->rgb) + at);
+        if (e == hipSuccess) e = launch_mean(b.jobs[i].accum, uint32_t(px), jobs[i].spp, rgb, s);
+        out.push_back(CopyOut{jobs[i].out_rgb, rgb, bytes});
+        at += bytes;
     }
     if (rc == PRT_OK && e == hipSuccess) e = copy_out(out.data(), out.size(), c.device, s);
     if (e != hipSuccess) rc = hip_fail(e, "batch readback");

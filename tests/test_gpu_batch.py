@@ -97,3 +97,23 @@ def test_calls_of_other_shapes_leave_each_others_memory(gpu):
         assert np.array_equal(images[0], want[k])
         left.append(device_free_bytes())
     assert len(set(left[2:])) == 1, left
+
+
+# Images of more than the block that they are copied from: they go in parts, and the block does
+# not grow with the batch.
+def test_images_of_a_large_batch(gpu):
+    from tests.helpers import device_free_bytes
+    scene = ca.Scene(W.cornell().mesh)
+    sides = [4096, 700, 4096, 33]
+    cams = [ca.camera_look_at((2.2, 0.548, 0.1), (0.0, 0.548, 0.0), (0.0, 1.0, 0.0), 39.3, s, s) for s in sides]
+    warm, _ = ca.render_batch([ca.BatchJob(scene, cams[-1], 1, 9)], max_depth=1, seed=4)
+    before = device_free_bytes()
+    images, _ = ca.render_batch([ca.BatchJob(scene, c, 1, v) for v, c in enumerate(cams)], max_depth=1, seed=4)
+    pixels = sum(s * s for s in sides)
+    held = before - device_free_bytes()
+    assert held < pixels * (168 + 16) + (300 << 20), held  # path slots, accumulators and the images' block
+    for v, (side, cam) in enumerate(zip(sides, cams)):
+        r = ca.ParallelRenderer(scene, side, side, 1, camera=cam, max_depth=1, seed=4, view_id=v)
+        r.render(1)
+        assert np.array_equal(images[v], r.radiance())
+        r.close()
