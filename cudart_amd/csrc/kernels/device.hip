@@ -255,10 +255,12 @@ extern "C" int prt_renderer_create(prt_scene* scene, const prt_camera* cam, uint
     r->tiles_x = (w + 7) / 8;
     r->tiles = r->tiles_x * ((h + 7) / 8);
     // What the renderer was made for needs no allocation later. (A wavefront renderer's queues
-    // have a spill area of their own; this one is made if first hits are asked for.)
-    if (c.integrator == PRT_INTEGRATOR_MEGAKERNEL)
-        rc = ensure_spill(r.get(), std::max(first_hit_columns(w, h), mega_columns(w, h, std::max(1u, spp), c.spp_per_launch,
-                                                                                  mega_resident(r.get()))));
+    // have a spill area of their own; this one is made if first hits are asked for. An image of
+    // more blocks than one launch can have threads for may still be rendered by launches whose
+    // lanes share pixels.)
+    const uint64_t columns = std::max(first_hit_columns(w, h),
+                                      mega_columns(w, h, std::max(1u, spp), c.spp_per_launch, mega_resident(r.get())));
+    if (c.integrator == PRT_INTEGRATOR_MEGAKERNEL && columns <= UINT32_MAX) rc = ensure_spill(r.get(), columns);
     if (rc != PRT_OK) return rc;
     HIP_TRY(hipStreamSynchronize(r->stream));
     *out = r.release();
